@@ -247,3 +247,36 @@ def tolerance(case):
     if case["algo"] == "trunk":
         return {"rel": 2e-5, "max": 2e-4}
     return {"rel": 3.5e-5, "max": 7e-4}
+
+
+def _conv64(x, w, bias, relu, stride, pad):
+    """The convolution as one product per window tap, summed in 64 bits."""
+    x = torch.nn.functional.pad(x, (pad, pad, pad, pad))
+    ks = w.shape[2]
+    oh, ow = (x.shape[2] - ks) // stride + 1, (x.shape[3] - ks) // stride + 1
+    y = torch.zeros((x.shape[0], w.shape[0], oh * ow), dtype=torch.float64, device=x.device)
+    for image in range(x.shape[0]):
+        for r in range(ks):
+            for s in range(ks):
+                tap = x[image, :, r:r + (oh - 1) * stride + 1:stride, s:s + (ow - 1) * stride + 1:stride]
+                y[image].addmm_(w[:, :, r, s].contiguous(), tap.reshape(tap.shape[0], oh * ow))
+    if bias is not None:
+        y += bias[:, None]
+    return (y.clamp_(min=0) if relu else y).view(x.shape[0], w.shape[0], oh, ow)
+
+
+def exact(case, seed):
+    """The outputs of run() in 64 bits, from the same draws of the generator as prepare()."""
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    if case["algo"] != "trunk":
+        x = _inputs(gen, case["n"], case["c"], case["h"], case["w"]).double()
+        w = _weights(gen, case["k"], case["c"], case["ks"]).double()
+        bias = _bias(gen, case["k"]).double() if case["bias_relu"] else None
+        return _conv64(x, w, bias, case["bias_relu"], case["stride"], case["pad"])
+    x = _inputs(gen, case["n"], 3, case["h"], case["h"]).double()
+    for block in TRUNK:
+        for c, k in block:
+            w, bias = _weights(gen, k, c, 3).double(), _bias(gen, k).double()
+            x = _conv64(x, w, bias, True, 1, 1)
+        x = torch.nn.functional.max_pool2d(x, 2)
+    return x
