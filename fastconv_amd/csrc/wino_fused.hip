@@ -11,6 +11,7 @@
 // global memory (L2) to registers: for reduction step (c, c+1) lane l of each
 // frequency loads U[f][c + l/32][k0 + l%32] and V[f][c + l/32][t0 + l%32], two
 // full 128-byte lines per load instruction.  Loads run three steps ahead.
+#include "split_mfma.h"
 #include "wino_fused_out.h"
 
 namespace {
@@ -31,17 +32,8 @@ __device__ __forceinline__ float ldg(const float *base, uint32_t byteOff) {
 constexpr int kDepth = 4;   // register slots of operand fragments (3 steps in flight + 1 in use)
 // (the offsets are 32-bit: the host checks that one frequency plane stays below 2^32 bytes)
 
-__global__ __launch_bounds__(kFusedThreads, 1) void wino_gemm_out_fused_kernel(const FusedParams p) {
-    extern __shared__ __attribute__((aligned(16))) float Ml[];   // [64 f][16 k][32 t]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lrow = lane >> 5, lcol = lane & 31;
-
-    // XCD-aware order: all output-channel blocks of one tile block run back to back on one XCD
-    const int b = blockIdx.x, xcd = b & 7, j = b >> 3;
-    const int tbl = j / p.nKB, kb = j - tbl * p.nKB;
-    const int tb = tbl * 8 + xcd;
-    if (tb >= p.nTB) return;
-
+// acc = the products of this wavefront's 8 frequencies, all channels.
+__device__ __forceinline__ void fused_products(const FusedParams &p, int wave, int lrow, int lcol, int kb, int tb, floatx16 (&acc)[kFW]) {
     // Per-frequency base pointers are wave-uniform (scalar registers); the lane's part of the
     // address is one 32-bit offset shared by all 16 frequencies.
     const int wv = __builtin_amdgcn_readfirstlane(wave);
@@ -52,7 +44,6 @@ __global__ __launch_bounds__(kFusedThreads, 1) void wino_gemm_out_fused_kernel(c
     uint32_t offU = 4u * ((uint32_t)lrow * p.K_pad + lcol), offV = 4u * ((uint32_t)lrow * (uint32_t)p.T_pad + lcol);
     const uint32_t stepU = 8u * p.K_pad, stepV = 8u * (uint32_t)p.T_pad;
 
-    floatx16 acc[kFW];
 #pragma unroll
     for (int f = 0; f < kFW; f++)
 #pragma unroll
@@ -99,7 +90,73 @@ __global__ __launch_bounds__(kFusedThreads, 1) void wino_gemm_out_fused_kernel(c
 #pragma unroll
         for (int f = 0; f < kFW; f++)
             acc[f] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][f], bv[u][f], acc[f], 0, 0, 0);
+}
 
+// The same on the bf16 matrix cores, in the order of the staged pipeline's GEMM (see split_mfma.h): 16 channels at a time,
+// a lane splits the 8 channels of its row and column.  The split is the larger part of the time: the operands of a
+// 32x32 block are split by every block that uses them.  C_pad is a multiple of 16.
+__device__ __forceinline__ void fused_split_products(const FusedParams &p, int wave, int lrow, int lcol, int kb, int tb, floatx16 (&acc)[kFW]) {
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    const size_t planeU = (size_t)p.C_pad * p.K_pad, planeV = (size_t)p.C_pad * p.T_pad;
+    const float *ub = p.U + (size_t)(wv * kFW) * planeU + (size_t)kb * 32;
+    const float *vb = p.V + (size_t)(wv * kFW) * planeV + (size_t)tb * 32;
+    uint32_t offU = 4u * (8u * lrow * p.K_pad + lcol), offV = 4u * (8u * lrow * (uint32_t)p.T_pad + lcol);
+    const uint32_t rowU = 4u * p.K_pad, rowV = 4u * (uint32_t)p.T_pad;
+#pragma unroll
+    for (int f = 0; f < kFW; f++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[f][i] = 0.f;
+    float u[2][8], v[2][8];
+    auto fetch = [&](int f, float (&a)[8], float (&b)[8]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            a[i] = ldg(ub + f * planeU, offU + i * rowU);
+            b[i] = ldg(vb + f * planeV, offV + i * rowV);
+        }
+    };
+    const int nStages = p.C_pad / 16;
+    fetch(0, u[0], v[0]);
+    for (int s = 0; s < nStages; s++) {
+#pragma unroll
+        for (int f = 0; f < kFW; f++) {
+            // the next frequency, or the first of the next 16 channels (the last ones again at the end)
+            if (f + 1 == kFW && s + 1 < nStages) {
+                offU += 16u * rowU;
+                offV += 16u * rowV;
+            }
+            fetch((f + 1) % kFW, u[(f + 1) & 1], v[(f + 1) & 1]);
+            fc_uintx4 a[3], b[3];
+            fc_split8(u[f & 1], a, 1);
+            fc_split8(v[f & 1], b, 1);
+            floatx16 one[1][1] = {{acc[f]}};
+            fc_split_products<1, 1, 1, 1>(a, b, one);
+            acc[f] = one[0][0];
+        }
+    }
+}
+
+template <bool SPLIT>
+__global__ __launch_bounds__(kFusedThreads, 1) void wino_gemm_out_fused_kernel(const FusedParams p) {
+    extern __shared__ __attribute__((aligned(16))) float Ml[];   // [64 f][16 k][32 t]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lrow = lane >> 5, lcol = lane & 31;
+
+    // XCD-aware order: all output-channel blocks of one tile block run back to back on one XCD
+    const int b = blockIdx.x, xcd = b & 7, j = b >> 3;
+    const int tbl = j / p.nKB, kb = j - tbl * p.nKB;
+    const int tb = tbl * 8 + xcd;
+    if (tb >= p.nTB) return;
+
+    floatx16 acc[kFW];
+    if constexpr (SPLIT) {
+        fused_split_products(p, wave, lrow, lcol, kb, tb, acc);
+        floatx16 all[1][kFW];
+#pragma unroll
+        for (int f = 0; f < kFW; f++) all[0][f] = acc[f];
+        if (__any(fc_not_finite<1, kFW>(all))) fused_products(p, wave, lrow, lcol, kb, tb, acc);
+    } else {
+        fused_products(p, wave, lrow, lcol, kb, tb, acc);
+    }
     fused_output_transform(p.out, acc, Ml, kb, tb);
 }
 
@@ -122,8 +179,8 @@ extern "C" int fc_wino_gemm_output_fused(fc_context *ctx, const fc_wino_plan *pl
     if (!ctx->fused_lds_granted) {
         if (ctx->capturing)
             return fc_set_error(ctx, FC_ERR_STATE, "fc_wino_gemm_output_fused: run this kernel once before recording a graph with it", hipSuccess);
-        FC_HIP_CHECK(ctx, hipFuncSetAttribute((const void *)wino_gemm_out_fused_kernel,
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFusedLdsBytes));
+        for (const void *kernel : {(const void *)wino_gemm_out_fused_kernel<false>, (const void *)wino_gemm_out_fused_kernel<true>})
+            FC_HIP_CHECK(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFusedLdsBytes));
         ctx->fused_lds_granted = true;
     }
     FusedParams p;
@@ -136,7 +193,10 @@ extern "C" int fc_wino_gemm_output_fused(fc_context *ctx, const fc_wino_plan *pl
     const long blocks = tbGroups * 8 * p.nKB;
     if (blocks >= (1l << 31)) return fc_set_error(ctx, FC_ERR_UNSUPPORTED, "fc_wino_gemm_output_fused: grid too large", hipSuccess);
     fc_stage_scope scope(ctx, FC_STAGE_FUSED_GEMM_OUT);
-    wino_gemm_out_fused_kernel<<<dim3((unsigned)blocks), dim3(kFusedThreads), kFusedLdsBytes, ctx->stream>>>(p);
+    if (fc_wino_gemm_splits(plan))
+        wino_gemm_out_fused_kernel<true><<<dim3((unsigned)blocks), dim3(kFusedThreads), kFusedLdsBytes, ctx->stream>>>(p);
+    else
+        wino_gemm_out_fused_kernel<false><<<dim3((unsigned)blocks), dim3(kFusedThreads), kFusedLdsBytes, ctx->stream>>>(p);
     FC_LAUNCH_CHECK(ctx, "wino_gemm_out_fused_kernel");
     return FC_OK;
 }

@@ -4,10 +4,12 @@
 // fastest, which is exactly the order v_mfma_f32_32x32x2_f32 wants its lanes in
 // (lane l holds row/col l%32 of reduction step l/32), so tiles go global -> LDS
 // as straight 16-byte copies and LDS -> registers as conflict-free dword reads.
+// Layers of more channels run on the bf16 matrix cores instead, at the same accuracy (split_tile below).
 #include <cmath>
 #include <utility>
 
 #include "fc_internal.h"
+#include "split_mfma.h"
 
 namespace {
 
@@ -60,6 +62,38 @@ struct GemmTile {
     static_assert(A_VEC % THREADS == 0 && B_VEC % THREADS == 0, "every thread copies the same number of float4");
     static_assert(A_LD >= 1 && B_LD >= 1, "tile smaller than one copy pass");
 };
+
+// PF = register sets of global prefetch.  Measured on MI355X: 2 or 4 sets change the rate of the
+// 64x64 tile by -2..+4 % depending on the layer and cost the larger tiles a resident workgroup
+// (their register count nearly doubles), so every configuration runs with one.
+template <int BM, int BN, int BK, int WGM, int WGN, int PF = 1>
+struct TileCfg : GemmTile<BM, BN, BK, WGM, WGN> {
+    static constexpr int BM_ = BM, BN_ = BN, BK_ = BK, WGM_ = WGM, WGN_ = WGN, PF_ = PF;
+};
+
+// The accumulators of a workgroup tile to M.
+template <class TL>
+__device__ __forceinline__ void store_tile(const floatx16 (&acc)[TL::MI][TL::NI], float *__restrict__ M, int K_pad, int T_pad, int f,
+                                           int kb, int tb, int wm0, int wn0, int lrow, int lcol) {
+    constexpr int BM = TL::BM_, BN = TL::BN_, MI = TL::MI, NI = TL::NI;
+    // D block layout: register i of lane l is row 8*(i/4) + 4*(l/32) + i%4, column l%32.
+    // The wavefront's block starts at a uniform address; the lane's share of it (4 * lrow rows down, lcol columns in) is one byte offset.
+    float *Mg = (M + ((size_t)f * K_pad + (size_t)kb * BM + wm0) * T_pad + (size_t)tb * BN + wn0);
+    const uint32_t mOff = 4u * (4u * (uint32_t)lrow * (uint32_t)T_pad + lcol);
+    const size_t rowBytes = (size_t)T_pad * 4;
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) {
+            // rows 0-3, 8-11, 16-19, 24-27 of the 32x32 block, stepped by addition in the scalar unit
+            char *pr = reinterpret_cast<char *>(uniform_ptr(Mg + (size_t)(mi * 32) * T_pad + ni * 32));
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                *reinterpret_cast<float *>(pr + mOff) = acc[mi][ni][i];
+                pr = uniform_ptr(pr + ((i % 4) == 3 ? 5 * rowBytes : rowBytes));
+            }
+        }
+}
 
 // One workgroup tile: M[f][kb*BM .. +BM][tb*BN .. +BN] = sum over all input channels.
 // `smem` holds the two LDS stages of both operands (2*BK*(BM+BN) floats).
@@ -204,23 +238,110 @@ __device__ __forceinline__ void gemm_tile(const float *__restrict__ U, const flo
     // the last nStages % PF stages
     stage_rest(stage, s0, nStages, std::make_integer_sequence<int, PF - 1>());
 
-    // D block layout: register i of lane l is row 8*(i/4) + 4*(l/32) + i%4, column l%32.
-    // The wavefront's block starts at a uniform address; the lane's share of it (4 * lrow rows down, lcol columns in) is one byte offset.
-    float *Mg = (M + ((size_t)f * K_pad + (size_t)kb * BM + wm0) * T_pad + (size_t)tb * BN + wn0);
-    const uint32_t mOff = 4u * (4u * (uint32_t)lrow * (uint32_t)T_pad + lcol);
-    const size_t rowBytes = (size_t)T_pad * 4;
+    store_tile<TL>(acc, M, K_pad, T_pad, f, kb, tb, wm0, wn0, lrow, lcol);
+}
+
+// The same tile on the bf16 matrix cores (see split_mfma.h): a wavefront takes 8 consecutive channels of 64 rows or
+// columns at a time, each lane one of them, splits the 8 floats it has fetched a stage ahead and writes one 16-byte
+// word per part.  Bound by the matrix cores and LDS (a 128x128 stage: 768 cycles of products, 48 KB read and 24 KB
+// written); the split runs beside the products of the other wavefronts, of which a SIMD needs three.  128x128 tiles,
+// batch 32, fp32 instructions -> this: 256 -> 256 channels at 56x56 218 -> 161 us (166 TFLOP/s), 512 -> 512 at 28x28
+// 223 -> 162, 128 -> 128 at 112x112 225 -> 181 (bound by memory, 4.2 TB/s); error against 64 bits 0.83 of the fp32 one's.
+// Spreading the split between the products by hand (sched_group_barrier) gained nothing.
+template <class TL>
+struct SplitTile {
+    static constexpr int ITEMS = 2 * (TL::BM_ + TL::BN_) / TL::THREADS;
+    typedef fc_split_stage<TL::BM_, TL::BN_> Stage;
+    static constexpr int LDS_WORDS = 2 * Stage::WORDS;
+    static_assert(TL::BM_ % 64 == 0 && TL::BN_ % 64 == 0, "a wavefront fetches 64 rows or columns of one operand");
+    static_assert(2 * (TL::BM_ + TL::BN_) % TL::THREADS == 0, "every wavefront fetches the same number of blocks");
+    static_assert(TL::BK_ == 16, "one product of depth 16 per stage");
+};
+
+template <class TL>
+__device__ __forceinline__ void split_tile(const float *__restrict__ U, const float *__restrict__ V,
+                                           float *__restrict__ M, int K_pad, int C_pad, int T_pad, int f, int kb,
+                                           int tb, fc_uintx4 *smem) {
+    typedef SplitTile<TL> S;
+    constexpr int BM = TL::BM_, BN = TL::BN_, MI = TL::MI, NI = TL::NI, ITEMS = S::ITEMS;
+    constexpr int A_PLANE = S::Stage::A_PLANE, B_PLANE = S::Stage::B_PLANE, WORDS = S::Stage::WORDS;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm0 = (wave / TL::WGN_) * TL::WM, wn0 = (wave % TL::WGN_) * TL::WN;
+    const int lrow = lane >> 5, lcol = lane & 31;
+    const int nStages = C_pad / 16;
+
+    // block j of this wavefront: 64 rows (columns) x 8 channels of A (B), from a uniform pointer
+    const float *src[ITEMS];
+    int dst[ITEMS], ld[ITEMS];
+    bool isA[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        int e = wave * 64 + j * TL::THREADS;
+        isA[j] = e < 2 * BM;
+        if (!isA[j]) e -= 2 * BM;
+        const int width = isA[j] ? BM : BN, g = e / width, c0 = e - g * width;
+        ld[j] = isA[j] ? K_pad : T_pad;
+        src[j] = uniform_ptr((isA[j] ? U + (size_t)f * C_pad * K_pad + (size_t)kb * BM
+                                     : V + (size_t)f * C_pad * T_pad + (size_t)tb * BN) + (size_t)(8 * g) * ld[j] + c0);
+        dst[j] = (isA[j] ? 0 : 3 * A_PLANE) + e;
+    }
+    float r[ITEMS][8];
+    uint32_t laneOff = 4u * lane;
+    // `more`: there is a stage to fetch (else the one before is fetched again, so that the loop has no branch)
+    auto fetch = [&](bool more) __attribute__((always_inline)) {
+        asm volatile("" : "+v"(laneOff));
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            src[j] = uniform_ptr(more ? src[j] + (size_t)16 * ld[j] : src[j]);
+            const float *b = src[j];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                r[j][i] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(b) + laneOff);
+                b = uniform_ptr(b + ld[j]);
+            }
+        }
+    };
+    auto park = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) fc_split8(r[j], smem + buf * WORDS + dst[j] + lane, isA[j] ? A_PLANE : B_PLANE);
+    };
+
+    floatx16 acc[MI][NI];
 #pragma unroll
     for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++) {
-            // rows 0-3, 8-11, 16-19, 24-27 of the 32x32 block, stepped by addition in the scalar unit
-            char *pr = reinterpret_cast<char *>(uniform_ptr(Mg + (size_t)(mi * 32) * T_pad + ni * 32));
+        for (int ni = 0; ni < NI; ni++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                *reinterpret_cast<float *>(pr + mOff) = acc[mi][ni][i];
-                pr = uniform_ptr(pr + ((i % 4) == 3 ? 5 * rowBytes : rowBytes));
-            }
-        }
+            for (int i = 0; i < 16; i++) acc[mi][ni][i] = 0.f;
+
+    fetch(false);
+    park(0);
+    fetch(nStages > 1);
+    __syncthreads();
+    const int aFrag = lrow * BM + wm0 + lcol, bFrag = 3 * A_PLANE + lrow * BN + wn0 + lcol;
+    int s = 0;
+    for (; s + 1 < nStages; s++) {
+        const fc_uintx4 *cur = smem + (s & 1) * WORDS;
+        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc);
+        park((s + 1) & 1);
+        fetch(s + 2 < nStages);
+        __syncthreads();
+    }
+    {
+        const fc_uintx4 *cur = smem + (s & 1) * WORDS;
+        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc);
+        __syncthreads();
+    }
+    if (__syncthreads_or(fc_not_finite<MI, NI>(acc))) {
+        // 64x64 at a time, which leaves the registers to the loop above
+        typedef TileCfg<64, 64, 16, 2, TL::THREADS / 128> Sub;
+        static_assert(Sub::THREADS == TL::THREADS && Sub::LDS_BYTES <= 16 * S::LDS_WORDS, "same workgroup");
+        for (int q = 0; q < (BM / 64) * (BN / 64); q++)
+            gemm_tile<Sub>(U, V, M, K_pad, C_pad, T_pad, f, kb * (BM / 64) + q / (BN / 64), tb * (BN / 64) + q % (BN / 64),
+                           reinterpret_cast<float *>(smem));
+        return;
+    }
+    store_tile<TL>(acc, M, K_pad, T_pad, f, kb, tb, wm0, wn0, lrow, lcol);
 }
 
 // Workgroups are dealt to the 8 XCDs round-robin by linear id.  All tiles of one
@@ -237,15 +358,19 @@ __device__ __forceinline__ void decode_tile(int b, int nKB, int nTB, int *f, int
     *kb = rem - *tb * nKB;
 }
 
-template <class TL>
-__global__ __launch_bounds__(TL::THREADS) void wino_gemm_kernel(const float *__restrict__ U,
-                                                                const float *__restrict__ V,
-                                                                float *__restrict__ M, int K_pad, int C_pad,
-                                                                int T_pad, int nKB, int nTB) {
-    __shared__ __attribute__((aligned(16))) float smem[2 * TL::BK_ * (TL::BM_ + TL::BN_)];
+// SPLIT: on the bf16 matrix cores; three wavefronts per SIMD (two cost 10-15 %) where the tile leaves the registers.
+template <class TL, bool SPLIT>
+__global__ __launch_bounds__(TL::THREADS, SPLIT && TL::BM_ * TL::BN_ <= 128 * 128 ? 3 : 1) void wino_gemm_kernel(
+    const float *__restrict__ U, const float *__restrict__ V, float *__restrict__ M, int K_pad, int C_pad, int T_pad, int nKB, int nTB) {
     int f, kb, tb;
     decode_tile(blockIdx.x, nKB, nTB, &f, &kb, &tb);
-    gemm_tile<TL>(U, V, M, K_pad, C_pad, T_pad, f, kb, tb, smem);
+    if constexpr (SPLIT) {
+        __shared__ fc_uintx4 words[SplitTile<TL>::LDS_WORDS];
+        split_tile<TL>(U, V, M, K_pad, C_pad, T_pad, f, kb, tb, words);
+    } else {
+        __shared__ __attribute__((aligned(16))) float smem[2 * TL::BK_ * (TL::BM_ + TL::BN_)];
+        gemm_tile<TL>(U, V, M, K_pad, C_pad, T_pad, f, kb, tb, smem);
+    }
 }
 
 // Same product, with the last `nTiles - nBig` tiles of the grid cut into quarters, so
@@ -272,14 +397,6 @@ __global__ __launch_bounds__(BIG::THREADS) void wino_gemm_tail_kernel(const floa
     }
 }
 
-// PF = register sets of global prefetch.  Measured on MI355X: 2 or 4 sets change the rate of the
-// 64x64 tile by -2..+4 % depending on the layer and cost the larger tiles a resident workgroup
-// (their register count nearly doubles), so every configuration runs with one.
-template <int BM, int BN, int BK, int WGM, int WGN, int PF = 1>
-struct TileCfg : GemmTile<BM, BN, BK, WGM, WGN> {
-    static constexpr int BM_ = BM, BN_ = BN, BK_ = BK, WGM_ = WGM, WGN_ = WGN, PF_ = PF;
-};
-
 typedef TileCfg<128, 128, 16, 2, 2> Cfg0;
 typedef TileCfg<64, 128, 16, 1, 2> Cfg1;
 typedef TileCfg<128, 64, 16, 2, 1> Cfg2;
@@ -294,18 +411,18 @@ typedef TileCfg<64, 32, 16, 2, 1> Cfg10;
 
 const fc_gemm_config kConfigs[] = {
 #define FC_CFG(id, T) {id, T::BM_, T::BN_, T::BK_, T::WGM_, T::WGN_, T::LDS_BYTES, 1}
-    FC_CFG(0, Cfg0), FC_CFG(1, Cfg1), FC_CFG(2, Cfg2), FC_CFG(3, Cfg3), FC_CFG(4, Cfg4), FC_CFG(5, Cfg5),
-    FC_CFG(6, Cfg6), FC_CFG(7, Cfg7), FC_CFG(8, Cfg8), FC_CFG(9, Cfg9), FC_CFG(10, Cfg10),
+    FC_CFG(0, Cfg0), FC_CFG(1, Cfg1), FC_CFG(2, Cfg2), FC_CFG(3, Cfg3), FC_CFG(4, Cfg4),
+    FC_CFG(5, Cfg5), FC_CFG(6, Cfg6), FC_CFG(7, Cfg7), FC_CFG(8, Cfg8), FC_CFG(9, Cfg9), FC_CFG(10, Cfg10),
 #undef FC_CFG
 };
 const int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 
-template <class TL>
+template <class TL, bool SPLIT = false>
 void launch(fc_context *ctx, const fc_wino_plan *plan, const float *U, const float *V, float *M) {
     const int nKB = plan->K_pad / TL::BM_, nTB = (int)(plan->T_pad / TL::BN_);
     const dim3 grid(64u * nKB * nTB);
-    wino_gemm_kernel<TL><<<grid, dim3(TL::THREADS), 0, ctx->stream>>>(U, V, M, plan->K_pad, plan->C_pad,
-                                                                      (int)plan->T_pad, nKB, nTB);
+    wino_gemm_kernel<TL, SPLIT><<<grid, dim3(TL::THREADS), 0, ctx->stream>>>(U, V, M, plan->K_pad, plan->C_pad,
+                                                                             (int)plan->T_pad, nKB, nTB);
 }
 
 // Tiles of the last, partly filled round that are worth quartering: none unless that
@@ -341,19 +458,33 @@ extern "C" int fc_wino_gemm_get_config(int id, fc_gemm_config *cfg) {
     return FC_OK;
 }
 
+static bool splits(long C, long K, const fc_gemm_config &c) {
+    return C * K > 8192 && c.bm % 64 == 0 && c.bn % 64 == 0 && c.bk == 16;
+}
+
+bool fc_wino_gemm_splits(const fc_wino_plan *plan) {
+    return splits(plan->shape.C, plan->shape.K, kConfigs[plan->gemm_config]);
+}
+
 // Cost model behind the untuned choice: padded multiply-adds, divided by a rate per tile shape
 // relative to 128x128x16 and by how evenly the grid fills the workgroup slots of the chip.  The
-// rates start from what each shape sustains on a large layer (256 -> 256 channels at 56x56,
-// batch 128) and are set so that the model picks a shape within 2 % of the best measured one on
-// fifteen VGG-16 / ResNet-50 layers at batch 1, 32 and 128: in practice 128x128 for large grids,
-// 64x64 for mid-sized ones (it loses less to padding and to uneven placement than its large-layer
-// rate suggests), 32x32 where a 64-wide tile would be mostly padding.
+// rates start from what each shape sustains on large layers (256 -> 256 channels at 56x56 and
+// 512 -> 512 at 28x28, batch 32).  The shapes of 64 and more run on the bf16 matrix cores
+// (128x128: 161 us against 220 with fp32 instructions on the first of these; 64x64: 195 against
+// 232), where the large tile is the furthest ahead: it writes and reads the least LDS per product.
+// 64x64 is level with it where it pads less (512 channels at 14x14: 68 us both) and ahead on
+// small grids; the shapes with a 32 stay on fp32 instructions, for layers whose 64-wide tile
+// would be mostly padding (512 channels at 28x28, batch 1: 14.7 us against 21).  Layers of few
+// channels stay on fp32 instructions whatever their tile: they are bound by memory (16 -> 64
+// channels, 28x28, batch 64: 7.1 us against 7.7), and keep the rates measured for those.
 extern "C" int fc_wino_gemm_default_config(const fc_conv_shape *s) {
     if (!fc_shape_ok(s)) return FC_ERR_INVALID;
-    static const double kRate[] = {1.00, 0.90, 0.90, 0.97, 0.72, 0.95, 0.88, 0.93, 0.93, 0.90, 0.76};
+    static const double kFp32Rate[] = {1.00, 0.90, 0.90, 0.97, 0.72, 0.95, 0.88, 0.93, 0.93, 0.90, 0.76};
+    static const double kRate[] = {1.00, 0.80, 0.80, 0.87, 0.63, 0.73, 0.70, 0.80, 0.80, 0.73, 0.65};
     static_assert(sizeof(kRate) / sizeof(kRate[0]) == sizeof(kConfigs) / sizeof(kConfigs[0]), "one rate per configuration");
     const int OH = fc_out_dim(s->H, s->pt, s->pb, 3, 1), OW = fc_out_dim(s->W, s->pl, s->pr, 3, 1);
     const double T = (double)s->N * ((OH + 5) / 6) * ((OW + 5) / 6);
+    const bool fewChannels = (long)s->C * s->K <= 8192;
     int best = 0;
     double bestCost = 1e300;
     for (int id = 0; id < kNumConfigs; id++) {
@@ -361,12 +492,15 @@ extern "C" int fc_wino_gemm_default_config(const fc_conv_shape *s) {
         const double kp = ceil((double)s->K / c.bm) * c.bm, tp = ceil(T / c.bn) * c.bn;
         const double cp = ceil((double)s->C / c.bk) * c.bk;
         const double blocks = 64.0 * (kp / c.bm) * (tp / c.bn);
-        const double slots = 256.0 * (c.bm * c.bn > 128 * 128 || c.bk == 32 ? 2 : 4);
+        const double slots = 256.0 * (c.bm * c.bn > 128 * 128 || c.bk == 32 ? 2 : id == 0 && !fewChannels ? 3 : 4);
         // the time of a launch is nearly linear in its tile count: a partly filled last round costs
-        // little, and nothing for configuration 0, whose last round runs as quartered tiles
+        // little, and nothing for configuration 0 on fp32 instructions, whose last round runs as quartered tiles
         double fill = blocks / (ceil(blocks / slots) * slots);
-        if (id == 0 && blocks > slots) fill = 1.0;
-        const double cost = kp * tp * cp / (kRate[id] * (0.8 + 0.2 * fill));
+        if (id == 0 && fewChannels && blocks > slots) fill = 1.0;
+        // the large tile on the bf16 matrix cores needs its three workgroups per CU to hide their barriers
+        // (256 -> 256 channels at 56x56, one image: 128 workgroups, 15.6 us against 11.4 for 64x64)
+        if (id == 0 && !fewChannels && blocks < slots) fill -= 2.0 * (1.0 - fill);
+        const double cost = kp * tp * cp / ((fewChannels ? kFp32Rate : kRate)[id] * (0.8 + 0.2 * fill));
         if (cost < bestCost) { bestCost = cost; best = id; }
     }
     return best;
@@ -390,20 +524,26 @@ extern "C" int fc_wino_gemm(fc_context *ctx, const fc_wino_plan *plan, const flo
     if (((uintptr_t)U_dev | (uintptr_t)V_dev | (uintptr_t)M_dev) & 15)
         return fc_set_error(ctx, FC_ERR_INVALID, "fc_wino_gemm: buffers must be 16-byte aligned", hipSuccess);
     fc_stage_scope scope(ctx, FC_STAGE_TENSOR_GEMM);
+    const bool split = fc_wino_gemm_splits(plan);
+#define FC_LAUNCH(T) (split ? launch<T, true>(ctx, plan, U_dev, V_dev, M_dev) : launch<T>(ctx, plan, U_dev, V_dev, M_dev))
     switch (plan->gemm_config) {
-        case 0: launch_with_tail<Cfg0, Cfg3>(ctx, plan, U_dev, V_dev, M_dev); break;
-        case 1: launch<Cfg1>(ctx, plan, U_dev, V_dev, M_dev); break;
-        case 2: launch<Cfg2>(ctx, plan, U_dev, V_dev, M_dev); break;
-        case 3: launch<Cfg3>(ctx, plan, U_dev, V_dev, M_dev); break;
+        case 0:
+            if (split) launch<Cfg0, true>(ctx, plan, U_dev, V_dev, M_dev);
+            else launch_with_tail<Cfg0, Cfg3>(ctx, plan, U_dev, V_dev, M_dev);
+            break;
+        case 1: FC_LAUNCH(Cfg1); break;
+        case 2: FC_LAUNCH(Cfg2); break;
+        case 3: FC_LAUNCH(Cfg3); break;
         case 4: launch<Cfg4>(ctx, plan, U_dev, V_dev, M_dev); break;
         case 5: launch<Cfg5>(ctx, plan, U_dev, V_dev, M_dev); break;
         case 6: launch<Cfg6>(ctx, plan, U_dev, V_dev, M_dev); break;
-        case 7: launch<Cfg7>(ctx, plan, U_dev, V_dev, M_dev); break;
-        case 8: launch<Cfg8>(ctx, plan, U_dev, V_dev, M_dev); break;
+        case 7: FC_LAUNCH(Cfg7); break;
+        case 8: FC_LAUNCH(Cfg8); break;
         case 9: launch<Cfg9>(ctx, plan, U_dev, V_dev, M_dev); break;
         case 10: launch<Cfg10>(ctx, plan, U_dev, V_dev, M_dev); break;
         default: return fc_set_error(ctx, FC_ERR_INVALID, "fc_wino_gemm: unknown tile configuration", hipSuccess);
     }
+#undef FC_LAUNCH
     FC_LAUNCH_CHECK(ctx, "wino_gemm_kernel");
     return FC_OK;
 }
