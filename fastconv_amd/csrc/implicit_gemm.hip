@@ -11,6 +11,7 @@
 #include <utility>
 
 #include "fc_internal.h"
+#include "split_mfma.h"
 
 namespace {
 
@@ -178,31 +179,128 @@ __device__ __forceinline__ void ig_gather_rows_buf(float (&r)[sizeof...(I)], __a
 // IG_TAP_*: the buffer gather for tap-major layers (see igemm_pack_filter_kernel).
 enum { IG_GATHER = 0, IG_POINTWISE = 1, IG_BUF_MASKED = 2, IG_TAP_MASKED = 3, IG_TAP_INSIDE = 4 };
 
+// Workgroups are dealt to the 8 XCDs round-robin by linear id, and every XCD has an L2 of its own.
+// Tiles are numbered pixel block major, output-channel block minor, and every XCD owns a contiguous
+// eighth of that sequence: the output-channel blocks that share one block of gathered pixels run
+// side by side on ONE XCD and find the pixels in its L2 (dealt round-robin, every XCD would fetch
+// every pixel block: measured 4-6x the algorithmic traffic on the ResNet-50 projections).
+// Returns false for a workgroup past the last tile.
+__device__ __forceinline__ bool ig_decode_tile(const IgemmParams &p, int *kb, int *pb) {
+    const int nTiles = p.nKB * p.nPB, perXcd = (nTiles + 7) >> 3;
+    const int tileId = (blockIdx.x & 7) * perXcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= perXcd || tileId >= nTiles) return false;
+    *pb = tileId / p.nKB;
+    *kb = tileId - *pb * p.nKB;
+    return true;
+}
+
+// The accumulators of a workgroup tile to y, or to this split's partial sums.
+template <class TL>
+__device__ __forceinline__ void ig_store_tile(const floatx16 (&acc)[TL::MI][TL::NI], const IgemmParams &p, int kb, int pb, int wm0,
+                                              int wn0, int lrow, int lcol) {
+    constexpr int BM = TL::BM_, BN = TL::BN_, MI = TL::MI, NI = TL::NI;
+    // epilogue: column = pixel (lane%32), rows = output channels.  Register i of an accumulator
+    // block is row 8*(i/4) + 4*(lane/32) + i%4: element (row r, column c) of the tile goes to
+    // dst[colOff(c) + (rowBase + r) * rowStride], with dst = y (colOff = n*K*OHW + pixel in image,
+    // rowStride = OHW) or the partial-sum slab of this split (colOff = pixel, rowStride = Npix).
+    const int OHW = p.OH * p.OW;
+    const bool partial = p.splitK > 1;
+    const int rowBase = kb * BM + wm0 + 4 * lrow;
+    if (p.fastStore) {
+        // every row of the tile is a real output channel and every byte offset fits 32 bits: a
+        // scalar base, one 32-bit offset per store, no predicates
+        char *dst = reinterpret_cast<char *>(partial ? p.ws : p.y);
+        const uint32_t rowStride = 4u * (partial ? (uint32_t)p.Npix : (uint32_t)OHW);      // bytes
+        const uint32_t slab = partial ? (uint32_t)blockIdx.y * (uint32_t)p.K * (uint32_t)p.Npix : 0u;
+        const bool plain = partial || (p.bias == nullptr && !p.relu);
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) {
+            const long opix = (long)pb * BN + wn0 + ni * 32 + lcol;
+            if (opix >= p.Npix) continue;
+            uint32_t off;
+            if (partial) {
+                off = slab + (uint32_t)opix;
+            } else {
+                const uint32_t n = fc_div((uint32_t)opix, p.divOHW);
+                off = n * (uint32_t)p.K * (uint32_t)OHW + ((uint32_t)opix - n * (uint32_t)OHW);
+            }
+            off = 4u * off + (uint32_t)rowBase * rowStride;
+            if (plain) {
+#pragma unroll
+                for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++)
+                        *reinterpret_cast<float *>(dst + (off + (uint32_t)(mi * 32 + 8 * (i / 4) + (i % 4)) * rowStride)) = acc[mi][ni][i];
+            } else {
+#pragma unroll
+                for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        floatx4 bq = {0.f, 0.f, 0.f, 0.f};
+                        if (p.bias) bq = *reinterpret_cast<const floatx4 *>(p.bias + rowBase + mi * 32 + 8 * q);
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            float v = acc[mi][ni][q * 4 + j] + bq[j];
+                            if (p.relu) v = __builtin_elementwise_maximum(v, 0.f);      // keeps a NaN
+                            *reinterpret_cast<float *>(dst + (off + (uint32_t)(mi * 32 + 8 * q + j) * rowStride)) = v;
+                        }
+                    }
+            }
+        }
+        return;
+    }
+    if (partial) {
+        // partial sums, [split][k][pixel]; igemm_reduce_kernel adds them up in split order
+        float *wz = p.ws + (size_t)blockIdx.y * p.K * p.Npix;
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) {
+            const long opix = (long)pb * BN + wn0 + ni * 32 + lcol;
+            if (opix >= p.Npix) continue;
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int k = rowBase + mi * 32 + 8 * (i / 4) + (i % 4);
+                    if (k < p.K) wz[(size_t)k * p.Npix + opix] = acc[mi][ni][i];
+                }
+        }
+        return;
+    }
+#pragma unroll
+    for (int ni = 0; ni < NI; ni++) {
+        const long opix = (long)pb * BN + wn0 + ni * 32 + lcol;
+        if (opix >= p.Npix) continue;
+        const uint32_t n = fc_div((uint32_t)opix, p.divOHW);
+        const uint32_t pp = (uint32_t)opix - n * (uint32_t)OHW;
+        float *yn = p.y + (size_t)n * p.K * OHW + pp;
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int k = rowBase + mi * 32 + 8 * (i / 4) + (i % 4);
+                if (k < p.K) {
+                    float v = acc[mi][ni][i];
+                    if (p.bias) v += p.bias[k];
+                    if (p.relu) v = __builtin_elementwise_maximum(v, 0.f);      // keeps a NaN
+                    yn[(size_t)k * OHW] = v;
+                }
+            }
+    }
+}
+
 // PW: pointwise layers (1x1, stride 1, no padding: the column matrix IS the input, row c of it
 // is channel c of x, contiguous over the pixels) whose pixels-per-image count is a multiple of 4
 // and whose channel count is a multiple of BK copy the B tile as 16-byte vectors, unconditionally:
 // a pixel group past the end re-reads the last group (its columns are never stored).
 template <class TL, int MODE>
-__global__ __launch_bounds__(TL::THREADS, TL::MIN_WAVES) void igemm_conv_kernel(const IgemmParams p) {
+__device__ __forceinline__ void ig_tile(const IgemmParams &p, const int kb, const int pb, float (*As)[TL::BK_ * TL::BM_],
+                                        float (*Bs)[TL::BK_ * TL::BN_]) {
     constexpr bool PW = MODE == IG_POINTWISE, TAP = MODE == IG_TAP_MASKED || MODE == IG_TAP_INSIDE;
     constexpr bool BUF = MODE == IG_BUF_MASKED || TAP;
     constexpr int BM = TL::BM_, BN = TL::BN_, BK = TL::BK_;
     constexpr int MI = TL::MI, NI = TL::NI, A_LD = TL::A_LD, B_LD = TL::B_LD;
-    __shared__ __attribute__((aligned(16))) float As[2][BK * BM];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BK * BN];
-
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm0 = (wave / TL::WGN_) * TL::WM, wn0 = (wave % TL::WGN_) * TL::WN;
-    // Workgroups are dealt to the 8 XCDs round-robin by linear id, and every XCD has an L2 of its own.
-    // Tiles are numbered pixel block major, output-channel block minor, and every XCD owns a contiguous
-    // eighth of that sequence: the output-channel blocks that share one block of gathered pixels run
-    // side by side on ONE XCD and find the pixels in its L2 (dealt round-robin, every XCD would fetch
-    // every pixel block: measured 4-6x the algorithmic traffic on the ResNet-50 projections).
-    const int nTiles = p.nKB * p.nPB, perXcd = (nTiles + 7) >> 3;
-    const int tileId = (blockIdx.x & 7) * perXcd + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= perXcd || tileId >= nTiles) return;
-    const int pb = tileId / p.nKB, kb = tileId - pb * p.nKB;
-
     // filter tile: straight 16-byte copies
     const int arow = tid / (BM / 4), acol = (tid % (BM / 4)) * 4;
     const float *ag = p.Wp + (size_t)kb * BM;                     // uniform; the lane adds aOff bytes
@@ -413,93 +511,191 @@ __global__ __launch_bounds__(TL::THREADS, TL::MIN_WAVES) void igemm_conv_kernel(
         __syncthreads();
     }
 
-    // epilogue: column = pixel (lane%32), rows = output channels.  Register i of an accumulator
-    // block is row 8*(i/4) + 4*(lane/32) + i%4: element (row r, column c) of the tile goes to
-    // dst[colOff(c) + (rowBase + r) * rowStride], with dst = y (colOff = n*K*OHW + pixel in image,
-    // rowStride = OHW) or the partial-sum slab of this split (colOff = pixel, rowStride = Npix).
-    const int OHW = p.OH * p.OW;
-    const bool partial = p.splitK > 1;
-    const int rowBase = kb * BM + wm0 + 4 * lrow;
-    if (p.fastStore) {
-        // every row of the tile is a real output channel and every byte offset fits 32 bits: a
-        // scalar base, one 32-bit offset per store, no predicates
-        char *dst = reinterpret_cast<char *>(partial ? p.ws : p.y);
-        const uint32_t rowStride = 4u * (partial ? (uint32_t)p.Npix : (uint32_t)OHW);      // bytes
-        const uint32_t slab = partial ? (uint32_t)blockIdx.y * (uint32_t)p.K * (uint32_t)p.Npix : 0u;
-        const bool plain = partial || (p.bias == nullptr && !p.relu);
+    ig_store_tile<TL>(acc, p, kb, pb, wm0, wn0, lrow, lcol);
+}
+
+template <class TL, int MODE>
+__global__ __launch_bounds__(TL::THREADS, TL::MIN_WAVES) void igemm_conv_kernel(const IgemmParams p) {
+    __shared__ __attribute__((aligned(16))) float As[2][TL::BK_ * TL::BM_];
+    __shared__ __attribute__((aligned(16))) float Bs[2][TL::BK_ * TL::BN_];
+    int kb, pb;
+    if (ig_decode_tile(p, &kb, &pb)) ig_tile<TL, MODE>(p, kb, pb, As, Bs);
+}
+
+// The same layer on the bf16 matrix cores at fp32 accuracy (see split_mfma.h), for inputs below 2 GiB.  A wavefront
+// takes 64 output channels or 64 pixels x 8 reduction rows at a time, a lane one channel or pixel: 8 loads through
+// buffer resources, a stage ahead, and one 16-byte word to LDS per part.  A lane's pixel is the same in every block it takes.
+// Bound by LDS for 64x64 tiles (288 cycles of a CU's LDS a stage, 192 of its matrix cores; 128x128: 576 and 768).
+// Measured at batch 32, fp32 instructions -> this: 256 -> 256 3x3/2 at 28x28 81.5 -> 76.2 us, 7x7/2 stem 91.4 -> 78.7,
+// 512 -> 2048 1x1 at 7x7 39.4 -> 31.0, 64 -> 64 3x3 at 56x56 73.1 -> 61.0.
+template <class TL>
+struct IgSplit {
+    static constexpr int A_WAVES = 2 * TL::BM_ / 64, B_WAVES = 2 * TL::BN_ / 64, WAVES = TL::THREADS / 64;   // blocks of a stage
+    // enough wavefronts for both operands at once: the first take A, the others B; else every wavefront takes both
+    static constexpr bool APART = A_WAVES + B_WAVES <= WAVES;
+    static constexpr int A_LD = (A_WAVES + WAVES - 1) / WAVES, B_LD = (B_WAVES + WAVES - 1) / WAVES;
+    typedef fc_split_stage<TL::BM_, TL::BN_> Stage;
+    static constexpr int LDS_WORDS = 2 * Stage::WORDS;
+    static constexpr int MIN_WAVES = TL::BM_ * TL::BN_ > 128 * 128 ? 1 : TL::BM_ * TL::BN_ == 64 * 64 ? 4 : 3;
+    static_assert(TL::BM_ % 64 == 0 && TL::BN_ % 64 == 0 && TL::BK_ == 16, "a wavefront fetches 64 rows or columns x 8 of the reduction");
+    static_assert(B_LD == 1 || B_WAVES % WAVES == 0, "no part-filled second block");
+    static_assert(B_LD == 1 || TL::THREADS % TL::BN_ == 0, "one pixel per lane");
+};
+
+template <class TL, int MODE, bool SPLIT>
+__global__ __launch_bounds__(TL::THREADS, IgSplit<TL>::MIN_WAVES) void igemm_conv_kernel(const IgemmParams p) {
+    static_assert(SPLIT, "the kernel above is the other one");
+    typedef IgSplit<TL> S;
+    constexpr bool TAP = MODE == IG_TAP_MASKED || MODE == IG_TAP_INSIDE;
+    constexpr int BM = TL::BM_, BN = TL::BN_, MI = TL::MI, NI = TL::NI, A_LD = S::A_LD, B_LD = S::B_LD, WAVES = S::WAVES;
+    constexpr int A_PLANE = S::Stage::A_PLANE, B_PLANE = S::Stage::B_PLANE, WORDS = S::Stage::WORDS;
+    __shared__ fc_uintx4 smem[S::LDS_WORDS];
+    int kb, pb;
+    if (!ig_decode_tile(p, &kb, &pb)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm0 = (wave / TL::WGN_) * TL::WM, wn0 = (wave % TL::WGN_) * TL::WN;
+    const int lrow = lane >> 5, lcol = lane & 31;
+    const int nStagesAll = p.Kred_pad / 16;
+    const int sBegin = blockIdx.y * p.stagesPerSplit, sEnd = min(sBegin + p.stagesPerSplit, nStagesAll);
+
+    // block numbers of this wavefront: depth half = block * 64 / width, first row or column = block * 64 % width
+    const int bWave = S::APART ? wave - S::A_WAVES : wave;
+    const bool takesA = wave < S::A_WAVES, takesB = bWave >= 0 && bWave < S::B_WAVES;
+
+    // filter: rows of Wp from a uniform pointer
+    const float *asrc[A_LD];
 #pragma unroll
-        for (int ni = 0; ni < NI; ni++) {
-            const long opix = (long)pb * BN + wn0 + ni * 32 + lcol;
-            if (opix >= p.Npix) continue;
-            uint32_t off;
-            if (partial) {
-                off = slab + (uint32_t)opix;
-            } else {
-                const uint32_t n = fc_div((uint32_t)opix, p.divOHW);
-                off = n * (uint32_t)p.K * (uint32_t)OHW + ((uint32_t)opix - n * (uint32_t)OHW);
+    for (int j = 0; j < A_LD; j++) {
+        const int e = (wave + j * WAVES) * 64;
+        asrc[j] = uniform_ptr(p.Wp + (size_t)(sBegin * 16 + 8 * (e / BM)) * p.K_pad + (size_t)kb * BM + e % BM);
+    }
+    // pixel: byte offset of its window in the tensor and the taps that lie outside the image
+    uint32_t pixByte = 0, invLo = ~0u, invHi = ~0u;
+    const long pix = (long)pb * BN + (bWave * 64) % BN + lane;
+    if (takesB && pix < p.Npix) {
+        const uint32_t n = fc_div((uint32_t)pix, p.divOHW);
+        const uint32_t pp = (uint32_t)pix - n * (uint32_t)(p.OH * p.OW);
+        const uint32_t oh = fc_div(pp, p.divOW), ow = pp - oh * p.OW;
+        const int ih0 = (int)oh * p.sh - p.pt, iw0 = (int)ow * p.sw - p.pl;
+        pixByte = 4u * (n * (uint32_t)(p.C * p.H * p.W) + (uint32_t)(ih0 * p.W + iw0));
+        if (MODE != IG_TAP_INSIDE) {
+            uint32_t rowBits = 0;
+            for (int q = 0; q < p.kw; q++) rowBits |= ((unsigned)(iw0 + q) < (unsigned)p.W) ? 0u : (1u << q);
+            uint64_t inv = 0;
+            for (int r = 0; r < p.kh; r++) {
+                const uint32_t bits = ((unsigned)(ih0 + r) < (unsigned)p.H) ? rowBits : ((1u << p.kw) - 1u);
+                if (r * p.kw < 64) inv |= (uint64_t)bits << (r * p.kw);
             }
-            off = 4u * off + (uint32_t)rowBase * rowStride;
-            if (plain) {
+            if (p.kh * p.kw < 64) inv |= ~0ull << (p.kh * p.kw);
+            invLo = (uint32_t)inv;
+            invHi = (uint32_t)(inv >> 32);
+        }
+    }
+    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.x), 0, (int)p.xBytes, 0x00020000);
+
+    // tap-major order: the tap and the first channel of the stage, counted in scalar registers
+    const uint32_t chanStep = 4u * (uint32_t)(p.H * p.W);
+    int tapT = 0, tapR = 0, tapS = 0, tapC = 0;
+    if (TAP) {
+        const int stagesPerTap = p.C / 16;
+        tapT = sBegin / stagesPerTap;
+        tapC = (sBegin - tapT * stagesPerTap) * 16;
+        tapR = tapT / p.kw;
+        tapS = tapT - tapR * p.kw;
+    }
+    float ra[A_LD][8], rb[B_LD][8];
+    uint32_t laneOff = 4u * lane;
+    // fetches stage s; stages are fetched in order
+    auto fetch = [&](const int s) __attribute__((always_inline)) {
+        if (takesA) {
+            asm volatile("" : "+v"(laneOff));
 #pragma unroll
-                for (int mi = 0; mi < MI; mi++)
+            for (int j = 0; j < A_LD; j++) {
+                const float *b = asrc[j];
 #pragma unroll
-                    for (int i = 0; i < 16; i++)
-                        *reinterpret_cast<float *>(dst + (off + (uint32_t)(mi * 32 + 8 * (i / 4) + (i % 4)) * rowStride)) = acc[mi][ni][i];
-            } else {
-#pragma unroll
-                for (int mi = 0; mi < MI; mi++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        floatx4 bq = {0.f, 0.f, 0.f, 0.f};
-                        if (p.bias) bq = *reinterpret_cast<const floatx4 *>(p.bias + rowBase + mi * 32 + 8 * q);
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            float v = acc[mi][ni][q * 4 + j] + bq[j];
-                            if (p.relu) v = __builtin_elementwise_maximum(v, 0.f);      // keeps a NaN
-                            *reinterpret_cast<float *>(dst + (off + (uint32_t)(mi * 32 + 8 * q + j) * rowStride)) = v;
-                        }
-                    }
+                for (int i = 0; i < 8; i++) {
+                    ra[j][i] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(b) + laneOff);
+                    b = uniform_ptr(b + p.K_pad);
+                }
+                asrc[j] = uniform_ptr(b + (size_t)8 * p.K_pad);
             }
         }
-        return;
-    }
-    if (partial) {
-        // partial sums, [split][k][pixel]; igemm_reduce_kernel adds them up in split order
-        float *wz = p.ws + (size_t)blockIdx.y * p.K * p.Npix;
-#pragma unroll
-        for (int ni = 0; ni < NI; ni++) {
-            const long opix = (long)pb * BN + wn0 + ni * 32 + lcol;
-            if (opix >= p.Npix) continue;
-#pragma unroll
-            for (int mi = 0; mi < MI; mi++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int k = rowBase + mi * 32 + 8 * (i / 4) + (i % 4);
-                    if (k < p.K) wz[(size_t)k * p.Npix + opix] = acc[mi][ni][i];
-                }
-        }
-        return;
-    }
-#pragma unroll
-    for (int ni = 0; ni < NI; ni++) {
-        const long opix = (long)pb * BN + wn0 + ni * 32 + lcol;
-        if (opix >= p.Npix) continue;
-        const uint32_t n = fc_div((uint32_t)opix, p.divOHW);
-        const uint32_t pp = (uint32_t)opix - n * (uint32_t)OHW;
-        float *yn = p.y + (size_t)n * p.K * OHW + pp;
-#pragma unroll
-        for (int mi = 0; mi < MI; mi++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int k = rowBase + mi * 32 + 8 * (i / 4) + (i % 4);
-                if (k < p.K) {
-                    float v = acc[mi][ni][i];
-                    if (p.bias) v += p.bias[k];
-                    if (p.relu) v = __builtin_elementwise_maximum(v, 0.f);      // keeps a NaN
-                    yn[(size_t)k * OHW] = v;
-                }
+        if (!takesB) return;
+        if (TAP) {
+            const uint32_t voff = pixByte + 4u * (uint32_t)(tapR * p.W + tapS);
+            // last, as a border pixel's window starts at a negative (wrapped) offset
+            uint32_t poison = 0;
+            if (MODE == IG_TAP_MASKED) {
+                const uint32_t word = tapT < 32 ? invLo : invHi;
+                poison = ((word >> (tapT & 31)) & 1u) << 31;
             }
+#pragma unroll
+            for (int j = 0; j < B_LD; j++) {
+                const uint32_t chan0 = (uint32_t)(tapC + 8 * ((bWave + j * WAVES) * 64 / BN)) * chanStep;
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    rb[j][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                   xres, (voff + (chan0 + (uint32_t)i * chanStep)) | poison, 0, 0));
+            }
+            tapC += 16;
+            if (tapC == p.C) {
+                tapC = 0;
+                tapT++;
+                if (++tapS == p.kw) { tapS = 0; tapR++; }
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < B_LD; j++)
+                ig_gather_rows_buf<true>(rb[j], xres, pixByte, invLo, invHi, p.table, s * 16 + 8 * ((bWave + j * WAVES) * 64 / BN), 1,
+                                         p.kw, std::make_integer_sequence<int, 8>());
+        }
+    };
+    auto park = [&](const int buf) __attribute__((always_inline)) {
+        fc_uintx4 *const dst = smem + buf * WORDS + lane;
+        if (takesA) {
+#pragma unroll
+            for (int j = 0; j < A_LD; j++) fc_split8(ra[j], dst + (wave + j * WAVES) * 64, A_PLANE);
+        }
+        if (takesB) {
+#pragma unroll
+            for (int j = 0; j < B_LD; j++) fc_split8(rb[j], dst + 3 * A_PLANE + (bWave + j * WAVES) * 64, B_PLANE);
+        }
+    };
+
+    floatx16 acc[MI][NI];
+#pragma unroll
+    for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[mi][ni][i] = 0.f;
+    const int aFrag = lrow * BM + wm0 + lcol, bFrag = 3 * A_PLANE + lrow * BN + wn0 + lcol;
+
+    fetch(sBegin);
+    park(0);
+    if (sBegin + 1 < sEnd) fetch(sBegin + 1);
+    __syncthreads();
+    for (int s = sBegin; s < sEnd; s++) {
+        const int buf = (s - sBegin) & 1;
+        const fc_uintx4 *cur = smem + buf * WORDS;
+        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc);
+        if (s + 1 < sEnd) {
+            park(buf ^ 1);
+            if (s + 2 < sEnd) fetch(s + 2);
+        }
+        __syncthreads();
     }
+    if (__syncthreads_or(fc_not_finite<MI, NI>(acc))) {
+        // 64x64 at a time, which leaves the registers to the loop above
+        typedef IgTile<64, 64, 16, 2, TL::THREADS / 128> Sub;
+        static_assert(Sub::THREADS == TL::THREADS && Sub::LDS_BYTES <= 16 * S::LDS_WORDS, "same workgroup");
+        float *const f = reinterpret_cast<float *>(smem);
+        for (int q = 0; q < (BM / 64) * (BN / 64); q++)
+            ig_tile<Sub, MODE>(p, kb * (BM / 64) + q / (BN / 64), pb * (BN / 64) + q % (BN / 64),
+                               reinterpret_cast<float (*)[16 * 64]>(f), reinterpret_cast<float (*)[16 * 64]>(f + 2 * 16 * 64));
+        return;
+    }
+    ig_store_tile<TL>(acc, p, kb, pb, wm0, wn0, lrow, lcol);
 }
 
 // Sums the partial results of a split reduction in split order (so the result does
@@ -549,11 +745,23 @@ void launch(fc_context *ctx, IgemmParams &p) {
     // one 32-bit byte offset with bit 31 to spare reaches every element of the tensor
     const bool buffer = p.xBytes < (1l << 31);
     const bool tapMajor = p.C % TL::BK_ == 0;      // the order fc_igemm_pack_filter laid the filter out in
-    if (pointwise) igemm_conv_kernel<TL, IG_POINTWISE><<<grid, dim3(TL::THREADS), 0, ctx->stream>>>(p);
-    else if (buffer && tapMajor && inside) igemm_conv_kernel<TL, IG_TAP_INSIDE><<<grid, dim3(TL::THREADS), 0, ctx->stream>>>(p);
-    else if (buffer && tapMajor && p.kh * p.kw <= 64) igemm_conv_kernel<TL, IG_TAP_MASKED><<<grid, dim3(TL::THREADS), 0, ctx->stream>>>(p);
-    else if (buffer && p.kh * p.kw <= 64) igemm_conv_kernel<TL, IG_BUF_MASKED><<<grid, dim3(TL::THREADS), 0, ctx->stream>>>(p);      // the taps of a window are one 64-bit mask
-    else igemm_conv_kernel<TL, IG_GATHER><<<grid, dim3(TL::THREADS), 0, ctx->stream>>>(p);
+    const dim3 block(TL::THREADS);
+    if constexpr (TL::BM_ % 64 == 0) {
+        // Bf16 matrix cores (a pointwise layer is a tap-major one whose only tap is inside) for inputs below 2 GiB, but
+        // not for a pointwise layer of up to 64 output channels: that is bound by reading x, which the fp32 kernel does
+        // 16 bytes a lane (256 -> 64 channels at 56x56, batch 32: 35.8 us against 37.6; 64 -> 256: 34.4 against 32.6);
+        // nor for a reduction of two or three stages, bound by its gathers and stores (3 -> 64 channels 3x3 at 224x224,
+        // batch 32: 129 us against 139).
+        const bool split = buffer && p.Kred_pad >= 64 && !(pointwise && p.K <= 64);
+        if (split && tapMajor && inside) { igemm_conv_kernel<TL, IG_TAP_INSIDE, true><<<grid, block, 0, ctx->stream>>>(p); return; }
+        if (split && tapMajor && p.kh * p.kw <= 64) { igemm_conv_kernel<TL, IG_TAP_MASKED, true><<<grid, block, 0, ctx->stream>>>(p); return; }
+        if (split && p.kh * p.kw <= 64) { igemm_conv_kernel<TL, IG_BUF_MASKED, true><<<grid, block, 0, ctx->stream>>>(p); return; }
+    }
+    if (pointwise) igemm_conv_kernel<TL, IG_POINTWISE><<<grid, block, 0, ctx->stream>>>(p);
+    else if (buffer && tapMajor && inside) igemm_conv_kernel<TL, IG_TAP_INSIDE><<<grid, block, 0, ctx->stream>>>(p);
+    else if (buffer && tapMajor && p.kh * p.kw <= 64) igemm_conv_kernel<TL, IG_TAP_MASKED><<<grid, block, 0, ctx->stream>>>(p);
+    else if (buffer && p.kh * p.kw <= 64) igemm_conv_kernel<TL, IG_BUF_MASKED><<<grid, block, 0, ctx->stream>>>(p);      // the taps of a window are one 64-bit mask
+    else igemm_conv_kernel<TL, IG_GATHER><<<grid, block, 0, ctx->stream>>>(p);
 }
 
 }  // namespace
@@ -591,12 +799,23 @@ extern "C" int fc_igemm_default_config(const fc_conv_shape *s) {
         const double cost = mp * np * kp / (kRate[id] * (0.8 + 0.2 * fill));
         if (cost < bestCost) { bestCost = cost; best = id; }
     }
+    // On the bf16 matrix cores 128x128 writes and reads the least LDS per product.  It takes over from 64x64 where the
+    // reduction is long enough to pay for its longer start, the grid is at least two rounds of its three workgroups per
+    // CU without a split, and it pads no more.  At batch 32 and the like:
+    // 256 -> 256 1x1 at 56x56 80 us against 92, 85 -> 128 3x3 at 150x150 303 against 403; with 32 rows 27.5 against 22.7.
+    if (best == 3 && Kr >= 256 && ceil(M / 128) * 128 == ceil(M / 64) * 64 && ceil(M / 128) * ceil(Np / 128) >= 1536) best = 0;
     // A layer that this tile shape can only fill the chip with by splitting the reduction over workgroups
     // (a pass of partial sums through memory and a second launch) goes to the kernels that split it inside
-    // the workgroup instead, while it is small enough for them.
+    // the workgroup instead, while it is small enough for them.  Where 64x64 tiles waste nothing and the partial sums
+    // fit the static workspace (so that fc_conv_implicit_gemm_static takes the plan, as before) the line is lower: at
+    // 1.85 GFLOP the others are ahead or level (3x3 on 256 channels, two 28x28 images: 23 us against 28; 1x1
+    // 2048 -> 512 on sixteen 7x7 images: 24 against 23), at 3.3 and 3.7 GFLOP behind (40 against 36 and 42 against
+    // 37-40, five layers).
     fc_igemm_plan plan;
     if (fc_igemm_make_plan(s, best, &plan) == FC_OK && plan.split_k > 1) {
-        const int ws = fc_igemm_ws_choose(s, plan.Npix);
+        const bool tiled = best == 3 && s->K % 64 == 0 && s->C % 16 == 0 && plan.split_k <= 15 && 2.0 * M * Kr * Np >= 3.2e9 &&
+                           plan.ws_bytes <= (size_t)FC_IGEMM_STATIC_WS_BYTES;
+        const int ws = tiled ? -1 : fc_igemm_ws_choose(s, plan.Npix);
         if (ws >= 0) return kNumIgConfigs + ws;
     }
     return best;
