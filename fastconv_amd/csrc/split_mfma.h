@@ -4,7 +4,7 @@
 // to nearest) and what is left, which fits 8 more.  Of the nine products of two such sums six are formed; the three left
 // out (mid*lo, lo*mid, lo*lo) are below 2^-22 of a product and of either sign.  Products of bf16 values are exact in the
 // matrix core and are added up in fp32.
-// Why: v_mfma_f32_32x32x2_f32 does 64 multiply-adds a cycle and SIMD unit, v_mfma_f32_32x32x16_bf16 512 and more, so six
+// Why: v_mfma_f32_32x32x2_f32 does 32 multiply-adds a cycle and SIMD unit, v_mfma_f32_32x32x16_bf16 512, so for 16384 six
 // passes of it take 192 cycles where the fp32 ones take 512, and the split costs about 6 vector instructions an element,
 // which run beside the bf16 matrix core.
 // An infinity has no such sum (inf - inf), so a tile whose result is not finite throughout is computed again with fp32

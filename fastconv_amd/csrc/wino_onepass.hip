@@ -401,8 +401,24 @@ extern "C" int fc_wino_prefer_onepass(const fc_conv_shape *s) {
     // bring a few blocks per CU (batch 1 layers do not).  Measured crossover against the staged
     // pipeline: about 200 blocks when one block covers all output channels, 500 otherwise.
     const long OH = fc_out_dim(s->H, s->pt, s->pb, 3, 1), OW = fc_out_dim(s->W, s->pl, s->pr, 3, 1);
-    const long blocks = ((long)s->N * ((OH + 5) / 6) * ((OW + 5) / 6) + kTB - 1) / kTB * ((s->K + kKB - 1) / kKB);
-    return blocks >= (s->K <= kKB ? 192 : 512) ? 1 : 0;
+    const long T = (long)s->N * ((OH + 5) / 6) * ((OW + 5) / 6);
+    const long blocks = (T + kTB - 1) / kTB * ((s->K + kKB - 1) / kKB);
+    if (blocks < (s->K <= kKB ? 192 : 512)) return 0;
+    if ((OW + 5) / 6 > kWinoMaxTilesW) return 1;      // the other pipelines do not take it
+    // What the pipelines with V and M in memory pay is bytes, what this one pays is products and, for every 64 output
+    // channels, an input transform: the line is a number of bytes per input channel.  It lies higher where the GEMM runs
+    // on the bf16 matrix cores (C*K > 8192).  Measured, us here / staged, at (V+M in MB):
+    //   64 -> 256 56x56 n32 (262) 171 / 130, 64 -> 512 28x28 n64 (236) 184 / 122, 64 -> 1024 110x110 n6 (603) 406 / 341,
+    //   64 -> 256 112x112 n32 (946) 518 / 538, 48 -> 512 76x76 n15 (363) 189 / 174, 48 -> 512 218x218 n4 (785) 404 / 486,
+    //   32 -> 512 69x69 n14 (281) 164 / 135, 32 -> 512 56x56 n32 (446) 198 / 200, 24 -> 512 202x202 n2 (317) 123 / 148;
+    //   C*K <= 8192: 64 -> 64 53x53 n54 (143) 109 / 65, 63x63 n50 (198) 109 / 97, 119x119 n20 (262) 115 / 129,
+    //   32 -> 64 141x141 n6 (85) 48 / 45, 32 -> 128 66x66 n37 (183) 85 / 87.
+    const double bytes = 256.0 * ((s->C + 15) / 16 * 16 + (s->K + 31) / 32 * 32) * (double)T;
+    if (bytes <= ((long)s->C * s->K > 8192 ? 10e6 : 3.5e6) * s->C) return 0;
+    // Few input and many output channels: the input transform of every 64 output channels outweighs writing V once, and
+    // the fused kernel needs no M.  Here / fused: 32 -> 256 62x62 n23 92 / 81, 159x159 n20 566 / 538, 32 -> 192 155x155
+    // n15 301 / 281, 24 -> 256 48x48 n48 78 / 70, 16 -> 512 112x112 n32 547 / 531; 32 -> 128 112x112 n32 169 / 183.
+    return s->C <= 32 && s->K >= 192 && bytes <= 2e9 && fc_wino_prefer_fused(s) ? 0 : 1;
 }
 
 extern "C" int fc_wino_forward_onepass(fc_context *ctx, const fc_wino_plan *plan, const float *x_dev, const float *w_dev,

@@ -440,8 +440,6 @@ __global__ __launch_bounds__(TPB / TPT) void wino_output_transform_kernel(const 
     }
 }
 
-constexpr int kWinoMaxTilesW = 170;
-
 // Largest of 128 / 64 / 32 tiles per block that divides the padded tile count.
 int tiles_per_block(long T_pad) { return (T_pad % 128 == 0) ? 128 : (T_pad % 64 == 0) ? 64 : 32; }
 

@@ -312,7 +312,9 @@ int fc_wino_forward_onepass(fc_context *ctx, const fc_wino_plan *plan, const flo
  * layer (measured on MI355X: 16 to 64 input channels, where the products are cheap next to
  * moving V and M through HBM, the image at least 8 columns wide, and at least 512 blocks of
  * 16 tiles x 64 output channels -- 192 when one block covers all output channels -- i.e. not
- * at batch 1; and every layer with at most four input channels, at any batch). */
+ * at batch 1, and V and M too large for the staged pipeline to be faster, from 3.5 MB per input
+ * channel on, 10 MB where C*K > 8192; and every layer with at most four input channels, at any
+ * batch), else 0. */
 int fc_wino_prefer_onepass(const fc_conv_shape *shape);
 
 /* All stages back to back: what winoF63_v1_single (winoF63ZC/winoF63ZC.h:5-6)

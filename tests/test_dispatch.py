@@ -1,0 +1,44 @@
+"""Which Winograd pipeline the library advises (host code only): where the single-kernel path hands a layer to the
+pipelines with V and M in memory, they accept it."""
+import ctypes as C
+
+import pytest
+
+from fastconv_amd import capi
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return capi.load_cdll()
+
+
+def shape(n, c, k, h, w=None):
+    return capi.ConvShape(n, c, h, h if w is None else w, k, 3, 3, 1, 1, 1, 1, 1, 1)
+
+
+@pytest.mark.parametrize("layer,onepass,fused", [
+    ((32, 64, 64, 224), 1, 0), ((32, 64, 128, 112), 1, 0), ((32, 64, 256, 112), 1, 0),   # V and M far beyond the last-level cache
+    ((32, 64, 64, 56), 0, 0), ((50, 64, 64, 63), 0, 0), ((20, 64, 64, 119), 1, 0),        # the line for fp32 instructions
+    ((32, 64, 256, 56), 0, 0), ((6, 64, 1024, 110), 0, 0), ((14, 32, 512, 69), 0, 0), ((2, 24, 512, 202), 1, 0),
+    ((23, 32, 256, 62), 0, 1), ((32, 16, 512, 112), 0, 1), ((32, 32, 128, 112), 1, 1),    # few channels in, many out
+    ((1, 64, 64, 56), 0, 0), ((4, 24, 64, 112, 1200), 1, 1),                              # too few blocks; too wide for a plan
+])
+def test_single_kernel_line(lib, layer, onepass, fused):
+    s = shape(*layer)
+    assert lib.fc_wino_prefer_onepass(C.byref(s)) == onepass
+    if not onepass:
+        assert lib.fc_wino_prefer_fused(C.byref(s)) == fused
+
+
+def test_layers_that_leave_the_single_kernel_path_have_a_plan(lib):
+    plan, seen = capi.WinoPlan(), 0
+    for c in (16, 17, 33, 48, 64):
+        for k in (1, 64, 65, 200, 512, 1031):
+            for n, h, w in ((1, 8, 1020), (1, 400, 1021), (3, 200, 5000), (64, 30, 31), (200, 223, 223), (4000, 7, 8)):
+                s = shape(n, c, k, h, w)
+                if not lib.fc_wino_prefer_onepass(C.byref(s)):
+                    rc = lib.fc_wino_make_plan(C.byref(s), lib.fc_wino_gemm_default_config(C.byref(s)), C.byref(plan))
+                    blocks = (n * ((h + 5) // 6) * ((w + 5) // 6) + 15) // 16 * ((k + 63) // 64)
+                    assert rc == 0 or blocks < 512, (c, k, n, h, w)
+                    seen += 1
+    assert seen > 30
