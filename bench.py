@@ -33,6 +33,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_MFMA_F32_TFLOPS = 157.3
+# fp32 products formed on the bf16 matrix cores (2.5 PFLOP/s) as six partial products each (csrc/split_mfma.h)
+PEAK_MFMA_SPLIT_TFLOPS = 2500.0 / 6
 PEAK_HBM_GBS = 8000.0
 # Measured HBM bytes per launch of the GEMM kernels (FETCH_SIZE and WRITE_SIZE of rocprofv3 --pmc, scaled by what
 # the same counters read for a plain copy): a text summary under profiles/, one line per layer and tile shape.
@@ -195,6 +197,25 @@ def takes_raw_filter_gemm(L, lay, filter_ready):
     has few tiles and the filter is not transformed beforehand: the rule fc_wino_forward applies."""
     return (lay.algo == "winograd" and lay.pipe == "staged" and not lay.fused and not filter_ready
             and lay.block_plans is None and L.wino_prefer_raw_filter_gemm(lay.plan))
+
+
+def product_peak(L, lay, filter_ready=False):
+    """Peak of the matrix instructions that form a layer's products, by the rules of the kernels' launches."""
+    if lay.algo == "im2col":
+        g = L.igemm_configs()[lay.iplan.config]
+        split = (g.waves_k <= 1 and g.bm % 64 == 0 and lay.iplan.Kred_pad >= 64 and lay.ks ** 2 <= 64 and
+                 4 * lay.N * lay.C * lay.H * lay.H < 1 << 31 and
+                 not (lay.ks == 1 and lay.st == 1 and lay.K <= 64 and lay.H * lay.H % 4 == 0 and lay.C % g.bk == 0))
+    else:
+        g = L.wino_configs()[lay.plan.gemm_config]
+        split = (lay.C * lay.K > 8192 and g.bm % 64 == 0 and g.bn % 64 == 0 and g.bk == 16 and
+                 lay.pipe != "onepass" and not takes_raw_filter_gemm(L, lay, filter_ready))
+    return PEAK_MFMA_SPLIT_TFLOPS if split else PEAK_MFMA_F32_TFLOPS
+
+
+def mean_peak(L, work, filter_ready=False):
+    """Peak of several layers' products together; work: (layer, flops)."""
+    return sum(f for _, f in work) / sum(f / product_peak(L, l, filter_ready) for l, f in work)
 
 
 def _time(L, fn, iters):
@@ -517,12 +538,13 @@ def run_workload(name, steps, warmup, o, detail=True, offline_filter=None):
             roofline["traffic_source"] = os.path.relpath(TRAFFIC_PROFILE, ROOT)
         roofline["algorithmic_bytes_per_launch_avg"] = round(
             sum(256.0 * (l.K * l.C + l.C * l.plan.T + l.K * l.plan.T) * l.repeats for l in staged) / launches_step)
-        roofline.update(achieved=round(ach, 2), frac=round(ach / PEAK_MFMA_F32_TFLOPS, 4),
+        peak = mean_peak(L, [(l, l.algorithmic()["gemm_flops"] * l.repeats) for l in staged], filter_ready)
+        roofline.update(achieved=round(ach, 2), peak=round(peak, 1), frac=round(ach / peak, 4),
                         launches=gemm_cnt, avg_launch_ms=round(gemm_ms / gemm_cnt, 5),
                         flops_per_launch_avg=gemm_flops_step / launches_step)
         if shader_clock:
-            # 256 CUs x 256 fp32 MFMA flops per clock: what the measured clock allows
-            at_clock = info["compute_units"] * 256 * shader_clock["mean_mhz"] * 1e6 / 1e12
+            # what the measured clock allows
+            at_clock = peak * shader_clock["mean_mhz"] / 2400.0
             roofline.update(peak_at_measured_clock=round(at_clock, 1), frac_at_measured_clock=round(ach / at_clock, 4))
     transforms = {}
     # online filter transforms of the staged and fused pipelines ride in the input transform's launch
@@ -594,8 +616,9 @@ def run_workload(name, steps, warmup, o, detail=True, offline_filter=None):
             igemm_events = "20 back-to-back calls per layer after the timed region, wall clock (a split reduction's second kernel included)"
         iflops = sum(l.flops * l.repeats for l in il) * (igemm_stage[1] / per_step)
         tf = iflops / (igemm_stage[0] * 1e-3) / 1e12
-        transforms["implicit_gemm"] = {"bound": "mfma", "achieved": round(tf, 2), "peak": PEAK_MFMA_F32_TFLOPS,
-                                       "unit": "TFLOP/s", "frac": round(tf / PEAK_MFMA_F32_TFLOPS, 4),
+        peak = mean_peak(L, [(l, l.flops * l.repeats) for l in il])
+        transforms["implicit_gemm"] = {"bound": "mfma", "achieved": round(tf, 2), "peak": round(peak, 1),
+                                       "unit": "TFLOP/s", "frac": round(tf / peak, 4),
                                        "launches": igemm_stage[1]}
     # the dominant kernel is the one with more time in the timed region: the implicit GEMM in the
     # ResNet-50 workloads, the staged Winograd GEMM in the VGG-16 ones
@@ -618,7 +641,7 @@ def run_workload(name, steps, warmup, o, detail=True, offline_filter=None):
         roofline = dict(transforms["implicit_gemm"], kernel=kname, traffic=tr,
                         avg_launch_ms=round(igemm_stage[0] / igemm_stage[1], 5))
         if shader_clock:
-            at_clock = info["compute_units"] * 256 * shader_clock["mean_mhz"] * 1e6 / 1e12
+            at_clock = roofline["peak"] * shader_clock["mean_mhz"] / 2400.0
             roofline.update(peak_at_measured_clock=round(at_clock, 1),
                             frac_at_measured_clock=round(roofline["achieved"] / at_clock, 4))
         if wino_gemm_line:
@@ -677,7 +700,7 @@ def run_workload(name, steps, warmup, o, detail=True, offline_filter=None):
         gf = lay.algorithmic()["gemm_flops"]
         row = {"ms": round(cand["ms"], 4), "gflops": round(lay.flops / (cand["ms"] * 1e-3) / 1e9, 1),
                "gemm_kernel_ms": round(gemm_ms, 4), "gemm_tflops": round(gf / (gemm_ms * 1e-3) / 1e12, 2),
-               "gemm_frac_mfma": round(gf / (gemm_ms * 1e-3) / 1e12 / PEAK_MFMA_F32_TFLOPS, 3)}
+               "gemm_frac_mfma": round(gf / (gemm_ms * 1e-3) / 1e12 / product_peak(L, lay), 3)}
         if cand["pipe"] == "staged":
             row.update(engine="four staged kernels, whole-layer U/V/M", tile=tile_name(g), waves="%dx%d" % (g.waves_m, g.waves_n),
                        input_tran_ms=round(st[ST_IT], 4), output_tran_ms=round(st[ST_OT], 4))
@@ -706,7 +729,7 @@ def run_workload(name, steps, warmup, o, detail=True, offline_filter=None):
             row.update(ms=round(ms, 4), gflops=round(lay.flops / (ms * 1e-3) / 1e9, 1), split_k=lay.iplan.split_k,
                        waves_over_reduction=g.waves_k,
                        gemm_tflops=round(lay.flops / (ms * 1e-3) / 1e12, 2),
-                       gemm_frac_mfma=round(lay.flops / (ms * 1e-3) / 1e12 / PEAK_MFMA_F32_TFLOPS, 3))
+                       gemm_frac_mfma=round(lay.flops / (ms * 1e-3) / 1e12 / product_peak(L, lay), 3))
         else:
             st = [L.stage_time(i)[0] / reps for i in range(4)]
             if lay.fused:      # one kernel does the GEMM and the output transform: listed under gemm
@@ -724,7 +747,7 @@ def run_workload(name, steps, warmup, o, detail=True, offline_filter=None):
                 "pipeline": lay.pipe, "ms": round(total, 4),
                 "gflops": round(lay.flops / (total * 1e-3) / 1e9, 1),
                 "gemm_tflops": round(a["gemm_flops"] / (st[ST_GEMM] * 1e-3) / 1e12, 2),
-                "gemm_frac_mfma": round(a["gemm_flops"] / (st[ST_GEMM] * 1e-3) / 1e12 / PEAK_MFMA_F32_TFLOPS, 3),
+                "gemm_frac_mfma": round(a["gemm_flops"] / (st[ST_GEMM] * 1e-3) / 1e12 / product_peak(L, lay, filter_ready), 3),
                 "input_tran_gbs": round((a["it_bytes"] + (0 if st[ST_KT] or raw_gemm else a["kt_bytes"])) / (st[ST_IT] * 1e-3) / 1e9, 0)
                 if st[ST_IT] else None,
                 "output_tran_gbs": round(a["ot_bytes"] / (st[ST_OT] * 1e-3) / 1e9, 0) if st[ST_OT] else None,
