@@ -208,7 +208,8 @@ def product_peak(L, lay, filter_ready=False):
                  not (lay.ks == 1 and lay.st == 1 and lay.K <= 64 and lay.H * lay.H % 4 == 0 and lay.C % g.bk == 0))
     else:
         g = L.wino_configs()[lay.plan.gemm_config]
-        split = (lay.C * lay.K > 8192 and g.bm % 64 == 0 and g.bn % 64 == 0 and g.bk == 16 and
+        split = (lay.C > 48 and lay.C * lay.K > 8192 and g.bm % 64 == 0 and g.bn % 64 == 0 and g.bk == 16 and
+                 (g.bm * g.bn > 64 * 64 or lay.C >= 160 or 256.0 * (lay.C + lay.K) * lay.plan.T_pad <= 256e6) and
                  lay.pipe != "onepass" and not takes_raw_filter_gemm(L, lay, filter_ready))
     return PEAK_MFMA_SPLIT_TFLOPS if split else PEAK_MFMA_F32_TFLOPS
 

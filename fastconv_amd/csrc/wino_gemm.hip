@@ -458,12 +458,18 @@ extern "C" int fc_wino_gemm_get_config(int id, fc_gemm_config *cfg) {
     return FC_OK;
 }
 
-static bool splits(long C, long K, const fc_gemm_config &c) {
-    return C * K > 8192 && c.bm % 64 == 0 && c.bn % 64 == 0 && c.bk == 16;
-}
+// Layers whose GEMM is bound by memory stay on fp32 instructions, which fetch 16 bytes a lane: up to 48 input channels
+// (fp32 / split: 29 -> 364 channels, 900 tiles 18.0 us / 18.4, 16 -> 700, 1089 tiles 28.3 / 33.5, 48 -> 512, 3136 tiles
+// 105 / 112; 64 -> 256, 1444 tiles 29.0 / 23.2), and with 64x64 tiles, whose operands are read most often, up to 160
+// where V and M outgrow the last-level cache (64 -> 160, 4900 tiles, 281 MB 84.7 / 93.9, but 2500 tiles, 143 MB 38.9 /
+// 31.8; 128 -> 300, 650 MB 250 / 261; 192 -> 300, 747 MB 343 / 322).
+static bool has_split_products(long C, long K) { return C > 48 && C * K > 8192; }
 
 bool fc_wino_gemm_splits(const fc_wino_plan *plan) {
-    return splits(plan->shape.C, plan->shape.K, kConfigs[plan->gemm_config]);
+    const fc_gemm_config &c = kConfigs[plan->gemm_config];
+    const long C = plan->shape.C, K = plan->shape.K;
+    if (!has_split_products(C, K) || c.bm % 64 != 0 || c.bn % 64 != 0 || c.bk != 16) return false;
+    return c.bm * c.bn > 64 * 64 || C >= 160 || 256.0 * (double)(C + K) * (double)plan->T_pad <= 256e6;
 }
 
 // Cost model behind the untuned choice: padded multiply-adds, divided by a rate per tile shape
@@ -484,7 +490,7 @@ extern "C" int fc_wino_gemm_default_config(const fc_conv_shape *s) {
     static_assert(sizeof(kRate) / sizeof(kRate[0]) == sizeof(kConfigs) / sizeof(kConfigs[0]), "one rate per configuration");
     const int OH = fc_out_dim(s->H, s->pt, s->pb, 3, 1), OW = fc_out_dim(s->W, s->pl, s->pr, 3, 1);
     const double T = (double)s->N * ((OH + 5) / 6) * ((OW + 5) / 6);
-    const bool fewChannels = (long)s->C * s->K <= 8192;
+    const bool fewChannels = !has_split_products(s->C, s->K);
     int best = 0;
     double bestCost = 1e300;
     for (int id = 0; id < kNumConfigs; id++) {
