@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdio>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "fc_internal.h"
@@ -525,9 +526,8 @@ __global__ __launch_bounds__(TL::THREADS, TL::MIN_WAVES) void igemm_conv_kernel(
 // The same layer on the bf16 matrix cores at fp32 accuracy (see split_mfma.h), for inputs below 2 GiB.  A wavefront
 // takes 64 output channels or 64 pixels x 8 reduction rows at a time, a lane one channel or pixel: 8 loads through
 // buffer resources, a stage ahead, and one 16-byte word to LDS per part.  A lane's pixel is the same in every block it takes.
-// Bound by LDS for 64x64 tiles (288 cycles of a CU's LDS a stage, 192 of its matrix cores; 128x128: 576 and 768).
-// Measured at batch 32, fp32 instructions -> this: 256 -> 256 3x3/2 at 28x28 81.5 -> 76.2 us, 7x7/2 stem 91.4 -> 78.7,
-// 512 -> 2048 1x1 at 7x7 39.4 -> 31.0, 64 -> 64 3x3 at 56x56 73.1 -> 61.0.
+// Measured at batch 32, fp32 instructions -> this, 64x64 tiles: 256 -> 256 3x3/2 at 28x28 82.5 -> 75.4 us, 7x7/2 stem
+// 91.3 -> 81.4, 512 -> 2048 1x1 at 7x7 39.2 -> 30.8, 64 -> 64 3x3 at 56x56 71.7 -> 60.7; 128x128: 256 -> 256 1x1 at 56x56 113 -> 83.
 template <class TL>
 struct IgSplit {
     static constexpr int A_WAVES = 2 * TL::BM_ / 64, B_WAVES = 2 * TL::BN_ / 64, WAVES = TL::THREADS / 64;   // blocks of a stage
@@ -536,7 +536,8 @@ struct IgSplit {
     static constexpr int A_LD = (A_WAVES + WAVES - 1) / WAVES, B_LD = (B_WAVES + WAVES - 1) / WAVES;
     typedef fc_split_stage<TL::BM_, TL::BN_> Stage;
     static constexpr int LDS_WORDS = 2 * Stage::WORDS;
-    static constexpr int MIN_WAVES = TL::BM_ * TL::BN_ > 128 * 128 ? 1 : TL::BM_ * TL::BN_ == 64 * 64 ? 4 : 3;
+    // wavefronts per SIMD the two sums leave registers for
+    static constexpr int MIN_WAVES = TL::MI * TL::NI > 4 ? 1 : TL::MI * TL::NI > 1 ? 2 : 4;
     static_assert(TL::BM_ % 64 == 0 && TL::BN_ % 64 == 0 && TL::BK_ == 16, "a wavefront fetches 64 rows or columns x 8 of the reduction");
     static_assert(B_LD == 1 || B_WAVES % WAVES == 0, "no part-filled second block");
     static_assert(B_LD == 1 || TL::THREADS % TL::BN_ == 0, "one pixel per lane");
@@ -662,13 +663,9 @@ __global__ __launch_bounds__(TL::THREADS, IgSplit<TL>::MIN_WAVES) void igemm_con
         }
     };
 
-    floatx16 acc[MI][NI];
-#pragma unroll
-    for (int mi = 0; mi < MI; mi++)
-#pragma unroll
-        for (int ni = 0; ni < NI; ni++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[mi][ni][i] = 0.f;
+    floatx16 acc[MI][NI], small[MI][NI];
+    fc_zero<MI, NI>(acc);
+    fc_zero<MI, NI>(small);
     const int aFrag = lrow * BM + wm0 + lcol, bFrag = 3 * A_PLANE + lrow * BN + wn0 + lcol;
 
     fetch(sBegin);
@@ -678,21 +675,23 @@ __global__ __launch_bounds__(TL::THREADS, IgSplit<TL>::MIN_WAVES) void igemm_con
     for (int s = sBegin; s < sEnd; s++) {
         const int buf = (s - sBegin) & 1;
         const fc_uintx4 *cur = smem + buf * WORDS;
-        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc);
+        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc, small);
         if (s + 1 < sEnd) {
             park(buf ^ 1);
             if (s + 2 < sEnd) fetch(s + 2);
         }
         __syncthreads();
     }
+    fc_add<MI, NI>(acc, small);
     if (__syncthreads_or(fc_not_finite<MI, NI>(acc))) {
         // 64x64 at a time, which leaves the registers to the loop above
-        typedef IgTile<64, 64, 16, 2, TL::THREADS / 128> Sub;
+        typedef std::conditional_t<TL::THREADS == 512, TL, IgTile<64, 64, 16, 2, TL::THREADS / 128>> Sub;
         static_assert(Sub::THREADS == TL::THREADS && Sub::LDS_BYTES <= 16 * S::LDS_WORDS, "same workgroup");
         float *const f = reinterpret_cast<float *>(smem);
-        for (int q = 0; q < (BM / 64) * (BN / 64); q++)
-            ig_tile<Sub, MODE>(p, kb * (BM / 64) + q / (BN / 64), pb * (BN / 64) + q % (BN / 64),
-                               reinterpret_cast<float (*)[16 * 64]>(f), reinterpret_cast<float (*)[16 * 64]>(f + 2 * 16 * 64));
+        constexpr int QM = BM / Sub::BM_, QN = BN / Sub::BN_;
+        for (int q = 0; q < QM * QN; q++)
+            ig_tile<Sub, MODE>(p, kb * QM + q / QN, pb * QN + q % QN, reinterpret_cast<float (*)[16 * Sub::BM_]>(f),
+                               reinterpret_cast<float (*)[16 * Sub::BN_]>(f + 2 * 16 * Sub::BM_));
         return;
     }
     ig_store_tile<TL>(acc, p, kb, pb, wm0, wn0, lrow, lcol);
@@ -717,6 +716,7 @@ __global__ __launch_bounds__(256) void igemm_reduce_kernel(const float *__restri
 }
 
 typedef IgTile<128, 128, 16, 2, 2> Ig0;
+typedef IgTile<128, 128, 16, 2, 4> Ig0Split;      // eight wavefronts, as in wino_gemm.hip
 typedef IgTile<64, 128, 16, 1, 2> Ig1;
 typedef IgTile<128, 64, 16, 2, 1> Ig2;
 typedef IgTile<64, 64, 16, 2, 2> Ig3;
@@ -747,15 +747,17 @@ void launch(fc_context *ctx, IgemmParams &p) {
     const bool tapMajor = p.C % TL::BK_ == 0;      // the order fc_igemm_pack_filter laid the filter out in
     const dim3 block(TL::THREADS);
     if constexpr (TL::BM_ % 64 == 0) {
+        typedef std::conditional_t<std::is_same<TL, Ig0>::value, Ig0Split, TL> TS;
+        const dim3 splitBlock(TS::THREADS);
         // Bf16 matrix cores (a pointwise layer is a tap-major one whose only tap is inside) for inputs below 2 GiB, but
         // not for a pointwise layer of up to 64 output channels: that is bound by reading x, which the fp32 kernel does
         // 16 bytes a lane (256 -> 64 channels at 56x56, batch 32: 35.8 us against 37.6; 64 -> 256: 34.4 against 32.6);
         // nor for a reduction of two or three stages, bound by its gathers and stores (3 -> 64 channels 3x3 at 224x224,
         // batch 32: 129 us against 139).
         const bool split = buffer && p.Kred_pad >= 64 && !(pointwise && p.K <= 64);
-        if (split && tapMajor && inside) { igemm_conv_kernel<TL, IG_TAP_INSIDE, true><<<grid, block, 0, ctx->stream>>>(p); return; }
-        if (split && tapMajor && p.kh * p.kw <= 64) { igemm_conv_kernel<TL, IG_TAP_MASKED, true><<<grid, block, 0, ctx->stream>>>(p); return; }
-        if (split && p.kh * p.kw <= 64) { igemm_conv_kernel<TL, IG_BUF_MASKED, true><<<grid, block, 0, ctx->stream>>>(p); return; }
+        if (split && tapMajor && inside) { igemm_conv_kernel<TS, IG_TAP_INSIDE, true><<<grid, splitBlock, 0, ctx->stream>>>(p); return; }
+        if (split && tapMajor && p.kh * p.kw <= 64) { igemm_conv_kernel<TS, IG_TAP_MASKED, true><<<grid, splitBlock, 0, ctx->stream>>>(p); return; }
+        if (split && p.kh * p.kw <= 64) { igemm_conv_kernel<TS, IG_BUF_MASKED, true><<<grid, splitBlock, 0, ctx->stream>>>(p); return; }
     }
     if (pointwise) igemm_conv_kernel<TL, IG_POINTWISE><<<grid, block, 0, ctx->stream>>>(p);
     else if (buffer && tapMajor && inside) igemm_conv_kernel<TL, IG_TAP_INSIDE><<<grid, block, 0, ctx->stream>>>(p);
@@ -800,9 +802,9 @@ extern "C" int fc_igemm_default_config(const fc_conv_shape *s) {
         if (cost < bestCost) { bestCost = cost; best = id; }
     }
     // On the bf16 matrix cores 128x128 writes and reads the least LDS per product.  It takes over from 64x64 where the
-    // reduction is long enough to pay for its longer start, the grid is at least two rounds of its three workgroups per
+    // reduction is long enough to pay for its longer start, the grid is at least three rounds of its two workgroups per
     // CU without a split, and it pads no more.  At batch 32 and the like:
-    // 256 -> 256 1x1 at 56x56 80 us against 92, 85 -> 128 3x3 at 150x150 303 against 403; with 32 rows 27.5 against 22.7.
+    // 256 -> 256 1x1 at 56x56 83 us against 95, 85 -> 128 3x3 at 150x150 337 against 420; with 32 rows 27.5 against 22.7.
     if (best == 3 && Kr >= 256 && ceil(M / 128) * 128 == ceil(M / 64) * 64 && ceil(M / 128) * ceil(Np / 128) >= 1536) best = 0;
     // A layer that this tile shape can only fill the chip with by splitting the reduction over workgroups
     // (a pass of partial sums through memory and a second launch) goes to the kernels that split it inside

@@ -93,45 +93,64 @@ __device__ __forceinline__ void fused_products(const FusedParams &p, int wave, i
 }
 
 // The same on the bf16 matrix cores, in the order of the staged pipeline's GEMM (see split_mfma.h): 16 channels at a time,
-// a lane splits the 8 channels of its row and column.  The split is the larger part of the time: the operands of a
-// 32x32 block are split by every block that uses them.  C_pad is a multiple of 16.
+// a lane splits the 8 channels of its row and column.  One frequency after another, so that only one has its second sum in
+// registers.  The split is the larger part of the time: the operands of a 32x32 block are split by every block that uses
+// them.  C_pad is a multiple of 16.
 __device__ __forceinline__ void fused_split_products(const FusedParams &p, int wave, int lrow, int lcol, int kb, int tb, floatx16 (&acc)[kFW]) {
     const int wv = __builtin_amdgcn_readfirstlane(wave);
     const size_t planeU = (size_t)p.C_pad * p.K_pad, planeV = (size_t)p.C_pad * p.T_pad;
     const float *ub = p.U + (size_t)(wv * kFW) * planeU + (size_t)kb * 32;
     const float *vb = p.V + (size_t)(wv * kFW) * planeV + (size_t)tb * 32;
-    uint32_t offU = 4u * (8u * lrow * p.K_pad + lcol), offV = 4u * (8u * lrow * (uint32_t)p.T_pad + lcol);
+    const uint32_t offU = 4u * (8u * lrow * p.K_pad + lcol), offV = 4u * (8u * lrow * (uint32_t)p.T_pad + lcol);
     const uint32_t rowU = 4u * p.K_pad, rowV = 4u * (uint32_t)p.T_pad;
-#pragma unroll
-    for (int f = 0; f < kFW; f++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) acc[f][i] = 0.f;
+    const int nStages = p.C_pad / 16;
     float u[2][8], v[2][8];
+    uint32_t atU, atV;      // of the next stage of a frequency
     auto fetch = [&](int f, float (&a)[8], float (&b)[8]) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            a[i] = ldg(ub + f * planeU, offU + i * rowU);
-            b[i] = ldg(vb + f * planeV, offV + i * rowV);
+            a[i] = ldg(ub + f * planeU, atU + i * rowU);
+            b[i] = ldg(vb + f * planeV, atV + i * rowV);
         }
+        atU += 16u * rowU;
+        atV += 16u * rowV;
     };
-    const int nStages = p.C_pad / 16;
+    floatx16 sum[1][1], small[1][1];
+    auto stage = [&](const float (&a)[8], const float (&b)[8]) __attribute__((always_inline)) {
+        fc_uintx4 as[3], bs[3];
+        fc_split8(a, as, 1);
+        fc_split8(b, bs, 1);
+        fc_split_products<1, 1, 1, 1>(as, bs, sum, small);
+    };
+    atU = offU;
+    atV = offV;
     fetch(0, u[0], v[0]);
-    for (int s = 0; s < nStages; s++) {
 #pragma unroll
-        for (int f = 0; f < kFW; f++) {
-            // the next frequency, or the first of the next 16 channels (the last ones again at the end)
-            if (f + 1 == kFW && s + 1 < nStages) {
-                offU += 16u * rowU;
-                offV += 16u * rowV;
-            }
-            fetch((f + 1) % kFW, u[(f + 1) & 1], v[(f + 1) & 1]);
-            fc_uintx4 a[3], b[3];
-            fc_split8(u[f & 1], a, 1);
-            fc_split8(v[f & 1], b, 1);
-            floatx16 one[1][1] = {{acc[f]}};
-            fc_split_products<1, 1, 1, 1>(a, b, one);
-            acc[f] = one[0][0];
+    for (int f = 0; f < kFW; f++) {
+        fc_zero<1, 1>(sum);
+        fc_zero<1, 1>(small);
+        // each stage is fetched one ahead, after the last the first of the next frequency (of the last one again at the end)
+        int s = 0;
+        for (; s + 2 < nStages; s += 2) {
+            fetch(f, u[1], v[1]);
+            stage(u[0], v[0]);
+            fetch(f, u[0], v[0]);
+            stage(u[1], v[1]);
         }
+        if (s + 2 == nStages) {
+            fetch(f, u[1], v[1]);
+            stage(u[0], v[0]);
+#pragma unroll
+            for (int i = 0; i < 8; i++) { u[0][i] = u[1][i]; v[0][i] = v[1][i]; }
+        }
+        atU = offU;
+        atV = offV;
+        fetch(min(f + 1, kFW - 1), u[1], v[1]);
+        stage(u[0], v[0]);
+#pragma unroll
+        for (int i = 0; i < 8; i++) { u[0][i] = u[1][i]; v[0][i] = v[1][i]; }
+        fc_add<1, 1>(sum, small);
+        acc[f] = sum[0][0];
     }
 }
 

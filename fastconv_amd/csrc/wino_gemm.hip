@@ -6,6 +6,7 @@
 // as straight 16-byte copies and LDS -> registers as conflict-free dword reads.
 // Layers of more channels run on the bf16 matrix cores instead, at the same accuracy (split_tile below).
 #include <cmath>
+#include <type_traits>
 #include <utility>
 
 #include "fc_internal.h"
@@ -243,10 +244,10 @@ __device__ __forceinline__ void gemm_tile(const float *__restrict__ U, const flo
 
 // The same tile on the bf16 matrix cores (see split_mfma.h): a wavefront takes 8 consecutive channels of 64 rows or
 // columns at a time, each lane one of them, splits the 8 floats it has fetched a stage ahead and writes one 16-byte
-// word per part.  Bound by the matrix cores and LDS (a 128x128 stage: 768 cycles of products, 48 KB read and 24 KB
-// written); the split runs beside the products of the other wavefronts, of which a SIMD needs three.  128x128 tiles,
-// batch 32, fp32 instructions -> this: 256 -> 256 channels at 56x56 218 -> 161 us (166 TFLOP/s), 512 -> 512 at 28x28
-// 223 -> 162, 128 -> 128 at 112x112 225 -> 181 (bound by memory, 4.2 TB/s); error against 64 bits 0.83 of the fp32 one's.
+// word per part.  The split runs beside the products of the other wavefronts.  128x128 tiles take eight wavefronts of 64x32
+// (four wavefronts of 64x64: 179 us where eight take 166, as two a SIMD do not cover each other's barriers).
+// Batch 32, fp32 instructions -> this: 256 -> 256 channels at 56x56 224 -> 166 us, 512 -> 512 at 28x28 239 -> 163,
+// 128 -> 128 at 112x112 220 -> 188 (bound by memory); 64x64 tiles: 512 -> 512 at 14x14 90 -> 71.
 // Spreading the split between the products by hand (sched_group_barrier) gained nothing.
 template <class TL>
 struct SplitTile {
@@ -306,13 +307,9 @@ __device__ __forceinline__ void split_tile(const float *__restrict__ U, const fl
         for (int j = 0; j < ITEMS; j++) fc_split8(r[j], smem + buf * WORDS + dst[j] + lane, isA[j] ? A_PLANE : B_PLANE);
     };
 
-    floatx16 acc[MI][NI];
-#pragma unroll
-    for (int mi = 0; mi < MI; mi++)
-#pragma unroll
-        for (int ni = 0; ni < NI; ni++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[mi][ni][i] = 0.f;
+    floatx16 acc[MI][NI], small[MI][NI];
+    fc_zero<MI, NI>(acc);
+    fc_zero<MI, NI>(small);
 
     fetch(false);
     park(0);
@@ -322,23 +319,24 @@ __device__ __forceinline__ void split_tile(const float *__restrict__ U, const fl
     int s = 0;
     for (; s + 1 < nStages; s++) {
         const fc_uintx4 *cur = smem + (s & 1) * WORDS;
-        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc);
+        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc, small);
         park((s + 1) & 1);
         fetch(s + 2 < nStages);
         __syncthreads();
     }
     {
         const fc_uintx4 *cur = smem + (s & 1) * WORDS;
-        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc);
+        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc, small);
         __syncthreads();
     }
+    fc_add<MI, NI>(acc, small);
     if (__syncthreads_or(fc_not_finite<MI, NI>(acc))) {
         // 64x64 at a time, which leaves the registers to the loop above
-        typedef TileCfg<64, 64, 16, 2, TL::THREADS / 128> Sub;
+        typedef std::conditional_t<TL::THREADS == 512, TL, TileCfg<64, 64, 16, 2, TL::THREADS / 128>> Sub;
         static_assert(Sub::THREADS == TL::THREADS && Sub::LDS_BYTES <= 16 * S::LDS_WORDS, "same workgroup");
-        for (int q = 0; q < (BM / 64) * (BN / 64); q++)
-            gemm_tile<Sub>(U, V, M, K_pad, C_pad, T_pad, f, kb * (BM / 64) + q / (BN / 64), tb * (BN / 64) + q % (BN / 64),
-                           reinterpret_cast<float *>(smem));
+        constexpr int QM = BM / Sub::BM_, QN = BN / Sub::BN_;
+        for (int q = 0; q < QM * QN; q++)
+            gemm_tile<Sub>(U, V, M, K_pad, C_pad, T_pad, f, kb * QM + q / QN, tb * QN + q % QN, reinterpret_cast<float *>(smem));
         return;
     }
     store_tile<TL>(acc, M, K_pad, T_pad, f, kb, tb, wm0, wn0, lrow, lcol);
@@ -358,9 +356,10 @@ __device__ __forceinline__ void decode_tile(int b, int nKB, int nTB, int *f, int
     *kb = rem - *tb * nKB;
 }
 
-// SPLIT: on the bf16 matrix cores; three wavefronts per SIMD (two cost 10-15 %) where the tile leaves the registers.
+// SPLIT: on the bf16 matrix cores; two wavefronts per SIMD where the tile leaves the registers (the two sums of 64x64 per
+// wavefront and the operands take 224 of 256).
 template <class TL, bool SPLIT>
-__global__ __launch_bounds__(TL::THREADS, SPLIT && TL::BM_ * TL::BN_ <= 128 * 128 ? 3 : 1) void wino_gemm_kernel(
+__global__ __launch_bounds__(TL::THREADS, SPLIT && TL::BM_ * TL::BN_ <= 128 * 128 ? 2 : 1) void wino_gemm_kernel(
     const float *__restrict__ U, const float *__restrict__ V, float *__restrict__ M, int K_pad, int C_pad, int T_pad, int nKB, int nTB) {
     int f, kb, tb;
     decode_tile(blockIdx.x, nKB, nTB, &f, &kb, &tb);
@@ -398,6 +397,7 @@ __global__ __launch_bounds__(BIG::THREADS) void wino_gemm_tail_kernel(const floa
 }
 
 typedef TileCfg<128, 128, 16, 2, 2> Cfg0;
+typedef TileCfg<128, 128, 16, 2, 4> Cfg0Split;      // eight wavefronts: two sums of 64x64 each leave a SIMD two wavefronts, of 64x32 four
 typedef TileCfg<64, 128, 16, 1, 2> Cfg1;
 typedef TileCfg<128, 64, 16, 2, 1> Cfg2;
 typedef TileCfg<64, 64, 16, 2, 2> Cfg3;
@@ -476,8 +476,8 @@ bool fc_wino_gemm_splits(const fc_wino_plan *plan) {
 // relative to 128x128x16 and by how evenly the grid fills the workgroup slots of the chip.  The
 // rates start from what each shape sustains on large layers (256 -> 256 channels at 56x56 and
 // 512 -> 512 at 28x28, batch 32).  The shapes of 64 and more run on the bf16 matrix cores
-// (128x128: 161 us against 220 with fp32 instructions on the first of these; 64x64: 195 against
-// 232), where the large tile is the furthest ahead: it writes and reads the least LDS per product.
+// (128x128: 166 us against 224 with fp32 instructions on the first of these; 64x64: 199 against
+// 229), where the large tile is the furthest ahead: it writes and reads the least LDS per product.
 // 64x64 is level with it where it pads less (512 channels at 14x14: 68 us both) and ahead on
 // small grids; the shapes with a 32 stay on fp32 instructions, for layers whose 64-wide tile
 // would be mostly padding (512 channels at 28x28, batch 1: 14.7 us against 21).  Layers of few
@@ -498,13 +498,13 @@ extern "C" int fc_wino_gemm_default_config(const fc_conv_shape *s) {
         const double kp = ceil((double)s->K / c.bm) * c.bm, tp = ceil(T / c.bn) * c.bn;
         const double cp = ceil((double)s->C / c.bk) * c.bk;
         const double blocks = 64.0 * (kp / c.bm) * (tp / c.bn);
-        const double slots = 256.0 * (c.bm * c.bn > 128 * 128 || c.bk == 32 ? 2 : id == 0 && !fewChannels ? 3 : 4);
+        const double slots = 256.0 * (c.bm * c.bn > 128 * 128 || c.bk == 32 ? 2 : id == 0 && !fewChannels ? 2 : 4);
         // the time of a launch is nearly linear in its tile count: a partly filled last round costs
         // little, and nothing for configuration 0 on fp32 instructions, whose last round runs as quartered tiles
         double fill = blocks / (ceil(blocks / slots) * slots);
         if (id == 0 && fewChannels && blocks > slots) fill = 1.0;
-        // the large tile on the bf16 matrix cores needs its three workgroups per CU to hide their barriers
-        // (256 -> 256 channels at 56x56, one image: 128 workgroups, 15.6 us against 11.4 for 64x64)
+        // the large tile on the bf16 matrix cores needs its two workgroups per CU to hide their barriers
+        // (256 -> 256 channels at 56x56, one image: 128 workgroups, 16.7 us against 11.4 for 64x64)
         if (id == 0 && !fewChannels && blocks < slots) fill -= 2.0 * (1.0 - fill);
         const double cost = kp * tp * cp / ((fewChannels ? kFp32Rate : kRate)[id] * (0.8 + 0.2 * fill));
         if (cost < bestCost) { bestCost = cost; best = id; }
@@ -534,7 +534,7 @@ extern "C" int fc_wino_gemm(fc_context *ctx, const fc_wino_plan *plan, const flo
 #define FC_LAUNCH(T) (split ? launch<T, true>(ctx, plan, U_dev, V_dev, M_dev) : launch<T>(ctx, plan, U_dev, V_dev, M_dev))
     switch (plan->gemm_config) {
         case 0:
-            if (split) launch<Cfg0, true>(ctx, plan, U_dev, V_dev, M_dev);
+            if (split) launch<Cfg0Split, true>(ctx, plan, U_dev, V_dev, M_dev);
             else launch_with_tail<Cfg0, Cfg3>(ctx, plan, U_dev, V_dev, M_dev);
             break;
         case 1: FC_LAUNCH(Cfg1); break;

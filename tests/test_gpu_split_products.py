@@ -7,9 +7,12 @@ from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# Of nine partial products three are left out, together below 2^-22 of a product; the six kept are summed in fp32
+# Of nine partial products three are left out, together below 2^-24 of a product; the six kept are summed in fp32
 # like the fp32 path's, whose own bound over n terms is n * 2^-24 of the sum of the magnitudes.
-EPS_PRODUCT, EPS_SUM = 2.0 ** -22, 2.0 ** -24
+EPS_PRODUCT, EPS_SUM = 2.0 ** -24, 2.0 ** -24
+# A sum of one term: what is left out, a last place of the last addition, which the matrix core does not round to nearest
+# (2^-23), and five additions of parts of 2^-8 and less.
+EPS_SINGLE = 3.1 * 2.0 ** -24
 
 
 @pytest.fixture(scope="module")
@@ -52,24 +55,82 @@ def test_implicit_gemm_split_products(lib, shp):
         assert (np.abs(lib.implicit_gemm_conv(cshape(s), x, w, config=cfg.id) - truth) <= tol).all(), cfg.id
 
 
-@pytest.mark.parametrize("C,K,T", [(16, 513, 9), (129, 64, 65), (100, 130, 129), (256, 33, 200)])
+def tiles_in_a_row(C, K, T):
+    return cshape(O.shape(1, C, 6, 6 * T, K)) if T <= 170 else cshape(O.shape(T // 100, C, 60, 60, K))
+
+
+def winograd_gemm(lib, plan, U, V):
+    mark = lib.mark()
+    M = lib.alloc(plan.M_bytes)
+    lib.wino_gemm(plan, lib.upload(U), lib.upload(V), M)
+    got = lib.download(M, (64, plan.K_pad, plan.T_pad))
+    lib.release(mark)
+    return got
+
+
+@pytest.mark.parametrize("C,K,T", [(64, 129, 9), (129, 64, 65), (100, 130, 129), (256, 33, 200), (160, 64, 65)])
 def test_winograd_gemm_split_products(lib, C, K, T):
-    """C*K above 8192: M = U * V per frequency against fp64, every tile shape; T tiles in one row of an image."""
-    s = cshape(O.shape(1, C, 6, 6 * T, K)) if T <= 170 else cshape(O.shape(T // 100, C, 60, 60, K))
+    """More than 48 channels and C*K above 8192: M = U * V per frequency against fp64, every tile shape; T tiles in one
+    row of an image."""
+    s = tiles_in_a_row(C, K, T)
     for cfg in lib.wino_configs():
         plan = lib.wino_plan(s, cfg.id)
-        mark = lib.mark()
         U = O.rng_uniform(C, (64, plan.C_pad, plan.K_pad))
         V = O.rng_uniform(K, (64, plan.C_pad, plan.T_pad))
-        M = lib.alloc(plan.M_bytes)
         print("split products", (C, K, T), cfg.bm, cfg.bn, cfg.bk, flush=True)
-        lib.wino_gemm(plan, lib.upload(U), lib.upload(V), M)
-        got = lib.download(M, (64, plan.K_pad, plan.T_pad))
-        lib.release(mark)
+        got = winograd_gemm(lib, plan, U, V)
         for f in (0, 9, 63):
             a, b = U[f].T.astype(np.float64), V[f].astype(np.float64)
             tol = (EPS_PRODUCT + (plan.C_pad + 40) * EPS_SUM) * (np.abs(a) @ np.abs(b))
             assert (np.abs(got[f] - a @ b) <= tol).all(), (cfg.id, f)
+
+
+def test_sums_of_one_term_keep_fp32_accuracy(lib):
+    """One channel of the filter is not zero: a partial product left out, or a first part that is cut off and not
+    rounded, shows in every result (test_split_products.py)."""
+    C, K, T = 160, 130, 129
+    s = tiles_in_a_row(C, K, T)
+    for cfg in lib.wino_configs():
+        plan = lib.wino_plan(s, cfg.id)
+        U = np.zeros((64, plan.C_pad, plan.K_pad), np.float32)
+        k = np.arange(plan.K_pad)
+        U[:, k % C, k] = O.rng_uniform(1, (64, plan.K_pad))
+        V = O.rng_uniform(2, (64, plan.C_pad, plan.T_pad))
+        print("one term", cfg.bm, cfg.bn, cfg.bk, flush=True)
+        got = winograd_gemm(lib, plan, U, V)
+        exact = U[:, k % C, k].astype(np.float64)[:, :, None] * V[:, k % C]
+        assert (np.abs(got - exact) <= EPS_SINGLE * np.abs(exact)).all(), cfg.id
+    s = O.shape(2, 64, 13, 11, 130, 1, 1, 1, 1, 0)
+    x, w = O.make_inputs(s, seed=7)
+    k = np.arange(s.K)
+    keep = w[k, k % s.C, 0, 0]
+    w[:] = 0.0
+    w[k, k % s.C, 0, 0] = keep
+    exact = keep.astype(np.float64)[None, :, None, None] * x[:, k % s.C]
+    for cfg in lib.igemm_configs():
+        print("one term, implicit gemm", cfg.bm, cfg.bn, cfg.waves_k, flush=True)
+        assert (np.abs(lib.implicit_gemm_conv(cshape(s), x, w, config=cfg.id) - exact) <= EPS_SINGLE * np.abs(exact)).all(), cfg.id
+
+
+def test_sums_with_few_terms_are_no_less_exact_than_with_fp32_products(lib):
+    """n of 256 channels of the filter are not zero: the 2-norm error of every tile shape against 64 bits is no larger
+    than that of the shapes that run on fp32 instructions (a tenth for the single term, whose parts are not rounded alike)."""
+    C, K, T = 256, 130, 129
+    s = tiles_in_a_row(C, K, T)
+    for n in (1, 4, 16, 64, 256):
+        err = {}
+        for cfg in lib.wino_configs():
+            plan = lib.wino_plan(s, cfg.id)
+            rng = np.random.default_rng(n)
+            U = rng.standard_normal((64, plan.C_pad, plan.K_pad), np.float32)
+            U *= np.argsort(rng.random((C, plan.K_pad)), axis=0) < n
+            V = rng.standard_normal((64, plan.C_pad, plan.T_pad), np.float32)
+            print("terms", n, cfg.bm, cfg.bn, cfg.bk, flush=True)
+            got = winograd_gemm(lib, plan, U, V)
+            exact = U[::9].transpose(0, 2, 1).astype(np.float64) @ V[::9].astype(np.float64)
+            err[cfg.bm % 64 == 0 and cfg.bn % 64 == 0 and cfg.bk == 16, cfg.id] = np.linalg.norm(got[::9] - exact) / np.linalg.norm(exact)
+        fp32 = min(e for (split, _), e in err.items() if not split)
+        assert all(e <= (1.1 if n == 1 else 1.0) * fp32 for (split, _), e in err.items() if split), (n, err)
 
 
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, np.finfo(np.float32).max])
