@@ -682,7 +682,7 @@ __global__ __launch_bounds__(TL::THREADS, IgSplit<TL>::MIN_WAVES) void igemm_con
         }
         __syncthreads();
     }
-    fc_add<MI, NI>(acc, small);
+    fc_join<MI, NI>(acc, small);
     if (__syncthreads_or(fc_not_finite<MI, NI>(acc))) {
         // 64x64 at a time, which leaves the registers to the loop above
         typedef std::conditional_t<TL::THREADS == 512, TL, IgTile<64, 64, 16, 2, TL::THREADS / 128>> Sub;

@@ -12,11 +12,14 @@
 // zero: 1.03 for n = 1, 0.67 for 4, 0.46 for 16, 0.38 for 64, 0.31 for 256.  (All six in one sum: 1.37, 1.82, 1.87, 1.47,
 // 0.82, and 10 % less time with 128x128 tiles, 2 % with 64x64 ones; the first part cut off instead of rounded: 1.64 for n = 1.)
 // Why: v_mfma_f32_32x32x2_f32 does 32 multiply-adds a cycle and SIMD unit, v_mfma_f32_32x32x16_bf16 512, so for 16384 six
-// passes of it take 192 cycles where the fp32 ones take 512, and the split costs about 6 vector instructions an element,
+// passes of it take 192 cycles where the fp32 ones take 512, and the split costs about 7 vector instructions an element,
 // which run beside the bf16 matrix core.
-// An infinity has no such sum (inf - inf), so a tile whose result is not finite throughout is computed again with fp32
-// instructions by the kernels that use this: NaN and infinities come out as they always did.  Parts below the smallest
-// bf16 number are lost: operands keep full precision down to 2^-110 (1e-33).
+// Operands are multiplied by 2^24 first and sums by 2^-48 last: the parts of the smallest subnormal float are then normal
+// bf16 numbers, and the split is exact over the whole lower range (without it parts below 2^-133 are lost, 2^-10 of an
+// operand of 2^-124).  One multiplication an element, 1 to 3 % of a launch.
+// An infinity has no such sum (inf - inf), and scaled operands from 2^104 and sums from 2^80 on overflow, so a tile whose
+// result is not finite throughout is computed again with fp32 instructions by the kernels that use this: NaN, infinities
+// and large values come out as they always did.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,11 +29,13 @@ typedef __bf16 fc_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float fc_floatx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t fc_uintx4 __attribute__((ext_vector_type(4)));
 
+constexpr float kSplitScale = 16777216.f, kSplitUnscale = 1.f / (kSplitScale * kSplitScale);      // 2^24, 2^-48
+
 // Two floats to their three parts, packed in pairs.
 __device__ __forceinline__ void fc_split2(float a, float b, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
-    const fc_floatx2 v = {a, b};
+    const fc_floatx2 v = {a * kSplitScale, b * kSplitScale};
     hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, fc_bf16x2));
-    fc_floatx2 r = {a - __builtin_bit_cast(float, hi << 16), b - __builtin_bit_cast(float, hi & 0xffff0000u)};
+    fc_floatx2 r = {v[0] - __builtin_bit_cast(float, hi << 16), v[1] - __builtin_bit_cast(float, hi & 0xffff0000u)};
     mid = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, fc_bf16x2));
     fc_floatx2 q = {r[0] - __builtin_bit_cast(float, mid << 16), r[1] - __builtin_bit_cast(float, mid & 0xffff0000u)};
     lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(q, fc_bf16x2));
@@ -95,14 +100,15 @@ __device__ __forceinline__ void fc_zero(Acc (&acc)[MI][NI]) {
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[mi][ni][i] = 0.f;
 }
+// The two sums together, at their true size.
 template <int MI, int NI, class Acc>
-__device__ __forceinline__ void fc_add(Acc (&acc)[MI][NI], const Acc (&small)[MI][NI]) {
+__device__ __forceinline__ void fc_join(Acc (&acc)[MI][NI], const Acc (&small)[MI][NI]) {
 #pragma unroll
     for (int mi = 0; mi < MI; mi++)
 #pragma unroll
         for (int ni = 0; ni < NI; ni++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc[mi][ni][i] += small[mi][ni][i];
+            for (int i = 0; i < 16; i++) acc[mi][ni][i] = (acc[mi][ni][i] + small[mi][ni][i]) * kSplitUnscale;
 }
 
 // Whether any of a lane's accumulators is an infinity or a NaN.

@@ -149,7 +149,7 @@ __device__ __forceinline__ void fused_split_products(const FusedParams &p, int w
         stage(u[0], v[0]);
 #pragma unroll
         for (int i = 0; i < 8; i++) { u[0][i] = u[1][i]; v[0][i] = v[1][i]; }
-        fc_add<1, 1>(sum, small);
+        fc_join<1, 1>(sum, small);
         acc[f] = sum[0][0];
     }
 }

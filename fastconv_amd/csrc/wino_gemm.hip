@@ -329,7 +329,7 @@ __device__ __forceinline__ void split_tile(const float *__restrict__ U, const fl
         fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc, small);
         __syncthreads();
     }
-    fc_add<MI, NI>(acc, small);
+    fc_join<MI, NI>(acc, small);
     if (__syncthreads_or(fc_not_finite<MI, NI>(acc))) {
         // 64x64 at a time, which leaves the registers to the loop above
         typedef std::conditional_t<TL::THREADS == 512, TL, TileCfg<64, 64, 16, 2, TL::THREADS / 128>> Sub;

@@ -133,6 +133,42 @@ def test_sums_with_few_terms_are_no_less_exact_than_with_fp32_products(lib):
         assert all(e <= (1.1 if n == 1 else 1.0) * fp32 for (split, _), e in err.items() if split), (n, err)
 
 
+def test_small_operands_keep_their_last_places(lib):
+    """Filter values down to the smallest subnormal float (one channel an output) meet large inputs, and the other way
+    round: the product is an ordinary number and as exact as any other."""
+    C, K, T = 160, 130, 129
+    s = tiles_in_a_row(C, K, T)
+    for cfg in lib.wino_configs():
+        plan = lib.wino_plan(s, cfg.id)
+        k, t = np.arange(plan.K_pad), np.arange(plan.T_pad)
+        for small_filter in (True, False):
+            small = np.exp2(-149.0 + np.arange(C) % 50)[None, :, None]      # 2^-149 .. 2^-100, by channel
+            large = np.exp2(90.0)
+            U = np.zeros((64, plan.C_pad, plan.K_pad), np.float32)
+            V = np.zeros((64, plan.C_pad, plan.T_pad), np.float32)
+            U[:, k % C, k] = O.rng_uniform(1, (64, plan.K_pad), 1.0, 2.0)
+            V[:, :C] = O.rng_uniform(2, (64, C, plan.T_pad), 1.0, 2.0)
+            if small_filter:
+                U[:, :C] *= small
+                V *= np.float32(large)
+            else:
+                U *= np.float32(large)
+                V[:, :C] *= small
+            print("small operands", cfg.bm, cfg.bn, cfg.bk, small_filter, flush=True)
+            got = winograd_gemm(lib, plan, U, V)
+            exact = U[:, k % C, k].astype(np.float64)[:, :, None] * V[:, k % C]
+            assert (np.abs(got - exact) <= EPS_SINGLE * np.abs(exact)).all(), (cfg.id, small_filter)
+    s = O.shape(1, 64, 13, 11, 130, 1, 1, 1, 1, 0)
+    x = O.rng_uniform(3, (s.N, s.C, s.H, s.W), 1.0, 2.0) * np.float32(2.0 ** 90)
+    w = np.zeros((s.K, s.C, 1, 1), np.float32)
+    k = np.arange(s.K)
+    w[k, k % s.C, 0, 0] = O.rng_uniform(4, (s.K,), 1.0, 2.0) * np.exp2(-149.0 + k % 50)
+    exact = w[k, k % s.C, 0, 0].astype(np.float64)[None, :, None, None] * x[:, k % s.C]
+    for cfg in lib.igemm_configs():
+        print("small operands, implicit gemm", cfg.bm, cfg.bn, cfg.waves_k, flush=True)
+        assert (np.abs(lib.implicit_gemm_conv(cshape(s), x, w, config=cfg.id) - exact) <= EPS_SINGLE * np.abs(exact)).all(), cfg.id
+
+
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, np.finfo(np.float32).max])
 def test_values_without_a_finite_split(lib, value):
     """An infinity meets weights of both signs and nothing else: infinities of the right sign, and no NaN next to
