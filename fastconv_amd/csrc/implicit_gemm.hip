@@ -195,10 +195,12 @@ __device__ __forceinline__ bool ig_decode_tile(const IgemmParams &p, int *kb, in
     return true;
 }
 
-// The accumulators of a workgroup tile to y, or to this split's partial sums.
-template <class TL>
-__device__ __forceinline__ void ig_store_tile(const floatx16 (&acc)[TL::MI][TL::NI], const IgemmParams &p, int kb, int pb, int wm0,
-                                              int wn0, int lrow, int lcol) {
+// The accumulators of a workgroup tile to y, with this bias and ReLU, or to this split's partial sums.
+// REPLACE: the sums are there already, without bias and ReLU; those that are not finite give way to the accumulators.
+template <class TL, bool REPLACE = false>
+__device__ __forceinline__ void ig_store_tile(const floatx16 (&acc)[TL::MI][TL::NI], const IgemmParams &p, const float *bias, int relu,
+                                              int kb, int pb, int wm0, int wn0, int lrow, int lcol) {
+    auto sum = [](const float *there, float v) __attribute__((always_inline)) { return REPLACE && __builtin_isfinite(*there) ? *there : v; };
     constexpr int BM = TL::BM_, BN = TL::BN_, MI = TL::MI, NI = TL::NI;
     // epilogue: column = pixel (lane%32), rows = output channels.  Register i of an accumulator
     // block is row 8*(i/4) + 4*(lane/32) + i%4: element (row r, column c) of the tile goes to
@@ -213,7 +215,7 @@ __device__ __forceinline__ void ig_store_tile(const floatx16 (&acc)[TL::MI][TL::
         char *dst = reinterpret_cast<char *>(partial ? p.ws : p.y);
         const uint32_t rowStride = 4u * (partial ? (uint32_t)p.Npix : (uint32_t)OHW);      // bytes
         const uint32_t slab = partial ? (uint32_t)blockIdx.y * (uint32_t)p.K * (uint32_t)p.Npix : 0u;
-        const bool plain = partial || (p.bias == nullptr && !p.relu);
+        const bool plain = partial || (bias == nullptr && !relu);
 #pragma unroll
         for (int ni = 0; ni < NI; ni++) {
             const long opix = (long)pb * BN + wn0 + ni * 32 + lcol;
@@ -230,20 +232,23 @@ __device__ __forceinline__ void ig_store_tile(const floatx16 (&acc)[TL::MI][TL::
 #pragma unroll
                 for (int mi = 0; mi < MI; mi++)
 #pragma unroll
-                    for (int i = 0; i < 16; i++)
-                        *reinterpret_cast<float *>(dst + (off + (uint32_t)(mi * 32 + 8 * (i / 4) + (i % 4)) * rowStride)) = acc[mi][ni][i];
+                    for (int i = 0; i < 16; i++) {
+                        float *d = reinterpret_cast<float *>(dst + (off + (uint32_t)(mi * 32 + 8 * (i / 4) + (i % 4)) * rowStride));
+                        *d = sum(d, acc[mi][ni][i]);
+                    }
             } else {
 #pragma unroll
                 for (int mi = 0; mi < MI; mi++)
 #pragma unroll
                     for (int q = 0; q < 4; q++) {
                         floatx4 bq = {0.f, 0.f, 0.f, 0.f};
-                        if (p.bias) bq = *reinterpret_cast<const floatx4 *>(p.bias + rowBase + mi * 32 + 8 * q);
+                        if (bias) bq = *reinterpret_cast<const floatx4 *>(bias + rowBase + mi * 32 + 8 * q);
 #pragma unroll
                         for (int j = 0; j < 4; j++) {
-                            float v = acc[mi][ni][q * 4 + j] + bq[j];
-                            if (p.relu) v = __builtin_elementwise_maximum(v, 0.f);      // keeps a NaN
-                            *reinterpret_cast<float *>(dst + (off + (uint32_t)(mi * 32 + 8 * q + j) * rowStride)) = v;
+                            float *d = reinterpret_cast<float *>(dst + (off + (uint32_t)(mi * 32 + 8 * q + j) * rowStride));
+                            float v = sum(d, acc[mi][ni][q * 4 + j]) + bq[j];
+                            if (relu) v = __builtin_elementwise_maximum(v, 0.f);      // keeps a NaN
+                            *d = v;
                         }
                     }
             }
@@ -262,7 +267,10 @@ __device__ __forceinline__ void ig_store_tile(const floatx16 (&acc)[TL::MI][TL::
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int k = rowBase + mi * 32 + 8 * (i / 4) + (i % 4);
-                    if (k < p.K) wz[(size_t)k * p.Npix + opix] = acc[mi][ni][i];
+                    if (k < p.K) {
+                        float *d = wz + (size_t)k * p.Npix + opix;
+                        *d = sum(d, acc[mi][ni][i]);
+                    }
                 }
         }
         return;
@@ -280,10 +288,11 @@ __device__ __forceinline__ void ig_store_tile(const floatx16 (&acc)[TL::MI][TL::
             for (int i = 0; i < 16; i++) {
                 const int k = rowBase + mi * 32 + 8 * (i / 4) + (i % 4);
                 if (k < p.K) {
-                    float v = acc[mi][ni][i];
-                    if (p.bias) v += p.bias[k];
-                    if (p.relu) v = __builtin_elementwise_maximum(v, 0.f);      // keeps a NaN
-                    yn[(size_t)k * OHW] = v;
+                    float *d = yn + (size_t)k * OHW;
+                    float v = sum(d, acc[mi][ni][i]);
+                    if (bias) v += bias[k];
+                    if (relu) v = __builtin_elementwise_maximum(v, 0.f);      // keeps a NaN
+                    *d = v;
                 }
             }
     }
@@ -293,7 +302,7 @@ __device__ __forceinline__ void ig_store_tile(const floatx16 (&acc)[TL::MI][TL::
 // is channel c of x, contiguous over the pixels) whose pixels-per-image count is a multiple of 4
 // and whose channel count is a multiple of BK copy the B tile as 16-byte vectors, unconditionally:
 // a pixel group past the end re-reads the last group (its columns are never stored).
-template <class TL, int MODE>
+template <class TL, int MODE, bool REPLACE = false>
 __device__ __forceinline__ void ig_tile(const IgemmParams &p, const int kb, const int pb, float (*As)[TL::BK_ * TL::BM_],
                                         float (*Bs)[TL::BK_ * TL::BN_]) {
     constexpr bool PW = MODE == IG_POINTWISE, TAP = MODE == IG_TAP_MASKED || MODE == IG_TAP_INSIDE;
@@ -512,7 +521,7 @@ __device__ __forceinline__ void ig_tile(const IgemmParams &p, const int kb, cons
         __syncthreads();
     }
 
-    ig_store_tile<TL>(acc, p, kb, pb, wm0, wn0, lrow, lcol);
+    ig_store_tile<TL, REPLACE>(acc, p, p.bias, p.relu, kb, pb, wm0, wn0, lrow, lcol);
 }
 
 template <class TL, int MODE>
@@ -683,18 +692,19 @@ __global__ __launch_bounds__(TL::THREADS, IgSplit<TL>::MIN_WAVES) void igemm_con
         __syncthreads();
     }
     fc_join<MI, NI>(acc, small);
-    if (__syncthreads_or(fc_not_finite<MI, NI>(acc))) {
+    const bool again = __syncthreads_or(fc_not_finite<MI, NI>(acc));
+    ig_store_tile<TL>(acc, p, again ? nullptr : p.bias, again ? 0 : p.relu, kb, pb, wm0, wn0, lrow, lcol);
+    if (again) {
         // 64x64 at a time, which leaves the registers to the loop above
         typedef std::conditional_t<TL::THREADS == 512, TL, IgTile<64, 64, 16, 2, TL::THREADS / 128>> Sub;
         static_assert(Sub::THREADS == TL::THREADS && Sub::LDS_BYTES <= 16 * S::LDS_WORDS, "same workgroup");
         float *const f = reinterpret_cast<float *>(smem);
         constexpr int QM = BM / Sub::BM_, QN = BN / Sub::BN_;
+        __syncthreads();      // the whole tile is in y, or in the partial sums
         for (int q = 0; q < QM * QN; q++)
-            ig_tile<Sub, MODE>(p, kb * QM + q / QN, pb * QN + q % QN, reinterpret_cast<float (*)[16 * Sub::BM_]>(f),
-                               reinterpret_cast<float (*)[16 * Sub::BN_]>(f + 2 * 16 * Sub::BM_));
-        return;
+            ig_tile<Sub, MODE, true>(p, kb * QM + q / QN, pb * QN + q % QN, reinterpret_cast<float (*)[16 * Sub::BM_]>(f),
+                                     reinterpret_cast<float (*)[16 * Sub::BN_]>(f + 2 * 16 * Sub::BM_));
     }
-    ig_store_tile<TL>(acc, p, kb, pb, wm0, wn0, lrow, lcol);
 }
 
 // Sums the partial results of a split reduction in split order (so the result does

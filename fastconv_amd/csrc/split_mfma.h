@@ -17,9 +17,11 @@
 // Operands are multiplied by 2^24 first and sums by 2^-48 last: the parts of the smallest subnormal float are then normal
 // bf16 numbers, and the split is exact over the whole lower range (without it parts below 2^-133 are lost, 2^-10 of an
 // operand of 2^-124).  One multiplication an element, 1 to 3 % of a launch.
-// An infinity has no such sum (inf - inf), and scaled operands from 2^104 and sums from 2^80 on overflow, so a tile whose
-// result is not finite throughout is computed again with fp32 instructions by the kernels that use this: NaN, infinities
-// and large values come out as they always did.
+// An infinity has no such sum (inf - inf), and scaled operands from 2^104 and sums from 2^80 on overflow.  Values that are
+// not finite are formed again with fp32 instructions by the kernels that use this, the others keep what they are: NaN,
+// infinities and large values come out as they always did, and a value depends on its own row and column alone.  A tile
+// with such a value runs through its reduction a second time: 256 -> 256 channels at 56x56, batch 32, one NaN 178 -> 194 us,
+// one in every tile 441 us (all on fp32 instructions: 225).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -92,6 +92,23 @@ __device__ __forceinline__ void fused_products(const FusedParams &p, int wave, i
             acc[f] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][f], bv[u][f], acc[f], 0, 0, 0);
 }
 
+// One of this wavefront's frequencies with fp32 instructions, in the order of fused_products.
+__device__ __forceinline__ floatx16 fused_one_product(const FusedParams &p, int wave, int f, int lrow, int lcol, int kb, int tb) {
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    const float *ub = p.U + (size_t)(wv * kFW + f) * p.C_pad * p.K_pad + (size_t)kb * 32;
+    const float *vb = p.V + (size_t)(wv * kFW + f) * p.C_pad * p.T_pad + (size_t)tb * 32;
+    uint32_t offU = 4u * ((uint32_t)lrow * p.K_pad + lcol), offV = 4u * ((uint32_t)lrow * (uint32_t)p.T_pad + lcol);
+    floatx16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i] = 0.f;
+    for (int s = 0; s < p.C_pad / 2; s++) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ldg(ub, offU), ldg(vb, offV), acc, 0, 0, 0);
+        offU += 8u * p.K_pad;
+        offV += 8u * (uint32_t)p.T_pad;
+    }
+    return acc;
+}
+
 // The same on the bf16 matrix cores, in the order of the staged pipeline's GEMM (see split_mfma.h): 16 channels at a time,
 // a lane splits the 8 channels of its row and column.  One frequency after another, so that only one has its second sum in
 // registers.  The split is the larger part of the time: the operands of a 32x32 block are split by every block that uses
@@ -150,6 +167,12 @@ __device__ __forceinline__ void fused_split_products(const FusedParams &p, int w
 #pragma unroll
         for (int i = 0; i < 8; i++) { u[0][i] = u[1][i]; v[0][i] = v[1][i]; }
         fc_join<1, 1>(sum, small);
+        if (__any(fc_not_finite<1, 1>(sum))) {
+            // values that are not finite, as in the GEMM of the staged pipeline
+            const floatx16 r = fused_one_product(p, wave, f, lrow, lcol, kb, tb);
+#pragma unroll
+            for (int i = 0; i < 16; i++) sum[0][0][i] = __builtin_isfinite(sum[0][0][i]) ? sum[0][0][i] : r[i];
+        }
         acc[f] = sum[0][0];
     }
 }
@@ -169,10 +192,6 @@ __global__ __launch_bounds__(kFusedThreads, 1) void wino_gemm_out_fused_kernel(c
     floatx16 acc[kFW];
     if constexpr (SPLIT) {
         fused_split_products(p, wave, lrow, lcol, kb, tb, acc);
-        floatx16 all[1][kFW];
-#pragma unroll
-        for (int f = 0; f < kFW; f++) all[0][f] = acc[f];
-        if (__any(fc_not_finite<1, kFW>(all))) fused_products(p, wave, lrow, lcol, kb, tb, acc);
     } else {
         fused_products(p, wave, lrow, lcol, kb, tb, acc);
     }

@@ -72,8 +72,8 @@ struct TileCfg : GemmTile<BM, BN, BK, WGM, WGN> {
     static constexpr int BM_ = BM, BN_ = BN, BK_ = BK, WGM_ = WGM, WGN_ = WGN, PF_ = PF;
 };
 
-// The accumulators of a workgroup tile to M.
-template <class TL>
+// The accumulators of a workgroup tile to M.  REPLACE: only where M holds no finite value.
+template <class TL, bool REPLACE = false>
 __device__ __forceinline__ void store_tile(const floatx16 (&acc)[TL::MI][TL::NI], float *__restrict__ M, int K_pad, int T_pad, int f,
                                            int kb, int tb, int wm0, int wn0, int lrow, int lcol) {
     constexpr int BM = TL::BM_, BN = TL::BN_, MI = TL::MI, NI = TL::NI;
@@ -90,7 +90,8 @@ __device__ __forceinline__ void store_tile(const floatx16 (&acc)[TL::MI][TL::NI]
             char *pr = reinterpret_cast<char *>(uniform_ptr(Mg + (size_t)(mi * 32) * T_pad + ni * 32));
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                *reinterpret_cast<float *>(pr + mOff) = acc[mi][ni][i];
+                float *dst = reinterpret_cast<float *>(pr + mOff);
+                if (!REPLACE || !__builtin_isfinite(*dst)) *dst = acc[mi][ni][i];
                 pr = uniform_ptr(pr + ((i % 4) == 3 ? 5 * rowBytes : rowBytes));
             }
         }
@@ -98,7 +99,7 @@ __device__ __forceinline__ void store_tile(const floatx16 (&acc)[TL::MI][TL::NI]
 
 // One workgroup tile: M[f][kb*BM .. +BM][tb*BN .. +BN] = sum over all input channels.
 // `smem` holds the two LDS stages of both operands (2*BK*(BM+BN) floats).
-template <class TL>
+template <class TL, bool REPLACE = false>
 __device__ __forceinline__ void gemm_tile(const float *__restrict__ U, const float *__restrict__ V,
                                           float *__restrict__ M, int K_pad, int C_pad, int T_pad, int f, int kb,
                                           int tb, float *smem) {
@@ -239,7 +240,7 @@ __device__ __forceinline__ void gemm_tile(const float *__restrict__ U, const flo
     // the last nStages % PF stages
     stage_rest(stage, s0, nStages, std::make_integer_sequence<int, PF - 1>());
 
-    store_tile<TL>(acc, M, K_pad, T_pad, f, kb, tb, wm0, wn0, lrow, lcol);
+    store_tile<TL, REPLACE>(acc, M, K_pad, T_pad, f, kb, tb, wm0, wn0, lrow, lcol);
 }
 
 // The same tile on the bf16 matrix cores (see split_mfma.h): a wavefront takes 8 consecutive channels of 64 rows or
@@ -330,16 +331,17 @@ __device__ __forceinline__ void split_tile(const float *__restrict__ U, const fl
         __syncthreads();
     }
     fc_join<MI, NI>(acc, small);
-    if (__syncthreads_or(fc_not_finite<MI, NI>(acc))) {
+    const bool again = __syncthreads_or(fc_not_finite<MI, NI>(acc));
+    store_tile<TL>(acc, M, K_pad, T_pad, f, kb, tb, wm0, wn0, lrow, lcol);
+    if (again) {
         // 64x64 at a time, which leaves the registers to the loop above
         typedef std::conditional_t<TL::THREADS == 512, TL, TileCfg<64, 64, 16, 2, TL::THREADS / 128>> Sub;
         static_assert(Sub::THREADS == TL::THREADS && Sub::LDS_BYTES <= 16 * S::LDS_WORDS, "same workgroup");
         constexpr int QM = BM / Sub::BM_, QN = BN / Sub::BN_;
+        __syncthreads();      // the whole tile is in M
         for (int q = 0; q < QM * QN; q++)
-            gemm_tile<Sub>(U, V, M, K_pad, C_pad, T_pad, f, kb * QM + q / QN, tb * QN + q % QN, reinterpret_cast<float *>(smem));
-        return;
+            gemm_tile<Sub, true>(U, V, M, K_pad, C_pad, T_pad, f, kb * QM + q / QN, tb * QN + q % QN, reinterpret_cast<float *>(smem));
     }
-    store_tile<TL>(acc, M, K_pad, T_pad, f, kb, tb, wm0, wn0, lrow, lcol);
 }
 
 // Workgroups are dealt to the 8 XCDs round-robin by linear id.  All tiles of one

@@ -195,3 +195,80 @@ def test_values_without_a_finite_split(lib, value):
         rest = np.ones((14, 14), bool)
         rest[5, 6] = False
         assert np.abs(y[0][:, rest] - truth[0][:, rest]).max() <= 1e-4
+
+
+POISON = [np.inf, -np.inf, np.nan, 3e38, 1e30]      # the last two are finite, but their scaled parts or sums are not
+
+
+@pytest.mark.parametrize("value", POISON)
+def test_winograd_gemm_forms_only_values_that_are_not_finite_again(lib, value):
+    """One value in V and one in U, in different quarters of the larger tiles: their column and row as fp64 has them,
+    everything else with the bits of a run without them."""
+    C, K, T = 160, 200, 200
+    s = tiles_in_a_row(C, K, T)
+    for cfg in lib.wino_configs():
+        plan = lib.wino_plan(s, cfg.id)
+        U = O.rng_uniform(C, (64, plan.C_pad, plan.K_pad))
+        V = O.rng_uniform(K, (64, plan.C_pad, plan.T_pad))
+        print("poison", value, cfg.bm, cfg.bn, cfg.bk, flush=True)
+        clean = winograd_gemm(lib, plan, U, V)
+        V[9, 100, 150] = value
+        U[9, 3, 70] = value
+        U[9, 100, 70] = V[9, 3, 150] = 0.5      # the two meet numbers
+        got = winograd_gemm(lib, plan, U, V)
+        rest = np.ones(got.shape, bool)
+        rest[9, 70, :] = rest[9, :, 150] = False
+        assert np.array_equal(got[rest], clean[rest]), cfg.id
+        with np.errstate(invalid="ignore"):
+            a, b = U[9].T.astype(np.float64), V[9].astype(np.float64)
+            exact, size = a @ b, np.abs(a) @ np.abs(b)
+        for line, e, z in ((got[9, 70], exact[70], size[70]), (got[9, :, 150], exact[:, 150], size[:, 150])):
+            fin = np.isfinite(e)
+            assert np.array_equal(line[~fin], e[~fin].astype(np.float32), equal_nan=True), cfg.id
+            assert (np.abs(line[fin] - e[fin]) <= (plan.C_pad + 40) * EPS_SUM * z[fin]).all(), cfg.id
+
+
+@pytest.mark.parametrize("value", POISON)
+def test_winograd_layer_with_values_that_are_not_finite(lib, value):
+    """One pixel of one image: the other images keep their bits, staged and fused pipeline give the same."""
+    s = O.shape(3, 160, 13, 12, 72)
+    x, w = O.make_inputs(s, seed=9)
+    bias = O.rng_uniform(5, (s.K,))
+    for cfg in lib.wino_configs():
+        print("poison", value, cfg.bm, cfg.bn, cfg.bk, flush=True)
+        clean = lib.winograd_conv(cshape(s), x, w, bias, True, config=cfg.id)
+        bad = x.copy()
+        bad[1, 100, 6, 5] = value
+        staged = lib.winograd_conv(cshape(s), bad, w, bias, True, config=cfg.id)
+        assert np.array_equal(staged[[0, 2]], clean[[0, 2]]), cfg.id
+        assert np.array_equal(lib.winograd_conv_fused(cshape(s), bad, w, bias, True, config=cfg.id), staged, equal_nan=True), cfg.id
+        hit = staged[1, :, 5:8, 4:7]      # the 3x3 windows that hold the pixel
+        assert np.isnan(hit).all() if np.isnan(value) else not np.array_equal(hit, clean[1, :, 5:8, 4:7])
+
+
+@pytest.mark.parametrize("value", POISON)
+@pytest.mark.parametrize("shp", [
+    (2, 64, 9, 10, 130, 3, 3, 1, 1, 1),      # split reduction, border taps, channels past a tile
+    (2, 64, 12, 12, 256, 1, 1, 1, 1, 0),     # whole tiles, no split reduction
+    (2, 7, 11, 12, 128, 3, 3, 1, 1, 1),      # table gather
+])
+def test_implicit_gemm_forms_only_values_that_are_not_finite_again(lib, shp, value):
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=11)
+    bias = O.rng_uniform(6, (s.K,))
+    bad = x.copy()
+    bad[1, 3, 4, 5] = value
+    truth = np.maximum(O.naive_conv_f64(s, bad, w, bias), 0.0)
+    size = O.naive_conv_f64(s, np.abs(bad), np.abs(w)) + 1.0
+    r = s.kh // 2
+    hit = np.zeros(truth.shape, bool)
+    hit[1, :, 4 - r:5 + r, 5 - r:6 + r] = True
+    for cfg in lib.igemm_configs():
+        print("poison", value, shp, cfg.bm, cfg.bn, cfg.waves_k, flush=True)
+        clean = lib.implicit_gemm_conv(cshape(s), x, w, bias, True, config=cfg.id)
+        got = lib.implicit_gemm_conv(cshape(s), bad, w, bias, True, config=cfg.id)
+        assert np.array_equal(got[~hit], clean[~hit]), cfg.id
+        fin = hit & np.isfinite(truth) & np.isfinite(size)
+        assert (np.abs(got[fin] - truth[fin]) <= (s.C * s.kh * s.kw + 40) * EPS_SUM * size[fin]).all(), cfg.id
+        odd = hit & ~(np.isfinite(truth) & np.isfinite(size))
+        assert np.array_equal(got[odd], truth[odd].astype(np.float32), equal_nan=True), cfg.id
