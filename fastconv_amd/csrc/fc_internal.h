@@ -69,9 +69,10 @@ int fc_igemm_ws_choose(const fc_conv_shape *s, long Npix);      // index of the 
 int fc_igemm_ws_pack(fc_context *ctx, const fc_igemm_plan *plan, const float *w_dev, float *Wq_dev, int32_t *table_dev);
 int fc_igemm_ws_run(fc_context *ctx, const fc_igemm_plan *plan, int index, const float *x_dev, const float *Wq_dev,
                     const int32_t *table_dev, const float *bias_dev, int relu, float *y_dev, bool timed);
-// wino_gemm.hip: whether the products of this plan run on the bf16 matrix cores (see split_mfma.h); the kernel that joins
-// GEMM and output transform follows, so that both pipelines give the same bits.  Tiles of whole 64s, 16 deep; layers
-// with C*K <= 8192, where the GEMM is bound by memory, stay on fp32 instructions.
+// wino_gemm.hip: whether the products of this plan run on the bf16 matrix cores (see split_mfma.h): tiles of whole 64s, 16
+// deep, more than 48 input channels, C*K above 8192 and, by tile, channels and the bytes of V and M, not bound by memory
+// (the lines stand beside it).  The kernel that joins GEMM and output transform follows, so that both pipelines give the
+// same bits for the same plan; plans of the same layer with other batches or tiles may round differently.
 bool fc_wino_gemm_splits(const fc_wino_plan *plan);
 // wino_smallc.hip: the single-kernel Winograd path of layers with at most four input channels.
 // Called by the fc_wino_*onepass* entry points after they have checked plan and pointers.

@@ -460,18 +460,29 @@ extern "C" int fc_wino_gemm_get_config(int id, fc_gemm_config *cfg) {
     return FC_OK;
 }
 
-// Layers whose GEMM is bound by memory stay on fp32 instructions, which fetch 16 bytes a lane: up to 48 input channels
-// (fp32 / split: 29 -> 364 channels, 900 tiles 18.0 us / 18.4, 16 -> 700, 1089 tiles 28.3 / 33.5, 48 -> 512, 3136 tiles
-// 105 / 112; 64 -> 256, 1444 tiles 29.0 / 23.2), and with 64x64 tiles, whose operands are read most often, up to 160
-// where V and M outgrow the last-level cache (64 -> 160, 4900 tiles, 281 MB 84.7 / 93.9, but 2500 tiles, 143 MB 38.9 /
-// 31.8; 128 -> 300, 650 MB 250 / 261; 192 -> 300, 747 MB 343 / 322).
+// Layers of up to 48 input channels stay on fp32 instructions, which fetch 16 bytes a lane: their GEMM is bound by memory
+// (fp32 / split us: 29 -> 364 channels, 900 tiles 18.0 / 18.4, 16 -> 700, 1089 tiles 28.3 / 33.5, 48 -> 512, 3136 tiles 105 / 112).
 static bool has_split_products(long C, long K) { return C > 48 && C * K > 8192; }
 
+// Beyond that the smaller tiles, whose operands are read most often, are bound by memory where V and M (here in MB)
+// outgrow the 256 MB of the last-level cache, and the 256-wide ones hold a single wavefront a SIMD.  Whole staged layer on
+// 60x60 images without the filter transform, us on fp32 instructions / split:
+//   128x128: 64 -> 256 (105) 56.7 / 55.1, (262) 140.9 / 141.5, (451) 261 / 270; 80 -> 256 (253) 148 / 145, (308) 178 / 176,
+//            (451) 249 / 257; 96 -> 256 (254) 156 / 148, (461) 267 / 267; 128 -> 256 (453) 293 / 279
+//   64x64:   64 -> 160 (101) 48.5 / 48.5, (180) 90.0 / 92.6; 80 -> 256 (105) 59.7 / 58.5, (253) 150.0 / 150.4; 96 -> 160 (179)
+//            98.7 / 97.0, (307) 171 / 177; 128 -> 256 (252) 166 / 162, (453) 296 / 302; 160 -> 256 (300) 203 / 197, (709) 488 / 490
+//   64x128, 128x64: 64 -> 256 (105) 58.6 / 59.0, 56.7 / 58.0; 96 -> 160 (179) 105 / 99, (219) 120 / 116; 128 -> 256 (453)
+//            296 / 306, 297 / 306; 160 -> 256 (450) 309 / 309, 310 / 310
+//   256x128, 128x256: 128 -> 256 (252) 169 / 173, 168 / 170; 160 -> 256 (300) 215 / 219, 214 / 214; 192 -> 256 (264) 201 / 201,
+//            207 / 202; 256 -> 256 (252) 206 / 194, 217 / 207
 bool fc_wino_gemm_splits(const fc_wino_plan *plan) {
     const fc_gemm_config &c = kConfigs[plan->gemm_config];
-    const long C = plan->shape.C, K = plan->shape.K;
-    if (!has_split_products(C, K) || c.bm % 64 != 0 || c.bn % 64 != 0 || c.bk != 16) return false;
-    return c.bm * c.bn > 64 * 64 || C >= 160 || 256.0 * (double)(C + K) * (double)plan->T_pad <= 256e6;
+    if (!has_split_products(plan->shape.C, plan->shape.K) || c.bm % 64 != 0 || c.bn % 64 != 0 || c.bk != 16) return false;
+    const int area = c.bm * c.bn, C = plan->C_pad;
+    const double bytes = (double)plan->V_bytes + (double)plan->M_bytes;
+    if (area > 128 * 128) return C >= 192;
+    if (area == 128 * 128) return C >= 96 || bytes <= 320e6;
+    return C >= 160 || (C >= 80 && bytes <= 256e6);
 }
 
 // Cost model behind the untuned choice: padded multiply-adds, divided by a rate per tile shape
@@ -484,7 +495,9 @@ bool fc_wino_gemm_splits(const fc_wino_plan *plan) {
 // small grids; the shapes with a 32 stay on fp32 instructions, for layers whose 64-wide tile
 // would be mostly padding (512 channels at 28x28, batch 1: 14.7 us against 21).  Layers of few
 // channels stay on fp32 instructions whatever their tile: they are bound by memory (16 -> 64
-// channels, 28x28, batch 64: 7.1 us against 7.7), and keep the rates measured for those.
+// channels, 28x28, batch 64: 7.1 us against 7.7), and keep the rates measured for those.  The smaller tiles of layers
+// whose V and M outgrow the cache (fc_wino_gemm_splits) are weighed with the same rates: for 60 layers of 64 to 160
+// channels, 100 to 880 MB, the choice is within 6 % of the best shape, 2 % but for seven.
 extern "C" int fc_wino_gemm_default_config(const fc_conv_shape *s) {
     if (!fc_shape_ok(s)) return FC_ERR_INVALID;
     static const double kFp32Rate[] = {1.00, 0.90, 0.90, 0.97, 0.72, 0.95, 0.88, 0.93, 0.93, 0.90, 0.76};

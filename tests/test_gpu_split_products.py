@@ -85,6 +85,22 @@ def test_winograd_gemm_split_products(lib, C, K, T):
             assert (np.abs(got[f] - a @ b) <= tol).all(), (cfg.id, f)
 
 
+@pytest.mark.parametrize("C,K,N", [
+    (48, 200, 1), (49, 200, 1),              # channels from which products are split, here with 128x128 tiles
+    (64, 130, 39), (64, 130, 40),            # V and M on either side of 320 MB with these
+    (64, 130, 1), (65, 130, 1),              # channels from which the smaller tiles follow
+    (80, 130, 36), (80, 130, 37),            # V and M on either side of 256 MB with 64x64 tiles
+    (144, 130, 30), (145, 130, 30),          # channels from which they follow at any size
+    (176, 130, 1), (177, 130, 1),            # and the 256-wide tiles
+])
+def test_fused_and_staged_pipeline_agree_at_the_lines_of_the_split(lib, C, K, N):
+    s = O.shape(N, C, 60, 60, K)
+    x, w = O.make_inputs(s, seed=C)
+    for cfg in (0, 1, 3, 7):
+        print("line", (C, K, N), cfg, flush=True)
+        assert np.array_equal(lib.winograd_conv_fused(cshape(s), x, w, config=cfg), lib.winograd_conv(cshape(s), x, w, config=cfg)), cfg
+
+
 def test_sums_of_one_term_keep_fp32_accuracy(lib):
     """One channel of the filter is not zero: a partial product left out, or a first part that is cut off and not
     rounded, shows in every result (test_split_products.py)."""
