@@ -74,9 +74,12 @@ int fc_igemm_ws_run(fc_context *ctx, const fc_igemm_plan *plan, int index, const
 // (the lines stand beside it).  The kernel that joins GEMM and output transform follows, so that both pipelines give the
 // same bits for the same plan; plans of the same layer with other batches or tiles may round differently.
 bool fc_wino_gemm_splits(const fc_wino_plan *plan);
+// What the staged pipeline takes: tiles in a row of the output (LDS of the input transform) and output channels (the output
+// transform has one workgroup row for each).
+constexpr int kWinoMaxTilesW = 170;
+constexpr int kWinoMaxChannels = 65535;
 // wino_smallc.hip: the single-kernel Winograd path of layers with at most four input channels.
 // Called by the fc_wino_*onepass* entry points after they have checked plan and pointers.
-constexpr int kWinoMaxTilesW = 170;      // tiles in a row of the output that the staged pipeline takes (LDS of the input transform)
 bool fc_wino_smallc_applies(const fc_conv_shape *s);
 int fc_wino_smallc_filter_transform(fc_context *ctx, const fc_wino_plan *plan, const float *w_dev, float *U_dev);
 // w_dev == nullptr: U_dev holds the transformed filter; otherwise the kernel transforms w_dev itself and fills U_dev

@@ -404,7 +404,7 @@ extern "C" int fc_wino_prefer_onepass(const fc_conv_shape *s) {
     const long T = (long)s->N * ((OH + 5) / 6) * ((OW + 5) / 6);
     const long blocks = (T + kTB - 1) / kTB * ((s->K + kKB - 1) / kKB);
     if (blocks < (s->K <= kKB ? 192 : 512)) return 0;
-    if ((OW + 5) / 6 > kWinoMaxTilesW) return 1;      // the other pipelines do not take it
+    if ((OW + 5) / 6 > kWinoMaxTilesW || s->K > kWinoMaxChannels) return 1;      // the staged pipeline does not take it
     // What the pipelines with V and M in memory pay is bytes, what this one pays is products and, for every 64 output
     // channels, an input transform: the line is a number of bytes per input channel.  It lies higher for C*K > 8192, with
     // more output channels and from 49 input channels on the bf16 matrix cores.  Us here / staged, at (V+M in MB):

@@ -623,7 +623,7 @@ extern "C" int fc_wino_output_transform(fc_context *ctx, const fc_wino_plan *pla
     }
     if (ldsBytes > 64 * 1024) return fc_set_error(ctx, FC_ERR_UNSUPPORTED, "fc_wino_output_transform: image too wide", hipSuccess);
     const dim3 grid((unsigned)((plan->T + tpb - 1) / tpb), s.K);
-    if (grid.y > 65535) return fc_set_error(ctx, FC_ERR_UNSUPPORTED, "fc_wino_output_transform: more than 65535 channels", hipSuccess);
+    if (s.K > kWinoMaxChannels) return fc_set_error(ctx, FC_ERR_UNSUPPORTED, "fc_wino_output_transform: more than 65535 channels", hipSuccess);
     if (((uintptr_t)y_dev & 15) != 0) return fc_set_error(ctx, FC_ERR_INVALID, "fc_wino_output_transform: y must be 16-byte aligned", hipSuccess);
     fc_stage_scope scope(ctx, FC_STAGE_OUTPUT_TRAN);
 #ifdef FC_OT_VEC2

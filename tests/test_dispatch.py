@@ -42,3 +42,13 @@ def test_layers_that_leave_the_single_kernel_path_have_a_plan(lib):
                     assert rc == 0 or blocks < 512, (c, k, n, h, w)
                     seen += 1
     assert seen > 30
+
+
+@pytest.mark.parametrize("k,onepass", [(65535, 0), (65536, 1), (70000, 1)])
+def test_more_output_channels_than_the_staged_pipeline_takes_stay_on_the_single_kernel(lib, k, onepass):
+    """The output transform of the staged pipeline refuses more than 65535 output channels; with as many the layer is
+    otherwise one for the staged pipeline."""
+    s = shape(1, 16, k, 12)
+    assert lib.fc_prefer_winograd(C.byref(s)) == 1
+    assert lib.fc_wino_prefer_onepass(C.byref(s)) == onepass
+    assert onepass or not lib.fc_wino_prefer_fused(C.byref(s))
