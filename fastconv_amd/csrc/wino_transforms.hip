@@ -400,6 +400,7 @@ __global__ __launch_bounds__(TPB / TPT) void wino_output_transform_kernel(const 
 
     constexpr int WAVES = TPB / TPT / 64;
     const size_t chan = (size_t)p.OH * p.OW;
+    const size_t y0 = reinterpret_cast<uintptr_t>(p.y) / sizeof(float);      // where y starts, for the alignment of its rows
     // one row of a partly covered band: columns xA .. xB-1 of `rows` rows
     auto copy_rows = [&](float *dst, const float *src, int rows, int xA, int xB) {
         for (int i = 0; i < rows; i++)
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(TPB / TPT) void wino_output_transform_kernel(const 
             float *dst = img + rowA * p.OW;
             const float *src = lds + (simg + rowA * p.OW);
             // 16-byte pieces where the run starts on a 16-byte boundary in y and in LDS and is a whole number of them
-            const bool vec4 = (len & 3) == 0 && ((((size_t)n * p.K + k) * chan + (size_t)rowA * p.OW) & 3) == 0 &&
+            const bool vec4 = (len & 3) == 0 && ((y0 + ((size_t)n * p.K + k) * chan + (size_t)rowA * p.OW) & 3) == 0 &&
                               ((simg + rowA * p.OW) & 3) == 0;
             if (vec4) {
                 typedef float vec4f __attribute__((ext_vector_type(4)));
@@ -624,7 +625,8 @@ extern "C" int fc_wino_output_transform(fc_context *ctx, const fc_wino_plan *pla
     if (ldsBytes > 64 * 1024) return fc_set_error(ctx, FC_ERR_UNSUPPORTED, "fc_wino_output_transform: image too wide", hipSuccess);
     const dim3 grid((unsigned)((plan->T + tpb - 1) / tpb), s.K);
     if (s.K > kWinoMaxChannels) return fc_set_error(ctx, FC_ERR_UNSUPPORTED, "fc_wino_output_transform: more than 65535 channels", hipSuccess);
-    if (((uintptr_t)y_dev & 15) != 0) return fc_set_error(ctx, FC_ERR_INVALID, "fc_wino_output_transform: y must be 16-byte aligned", hipSuccess);
+    // (what the single kernel takes: fc_wino_prefer_onepass chooses between them without knowing y)
+    if (((uintptr_t)y_dev & 7) != 0) return fc_set_error(ctx, FC_ERR_INVALID, "fc_wino_output_transform: y must be 8-byte aligned", hipSuccess);
     fc_stage_scope scope(ctx, FC_STAGE_OUTPUT_TRAN);
 #ifdef FC_OT_VEC2
     if (tpb == 128) wino_output_transform_kernel<128, 2><<<grid, dim3(64), ldsBytes, ctx->stream>>>(p);

@@ -481,6 +481,32 @@ def test_winograd_single_kernel_plan_is_not_accepted_by_the_staged_calls(lib):
         lib.wino_conv_onepass(lib.wino_plan(s, 0), buf, buf, buf)
 
 
+@pytest.mark.parametrize("shp", [(3, 16, 28, 28, 40), (2, 24, 13, 14, 33), (1, 17, 20, 50, 70), (2, 64, 8, 9, 64)])
+def test_every_winograd_pipeline_takes_an_output_aligned_to_8_bytes(lib, shp):
+    """The library advises a pipeline without knowing y: with y at an odd multiple of 8 bytes each gives the bits it
+    gives at a 256-byte boundary, and writes nothing beside y."""
+    s = O.shape(*shp)
+    cs = cshape(s)
+    x, w = O.make_inputs(s, seed=4)
+    n = s.N * s.K * s.H * s.W
+    announce("8-byte aligned output", shp)
+    plan, one = lib.wino_plan(cs, lib.wino_default_config(cs)), lib.wino_onepass_plan(cs)
+    mark = lib.mark()
+    dx, dw = lib.upload(x), lib.upload(w)
+    U, V, M = lib.alloc(max(plan.U_bytes, one.U_bytes)), lib.alloc(plan.V_bytes), lib.alloc(plan.M_bytes)
+    for run in (lambda y: lib.wino_forward(plan, dx, dw, U, V, M, y), lambda y: lib.wino_forward_fused(plan, dx, dw, U, V, y),
+                lambda y: lib.wino_forward_onepass(one, dx, dw, U, y)):
+        got = []
+        for first in (64, 2, 66, 70):      # floats past a 256-byte boundary
+            buf = lib.upload(np.full(n + 128, 7.0, np.float32))
+            run(type(buf)(buf.value + 4 * first))
+            out = lib.download(buf, (n + 128,))
+            assert (out[:first] == 7.0).all() and (out[first + n:] == 7.0).all()
+            got.append(out[first:first + n])
+        assert all(np.array_equal(g, got[0]) for g in got[1:])
+    lib.release(mark)
+
+
 def test_winograd_rejects_unsupported(lib):
     import fastconv_amd as F
     for bad in [O.shape(1, 4, 8, 8, 4, 3, 3, 2, 2, 1), O.shape(1, 4, 8, 8, 4, 5, 5, 1, 1, 2),
