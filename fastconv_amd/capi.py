@@ -109,6 +109,7 @@ _ABI = {
     "fc_wino_conv_onepass": (C.c_int, [_vp, C.POINTER(WinoPlan), _vp, _vp, _vp, C.c_int, _vp]),
     "fc_wino_forward_onepass": (C.c_int, [_vp, C.POINTER(WinoPlan), _vp, _vp, _vp, C.c_int, C.c_int, _vp, _vp]),
     "fc_wino_prefer_onepass": (C.c_int, [C.POINTER(ConvShape)]),
+    "fc_wino_prefer_onepass_to_fused": (C.c_int, [C.POINTER(ConvShape)]),
     "fc_wino_forward_fused": (C.c_int, [_vp, C.POINTER(WinoPlan), _vp, _vp, _vp, C.c_int, C.c_int, _vp, _vp, _vp]),
     "fc_wino_forward": (C.c_int, [_vp, C.POINTER(WinoPlan), _vp, _vp, _vp, C.c_int, C.c_int,
                                   _vp, _vp, _vp, _vp]),

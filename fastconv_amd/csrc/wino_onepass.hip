@@ -392,18 +392,26 @@ extern "C" int fc_wino_conv_onepass(fc_context *ctx, const fc_wino_plan *plan, c
     return FC_OK;
 }
 
-extern "C" int fc_wino_prefer_onepass(const fc_conv_shape *s) {
-    if (!fc_shape_ok(s) || s->kh != 3 || s->kw != 3 || s->sh != 1 || s->sw != 1 || s->W < 8) return 0;
+// Whether the layer is one for the single kernel where V and M in memory are not the better way.
+static bool onepass_fills(const fc_conv_shape *s) {
+    if (!fc_shape_ok(s) || s->kh != 3 || s->kw != 3 || s->sh != 1 || s->sw != 1 || s->W < 8) return false;
     // at most four channels: a kernel of its own on the vector ALUs, the fastest Winograd path at every batch
-    if (fc_wino_smallc_applies(s)) return 1;
-    if (s->C < 16 || s->C > 64) return 0;
+    if (fc_wino_smallc_applies(s)) return true;
+    if (s->C < 16 || s->C > 64) return false;
     // one 16-tile x 64-channel block per workgroup, one workgroup per CU at a time: the layer must
     // bring a few blocks per CU (batch 1 layers do not).  Measured crossover against the staged
     // pipeline: about 200 blocks when one block covers all output channels, 500 otherwise.
     const long OH = fc_out_dim(s->H, s->pt, s->pb, 3, 1), OW = fc_out_dim(s->W, s->pl, s->pr, 3, 1);
     const long T = (long)s->N * ((OH + 5) / 6) * ((OW + 5) / 6);
     const long blocks = (T + kTB - 1) / kTB * ((s->K + kKB - 1) / kKB);
-    if (blocks < (s->K <= kKB ? 192 : 512)) return 0;
+    return blocks >= (s->K <= kKB ? 192 : 512);
+}
+
+extern "C" int fc_wino_prefer_onepass(const fc_conv_shape *s) {
+    if (!onepass_fills(s)) return 0;
+    if (fc_wino_smallc_applies(s)) return 1;
+    const long OH = fc_out_dim(s->H, s->pt, s->pb, 3, 1), OW = fc_out_dim(s->W, s->pl, s->pr, 3, 1);
+    const long T = (long)s->N * ((OH + 5) / 6) * ((OW + 5) / 6);
     if ((OW + 5) / 6 > kWinoMaxTilesW || s->K > kWinoMaxChannels) return 1;      // the staged pipeline does not take it
     // What the pipelines with V and M in memory pay is bytes, what this one pays is products and, for every 64 output
     // channels, an input transform: the line is a number of bytes per input channel.  It lies higher for C*K > 8192, with
@@ -419,6 +427,15 @@ extern "C" int fc_wino_prefer_onepass(const fc_conv_shape *s) {
     // the fused kernel needs no M.  Here / fused: 32 -> 256 62x62 n23 92 / 81, 159x159 n20 566 / 538, 32 -> 192 155x155
     // n15 301 / 281, 24 -> 256 48x48 n48 78 / 70, 16 -> 512 112x112 n32 547 / 531; 32 -> 128 112x112 n32 169 / 183.
     return s->C <= 32 && s->K >= 192 && bytes <= 2e9 && fc_wino_prefer_fused(s) ? 0 : 1;
+}
+
+// Against the fused pipeline (V in memory) the line lies elsewhere.  One block of output channels: the fused kernel brings
+// half as many workgroups up to 32 of them and is level up to 64.  More: the input transform of every 64 output channels
+// outweighs writing V once, but for the layers above.  Us here / fused: 40 -> 24 112x112 n9 34.8 / 41.8, 48 -> 32 87x87 n17
+// 45.8 / 48.2, 32 -> 32 120x120 n10 33.1 / 35.0, 48 -> 64 87x87 n17 55.7 / 54.1, 64 -> 64 56x56 n32 51.2 / 52.2, 53x53 n54 108.2 /
+// 99.9, 63x63 n50 108.0 / 107.9; 48 -> 96 100x100 n10 75.6 / 69.3, 64 -> 256 56x56 n32 170 / 153, 64 -> 1024 110x110 n6 406 / 361.
+extern "C" int fc_wino_prefer_onepass_to_fused(const fc_conv_shape *s) {
+    return onepass_fills(s) && (s->K <= kKB || fc_wino_prefer_onepass(s)) ? 1 : 0;
 }
 
 extern "C" int fc_wino_forward_onepass(fc_context *ctx, const fc_wino_plan *plan, const float *x_dev, const float *w_dev,

@@ -27,7 +27,7 @@ ConvWinoF63Layer::ConvWinoF63Layer(float *input, float *kernel, float *biasw, fl
     imgBlock_best = DefaultImagesPerBlock(oc, ic, tileN, n, kCacheBudget);
     gemmConfig_best = ConvWinoF63ZCLayer::DefaultConfig(oc, ic, ih, iw, pad_top, imgBlock_best);
     const fc_conv_shape whole = Shape((int)n);
-    if (fc_wino_prefer_onepass(&whole)) imgBlock_best = 0;      // 0: the single-kernel engine, whole batch
+    if (fc_wino_prefer_onepass_to_fused(&whole)) imgBlock_best = 0;      // 0: the single-kernel engine, whole batch
     enableOffKernel = enableOffKernel_best = 0;      // online, as the driver's -ts default
     tileBlock = ocBlock = icBlock = ocRegBlock = tileRegBlock = imgBlock = 0;
 }

@@ -313,9 +313,16 @@ int fc_wino_forward_onepass(fc_context *ctx, const fc_wino_plan *plan, const flo
  * moving V and M through HBM, the image at least 8 columns wide, and at least 512 blocks of
  * 16 tiles x 64 output channels -- 192 when one block covers all output channels -- i.e. not
  * at batch 1, and V and M too large for the staged pipeline to be faster, from 3.5 MB per input
- * channel on, 10 MB where C*K > 8192; and every layer with at most four input channels, at any
- * batch), else 0. */
+ * channel on, 10 MB where C*K > 8192; layers that the staged pipeline does not take; and every
+ * layer with at most four input channels, at any batch), else 0.  A layer for which it is 0
+ * runs fastest with V and, unless fc_wino_prefer_fused is 1, M in memory: up to 640 MB for the
+ * two (fc_wino_make_plan gives the sizes).  Where there is no room for them the single kernel
+ * still takes the layer if fc_wino_make_onepass_plan does. */
 int fc_wino_prefer_onepass(const fc_conv_shape *shape);
+
+/* 1 when the single-kernel path is expected to be faster than fc_wino_forward_fused, the choice
+ * of a caller with these two ways only (the blocked layer class, which has no M), else 0. */
+int fc_wino_prefer_onepass_to_fused(const fc_conv_shape *shape);
 
 /* All stages back to back: what winoF63_v1_single (winoF63ZC/winoF63ZC.h:5-6)
  * does in one call.  filter_ready != 0 skips the filter transform (U already

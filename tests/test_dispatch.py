@@ -52,3 +52,15 @@ def test_more_output_channels_than_the_staged_pipeline_takes_stay_on_the_single_
     assert lib.fc_prefer_winograd(C.byref(s)) == 1
     assert lib.fc_wino_prefer_onepass(C.byref(s)) == onepass
     assert onepass or not lib.fc_wino_prefer_fused(C.byref(s))
+
+
+@pytest.mark.parametrize("layer,onepass", [
+    ((17, 48, 32, 87), 1), ((9, 40, 24, 112), 1), ((10, 32, 32, 120), 1), ((32, 64, 64, 56), 1),      # staged is faster still
+    ((32, 64, 256, 56), 0), ((6, 64, 1024, 110), 0), ((10, 48, 96, 100), 0), ((23, 32, 256, 62), 0),
+    ((32, 64, 64, 224), 1), ((32, 64, 128, 112), 1), ((32, 3, 64, 224), 1), ((1, 64, 64, 56), 0),
+])
+def test_single_kernel_against_the_fused_pipeline_alone(lib, layer, onepass):
+    """What the blocked layer class asks, which has no staged pipeline."""
+    s = shape(*layer)
+    assert lib.fc_wino_prefer_onepass_to_fused(C.byref(s)) == onepass
+    assert onepass or not lib.fc_wino_prefer_onepass(C.byref(s))

@@ -163,6 +163,14 @@ def test_blocked_variant_uses_the_single_kernel_engine_and_tunes(tmp_path):
     assert "single kernel" not in out and "PASS" in out
 
 
+@pytest.mark.parametrize("ic,oc,size,batch,single", [(48, 32, 87, 17, True), (64, 256, 28, 64, False)])
+def test_blocked_class_chooses_between_its_own_two_ways(ic, oc, size, batch, single):
+    """Both layers are fastest on the staged pipeline, which the class does not have."""
+    out = _run([_exe("conv_test"), "-ic", str(ic), "-oc", str(oc), "-is", str(size), str(size), "-ks", "3", "3", "-ip", "1",
+                "-n", str(batch), "-i", "2", "-t", "16", "--strict", "--check-images", "1", "-a", "winograd", "--variant", "blocked"])
+    assert "PASS" in out and ("single kernel" in out) == single
+
+
 def test_layer_graph_runs_a_vgg_trunk_and_matches_the_host_chain():
     out = _run([_exe("net_test"), "-n", "2", "-is", "64", "-w", "4", "-i", "2"])
     m = re.search(r"Max relative error vs host chain: (\S+)", out)
