@@ -1,7 +1,7 @@
 // Runs a VGG-16 style convolution trunk (13 x [3x3 conv + bias + ReLU], 2x2 max pooling
 // between the blocks) back to back on the device through the layer graph of layer.h, and
 // checks the result against the same chain on the host (ConvNaiveLayer + ReLU + pooling).
-//   net_test [-n batch] [-is size] [-w width_divisor] [-i iterations] [--no-check] [--graph]
+//   net_test [-n batch] [-is size] [-w width_divisor] [-i iterations] [--no-check] [--graph] [--arena KB]
 // --graph records the trunk once and replays the recording (one launch call per forward pass).
 // -w 4 divides every channel count by 4 (a small trunk whose host check takes seconds).
 #include <math.h>
@@ -19,12 +19,14 @@
 
 int main(int argc, char **argv) {
     size_t batch = 1, size = 32, divisor = 4, iterations = 5;
+    size_t arena_kb = 0;
     bool check = true, graph = false;
     for (int i = 1; i < argc; i++) {
         if (!strcmp(argv[i], "-n") && i + 1 < argc) batch = strtoul(argv[++i], NULL, 10);
         else if (!strcmp(argv[i], "-is") && i + 1 < argc) size = strtoul(argv[++i], NULL, 10);
         else if (!strcmp(argv[i], "-w") && i + 1 < argc) divisor = strtoul(argv[++i], NULL, 10);
         else if (!strcmp(argv[i], "-i") && i + 1 < argc) iterations = strtoul(argv[++i], NULL, 10);
+        else if (!strcmp(argv[i], "--arena") && i + 1 < argc) arena_kb = strtoul(argv[++i], NULL, 10);
         else if (!strcmp(argv[i], "--no-check")) check = false;
         else if (!strcmp(argv[i], "--graph")) graph = true;
         else { fprintf(stderr, "Error: unknown argument '%s'\n", argv[i]); return 1; }
@@ -59,6 +61,7 @@ int main(int argc, char **argv) {
     size_t arena = (size_t)256 << 20;
     arena += batch * size * size * (64 / divisor) * 4 * 40;            // activations
     arena += batch * ((size + 5) / 6) * ((size + 5) / 6) * 256 * 2 * (128 / divisor + 32) + ((size_t)1 << 28);
+    if (arena_kb) arena = arena_kb * 1024;
     fastconv::Device::Configure(arena + ((size_t)64 << 20));
     feather::Net net(arena);
     net.SetInput(batch, 3, size, size);
@@ -75,8 +78,8 @@ int main(int argc, char **argv) {
         }
     }
     if (net.Init() != 0) return 1;
-    printf("Layer graph: %zu layers, shared scratch %zu KB, direct-convolution FLOP count %.3f GFLOP\n", net.num_layers(),
-           net.common_bytes() / 1024, flops / 1e9);
+    printf("Layer graph: %zu layers, shared scratch %zu KB, arena used %zu KB, direct-convolution FLOP count %.3f GFLOP\n",
+           net.num_layers(), net.common_bytes() / 1024, net.arena_used() / 1024, flops / 1e9);
     fastconv::Device &d = fastconv::Device::Get();
     net.Forward(input.data());
     d.Check(fc_sync(d.ctx()), "fc_sync");

@@ -42,7 +42,9 @@ int ConvolutionLayer::Init() {
     nnp_size ks = {k_, k_}, st = {s_, s_}, os = {_top_blobs[_name]->width(), _top_blobs[_name]->height()};
     const nnp_convolution_algorithm algo = select_algorithm(ks, st, os, shape_.C, oc_, shape_.N);
     winograd_ = algo == nnp_convolution_algorithm_winograd;
-    onepass_ = winograd_ && fc_wino_prefer_onepass(&shape_) != 0;
+    // the single kernel has neither V nor M: slower on some layers of few channels (up to 64), but without scratch
+    onepass_ = winograd_ && (fc_wino_prefer_onepass(&shape_) != 0 ||
+                             (no_scratch_ && shape_.C <= 64 && fc_wino_make_onepass_plan(&shape_, &wplan_) == FC_OK));
     if (onepass_) {
         // the whole layer in one kernel: no shared scratch at all
         d.Check(fc_wino_make_onepass_plan(&shape_, &wplan_), "fc_wino_make_onepass_plan");
@@ -59,6 +61,16 @@ int ConvolutionLayer::Init() {
         common_mempool->Request(m_off_ + (fused_ ? 0 : wplan_.M_bytes));
     } else {
         d.Check(fc_igemm_make_plan(&shape_, fc_igemm_default_config(&shape_), &iplan_), "fc_igemm_make_plan");
+        // the largest tile whose workgroups split the reduction among themselves needs no partial sums in memory
+        int area = 0;
+        for (int id = 0; no_scratch_ && iplan_.ws_bytes && id < fc_igemm_num_configs(); id++) {
+            fc_gemm_config c;
+            fc_igemm_plan plan;
+            if (fc_igemm_get_config(id, &c) != FC_OK || c.waves_k != 8 || c.bm * c.bn <= area) continue;
+            if (fc_igemm_make_plan(&shape_, id, &plan) != FC_OK) continue;
+            area = c.bm * c.bn;
+            iplan_ = plan;
+        }
         POOL_OK_OR_FAIL(private_mempool->Alloc(&Wp_, iplan_.Wp_bytes));
         float *tab = NULL;
         POOL_OK_OR_FAIL(private_mempool->Alloc(&tab, iplan_.table_bytes));
@@ -142,14 +154,21 @@ void Net::Add(Layer *layer) {
     layers_.push_back(layer);
 }
 
-int Net::Init() {
+bool Net::InitLayers() {
     for (size_t i = 0; i < layers_.size(); i++)
-        if (layers_[i]->Init() != 0) return -1;
-    if (common_->common_bytes() > 0 && !common_->Alloc()) {
-        fprintf(stderr, "Error: the arena is too small for the shared scratch (%zu bytes)\n", common_->common_bytes());
-        return -1;
-    }
-    return 0;
+        if (layers_[i]->Init() != 0) return false;
+    const size_t bytes = common_->common_bytes();
+    return bytes == 0 || (alloc_->largest_free() >= bytes && common_->Alloc());
+}
+
+int Net::Init() {
+    if (InitLayers()) return 0;
+    fprintf(stderr, "Net: the arena is too small for the shared scratch (%zu bytes); layers that can do without it will\n", common_->common_bytes());
+    common_->FreeAll();
+    for (size_t i = 0; i < layers_.size(); i++) layers_[i]->LeaveScratch();
+    if (InitLayers()) return 0;
+    fprintf(stderr, "Error: the arena is too small for the shared scratch (%zu bytes)\n", common_->common_bytes());
+    return -1;
 }
 
 int Net::Forward(const float *input_host) {

@@ -38,8 +38,14 @@ class Layer {
     }
     // Shapes (and allocates) the output blobs from the bottom blobs.
     virtual int GenerateTopBlobs() = 0;
-    // Other initialisation: plans, filter transforms, scratch requests to the common pool.
+    // Other initialisation: plans, filter transforms, scratch requests to the common pool.  Called again, after
+    // LeaveScratch(), when the arena has no room for the scratch of the fastest ways.
     virtual int Init() { return 0; }
+    // From now on without scratch where the layer has such a way; its buffers go back.
+    void LeaveScratch() {
+        private_mempool->FreeAll();
+        no_scratch_ = true;
+    }
     virtual int Forward() = 0;
 
     std::string name() { return _name; }
@@ -66,6 +72,7 @@ class Layer {
     CommonMemPool<float> *common_mempool;
     PrivateMemPool<float> *private_mempool;
     fastconv::RangeAllocator *_alloc = NULL;
+    bool no_scratch_ = false;
 };
 
 // kernel x kernel convolution, optional per-channel bias and ReLU fused into the epilogue.
@@ -118,8 +125,10 @@ class Net {
     size_t num_layers() const { return layers_.size(); }
     Layer *layer(size_t i) { return layers_[i]; }
     size_t common_bytes() const { return common_->common_bytes(); }
+    size_t arena_used() const { return alloc_->used(); }
 
    private:
+    bool InitLayers();
     fastconv::RangeAllocator *alloc_;
     CommonMemPool<float> *common_;
     Blob<float> *input_;

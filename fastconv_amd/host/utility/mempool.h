@@ -134,6 +134,7 @@ class CommonMemPool {
             if (it->second) alloc_->Free(it->second);
         common_ptr_map.clear();
         common_size_map.clear();
+        common_size = 0;
         return true;
     }
     void PrintStats() {

@@ -178,6 +178,16 @@ def test_layer_graph_runs_a_vgg_trunk_and_matches_the_host_chain():
     assert "17 layers" in out
 
 
+def test_layer_graph_fits_an_arena_without_room_for_the_fastest_way():
+    """Twelve 128x128 images: the 32-channel layers are fastest with V and M in memory, 95 MB that the layers after
+    them do not need.  An arena 30 MB short of that still runs the trunk, with those layers in the single kernel."""
+    args = [_exe("net_test"), "-n", "12", "-is", "128", "-w", "2", "-i", "2"]
+    scratch, used = (int(v) for v in re.search(r"shared scratch (\d+) KB, arena used (\d+) KB", _run(args + ["--no-check"])).groups())
+    assert scratch > 80 << 10
+    out = _run(args + ["--arena", str(used - (30 << 10))])
+    assert "PASS" in out and int(re.search(r"shared scratch (\d+) KB", out).group(1)) < 60 << 10
+
+
 def test_layer_graph_replayed_from_a_recording_matches_the_host_chain():
     out = _run([_exe("net_test"), "-n", "1", "-is", "64", "-w", "4", "-i", "3", "--graph"])
     m = re.search(r"Max relative error vs host chain: (\S+)", out)
