@@ -743,31 +743,47 @@ const fc_gemm_config kIgConfigs[] = {
 };
 const int kNumIgConfigs = sizeof(kIgConfigs) / sizeof(kIgConfigs[0]);
 
+// The column matrix of a pointwise layer is its input, read 16 bytes a lane where that is possible.
+bool ig_pointwise(const fc_conv_shape &s, int bk, bool x16) {
+    return s.kh == 1 && s.kw == 1 && s.sh == 1 && s.sw == 1 && s.pt == 0 && s.pb == 0 && s.pl == 0 && s.pr == 0 &&
+           (s.H * s.W) % 4 == 0 && s.C % bk == 0 && x16 && 4l * s.N * s.C * s.H * s.W < (1l << 32);
+}
+
+// No tap of any window leaves the image, and the reduction has no padding rows.
+bool ig_inside(const fc_conv_shape &s, int bk) {
+    const int OH = fc_out_dim(s.H, s.pt, s.pb, s.kh, s.sh), OW = fc_out_dim(s.W, s.pl, s.pr, s.kw, s.sw);
+    return s.pt == 0 && s.pl == 0 && (OH - 1) * s.sh + s.kh <= s.H && (OW - 1) * s.sw + s.kw <= s.W && (s.C * s.kh * s.kw) % bk == 0;
+}
+
+// Whether the products run on the bf16 matrix cores (a pointwise layer is a tap-major one whose only tap is inside): for
+// inputs below 2 GiB, but not for a pointwise layer of up to 64 output channels: that is bound by reading x, which the fp32
+// kernel does 16 bytes a lane (256 -> 64 channels at 56x56, batch 32: 35.8 us against 37.6; 64 -> 256: 35.0 against 34.4);
+// nor for a reduction of two or three stages, bound by its gathers and stores (3 -> 64 channels 3x3 at 224x224, batch 32:
+// 129 us against 139).
+bool ig_splits(const fc_conv_shape &s, const fc_gemm_config &c, bool x16) {
+    if (c.waves_k > 1 || c.bm % 64 != 0 || 4l * s.N * s.C * s.H * s.W >= (1l << 31) || (long)s.C * s.kh * s.kw <= 48) return false;
+    if (ig_pointwise(s, c.bk, x16) && s.K <= 64) return false;
+    return s.kh * s.kw <= 64 || (s.C % c.bk == 0 && ig_inside(s, c.bk));
+}
+
 template <class TL>
-void launch(fc_context *ctx, IgemmParams &p) {
+void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, IgemmParams &p) {
     const dim3 grid((unsigned)(((p.nKB * p.nPB + 7) / 8) * 8), (unsigned)p.splitK);
-    const bool pointwise = p.kh == 1 && p.kw == 1 && p.sh == 1 && p.sw == 1 && p.pt == 0 && p.pl == 0 &&
-                           p.OH == p.H && p.OW == p.W && (p.H * p.W) % 4 == 0 && p.C % TL::BK_ == 0 &&
-                           ((uintptr_t)p.x & 15) == 0 && p.xBytes < (1l << 32);
-    // no tap of any window leaves the image, and no padding rows in the reduction
-    const bool inside = p.pt == 0 && p.pl == 0 && (p.OH - 1) * p.sh + p.kh <= p.H && (p.OW - 1) * p.sw + p.kw <= p.W &&
-                        (p.C * p.kh * p.kw) % TL::BK_ == 0;
+    const bool x16 = ((uintptr_t)p.x & 15) == 0;
+    const bool pointwise = ig_pointwise(s, TL::BK_, x16), inside = ig_inside(s, TL::BK_);
     // one 32-bit byte offset with bit 31 to spare reaches every element of the tensor
     const bool buffer = p.xBytes < (1l << 31);
     const bool tapMajor = p.C % TL::BK_ == 0;      // the order fc_igemm_pack_filter laid the filter out in
     const dim3 block(TL::THREADS);
     if constexpr (TL::BM_ % 64 == 0) {
-        typedef std::conditional_t<std::is_same<TL, Ig0>::value, Ig0Split, TL> TS;
-        const dim3 splitBlock(TS::THREADS);
-        // Bf16 matrix cores (a pointwise layer is a tap-major one whose only tap is inside) for inputs below 2 GiB, but
-        // not for a pointwise layer of up to 64 output channels: that is bound by reading x, which the fp32 kernel does
-        // 16 bytes a lane (256 -> 64 channels at 56x56, batch 32: 35.8 us against 37.6; 64 -> 256: 34.4 against 32.6);
-        // nor for a reduction of two or three stages, bound by its gathers and stores (3 -> 64 channels 3x3 at 224x224,
-        // batch 32: 129 us against 139).
-        const bool split = buffer && p.Kred_pad >= 64 && !(pointwise && p.K <= 64);
-        if (split && tapMajor && inside) { igemm_conv_kernel<TS, IG_TAP_INSIDE, true><<<grid, splitBlock, 0, ctx->stream>>>(p); return; }
-        if (split && tapMajor && p.kh * p.kw <= 64) { igemm_conv_kernel<TS, IG_TAP_MASKED, true><<<grid, splitBlock, 0, ctx->stream>>>(p); return; }
-        if (split && p.kh * p.kw <= 64) { igemm_conv_kernel<TS, IG_BUF_MASKED, true><<<grid, splitBlock, 0, ctx->stream>>>(p); return; }
+        if (ig_splits(s, cfg, x16)) {
+            typedef std::conditional_t<std::is_same<TL, Ig0>::value, Ig0Split, TL> TS;
+            const dim3 splitBlock(TS::THREADS);
+            if (tapMajor && inside) igemm_conv_kernel<TS, IG_TAP_INSIDE, true><<<grid, splitBlock, 0, ctx->stream>>>(p);
+            else if (tapMajor) igemm_conv_kernel<TS, IG_TAP_MASKED, true><<<grid, splitBlock, 0, ctx->stream>>>(p);
+            else igemm_conv_kernel<TS, IG_BUF_MASKED, true><<<grid, splitBlock, 0, ctx->stream>>>(p);
+            return;
+        }
     }
     if (pointwise) igemm_conv_kernel<TL, IG_POINTWISE><<<grid, block, 0, ctx->stream>>>(p);
     else if (buffer && tapMajor && inside) igemm_conv_kernel<TL, IG_TAP_INSIDE><<<grid, block, 0, ctx->stream>>>(p);
@@ -815,17 +831,20 @@ extern "C" int fc_igemm_default_config(const fc_conv_shape *s) {
     // reduction is long enough to pay for its longer start, the grid is at least three rounds of its two workgroups per
     // CU without a split, and it pads no more.  At batch 32 and the like:
     // 256 -> 256 1x1 at 56x56 83 us against 95, 85 -> 128 3x3 at 150x150 337 against 420; with 32 rows 27.5 against 22.7.
-    if (best == 3 && Kr >= 256 && ceil(M / 128) * 128 == ceil(M / 64) * 64 && ceil(M / 128) * ceil(Np / 128) >= 1536) best = 0;
+    const bool split = ig_splits(*s, kIgConfigs[3], true);      // the rates above are those of the fp32 instructions
+    if (split && best == 3 && Kr >= 256 && ceil(M / 128) * 128 == ceil(M / 64) * 64 && ceil(M / 128) * ceil(Np / 128) >= 1536) best = 0;
     // A layer that this tile shape can only fill the chip with by splitting the reduction over workgroups
     // (a pass of partial sums through memory and a second launch) goes to the kernels that split it inside
     // the workgroup instead, while it is small enough for them.  Where 64x64 tiles waste nothing and the partial sums
     // fit the static workspace (so that fc_conv_implicit_gemm_static takes the plan, as before) the line is lower: at
     // 1.85 GFLOP the others are ahead or level (3x3 on 256 channels, two 28x28 images: 23 us against 28; 1x1
-    // 2048 -> 512 on sixteen 7x7 images: 24 against 23), at 3.3 and 3.7 GFLOP behind (40 against 36 and 42 against
-    // 37-40, five layers).
+    // 2048 -> 512 on sixteen 7x7 images: 24 against 23), at 3.7 GFLOP level or behind (42.8 against 41.5 and 42.1, 512
+    // channels, one 28x28 or four 14x14 images).  More than 15 parts are added up by too few workgroups: the others are
+    // ahead or level (512 channels, fourteen 7x7 images, 18 parts: 37.0 against 39.2; 1024 -> 512, eight, 28 parts: 47.2
+    // against 47.7; 5x5 512 -> 256, two 20x20 images, 30 parts, is the exception: 69 against 60).
     fc_igemm_plan plan;
     if (fc_igemm_make_plan(s, best, &plan) == FC_OK && plan.split_k > 1) {
-        const bool tiled = best == 3 && s->K % 64 == 0 && s->C % 16 == 0 && plan.split_k <= 15 && 2.0 * M * Kr * Np >= 3.2e9 &&
+        const bool tiled = split && best == 3 && s->K % 64 == 0 && s->C % 16 == 0 && plan.split_k <= 15 && 2.0 * M * Kr * Np >= 3.2e9 &&
                            plan.ws_bytes <= (size_t)FC_IGEMM_STATIC_WS_BYTES;
         const int ws = tiled ? -1 : fc_igemm_ws_choose(s, plan.Npix);
         if (ws >= 0) return kNumIgConfigs + ws;
@@ -1024,14 +1043,14 @@ static int igemm_run(fc_context *ctx, const fc_igemm_plan *plan, const float *x_
     if ((long)p.nKB * p.nPB >= (1l << 31)) return fail(FC_ERR_UNSUPPORTED, "grid too large");
     fc_stage_scope scope(ctx, timed ? FC_STAGE_IMPLICIT_GEMM : -1);
     switch (plan->config) {
-        case 0: launch<Ig0>(ctx, p); break;
-        case 1: launch<Ig1>(ctx, p); break;
-        case 2: launch<Ig2>(ctx, p); break;
-        case 3: launch<Ig3>(ctx, p); break;
-        case 4: launch<Ig4>(ctx, p); break;
-        case 5: launch<Ig5>(ctx, p); break;
-        case 6: launch<Ig6>(ctx, p); break;
-        case 7: launch<Ig7>(ctx, p); break;
+        case 0: launch<Ig0>(ctx, s, cfg, p); break;
+        case 1: launch<Ig1>(ctx, s, cfg, p); break;
+        case 2: launch<Ig2>(ctx, s, cfg, p); break;
+        case 3: launch<Ig3>(ctx, s, cfg, p); break;
+        case 4: launch<Ig4>(ctx, s, cfg, p); break;
+        case 5: launch<Ig5>(ctx, s, cfg, p); break;
+        case 6: launch<Ig6>(ctx, s, cfg, p); break;
+        case 7: launch<Ig7>(ctx, s, cfg, p); break;
         default: return fail(FC_ERR_INVALID, "unknown tile configuration");
     }
     FC_LAUNCH_CHECK(ctx, "igemm_conv_kernel");

@@ -64,3 +64,16 @@ def test_single_kernel_against_the_fused_pipeline_alone(lib, layer, onepass):
     s = shape(*layer)
     assert lib.fc_wino_prefer_onepass_to_fused(C.byref(s)) == onepass
     assert onepass or not lib.fc_wino_prefer_onepass(C.byref(s))
+
+
+@pytest.mark.parametrize("geo,bm", [
+    ((32, 256, 56, 56, 256, 1, 1, 1, 0), 128), ((12, 85, 150, 150, 128, 3, 3, 1, 1), 128),
+    ((39, 256, 230, 230, 256, 1, 1, 1, 0), 128), ((40, 256, 230, 230, 256, 1, 1, 1, 0), 64),      # 2 GiB of input between them
+    ((64, 64, 400, 400, 256, 3, 3, 2, 1), 64),
+])
+def test_large_implicit_gemm_tiles_only_where_they_run_on_the_bf16_matrix_cores(lib, geo, bm):
+    """128x128 tiles are ahead of 64x64 ones there, and behind on fp32 instructions, which inputs of 2 GiB run on."""
+    n, c, h, w, k, kh, kw, st, p = geo
+    s, g = capi.ConvShape(n, c, h, w, k, kh, kw, st, st, p, p, p, p), capi.GemmConfig()
+    assert lib.fc_igemm_get_config(lib.fc_igemm_default_config(C.byref(s)), C.byref(g)) == 0
+    assert (g.bm, g.bn, g.waves_k) == (bm, bm, 1)
