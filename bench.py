@@ -200,17 +200,12 @@ def takes_raw_filter_gemm(L, lay, filter_ready):
 
 
 def product_peak(L, lay, filter_ready=False):
-    """Peak of the matrix instructions that form a layer's products, by the rules of the kernels' launches."""
+    """Peak of the matrix instructions that form a layer's products."""
     if lay.algo == "im2col":
-        g = L.igemm_configs()[lay.iplan.config]
-        split = (g.waves_k <= 1 and g.bm % 64 == 0 and lay.iplan.Kred_pad >= 64 and lay.ks ** 2 <= 64 and
-                 4 * lay.N * lay.C * lay.H * lay.H < 1 << 31 and
-                 not (lay.ks == 1 and lay.st == 1 and lay.K <= 64 and lay.H * lay.H % 4 == 0 and lay.C % g.bk == 0))
+        split = L.igemm_splits_products(lay.iplan)
     else:
-        g = L.wino_configs()[lay.plan.gemm_config]
-        split = (lay.C > 48 and lay.C * lay.K > 8192 and g.bm % 64 == 0 and g.bn % 64 == 0 and g.bk == 16 and
-                 (g.bm * g.bn > 64 * 64 or lay.C >= 160 or 256.0 * (lay.C + lay.K) * lay.plan.T_pad <= 256e6) and
-                 lay.pipe != "onepass" and not takes_raw_filter_gemm(L, lay, filter_ready))
+        split = (lay.pipe != "onepass" and not takes_raw_filter_gemm(L, lay, filter_ready) and
+                 L.wino_splits_products(lay.plan))
     return PEAK_MFMA_SPLIT_TFLOPS if split else PEAK_MFMA_F32_TFLOPS
 
 

@@ -97,6 +97,7 @@ _ABI = {
     "fc_wino_filter_transform": (C.c_int, [_vp, C.POINTER(WinoPlan), _vp, _vp]),
     "fc_wino_input_transform": (C.c_int, [_vp, C.POINTER(WinoPlan), _vp, _vp]),
     "fc_wino_gemm": (C.c_int, [_vp, C.POINTER(WinoPlan), _vp, _vp, _vp]),
+    "fc_wino_gemm_splits_products": (C.c_int, [C.POINTER(WinoPlan)]),
     "fc_wino_gemm_raw_filter": (C.c_int, [_vp, C.POINTER(WinoPlan), _vp, _vp, _vp, C.c_int, C.c_int]),
     "fc_wino_raw_filter_gemm_applies": (C.c_int, [C.POINTER(WinoPlan)]),
     "fc_wino_prefer_raw_filter_gemm": (C.c_int, [C.POINTER(WinoPlan)]),
@@ -116,6 +117,7 @@ _ABI = {
     "fc_igemm_num_configs": (C.c_int, []),
     "fc_igemm_get_config": (C.c_int, [C.c_int, C.POINTER(GemmConfig)]),
     "fc_igemm_make_plan": (C.c_int, [C.POINTER(ConvShape), C.c_int, C.POINTER(IgemmPlan)]),
+    "fc_igemm_splits_products": (C.c_int, [C.POINTER(IgemmPlan)]),
     "fc_igemm_pack_filter": (C.c_int, [_vp, C.POINTER(IgemmPlan), _vp, _vp, _vp]),
     "fc_conv_implicit_gemm": (C.c_int, [_vp, C.POINTER(IgemmPlan), _vp, _vp, _vp, _vp, C.c_int, _vp, _vp]),
     "fc_conv_implicit_gemm_static": (C.c_int, [_vp, C.POINTER(IgemmPlan), _vp, _vp, _vp, _vp, C.c_int, _vp]),
@@ -344,6 +346,13 @@ class Library:
         if rc:
             raise FastConvError(rc, self.c.fc_status_string(rc).decode())
         return plan
+
+    def wino_splits_products(self, plan):
+        """Whether the products of this plan run on the bf16 matrix cores."""
+        return bool(self.c.fc_wino_gemm_splits_products(C.byref(plan)))
+
+    def igemm_splits_products(self, plan):
+        return bool(self.c.fc_igemm_splits_products(C.byref(plan)))
 
     # ---- Winograd stages
     def wino_filter_transform(self, plan, w, U):

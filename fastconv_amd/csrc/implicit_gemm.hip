@@ -901,6 +901,10 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
     return FC_OK;
 }
 
+extern "C" int fc_igemm_splits_products(const fc_igemm_plan *plan) {
+    return plan && plan->config >= 0 && plan->config < kNumIgConfigs && ig_splits(plan->shape, kIgConfigs[plan->config], true) ? 1 : 0;
+}
+
 static int ig_plan_check(fc_context *ctx, const fc_igemm_plan *plan) {
     if (!fc_ctx_ok(ctx)) return FC_ERR_STATE;
     if (!plan) return fc_set_error(ctx, FC_ERR_INVALID, "null plan", hipSuccess);

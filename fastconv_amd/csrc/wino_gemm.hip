@@ -527,6 +527,10 @@ extern "C" int fc_wino_gemm_default_config(const fc_conv_shape *s) {
     return best;
 }
 
+extern "C" int fc_wino_gemm_splits_products(const fc_wino_plan *plan) {
+    return plan && plan->gemm_config >= 0 && plan->gemm_config < kNumConfigs && fc_wino_gemm_splits(plan) ? 1 : 0;
+}
+
 extern "C" int fc_wino_gemm(fc_context *ctx, const fc_wino_plan *plan, const float *U_dev, const float *V_dev,
                             float *M_dev) {
     if (!fc_ctx_ok(ctx)) return FC_ERR_STATE;

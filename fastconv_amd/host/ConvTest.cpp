@@ -438,7 +438,9 @@ int main(int argc, char *argv[]) {
             // from the algorithmic work of the stage: Winograd products 2*64*K*C*T flop over T = N*ceil(OH/6)*ceil(OW/6)
             // tiles (the implicit GEMM: the direct-convolution count), input transform x once + V once, output
             // transform M once + y once, filter transform w once + U once.
-            const double kPeakTflops = 157.3, kPeakGbs = 8000.0;
+            // gemm_frac_mfma is of that fp32 peak and passes 1 where the products are split over the bf16 matrix cores (six bf16
+            // products for one, 2500 / 6 TFLOP/s); gemm_frac_peak is of the peak of the instructions that ran.
+            const double kPeakTflops = 157.3, kPeakSplitTflops = 2500.0 / 6.0, kPeakGbs = 8000.0;
             const bool wino = options.algorithm == nnp_convolution_algorithm_winograd;
             const double N = (double)options.batch, C = (double)input_channels, K = (double)output_channels;
             const double T = N * (double)((output_size.height + 5) / 6) * (double)((output_size.width + 5) / 6);
@@ -456,6 +458,20 @@ int main(int argc, char *argv[]) {
                     at += snprintf(roof + at, sizeof roof - at, ", \"%s\": null, \"%s\": null", name, frac_name);
                 }
             };
+            fc_conv_shape shp = {(int)options.batch, (int)input_channels, (int)input_size.height, (int)input_size.width,
+                                 (int)output_channels, (int)kernel_size.height, (int)kernel_size.width, (int)output_subsampling.height,
+                                 (int)output_subsampling.width, (int)input_padding.top, (int)input_padding.bottom,
+                                 (int)input_padding.left, (int)input_padding.right};
+            bool split = false;
+            fc_igemm_plan iplan;
+            fc_wino_plan wplan;
+            if (!wino) {
+                split = fc_igemm_make_plan(&shp, chosen_config, &iplan) == FC_OK && fc_igemm_splits_products(&iplan);
+            } else if (chosen_option != 0) {      // not the single kernel
+                if (chosen_option > 0) shp.N = chosen_option;
+                split = fc_wino_make_plan(&shp, chosen_config, &wplan) == FC_OK && fc_wino_gemm_splits_products(&wplan) &&
+                        (options.blocked_variant || kernel_transform_offline || !fc_wino_prefer_raw_filter_gemm(&wplan));
+            }
             field("gemm_tflops", gemm_flops, stage_ms[2], 1e12, kPeakTflops, "gemm_frac_mfma");
             field("input_tran_gbs", it_bytes, wino ? stage_ms[0] : 0.0, 1e9, kPeakGbs, "input_tran_frac_hbm");
             field("output_tran_gbs", ot_bytes, wino ? stage_ms[3] : 0.0, 1e9, kPeakGbs, "output_tran_frac_hbm");
@@ -465,14 +481,15 @@ int main(int argc, char *argv[]) {
                    "\"gflops\": %.2f, \"input_tran_ms\": %.6f, \"kernel_tran_ms\": %.6f, \"gemm_ms\": %.6f, "
                    "\"output_tran_ms\": %.6f, \"max_rel_err\": %.4e, \"naive_ms\": %.3f, \"naive_threads\": %zu, "
                    "\"checked_images\": %zu, \"images_per_block\": %d, \"kernel_transform\": \"%s\"%s, "
-                   "\"peak_mfma_tflops\": %.1f, \"peak_hbm_gbs\": %.0f}\n",
+                   "\"split_products\": %d, \"gemm_frac_peak\": %.4f, \"peak_mfma_tflops\": %.1f, \"peak_hbm_gbs\": %.0f}\n",
                    algorithm_name(options.algorithm),
                    (options.algorithm == nnp_convolution_algorithm_winograd && options.blocked_variant) ? "_blocked" : "",
                    options.batch, input_channels, output_channels, input_size.height, input_size.width,
                    kernel_size.height, kernel_size.width, output_subsampling.height, options.input_padding,
                    chosen_config, ms, gflops, stage_ms[0], stage_ms[1], stage_ms[2], stage_ms[3], err, naive_ms,
                    options.threads, options.check ? checked : (size_t)0, chosen_option,
-                   kernel_transform_offline < 0 ? "n/a" : kernel_transform_offline ? "offline" : "online", roof,
+                   kernel_transform_offline < 0 ? "n/a" : kernel_transform_offline ? "offline" : "online", roof, split ? 1 : 0,
+                   stage_ms[2] > 0.0 ? gemm_flops / (stage_ms[2] * 1e-3) / 1e12 / (split ? kPeakSplitTflops : kPeakTflops) : 0.0,
                    kPeakTflops, kPeakGbs);
         }
     }

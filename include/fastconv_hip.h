@@ -143,7 +143,10 @@ int fc_clock_probe_end(fc_context *ctx, double *mhz, int capacity, int *n_sample
  * (convLayer/winoF63ConvZC.cpp:25-174); here a configuration is a workgroup
  * tile BM (output channels) x BN (tiles) x BK (input channels) and a wave grid
  * (waves_m x waves_n wavefronts side by side over the tile, times waves_k
- * wavefronts that each take a share of the reduction). */
+ * wavefronts that each take a share of the reduction).  lds_bytes and the wave grid are
+ * those of the kernel that runs on fp32 matrix instructions; where a plan's products are
+ * split (fc_wino_gemm_splits_products, fc_igemm_splits_products) a tile takes
+ * 192 * (bm + bn) bytes of LDS, up to 72 KB, and the 128x128 one eight wavefronts. */
 typedef struct {
     int id;
     int bm, bn, bk;
@@ -212,11 +215,18 @@ int fc_wino_filter_input_transform(fc_context *ctx, const fc_wino_plan *plan,
                                    const float *x_dev, float *V_dev);
 
 /* M[f] = U[f]^T-layout product over input channels for all 64 frequencies in
- * one launch, on fp32 MFMA.  Replaces the depth x oc x tile loop nest calling
+ * one launch, at fp32 accuracy: on fp32 MFMA, or, where that is faster, as six products
+ * of three bf16 parts of each operand, which add up to it exactly.  Replaces the depth x oc x tile loop nest calling
  * TensorGEMMInnerKernel4x4x4_v3 (winoF63ZC/winoF63ZC.cpp:818-860,
  * winoF63ZC/TensorGEMMZC.cpp:443-583).  M is overwritten, never accumulated. */
 int fc_wino_gemm(fc_context *ctx, const fc_wino_plan *plan,
                  const float *U_dev, const float *V_dev, float *M_dev);
+/* 1 when the products of this plan are formed from bf16 parts (above; fc_wino_gemm_output_fused
+ * does as fc_wino_gemm, so that the two give the same bits for one plan), else 0.  The error of such a sum
+ * against 64 bits is 0.3 to 0.7 of the fp32 instructions', 1.03 where a single term is not zero;
+ * one plan always rounds alike, but plans of one layer with other batches or tiles may not.
+ * Values that are not finite, and sums from 2^80 on, are formed on fp32 MFMA in a second pass. */
+int fc_wino_gemm_splits_products(const fc_wino_plan *plan);
 
 /* The same stage fed by the untransformed filter w[K][C][3][3]: U = G g G^T is formed
  * in registers, lane by lane in the layout the MFMA takes its first operand in, and never
@@ -360,6 +370,9 @@ typedef struct {
 } fc_igemm_plan;
 
 int fc_igemm_make_plan(const fc_conv_shape *shape, int config, fc_igemm_plan *plan);
+/* As fc_wino_gemm_splits_products, for x at a multiple of 16 bytes (else a pointwise layer of up to 64
+ * output channels is split as well). */
+int fc_igemm_splits_products(const fc_igemm_plan *plan);
 
 /* Replaces pack_a_v2 (im2col/gemm_pack.cpp:192-260) as a one-time step. */
 int fc_igemm_pack_filter(fc_context *ctx, const fc_igemm_plan *plan, const float *w_dev,

@@ -77,3 +77,36 @@ def test_large_implicit_gemm_tiles_only_where_they_run_on_the_bf16_matrix_cores(
     s, g = capi.ConvShape(n, c, h, w, k, kh, kw, st, st, p, p, p, p), capi.GemmConfig()
     assert lib.fc_igemm_get_config(lib.fc_igemm_default_config(C.byref(s)), C.byref(g)) == 0
     assert (g.bm, g.bn, g.waves_k) == (bm, bm, 1)
+
+
+@pytest.mark.parametrize("n,c,k,h,tile,split", [
+    (1, 48, 200, 60, (128, 128), 0), (1, 49, 200, 60, (128, 128), 1), (1, 64, 128, 60, (128, 128), 0), (1, 64, 129, 60, (128, 128), 1),
+    (38, 64, 130, 60, (128, 128), 1), (39, 64, 130, 60, (128, 128), 0), (40, 96, 130, 60, (128, 128), 1),      # V and M of 320 MB
+    (1, 64, 130, 60, (64, 64), 0), (1, 65, 130, 60, (64, 64), 1), (36, 80, 130, 60, (64, 64), 1), (37, 80, 130, 60, (64, 64), 0),      # 256 MB
+    (30, 144, 130, 60, (64, 64), 0), (30, 145, 130, 60, (64, 64), 1), (1, 176, 200, 60, (256, 128), 0), (1, 177, 200, 60, (256, 128), 1),
+    (8, 512, 512, 28, (64, 32), 0),
+])
+def test_which_winograd_products_are_split(lib, n, c, k, h, tile, split):
+    s, g, plan = shape(n, c, k, h), capi.GemmConfig(), capi.WinoPlan()
+    for i in range(lib.fc_wino_gemm_num_configs()):
+        assert lib.fc_wino_gemm_get_config(i, C.byref(g)) == 0
+        if (g.bm, g.bn) != tile:
+            continue
+        assert lib.fc_wino_make_plan(C.byref(s), i, C.byref(plan)) == 0
+        assert lib.fc_wino_gemm_splits_products(C.byref(plan)) == (split if g.bk == 16 else 0)
+    assert lib.fc_wino_make_onepass_plan(C.byref(s), C.byref(plan)) == 0
+    assert lib.fc_wino_gemm_splits_products(C.byref(plan)) == 0 and lib.fc_wino_gemm_splits_products(None) == 0
+
+
+@pytest.mark.parametrize("geo,split", [
+    ((32, 256, 56, 56, 256, 1, 1, 0), 1), ((32, 256, 56, 56, 64, 1, 1, 0), 0), ((32, 256, 56, 56, 64, 1, 2, 0), 1),
+    ((1, 3, 32, 32, 64, 3, 1, 1), 0), ((1, 3, 32, 32, 64, 5, 1, 2), 1), ((1, 3, 32, 32, 64, 9, 1, 4), 0), ((1, 16, 32, 32, 64, 9, 1, 0), 1),
+    ((40, 256, 230, 230, 256, 1, 1, 0), 0),
+])
+def test_which_implicit_gemm_products_are_split(lib, geo, split):
+    n, c, h, w, k, ks, st, p = geo
+    s, g, plan = capi.ConvShape(n, c, h, w, k, ks, ks, st, st, p, p, p, p), capi.GemmConfig(), capi.IgemmPlan()
+    for i in range(lib.fc_igemm_num_configs()):
+        assert lib.fc_igemm_get_config(i, C.byref(g)) == 0
+        if lib.fc_igemm_make_plan(C.byref(s), i, C.byref(plan)) == 0:
+            assert lib.fc_igemm_splits_products(C.byref(plan)) == (split if g.waves_k == 1 and g.bm % 64 == 0 else 0), i

@@ -74,6 +74,18 @@ def test_json_line_reports_every_stage_against_its_roofline():
     assert 0.0 < j["gemm_frac_mfma"] < 1.0 and j["input_tran_gbs"] is None and j["output_tran_frac_hbm"] is None
 
 
+def test_json_line_names_the_peak_of_the_instructions_that_ran():
+    """A layer whose products are split over the bf16 matrix cores passes the fp32 peak; of their own it stays below."""
+    base = [_exe("conv_test"), "-ks", "3", "3", "-ip", "1", "-i", "5", "-t", "16", "--check-images", "1", "--strict", "--json",
+            "-a", "winograd"]
+    j = _json_line(_run(base + ["-ic", "512", "-oc", "512", "-is", "28", "28", "-n", "32"]))
+    assert j["split_products"] == 1 and j["gemm_frac_peak"] == pytest.approx(j["gemm_tflops"] / (2500 / 6), abs=2e-4)
+    assert 0.2 < j["gemm_frac_peak"] < 1.0
+    for args in (["-ic", "16", "-oc", "64", "-is", "56", "56", "-n", "4"], ["-ic", "512", "-oc", "512", "-is", "14", "14", "-n", "1"]):
+        j = _json_line(_run(base + args))      # few channels; straight from the 3x3 filter
+        assert j["split_products"] == 0 and j["gemm_frac_peak"] == pytest.approx(j["gemm_frac_mfma"], abs=2e-4)
+
+
 @pytest.mark.parametrize("variant", ["zc", "blocked"])
 @pytest.mark.parametrize("batch,C,H", [(64, 256, 56), (128, 256, 56), (64, 512, 28), (128, 512, 28), (64, 512, 14),
                                        (128, 512, 14)])

@@ -87,7 +87,7 @@ def test_winograd_gemm_split_products(lib, C, K, T):
 
 @pytest.mark.parametrize("C,K,N", [
     (48, 200, 1), (49, 200, 1),              # channels from which products are split, here with 128x128 tiles
-    (64, 130, 39), (64, 130, 40),            # V and M on either side of 320 MB with these
+    (64, 130, 38), (64, 130, 39),            # V and M on either side of 320 MB with these
     (64, 130, 1), (65, 130, 1),              # channels from which the smaller tiles follow
     (80, 130, 36), (80, 130, 37),            # V and M on either side of 256 MB with 64x64 tiles
     (144, 130, 30), (145, 130, 30),          # channels from which they follow at any size
