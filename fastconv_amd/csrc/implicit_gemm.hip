@@ -535,8 +535,9 @@ __global__ __launch_bounds__(TL::THREADS, TL::MIN_WAVES) void igemm_conv_kernel(
 // The same layer on the bf16 matrix cores at fp32 accuracy (see split_mfma.h), for inputs below 2 GiB.  A wavefront
 // takes 64 output channels or 64 pixels x 8 reduction rows at a time, a lane one channel or pixel: 8 loads through
 // buffer resources, a stage ahead, and one 16-byte word to LDS per part.  A lane's pixel is the same in every block it takes.
-// Measured at batch 32, fp32 instructions -> this, 64x64 tiles: 256 -> 256 3x3/2 at 28x28 82.5 -> 75.4 us, 7x7/2 stem
-// 91.3 -> 81.4, 512 -> 2048 1x1 at 7x7 39.2 -> 30.8, 64 -> 64 3x3 at 56x56 71.7 -> 60.7; 128x128: 256 -> 256 1x1 at 56x56 113 -> 83.
+// Measured at batch 32, fp32 instructions -> this, 64x64 tiles: 256 -> 256 3x3/2 at 28x28 84.2 -> 76.6 us, 7x7/2 stem
+// 91.4 -> 81.1, 512 -> 2048 1x1 at 7x7 39.4 -> 32.7, 64 -> 64 3x3 at 56x56 73.7 -> 63.0; 128x128: 256 -> 256 1x1 at 56x56
+// 113 -> 85.  The 64x64 one on a 3x3/2 layer: matrix pipes busy 31 % of the cycles, other vector instructions 48 %, LDS 31 %.
 template <class TL>
 struct IgSplit {
     static constexpr int A_WAVES = 2 * TL::BM_ / 64, B_WAVES = 2 * TL::BN_ / 64, WAVES = TL::THREADS / 64;   // blocks of a stage
@@ -835,7 +836,7 @@ extern "C" int fc_igemm_default_config(const fc_conv_shape *s) {
     // On the bf16 matrix cores 128x128 writes and reads the least LDS per product.  It takes over from 64x64 where the
     // reduction is long enough to pay for its longer start, the grid is at least three rounds of its two workgroups per
     // CU without a split, and it pads no more.  At batch 32 and the like:
-    // 256 -> 256 1x1 at 56x56 83 us against 95, 85 -> 128 3x3 at 150x150 337 against 420; with 32 rows 27.5 against 22.7.
+    // 256 -> 256 1x1 at 56x56 85 us against 98, 85 -> 128 3x3 at 150x150 345 against 418; with 32 rows 27.5 against 22.7.
     const bool split = ig_splits(*s, kIgConfigs[3], true);      // the rates above are those of the fp32 instructions
     if (split && best == 3 && Kr >= 256 && ceil(M / 128) * 128 == ceil(M / 64) * 64 && ceil(M / 128) * ceil(Np / 128) >= 1536) best = 0;
     // A layer that this tile shape can only fill the chip with by splitting the reduction over workgroups

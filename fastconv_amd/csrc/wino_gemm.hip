@@ -247,8 +247,9 @@ __device__ __forceinline__ void gemm_tile(const float *__restrict__ U, const flo
 // columns at a time, each lane one of them, splits the 8 floats it has fetched a stage ahead and writes one 16-byte
 // word per part.  The split runs beside the products of the other wavefronts.  128x128 tiles take eight wavefronts of 64x32
 // (four wavefronts of 64x64: 179 us where eight take 166, as two a SIMD do not cover each other's barriers).
-// Batch 32, fp32 instructions -> this: 256 -> 256 channels at 56x56 224 -> 166 us, 512 -> 512 at 28x28 239 -> 163,
-// 128 -> 128 at 112x112 220 -> 188 (bound by memory); 64x64 tiles: 512 -> 512 at 14x14 90 -> 71.
+// Batch 32, fp32 instructions -> this: 256 -> 256 channels at 56x56 225 -> 169 us (156 TFLOP/s; the matrix pipes are busy
+// 65 % of the cycles at the 1.6 GHz the power leaves, LDS 41 %), 512 -> 512 at 28x28 242 -> 166, 128 -> 128 at 112x112
+// 221 -> 191 (bound by memory); 64x64 tiles: 512 -> 512 at 14x14 95 -> 73.
 // Spreading the split between the products by hand (sched_group_barrier) gained nothing.
 template <class TL>
 struct SplitTile {
@@ -489,9 +490,9 @@ bool fc_wino_gemm_splits(const fc_wino_plan *plan) {
 // relative to 128x128x16 and by how evenly the grid fills the workgroup slots of the chip.  The
 // rates start from what each shape sustains on large layers (256 -> 256 channels at 56x56 and
 // 512 -> 512 at 28x28, batch 32).  The shapes of 64 and more run on the bf16 matrix cores
-// (128x128: 166 us against 224 with fp32 instructions on the first of these; 64x64: 199 against
-// 229), where the large tile is the furthest ahead: it writes and reads the least LDS per product.
-// 64x64 is level with it where it pads less (512 channels at 14x14: 68 us both) and ahead on
+// (128x128: 169 us against 225 with fp32 instructions on the first of these; 64x64: 199 against
+// 230), where the large tile is the furthest ahead: it writes and reads the least LDS per product.
+// 64x64 is level with it where it pads less (512 channels at 14x14: 70 us and 73) and ahead on
 // small grids; the shapes with a 32 stay on fp32 instructions, for layers whose 64-wide tile
 // would be mostly padding (512 channels at 28x28, batch 1: 14.7 us against 21).  Layers of few
 // channels stay on fp32 instructions whatever their tile: they are bound by memory (16 -> 64
@@ -519,7 +520,7 @@ extern "C" int fc_wino_gemm_default_config(const fc_conv_shape *s) {
         double fill = blocks / (ceil(blocks / slots) * slots);
         if (id == 0 && fewChannels && blocks > slots) fill = 1.0;
         // the large tile on the bf16 matrix cores needs its two workgroups per CU to hide their barriers
-        // (256 -> 256 channels at 56x56, one image: 128 workgroups, 16.7 us against 11.4 for 64x64)
+        // (256 -> 256 channels at 56x56, one image: 128 workgroups, 13.7 us against 11.5 for 64x64)
         if (id == 0 && !fewChannels && blocks < slots) fill -= 2.0 * (1.0 - fill);
         const double cost = kp * tp * cp / ((fewChannels ? kFp32Rate : kRate)[id] * (0.8 + 0.2 * fill));
         if (cost < bestCost) { bestCost = cost; best = id; }

@@ -416,7 +416,7 @@ extern "C" int fc_wino_prefer_onepass(const fc_conv_shape *s) {
     // What the pipelines with V and M in memory pay is bytes, what this one pays is products and, for every 64 output
     // channels, an input transform: the line is a number of bytes per input channel.  It lies higher for C*K > 8192, with
     // more output channels and from 49 input channels on the bf16 matrix cores.  Us here / staged, at (V+M in MB):
-    //   64 -> 256 56x56 n32 (262) 171 / 130, 64 -> 512 28x28 n64 (236) 184 / 122, 64 -> 1024 110x110 n6 (603) 406 / 341,
+    //   64 -> 256 56x56 n32 (262) 171 / 138, 64 -> 512 28x28 n64 (236) 184 / 126, 64 -> 1024 110x110 n6 (603) 406 / 343,
     //   64 -> 256 112x112 n32 (946) 518 / 538, 48 -> 320 111x111 n5 (170) 139 / 96, 48 -> 512 218x218 n4 (785) 404 / 486,
     //   32 -> 675 90x90 n5 (204) 116 / 104, 40 -> 812 215x215 n1 (283) 199 / 163, 24 -> 512 202x202 n2 (317) 123 / 148;
     //   C*K <= 8192: 64 -> 64 53x53 n54 (143) 109 / 65, 63x63 n50 (198) 109 / 97, 119x119 n20 (262) 115 / 129,
