@@ -25,42 +25,61 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));   // native vector: a
 // stage share one filter tap -- one in-image test and one window offset per stage instead of one per
 // gathered element, and consecutive rows are consecutive channels (no table lookups in the loop).
 // The packed filter and the row table follow whichever order the layer uses.
+// The split kernel (igemm_split_kernel) has orders of its own, padded so that a lane's 8 rows can be read without a look at
+// each: blocks of 16 channels, tap by tap within a block, so that the taps of a block find its pixels in the cache (tap-major
+// reads the whole input once per tap: 400 -> 32 channels 3x3/2 at 153x153, batch 12, 370 us against 221); or channel-major with every window row in runs of 8 or 4 columns.
 // Row table entry for reduction row kred (tap (r, s) of channel c):
 //   [2*kred]   = c*H*W + r*W + s      (offset from the window origin)
 //   [2*kred+1] = r << 16 | s          (31 << 16 | 31 for padding rows: a mask bit that is never set)
+enum { IG_ORDER_CHANNEL, IG_ORDER_TAP, IG_ORDER_BLOCK, IG_ORDER_ROW8, IG_ORDER_ROW4 };
+
 __global__ __launch_bounds__(256) void igemm_pack_filter_kernel(const float *__restrict__ w,
                                                                 float *__restrict__ Wp,
                                                                 int32_t *__restrict__ table, int K, int C,
-                                                                int kh, int kw, int H, int W, int Kred,
-                                                                int Kred_pad, int K_pad, int tapMajor) {
+                                                                int kh, int kw, int H, int W, int rows,
+                                                                int Kred_pad, int K_pad, int order) {
     const int k = blockIdx.x * 64 + (threadIdx.x & 63);
     const int kred = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (kred >= Kred_pad) return;
     int c = 0, r = 31, s = 31;
-    if (kred < Kred) {
-        if (tapMajor) {
+    bool real = kred < rows;
+    if (real) {
+        if (order == IG_ORDER_TAP) {
             const int t = kred / C;
             c = kred - t * C;
             r = t / kw;
             s = t - r * kw;
+        } else if (order == IG_ORDER_BLOCK) {
+            const int stage = kred / 16, block = stage / (kh * kw), t = stage - block * (kh * kw);
+            c = block * 16 + kred % 16;
+            r = t / kw;
+            s = t - r * kw;
+            real = c < C;
         } else {
-            c = kred / (kh * kw);
-            const int rs = kred - c * kh * kw;
-            r = rs / kw;
-            s = rs - r * kw;
+            const int run = order == IG_ORDER_ROW8 ? 8 : order == IG_ORDER_ROW4 ? 4 : 1;
+            const int width = (kw + run - 1) / run * run;      // rows of the reduction per window row
+            c = kred / (kh * width);
+            const int rs = kred - c * kh * width;
+            r = rs / width;
+            s = rs - r * width;
+            real = s < kw;
         }
     }
     if (k < K_pad)
-        Wp[(size_t)kred * K_pad + k] = (k < K && kred < Kred) ? w[((size_t)k * C + c) * (kh * kw) + r * kw + s] : 0.f;
+        Wp[(size_t)kred * K_pad + k] = (k < K && real) ? w[((size_t)k * C + c) * (kh * kw) + r * kw + s] : 0.f;
     if (blockIdx.x == 0 && (threadIdx.x & 63) == 0) {
-        table[2 * kred] = kred < Kred ? c * H * W + r * W + s : 0;
-        table[2 * kred + 1] = (r << 16) | s;
+        table[2 * kred] = real ? c * H * W + r * W + s : 0;
+        table[2 * kred + 1] = real ? (r << 16) | s : (31 << 16) | 31;
     }
 }
+
+// 16-byte words of 32 output channels and one stage of the split filter: three parts x two halves of 8 rows x 32 channels.
+constexpr int kSplitBlockWords = 3 * 64;
 
 struct IgemmParams {
     const float *x;
     const float *Wp;
+    const fc_uintx4 *Ws;           // the filter split into its parts, where products are split
     const int32_t *table;
     const float *bias;
     float *y;
@@ -532,185 +551,286 @@ __global__ __launch_bounds__(TL::THREADS, TL::MIN_WAVES) void igemm_conv_kernel(
     if (ig_decode_tile(p, &kb, &pb)) ig_tile<TL, MODE>(p, kb, pb, As, Bs);
 }
 
-// The same layer on the bf16 matrix cores at fp32 accuracy (see split_mfma.h), for inputs below 2 GiB.  A wavefront
-// takes 64 output channels or 64 pixels x 8 reduction rows at a time, a lane one channel or pixel: 8 loads through
-// buffer resources, a stage ahead, and one 16-byte word to LDS per part.  A lane's pixel is the same in every block it takes.
-// Measured at batch 32, fp32 instructions -> this, 64x64 tiles: 256 -> 256 3x3/2 at 28x28 84.2 -> 76.6 us, 7x7/2 stem
-// 91.4 -> 81.1, 512 -> 2048 1x1 at 7x7 39.4 -> 32.7, 64 -> 64 3x3 at 56x56 73.7 -> 63.0; 128x128: 256 -> 256 1x1 at 56x56
-// 113 -> 85.  The 64x64 one on a 3x3/2 layer: matrix pipes busy 31 % of the cycles, other vector instructions 48 %, LDS 31 %.
-template <class TL>
+// The same layer on the bf16 matrix cores at fp32 accuracy (see split_mfma.h), for inputs below 2 GiB.
+//
+// A wavefront owns all rows of 32 pixel columns, so that a column is gathered and split by the
+// wavefront that multiplies it and goes from memory to the matrix core without leaving its registers: a lane holds 8
+// consecutive reduction rows of one pixel, which is its share of a 32x32x16 product.  The filter has been split when it was
+// packed and goes to LDS by direct loads, one stage ahead, for all wavefronts of the workgroup.
+// What bounds it is the issue of vector memory: a load takes a CU about 20 cycles whatever its width, and a stage of a 128x128
+// tile takes 32 loads of columns and 12 of the filter, 880 cycles, beside 768 of products (both operands through registers,
+// 4 bytes a lane, took 64 loads).  Window rows in runs are 16 bytes a lane, 8 loads a stage.
+// Measured at batch 32, fp32 instructions -> both operands split in the kernel -> this: 256 -> 256 3x3/2 at 28x28 84 -> 75.5 -> 66.7
+// us, 7x7/2 stem 91 -> 79 -> 57, 64 -> 64 3x3 at 56x56 74 -> 62 -> 48, 256 -> 256 1x1 at 56x56 113 -> 83 -> 74.5, 512 -> 2048 1x1 at
+// 7x7 39 -> 32 -> 27.8; 32 -> 16 3x3 at 97x97, batch 55, (32 rows a tile) 112 -> 66.  Prefetch of the operands across a whole
+// stage with three LDS buffers in place of two: -3 to +8 %, two wavefronts a SIMD in place of four.
+template <int BM, int BN, int WAVES>
 struct IgSplit {
-    static constexpr int A_WAVES = 2 * TL::BM_ / 64, B_WAVES = 2 * TL::BN_ / 64, WAVES = TL::THREADS / 64;   // blocks of a stage
-    // enough wavefronts for both operands at once: the first take A, the others B; else every wavefront takes both
-    static constexpr bool APART = A_WAVES + B_WAVES <= WAVES;
-    static constexpr int A_LD = (A_WAVES + WAVES - 1) / WAVES, B_LD = (B_WAVES + WAVES - 1) / WAVES;
-    typedef fc_split_stage<TL::BM_, TL::BN_> Stage;
-    static constexpr int LDS_WORDS = 2 * Stage::WORDS;
+    static constexpr int BM_ = BM, BN_ = BN, THREADS = 64 * WAVES;
+    static constexpr int WN = BN / WAVES, MI = BM / 32, NI = WN / 32;
+    static constexpr int STAGE_WORDS = kSplitBlockWords * (BM / 32);      // of the filter
+    // the tile that forms values again that are not finite: same threads
+    typedef IgTile<64, 64, 16, 2, THREADS / 128> Again;
+    static constexpr int LDS_WORDS = 2 * STAGE_WORDS > Again::LDS_BYTES / 16 ? 2 * STAGE_WORDS : Again::LDS_BYTES / 16;
     // wavefronts per SIMD the two sums leave registers for
-    static constexpr int MIN_WAVES = TL::MI * TL::NI > 4 ? 1 : TL::MI * TL::NI > 1 ? 2 : 4;
-    static_assert(TL::BM_ % 64 == 0 && TL::BN_ % 64 == 0 && TL::BK_ == 16, "a wavefront fetches 64 rows or columns x 8 of the reduction");
-    static_assert(B_LD == 1 || B_WAVES % WAVES == 0, "no part-filled second block");
-    static_assert(B_LD == 1 || TL::THREADS % TL::BN_ == 0, "one pixel per lane");
+    static constexpr int MIN_WAVES = MI * NI > 2 ? 2 : 4;
+    static_assert(Again::THREADS == THREADS && BM % Again::BM_ == 0 && BN % Again::BN_ == 0, "same workgroup");
+};
+// Tile shape of a public configuration on the bf16 matrix cores (void: none).
+template <class TL> struct IgSplitOf { typedef void type; };
+
+// How the reduction rows of a stage lie in the input (orders of the reduction: ig_order).
+//   SP_INSIDE      16 channels of one window tap, no tap outside the image
+//   SP_MASKED      the same with taps outside the image
+//   SP_PAD         the same with channels past the last one
+//   SP_ROW8        two runs of 8 columns of a window row of one channel: 16-byte loads
+//   SP_ROW4        four runs of 4 columns
+enum { SP_INSIDE, SP_MASKED, SP_PAD, SP_ROW8, SP_ROW4 };
+
+template <int MI_, class S>
+struct IgSplitPart {
+    static constexpr int BM_ = S::BM_, BN_ = S::BN_, MI = MI_, NI = S::NI;
 };
 
-template <class TL, int MODE, bool SPLIT>
-__global__ __launch_bounds__(TL::THREADS, IgSplit<TL>::MIN_WAVES) void igemm_conv_kernel(const IgemmParams p) {
-    static_assert(SPLIT, "the kernel above is the other one");
-    typedef IgSplit<TL> S;
-    constexpr bool TAP = MODE == IG_TAP_MASKED || MODE == IG_TAP_INSIDE;
-    constexpr int BM = TL::BM_, BN = TL::BN_, MI = TL::MI, NI = TL::NI, A_LD = S::A_LD, B_LD = S::B_LD, WAVES = S::WAVES;
-    constexpr int A_PLANE = S::Stage::A_PLANE, B_PLANE = S::Stage::B_PLANE, WORDS = S::Stage::WORDS;
-    __shared__ fc_uintx4 smem[S::LDS_WORDS];
-    int kb, pb;
-    if (!ig_decode_tile(p, &kb, &pb)) return;
+// One workgroup tile, of which the first MI blocks of 32 rows of each wavefront hold output channels.
+template <class S, int MODE, int MI>
+__device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb, const int pb, fc_uintx4 *smem) {
+    constexpr bool ROW = MODE == SP_ROW8 || MODE == SP_ROW4;
+    constexpr int NI = S::NI, WAVES = S::THREADS / 64;
+    constexpr uint32_t OUTSIDE = 0x80000000u;      // past the end of x whatever scalar offset is added: reads 0
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm0 = (wave / TL::WGN_) * TL::WM, wn0 = (wave % TL::WGN_) * TL::WN;
+    const int wn0 = wave * S::WN;
     const int lrow = lane >> 5, lcol = lane & 31;
     const int nStagesAll = p.Kred_pad / 16;
     const int sBegin = blockIdx.y * p.stagesPerSplit, sEnd = min(sBegin + p.stagesPerSplit, nStagesAll);
 
-    // block numbers of this wavefront: depth half = block * 64 / width, first row or column = block * 64 % width
-    const int bWave = S::APART ? wave - S::A_WAVES : wave;
-    const bool takesA = wave < S::A_WAVES, takesB = bWave >= 0 && bWave < S::B_WAVES;
-
-    // filter: rows of Wp from a uniform pointer
-    const float *asrc[A_LD];
+    // pixels of this lane: byte offset of the window in the tensor, window rows and columns outside the image
+    uint32_t pixByte[NI], rowBad[NI], colBad[NI];
+    bool before = false;      // a window that starts before the first element of x
 #pragma unroll
-    for (int j = 0; j < A_LD; j++) {
-        const int e = (wave + j * WAVES) * 64;
-        asrc[j] = uniform_ptr(p.Wp + (size_t)(sBegin * 16 + 8 * (e / BM)) * p.K_pad + (size_t)kb * BM + e % BM);
-    }
-    // pixel: byte offset of its window in the tensor and the taps that lie outside the image
-    uint32_t pixByte = 0, invLo = ~0u, invHi = ~0u;
-    const long pix = (long)pb * BN + (bWave * 64) % BN + lane;
-    if (takesB && pix < p.Npix) {
-        const uint32_t n = fc_div((uint32_t)pix, p.divOHW);
-        const uint32_t pp = (uint32_t)pix - n * (uint32_t)(p.OH * p.OW);
-        const uint32_t oh = fc_div(pp, p.divOW), ow = pp - oh * p.OW;
-        const int ih0 = (int)oh * p.sh - p.pt, iw0 = (int)ow * p.sw - p.pl;
-        pixByte = 4u * (n * (uint32_t)(p.C * p.H * p.W) + (uint32_t)(ih0 * p.W + iw0));
-        if (MODE != IG_TAP_INSIDE) {
-            uint32_t rowBits = 0;
-            for (int q = 0; q < p.kw; q++) rowBits |= ((unsigned)(iw0 + q) < (unsigned)p.W) ? 0u : (1u << q);
-            uint64_t inv = 0;
-            for (int r = 0; r < p.kh; r++) {
-                const uint32_t bits = ((unsigned)(ih0 + r) < (unsigned)p.H) ? rowBits : ((1u << p.kw) - 1u);
-                if (r * p.kw < 64) inv |= (uint64_t)bits << (r * p.kw);
+    for (int ni = 0; ni < NI; ni++) {
+        const long pix = (long)pb * S::BN_ + wn0 + ni * 32 + lcol;
+        pixByte[ni] = OUTSIDE;
+        rowBad[ni] = colBad[ni] = ~0u;
+        if (pix < p.Npix) {
+            const uint32_t n = fc_div((uint32_t)pix, p.divOHW);
+            const uint32_t pp = (uint32_t)pix - n * (uint32_t)(p.OH * p.OW);
+            const uint32_t oh = fc_div(pp, p.divOW), ow = pp - oh * p.OW;
+            const int ih0 = (int)oh * p.sh - p.pt, iw0 = (int)ow * p.sw - p.pl;
+            pixByte[ni] = 4u * (n * (uint32_t)(p.C * p.H * p.W) + (uint32_t)(ih0 * p.W + iw0));
+            if (!ROW) pixByte[ni] += 8u * lrow * 4u * (uint32_t)(p.H * p.W);      // the lane's first channel of a stage
+            if (MODE != SP_INSIDE) {
+                for (int r = 0; r < p.kh; r++) rowBad[ni] &= (unsigned)(ih0 + r) < (unsigned)p.H ? ~(1u << r) : ~0u;
+                for (int q = 0; q < p.kw; q++) colBad[ni] &= (unsigned)(iw0 + q) < (unsigned)p.W ? ~(1u << q) : ~0u;
             }
-            if (p.kh * p.kw < 64) inv |= ~0ull << (p.kh * p.kw);
-            invLo = (uint32_t)inv;
-            invHi = (uint32_t)(inv >> 32);
+            before |= (int)pixByte[ni] < 0;
         }
     }
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.x), 0, (int)p.xBytes, 0x00020000);
+    auto load1 = [&](const uint32_t voff, const uint32_t soff) __attribute__((always_inline)) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xres, voff, soff, 0));
+    };
 
-    // tap-major order: the tap and the first channel of the stage, counted in scalar registers
+    float raw[NI][8];
+    // -- blocks of channels: the tap and the first channel of the stage, counted in scalar registers
     const uint32_t chanStep = 4u * (uint32_t)(p.H * p.W);
-    int tapT = 0, tapR = 0, tapS = 0, tapC = 0;
-    if (TAP) {
-        const int stagesPerTap = p.C / 16;
-        tapT = sBegin / stagesPerTap;
-        tapC = (sBegin - tapT * stagesPerTap) * 16;
-        tapR = tapT / p.kw;
-        tapS = tapT - tapR * p.kw;
-    }
-    // Where the operands are fetched by different wavefronts and the taps' masks take registers too they share theirs: six
-    // wavefronts a SIMD in place of five (7x7/2 stem, batch 32: 81.1 us for 82.9; the other gathers lose 1 to 3 % by it).
-    constexpr bool SHARED = S::APART && MODE == IG_BUF_MASKED;
-    static_assert(!SHARED || (A_LD == 1 && B_LD == 1), "one block a wavefront");
-    float ra[A_LD][8], rb2[SHARED ? 1 : B_LD][8];
-    float (*const rb)[8] = SHARED ? ra : rb2;
-    uint32_t laneOff = 4u * lane;
-    // fetches stage s; stages are fetched in order
-    auto fetch = [&](const int s) __attribute__((always_inline)) {
-        if (takesA) {
-            asm volatile("" : "+v"(laneOff));
+    int tapR = 0, tapS = 0, tapC = 0;
+    uint32_t voff[NI];
+    auto tap = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < A_LD; j++) {
-                const float *b = asrc[j];
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    ra[j][i] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(b) + laneOff);
-                    b = uniform_ptr(b + p.K_pad);
-                }
-                asrc[j] = uniform_ptr(b + (size_t)8 * p.K_pad);
-            }
-        }
-        if (!takesB) return;
-        if (TAP) {
-            const uint32_t voff = pixByte + 4u * (uint32_t)(tapR * p.W + tapS);
-            // last, as a border pixel's window starts at a negative (wrapped) offset
-            uint32_t poison = 0;
-            if (MODE == IG_TAP_MASKED) {
-                const uint32_t word = tapT < 32 ? invLo : invHi;
-                poison = ((word >> (tapT & 31)) & 1u) << 31;
-            }
-#pragma unroll
-            for (int j = 0; j < B_LD; j++) {
-                const uint32_t chan0 = (uint32_t)(tapC + 8 * ((bWave + j * WAVES) * 64 / BN)) * chanStep;
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    rb[j][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                   xres, (voff + (chan0 + (uint32_t)i * chanStep)) | poison, 0, 0));
-            }
-            tapC += 16;
-            if (tapC == p.C) {
-                tapC = 0;
-                tapT++;
-                if (++tapS == p.kw) { tapS = 0; tapR++; }
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < B_LD; j++)
-                ig_gather_rows_buf<true>(rb[j], xres, pixByte, invLo, invHi, p.table, s * 16 + 8 * ((bWave + j * WAVES) * 64 / BN), 1,
-                                         p.kw, std::make_integer_sequence<int, 8>());
+        for (int ni = 0; ni < NI; ni++) {
+            voff[ni] = pixByte[ni] + 4u * (uint32_t)(tapR * p.W + tapS);
+            if (MODE != SP_INSIDE) voff[ni] = ((rowBad[ni] >> tapR) | (colBad[ni] >> tapS)) & 1u ? OUTSIDE : voff[ni];
         }
     };
-    auto park = [&](const int buf) __attribute__((always_inline)) {
-        fc_uintx4 *const dst = smem + buf * WORDS + lane;
-        if (takesA) {
+    // -- row orders: table entries of the runs of the stage to fetch, fetched themselves a stage before
+    constexpr int RUNS = MODE == SP_ROW8 ? 2 : 4, RUN = 16 / RUNS;
+    int runOff[RUNS], runTap[RUNS];
+    uint32_t cols[NI][2], rowVoff[NI][2];      // of the stage in `raw`: columns of the runs inside the image, offsets
+    auto table = [&](const int s) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < A_LD; j++) fc_split8(ra[j], dst + (wave + j * WAVES) * 64, A_PLANE);
+        for (int u = 0; u < RUNS; u++) {
+            runOff[u] = p.table[2 * (16 * s + RUN * u)];
+            runTap[u] = p.table[2 * (16 * s + RUN * u) + 1];
         }
-        if (takesB) {
+    };
+    if (ROW) {
+        table(sBegin);
+    } else {
+        const int block = sBegin / (p.kh * p.kw), t = sBegin - block * (p.kh * p.kw);
+        tapC = block * 16;
+        tapR = t / p.kw;
+        tapS = t - tapR * p.kw;
+        tap();
+    }
+    // fetches stage s; stages are fetched in order
+    auto fetch = [&](const int s) __attribute__((always_inline)) {
+        if (ROW) {
 #pragma unroll
-            for (int j = 0; j < B_LD; j++) fc_split8(rb[j], dst + 3 * A_PLANE + (bWave + j * WAVES) * 64, B_PLANE);
+            for (int v = 0; v < RUNS / 2; v++) {
+                const int off = lrow ? runOff[RUNS / 2 + v] : runOff[v], rs = lrow ? runTap[RUNS / 2 + v] : runTap[v];
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++) {
+                    const uint32_t vo = (rowBad[ni] >> (rs >> 16)) & 1u ? OUTSIDE : pixByte[ni] + 4u * (uint32_t)off;
+                    cols[ni][v] = ~colBad[ni] >> (rs & 0xffff);
+                    rowVoff[ni][v] = vo;
+#pragma unroll
+                    for (int h = 0; h < RUN / 4; h++) {
+                        const floatx4 d = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xres, vo, 16 * h, 0));
+#pragma unroll
+                        for (int j = 0; j < 4; j++) raw[ni][v * RUN + 4 * h + j] = d[j];
+                    }
+                }
+            }
+            table(min(s + 1, nStagesAll - 1));
+            return;
         }
+        const int left = p.C - tapC - 8 * lrow;      // channels of the lane's 8 that exist
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int c = MODE == SP_PAD ? min(tapC + i, p.C - 1) : tapC + i;
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++)
+                raw[ni][i] = load1(MODE == SP_PAD && i >= left ? OUTSIDE : voff[ni], (uint32_t)c * chanStep);
+        }
+        tapS++;
+        const bool row = tapS == p.kw;
+        tapS = row ? 0 : tapS;
+        tapR += row ? 1 : 0;
+        const bool all = tapR == p.kh;
+        tapR = all ? 0 : tapR;
+        tapC += all ? 16 : 0;
+        tap();
+    };
+    // the stage in `raw` as operand words of the three parts
+    fc_uintx4 b[NI][3];
+    // readAgain: runs that start before x are read again, element by element (whether a 16-byte load there gives the elements
+    // inside x is left open)
+    auto split = [&](auto readAgain) __attribute__((always_inline)) {
+        if (ROW) {
+            if constexpr (decltype(readAgain)::value) {
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const uint32_t vo = rowVoff[ni][i / RUN], at = vo + 4u * (uint32_t)(i % RUN);
+                        const float d = load1((int)at < 0 ? OUTSIDE : at, 0);      // (an immediate offset would not wrap)
+                        raw[ni][i] = vo != OUTSIDE && (int)vo < 0 ? d : raw[ni][i];
+                    }
+            }
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const int keep = (int)(cols[ni][i / RUN] << (31 - i % RUN)) >> 31;
+                    raw[ni][i] = __builtin_bit_cast(float, __builtin_bit_cast(int, raw[ni][i]) & keep);
+                }
+        }
+#pragma unroll
+        for (int ni = 0; ni < NI; ni++) fc_split8(raw[ni], b[ni], 1);
+    };
+    // filter words of the next stage to LDS: whole wavefronts, 16 bytes a lane
+    constexpr int PIECES = MI * kSplitBlockWords / 64;
+    const fc_uintx4 *fbase = p.Ws + ((size_t)sBegin * (p.K_pad / 32) + (size_t)kb * (S::BM_ / 32)) * kSplitBlockWords;
+    const size_t fstep = (size_t)(p.K_pad / 32) * kSplitBlockWords;
+    auto filter = [&](const int buf) __attribute__((always_inline)) {
+        const fc_uintx4 *src = uniform_ptr(fbase);
+#pragma unroll
+        for (int i = 0; i < (PIECES + WAVES - 1) / WAVES; i++) {
+            const int piece = wave + i * WAVES;
+            if (PIECES % WAVES == 0 || piece < PIECES)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + piece * 64 + lane),
+                                                 (__attribute__((address_space(3))) void *)(smem + buf * S::STAGE_WORDS + piece * 64), 16, 0, 0);
+        }
+        fbase = uniform_ptr(fbase + fstep);
     };
 
     floatx16 acc[MI][NI], small[MI][NI];
     fc_zero<MI, NI>(acc);
     fc_zero<MI, NI>(small);
-    const int aFrag = lrow * BM + wm0 + lcol, bFrag = 3 * A_PLANE + lrow * BN + wn0 + lcol;
-
-    fetch(sBegin);
-    park(0);
-    if (sBegin + 1 < sEnd) fetch(sBegin + 1);
-    __syncthreads();
-    for (int s = sBegin; s < sEnd; s++) {
+    // more: a stage follows
+    auto stage = [&](const int s, const bool more, auto readAgain) __attribute__((always_inline)) {
         const int buf = (s - sBegin) & 1;
-        const fc_uintx4 *cur = smem + buf * WORDS;
-        fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc, small);
-        if (s + 1 < sEnd) {
-            park(buf ^ 1);
-            if (s + 2 < sEnd) fetch(s + 2);
+        split(readAgain);
+        __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): this wavefront's filter words of the stage are in LDS
+        __syncthreads();                         // and those of the others, which have read the stage before
+        const fc_uintx4 *as = smem + buf * S::STAGE_WORDS + lane;
+        fc_bf16x8 a[3][MI];
+#pragma unroll
+        for (int q = 2; q >= 0; q--)
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++) a[q][mi] = __builtin_bit_cast(fc_bf16x8, as[mi * kSplitBlockWords + q * 64]);
+        if (more) {      // (behind the reads: the compiler has reads of LDS wait for direct loads before them)
+            filter(buf ^ 1);
+            fetch(s + 1);
         }
-        __syncthreads();
+        constexpr int pa[5] = {2, 1, 0, 1, 0}, pb[5] = {0, 1, 2, 0, 1};
+#pragma unroll
+        for (int q = 0; q < 5; q++)
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                for (int ni = 0; ni < NI; ni++)
+                    small[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[q]][mi], __builtin_bit_cast(fc_bf16x8, b[ni][pb[q]]), small[mi][ni], 0, 0, 0);
+#pragma unroll
+        for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][mi], __builtin_bit_cast(fc_bf16x8, b[ni][0]), acc[mi][ni], 0, 0, 0);
+    };
+    filter(0);
+    fetch(sBegin);
+    int s = sBegin;
+    if constexpr (ROW) {
+        // stages of the first channel, where windows of the first image may start before x
+        const int stagesBefore = __builtin_amdgcn_readfirstlane(__any(before) ? (p.kh * ((p.kw + RUN - 1) / RUN) * RUN + 15) / 16 : 0);
+#pragma unroll 1
+        for (; s < sEnd && s < stagesBefore; s++) stage(s, s + 1 < sEnd, std::true_type());
+#pragma unroll 1
+        for (; s < sEnd; s++) stage(s, s + 1 < sEnd, std::false_type());
+    } else {
+#pragma unroll 1
+        for (; s + 1 < sEnd; s++) stage(s, true, std::false_type());
+        stage(s, false, std::false_type());
     }
     fc_join<MI, NI>(acc, small);
     const bool again = __syncthreads_or(fc_not_finite<MI, NI>(acc));
-    ig_store_tile<TL>(acc, p, again ? nullptr : p.bias, again ? 0 : p.relu, kb, pb, wm0, wn0, lrow, lcol);
+    ig_store_tile<IgSplitPart<MI, S>>(acc, p, again ? nullptr : p.bias, again ? 0 : p.relu, kb, pb, 0, wn0, lrow, lcol);
     if (again) {
-        // 64x64 at a time, which leaves the registers to the loop above
-        typedef std::conditional_t<TL::THREADS == 512, TL, IgTile<64, 64, 16, 2, TL::THREADS / 128>> Sub;
-        static_assert(Sub::THREADS == TL::THREADS && Sub::LDS_BYTES <= 16 * S::LDS_WORDS, "same workgroup");
+        // a smaller tile at a time, which leaves the registers to the loop above; the table knows any order
+        typedef typename S::Again Sub;
         float *const f = reinterpret_cast<float *>(smem);
-        constexpr int QM = BM / Sub::BM_, QN = BN / Sub::BN_;
+        constexpr int QM = S::BM_ / Sub::BM_, QN = S::BN_ / Sub::BN_;
         __syncthreads();      // the whole tile is in y, or in the partial sums
         for (int q = 0; q < QM * QN; q++)
-            ig_tile<Sub, MODE, true>(p, kb * QM + q / QN, pb * QN + q % QN, reinterpret_cast<float (*)[16 * Sub::BM_]>(f),
+            ig_tile<Sub, IG_GATHER, true>(p, kb * QM + q / QN, pb * QN + q % QN, reinterpret_cast<float (*)[16 * Sub::BM_]>(f),
                                      reinterpret_cast<float (*)[16 * Sub::BN_]>(f + 2 * 16 * Sub::BM_));
     }
+}
+
+template <class S, int MODE>
+__global__ __launch_bounds__(S::THREADS, (MODE == SP_ROW4 || MODE == SP_INSIDE) && S::MIN_WAVES > 3 ? 3 : S::MIN_WAVES) void igemm_split_kernel(const IgemmParams p) {
+    __shared__ fc_uintx4 smem[S::LDS_WORDS];
+    int kb, pb;
+    if (!ig_decode_tile(p, &kb, &pb)) return;
+    // 32 rows of a 64-row tile past the last output channel are not multiplied
+    if (S::BM_ == 64 && p.K - kb * 64 <= 32) ig_split_tile<S, MODE, 1>(p, kb, pb, smem);
+    else ig_split_tile<S, MODE, S::MI>(p, kb, pb, smem);
+}
+
+// The packed filter as operand words: [stage][block of 32 output channels][part][half of the stage][channel], 16 bytes each,
+// after the fp32 filter (which forms values again that are not finite).
+__global__ __launch_bounds__(256) void igemm_split_filter_kernel(const float *__restrict__ Wp, fc_uintx4 *__restrict__ Ws, int K_pad, long total) {
+    const long id = (long)blockIdx.x * 256 + threadIdx.x;
+    if (id >= total) return;
+    const int lane = (int)(id & 63), row = lane & 31, half = lane >> 5;
+    const long block = id >> 6;      // stage * (K_pad / 32) + block of channels
+    const long stage = block / (K_pad / 32), kb = block - stage * (K_pad / 32);
+    const float *src = Wp + (size_t)(16 * stage + 8 * half) * K_pad + kb * 32 + row;
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = src[(size_t)i * K_pad];
+    fc_split8(v, Ws + (size_t)block * kSplitBlockWords + lane, 64);
 }
 
 // Sums the partial results of a split reduction in split order (so the result does
@@ -732,7 +852,6 @@ __global__ __launch_bounds__(256) void igemm_reduce_kernel(const float *__restri
 }
 
 typedef IgTile<128, 128, 16, 2, 2> Ig0;
-typedef IgTile<128, 128, 16, 2, 4> Ig0Split;      // eight wavefronts, as in wino_gemm.hip
 typedef IgTile<64, 128, 16, 1, 2> Ig1;
 typedef IgTile<128, 64, 16, 2, 1> Ig2;
 typedef IgTile<64, 64, 16, 2, 2> Ig3;
@@ -740,6 +859,14 @@ typedef IgTile<32, 64, 16, 1, 1> Ig4;
 typedef IgTile<256, 128, 16, 2, 2> Ig5;
 typedef IgTile<128, 256, 16, 2, 2> Ig6;
 typedef IgTile<64, 256, 16, 1, 4> Ig7;
+template <> struct IgSplitOf<Ig0> { typedef IgSplit<128, 128, 4> type; };
+template <> struct IgSplitOf<Ig1> { typedef IgSplit<64, 128, 4> type; };
+template <> struct IgSplitOf<Ig2> { typedef IgSplit<128, 64, 2> type; };
+template <> struct IgSplitOf<Ig3> { typedef IgSplit<64, 64, 2> type; };
+// (a wavefront's registers hold the two sums of 128x32 at most)
+template <> struct IgSplitOf<Ig5> { typedef IgSplit<128, 128, 4> type; };
+template <> struct IgSplitOf<Ig6> { typedef IgSplit<128, 128, 4> type; };
+template <> struct IgSplitOf<Ig7> { typedef IgSplit<64, 128, 4> type; };
 
 const fc_gemm_config kIgConfigs[] = {
 #define FC_CFG(id, T) {id, T::BM_, T::BN_, T::BK_, T::WGM_, T::WGN_, T::LDS_BYTES, 1}
@@ -766,36 +893,115 @@ bool ig_inside(const fc_conv_shape &s, int bk) {
 // kernel does 16 bytes a lane (256 -> 64 channels at 56x56, batch 32: 35.8 us against 37.6; 64 -> 256: 35.0 against 34.4);
 // nor for a reduction of two or three stages, bound by its gathers and stores (3 -> 64 channels 3x3 at 224x224, batch 32:
 // 129 us against 139).
-bool ig_splits(const fc_conv_shape &s, const fc_gemm_config &c, bool x16) {
+bool ig_splits(const fc_conv_shape &s, const fc_gemm_config &c) {
     if (c.waves_k > 1 || c.bm % 64 != 0 || 4l * s.N * s.C * s.H * s.W >= (1l << 31) || (long)s.C * s.kh * s.kw <= 48) return false;
-    if (ig_pointwise(s, c.bk, x16) && s.K <= 64) return false;
+    if (ig_pointwise(s, c.bk, true) && s.K <= 64) return false;
     return s.kh * s.kw <= 64 || (s.C % c.bk == 0 && ig_inside(s, c.bk));
+}
+
+// Order of the reduction rows and their number (before rounding up to a stage).
+int ig_order(const fc_conv_shape &s, const fc_gemm_config &c, long *rows) {
+    const long taps = (long)s.kh * s.kw;
+    *rows = s.C * taps;
+    if (!ig_splits(s, c)) return s.C % c.bk == 0 ? IG_ORDER_TAP : IG_ORDER_CHANNEL;
+    if (s.C % 16 == 0) return IG_ORDER_BLOCK;
+    const long block = fc_round_up(s.C, 16) * taps;
+    const long row8 = 8l * s.C * s.kh * ((s.kw + 7) / 8), row4 = 4l * s.C * s.kh * ((s.kw + 3) / 4);
+    const double costBlock = 1.0 * block, costRow8 = 0.85 * fc_round_up(row8, 16), costRow4 = 0.9 * fc_round_up(row4, 16);
+    if (costBlock <= costRow8 && costBlock <= costRow4) { *rows = block; return IG_ORDER_BLOCK; }
+    if (costRow8 <= costRow4) { *rows = row8; return IG_ORDER_ROW8; }
+    *rows = row4;
+    return IG_ORDER_ROW4;
 }
 
 template <class TL>
 void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, IgemmParams &p) {
-    const dim3 grid((unsigned)(((p.nKB * p.nPB + 7) / 8) * 8), (unsigned)p.splitK);
+    if constexpr (!std::is_void<typename IgSplitOf<TL>::type>::value) {
+        if (ig_splits(s, cfg)) {
+            typedef typename IgSplitOf<TL>::type S;
+            p.nKB = p.K_pad / S::BM_;
+            p.nPB = (int)((p.Npix + S::BN_ - 1) / S::BN_);
+            const dim3 grid((unsigned)(((long)p.nKB * p.nPB + 7) / 8 * 8), (unsigned)p.splitK), block(S::THREADS);
+            long rows;
+            const int order = ig_order(s, cfg, &rows);
+            if (order == IG_ORDER_ROW8) igemm_split_kernel<S, SP_ROW8><<<grid, block, 0, ctx->stream>>>(p);
+            else if (order == IG_ORDER_ROW4) igemm_split_kernel<S, SP_ROW4><<<grid, block, 0, ctx->stream>>>(p);
+            else if (s.C % 16 != 0) igemm_split_kernel<S, SP_PAD><<<grid, block, 0, ctx->stream>>>(p);
+            else if (ig_inside(s, 16)) igemm_split_kernel<S, SP_INSIDE><<<grid, block, 0, ctx->stream>>>(p);
+            else igemm_split_kernel<S, SP_MASKED><<<grid, block, 0, ctx->stream>>>(p);
+            return;
+        }
+    }
     const bool x16 = ((uintptr_t)p.x & 15) == 0;
     const bool pointwise = ig_pointwise(s, TL::BK_, x16), inside = ig_inside(s, TL::BK_);
     // one 32-bit byte offset with bit 31 to spare reaches every element of the tensor
     const bool buffer = p.xBytes < (1l << 31);
     const bool tapMajor = p.C % TL::BK_ == 0;      // the order fc_igemm_pack_filter laid the filter out in
-    const dim3 block(TL::THREADS);
-    if constexpr (TL::BM_ % 64 == 0) {
-        if (ig_splits(s, cfg, x16)) {
-            typedef std::conditional_t<std::is_same<TL, Ig0>::value, Ig0Split, TL> TS;
-            const dim3 splitBlock(TS::THREADS);
-            if (tapMajor && inside) igemm_conv_kernel<TS, IG_TAP_INSIDE, true><<<grid, splitBlock, 0, ctx->stream>>>(p);
-            else if (tapMajor) igemm_conv_kernel<TS, IG_TAP_MASKED, true><<<grid, splitBlock, 0, ctx->stream>>>(p);
-            else igemm_conv_kernel<TS, IG_BUF_MASKED, true><<<grid, splitBlock, 0, ctx->stream>>>(p);
-            return;
-        }
-    }
+    const dim3 grid((unsigned)(((p.nKB * p.nPB + 7) / 8) * 8), (unsigned)p.splitK), block(TL::THREADS);
     if (pointwise) igemm_conv_kernel<TL, IG_POINTWISE><<<grid, block, 0, ctx->stream>>>(p);
     else if (buffer && tapMajor && inside) igemm_conv_kernel<TL, IG_TAP_INSIDE><<<grid, block, 0, ctx->stream>>>(p);
     else if (buffer && tapMajor && p.kh * p.kw <= 64) igemm_conv_kernel<TL, IG_TAP_MASKED><<<grid, block, 0, ctx->stream>>>(p);
     else if (buffer && p.kh * p.kw <= 64) igemm_conv_kernel<TL, IG_BUF_MASKED><<<grid, block, 0, ctx->stream>>>(p);      // the taps of a window are one 64-bit mask
     else igemm_conv_kernel<TL, IG_GATHER><<<grid, block, 0, ctx->stream>>>(p);
+}
+
+// Expected time of a layer on the bf16 matrix cores, in us, under one of the tile shapes 128x128, 64x128, 128x64 and 64x64
+// (configurations 0 to 3).  A CU takes a stage of a workgroup every `cycles` (block or row order), however many it holds, and
+// one workgroup takes at least `latency` for it; beside that the start of a round, memory, and for a split reduction the pass
+// over the partial sums.  Constants: least squares over 6348 times of 1894 layers (1x1, 3x3, 5x5 and 7x7, one to 64 images,
+// 1 to 1024 channels, 0.1 to 120 GFLOP), standard deviation 13 %; the choice among the four is 1.5 % behind the best of them.
+struct IgSplitCost {
+    int bm, bn, perCu;
+    double cyclesBlock, cyclesRow, latency, start;
+};
+const IgSplitCost kIgSplitCost[] = {{128, 128, 2, 1121, 1032, 1602, 928}, {64, 128, 4, 756, 713, 1041, 535},
+                                    {128, 64, 4, 621, 563, 1821, 711}, {64, 64, 8, 420, 398, 1031, 313}};
+
+double ig_split_us(const fc_conv_shape &s, int config, const fc_igemm_plan &plan) {
+    const IgSplitCost &c = kIgSplitCost[config];
+    long rows;
+    const int order = ig_order(s, kIgConfigs[config], &rows);
+    const double stages = ceil(ceil(rows / 16.0) / plan.split_k), kBlocks = ceil((double)s.K / c.bm);
+    double cycles = order == IG_ORDER_BLOCK ? c.cyclesBlock : c.cyclesRow;
+    if (c.bm == 64 && s.K % 64 != 0 && s.K % 64 <= 32) cycles *= (kBlocks - 1 + 0.59) / kBlocks;      // half of the last rows
+    const double blocks = kBlocks * ceil((double)plan.Npix / c.bn) * plan.split_k, slots = 256.0 * c.perCu;
+    auto round = [&](double perCu) { return stages * fmax(c.latency, perCu * cycles) + c.start * (1 + 2.3 * perCu); };
+    const double full = floor(blocks / slots), rest = blocks - full * slots;
+    const double compute = (full * round(c.perCu) + (rest > 0 ? round(ceil(rest / 256)) : 0)) / 2000;
+    const double bytes = 4.0 * ((double)s.N * s.C * s.H * s.W / (s.kh * s.kw == 1 ? s.sh * s.sw : 1) + (double)s.K * plan.Npix);
+    const double us = 4.5 + pow(pow(compute, 4) + pow(bytes / 4.99e6, 4), 0.25);
+    return plan.split_k > 1 ? us + 3.4 + 2.0 * plan.ws_bytes / 6.65e6 : us;
+}
+
+// The same for a kernel that splits the reduction over the wavefronts of a workgroup (6001 times, 16 %).
+double ig_ws_us(const fc_conv_shape &s, const fc_gemm_config &c, long npix) {
+    const double mt = c.bm / 16, nt = c.bn / 16, units = ceil((double)s.C * s.kh * s.kw / 16);
+    const double perCu = ceil(ceil((double)s.K / c.bm) * ceil((double)npix / c.bn) / 256);
+    const bool table = s.C % 16 != 0, row3 = !table && s.kw == 3;
+    const double loads = (mt + 4 * nt / (row3 ? 3 : 1)) * 7.06;
+    const double cycles = fmax(loads, 17.1 * mt * nt) + 18.8 * (mt + nt) + (table ? 36.7 * nt : 0);
+    return 3.5 + (perCu * units * cycles + 52.8 * perCu * mt * nt * c.waves_k) / 2000;
+}
+
+// A layer whose reduction the best tile would split over workgroups goes to the kernels that split it inside the workgroup
+// where those are expected ahead, from 9 parts on also where they are 15 % behind and from 21 on 50 %: the model then favours
+// the tiles (most of the layers that lost more than 15 % by it: 9 to 32 parts, reductions of 1000 to 9000 rows, 15 to 25 us).
+int ig_split_default_config(const fc_conv_shape *s) {
+    int best = 3;
+    double bestUs = 1e300;
+    fc_igemm_plan plan, bestPlan = {};
+    for (int id = 0; id < 4; id++) {
+        if (fc_igemm_make_plan(s, id, &plan) != FC_OK) continue;
+        const double us = ig_split_us(*s, id, plan);
+        if (us < bestUs) { bestUs = us; best = id; bestPlan = plan; }
+    }
+    const int ws = bestPlan.split_k > 1 ? fc_igemm_ws_choose(s, plan.Npix) : -1;
+    if (ws >= 0) {
+        fc_gemm_config c;
+        fc_igemm_ws_get_config(ws, kNumIgConfigs + ws, &c);
+        if (ig_ws_us(*s, c, plan.Npix) < bestUs * (bestPlan.split_k > 20 ? 1.5 : bestPlan.split_k > 8 ? 1.15 : 1.0)) return kNumIgConfigs + ws;
+    }
+    return best;
 }
 
 }  // namespace
@@ -810,12 +1016,14 @@ extern "C" int fc_igemm_get_config(int id, fc_gemm_config *cfg) {
     return FC_OK;
 }
 
-// Untuned choice: padded multiply-adds divided by the rate each tile shape sustains relative to
+// Untuned choice on fp32 instructions: padded multiply-adds divided by the rate each tile shape sustains relative to
 // 64x64x16 (measured on MI355X over pointwise, strided and 3x3 layers at batch 32; the shapes with
 // 128 accumulators per wavefront run one or two workgroups per CU and fall far behind) and by how
 // evenly the grid fills the chip.
 extern "C" int fc_igemm_default_config(const fc_conv_shape *s) {
     if (!fc_shape_ok(s)) return FC_ERR_INVALID;
+    // (a 1x1 layer of at most 32 output channels is bound by reading x: 32 rows a tile and more workgroups are ahead there)
+    if (ig_splits(*s, kIgConfigs[3]) && !(s->kh * s->kw == 1 && s->K <= 32 && s->C % 16 == 0)) return ig_split_default_config(s);
     static const double kRate[] = {0.93, 0.81, 0.82, 1.00, 0.75, 0.60, 0.62, 0.84};
     static_assert(sizeof(kRate) / sizeof(kRate[0]) == sizeof(kIgConfigs) / sizeof(kIgConfigs[0]), "one rate per configuration");
     const double M = s->K, Kr = (double)s->C * s->kh * s->kw;
@@ -833,26 +1041,12 @@ extern "C" int fc_igemm_default_config(const fc_conv_shape *s) {
         const double cost = mp * np * kp / (kRate[id] * (0.8 + 0.2 * fill));
         if (cost < bestCost) { bestCost = cost; best = id; }
     }
-    // On the bf16 matrix cores 128x128 writes and reads the least LDS per product.  It takes over from 64x64 where the
-    // reduction is long enough to pay for its longer start, the grid is at least three rounds of its two workgroups per
-    // CU without a split, and it pads no more.  At batch 32 and the like:
-    // 256 -> 256 1x1 at 56x56 85 us against 98, 85 -> 128 3x3 at 150x150 345 against 418; with 32 rows 27.5 against 22.7.
-    const bool split = ig_splits(*s, kIgConfigs[3], true);      // the rates above are those of the fp32 instructions
-    if (split && best == 3 && Kr >= 256 && ceil(M / 128) * 128 == ceil(M / 64) * 64 && ceil(M / 128) * ceil(Np / 128) >= 1536) best = 0;
     // A layer that this tile shape can only fill the chip with by splitting the reduction over workgroups
     // (a pass of partial sums through memory and a second launch) goes to the kernels that split it inside
-    // the workgroup instead, while it is small enough for them.  Where 64x64 tiles waste nothing and the partial sums
-    // fit the static workspace (so that fc_conv_implicit_gemm_static takes the plan, as before) the line is lower: at
-    // 1.85 GFLOP the others are ahead or level (3x3 on 256 channels, two 28x28 images: 23 us against 28; 1x1
-    // 2048 -> 512 on sixteen 7x7 images: 24 against 23), at 3.7 GFLOP level or behind (42.8 against 41.5 and 42.1, 512
-    // channels, one 28x28 or four 14x14 images).  More than 15 parts are added up by too few workgroups: the others are
-    // ahead or level (512 channels, fourteen 7x7 images, 18 parts: 37.0 against 39.2; 1024 -> 512, eight, 28 parts: 47.2
-    // against 47.7; 5x5 512 -> 256, two 20x20 images, 30 parts, is the exception: 69 against 60).
+    // the workgroup instead, while it is small enough for them.
     fc_igemm_plan plan;
     if (fc_igemm_make_plan(s, best, &plan) == FC_OK && plan.split_k > 1) {
-        const bool tiled = split && best == 3 && s->K % 64 == 0 && s->C % 16 == 0 && plan.split_k <= 15 && 2.0 * M * Kr * Np >= 3.2e9 &&
-                           plan.ws_bytes <= (size_t)FC_IGEMM_STATIC_WS_BYTES;
-        const int ws = tiled ? -1 : fc_igemm_ws_choose(s, plan.Npix);
+        const int ws = fc_igemm_ws_choose(s, plan.Npix);
         if (ws >= 0) return kNumIgConfigs + ws;
     }
     return best;
@@ -871,11 +1065,19 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
     const long npix = (long)s->N * plan->OH * plan->OW;
     if (kred >= (1l << 28) || npix >= (1l << 31) || (long)s->C * s->H * s->W >= (1l << 31)) return FC_ERR_UNSUPPORTED;
     plan->Kred = (int)kred;
-    plan->Kred_pad = (int)fc_round_up(kred, cfg.bk);
+    long rows = kred;
+    bool split = false;
+    if (config < kNumIgConfigs) {
+        split = ig_splits(*s, cfg);
+        ig_order(*s, cfg, &rows);
+        if (rows >= (1l << 28)) return FC_ERR_UNSUPPORTED;
+    }
+    plan->Kred_pad = (int)fc_round_up(rows, cfg.bk);
     plan->K_pad = (int)fc_round_up(s->K, cfg.bm);
     plan->Npix = npix;
     plan->config = config;
-    plan->Wp_bytes = sizeof(float) * (size_t)plan->Kred_pad * plan->K_pad;
+    // in fp32 and, where products are split, in three bf16 parts
+    plan->Wp_bytes = (sizeof(float) + (split ? 6 : 0)) * (size_t)plan->Kred_pad * plan->K_pad;
     plan->table_bytes = sizeof(int32_t) * 2 * (size_t)plan->Kred_pad;
     if (config >= kNumIgConfigs) {
         // the reduction is split inside the workgroups: one launch, no workspace
@@ -888,7 +1090,7 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
     // reduction until about three workgroups per CU exist, keeping >= 4 LDS stages per part.
     const long blocks = (long)(plan->K_pad / cfg.bm) * ((npix + cfg.bn - 1) / cfg.bn);
     const int stages = plan->Kred_pad / cfg.bk;
-    int split = 1;
+    int splitK = 1;
     // A grid of two to four workgroups per CU is placed unevenly by the dispatcher (some CUs get
     // one more than their share and set the time of the launch): with a long reduction, splitting
     // it to about six per CU is worth the second pass (measured: 3x3 stride-2 layers of ResNet-50
@@ -896,19 +1098,19 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
     const bool longReduction = stages >= 64;
     const long below = longReduction ? 1024 : 512, target = longReduction ? 1536 : 768;
     if (blocks < below) {
-        split = (int)((target + blocks - 1) / blocks);
-        if (split > stages / 4) split = stages / 4;
-        if (split > 32) split = 32;
-        if (split < 1) split = 1;
+        splitK = (int)((target + blocks - 1) / blocks);
+        if (splitK > stages / 4) splitK = stages / 4;
+        if (splitK > 32) splitK = 32;
+        if (splitK < 1) splitK = 1;
     }
-    const int per = (stages + split - 1) / split;
+    const int per = (stages + splitK - 1) / splitK;
     plan->split_k = (stages + per - 1) / per;          // no empty parts
     plan->ws_bytes = plan->split_k > 1 ? sizeof(float) * (size_t)plan->split_k * s->K * npix : 0;
     return FC_OK;
 }
 
 extern "C" int fc_igemm_splits_products(const fc_igemm_plan *plan) {
-    return plan && plan->config >= 0 && plan->config < kNumIgConfigs && ig_splits(plan->shape, kIgConfigs[plan->config], true) ? 1 : 0;
+    return plan && plan->config >= 0 && plan->config < kNumIgConfigs && ig_splits(plan->shape, kIgConfigs[plan->config]) ? 1 : 0;
 }
 
 static int ig_plan_check(fc_context *ctx, const fc_igemm_plan *plan) {
@@ -933,11 +1135,19 @@ extern "C" int fc_igemm_pack_filter(fc_context *ctx, const fc_igemm_plan *plan, 
     if (plan->config >= kNumIgConfigs) return fc_igemm_ws_pack(ctx, plan, w_dev, Wp_dev, table_dev);
     fc_gemm_config cfg;
     fc_igemm_get_config(plan->config, &cfg);
-    const int tapMajor = s.C % cfg.bk == 0 ? 1 : 0;      // must match the kernel's choice in launch()
+    long rows;
+    const int order = ig_order(s, cfg, &rows);
     fc_stage_scope scope(ctx, FC_STAGE_FILTER_PACK);
     igemm_pack_filter_kernel<<<grid, dim3(256), 0, ctx->stream>>>(w_dev, Wp_dev, table_dev, s.K, s.C, s.kh, s.kw, s.H,
-                                                                 s.W, plan->Kred, plan->Kred_pad, plan->K_pad, tapMajor);
+                                                                 s.W, (int)rows, plan->Kred_pad, plan->K_pad, order);
     FC_LAUNCH_CHECK(ctx, "igemm_pack_filter_kernel");
+    if (ig_splits(s, cfg)) {
+        const long total = (long)(plan->Kred_pad / 16) * (plan->K_pad / 32) * 64;
+        if ((total + 255) / 256 >= (1l << 31)) return fc_set_error(ctx, FC_ERR_UNSUPPORTED, "fc_igemm_pack_filter: filter too large", hipSuccess);
+        igemm_split_filter_kernel<<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream>>>(
+            Wp_dev, reinterpret_cast<fc_uintx4 *>(Wp_dev + (size_t)plan->Kred_pad * plan->K_pad), plan->K_pad, total);
+        FC_LAUNCH_CHECK(ctx, "igemm_split_filter_kernel");
+    }
     return FC_OK;
 }
 
@@ -1037,6 +1247,7 @@ static int igemm_run(fc_context *ctx, const fc_igemm_plan *plan, const float *x_
     const fc_conv_shape &s = plan->shape;
     IgemmParams p;
     p.x = x_dev; p.Wp = Wp_dev; p.table = table_dev; p.bias = bias_dev; p.y = y_dev;
+    p.Ws = reinterpret_cast<const fc_uintx4 *>(Wp_dev + (size_t)plan->Kred_pad * plan->K_pad);
     p.N = s.N; p.C = s.C; p.H = s.H; p.W = s.W; p.K = s.K; p.OH = plan->OH; p.OW = plan->OW;
     p.kh = s.kh; p.kw = s.kw; p.sh = s.sh; p.sw = s.sw; p.pt = s.pt; p.pl = s.pl; p.relu = relu;
     p.Kred_pad = plan->Kred_pad; p.K_pad = plan->K_pad; p.Npix = plan->Npix;
