@@ -5,10 +5,9 @@
 //
 // A workgroup owns 16 consecutive tiles x 64 output channels and walks the input channels in
 // chunks of 4.  Three chunks are in flight; in every barrier-delimited region each thread
-//   1. takes one 8-float row of an 8x8 input patch, fetched two regions earlier as the 8
-//      floats of the image row nearest to it (two 16-byte loads, no branches, nothing consumed
-//      at load time so the loads stay in flight); rows touching the image border are shifted
-//      and zero-filled through a private LDS slot; applies B along the row and parks the
+//   1. takes one 8-float row of an 8x8 input patch, fetched two regions earlier (two 16-byte
+//      loads, no branches, nothing consumed at load time so the loads stay in flight); what
+//      lies beyond the image border is zeroed; applies B along the row and parks the
 //      result in LDS                                             (tmp[2][4 c][16 t][8][8]),
 //   2. applies B^T down one column of the chunk parked in the previous region and writes it as
 //      the B operand of the products                             (Vs[2][64 f][4 c][16 t]),
@@ -17,6 +16,9 @@
 //      chunk is one MFMA reduction step.  A comes from the transformed filter in L2 as one
 //      16-byte load per frequency and chunk (the four 16-channel blocks of a lane side by
 //      side, fetched two regions ahead), B from Vs.
+// Windows read past the border and masked, not clamped to the image row and shifted through LDS (all but the first and the
+// last rows of x): about half of the workgroups of a 224x224 image hold border tiles, and the shift took each of their
+// rows 10 LDS instructions and 16 vector ones.  64 -> 64 at 224x224, batch 32: 483 -> 460 us; VGG-16 stack 3134 -> 3087 us.
 // fp32 MFMA and fp32 vector arithmetic share the SIMD's ALUs on this chip (a measured fact:
 // their times add, they do not overlap), so the transform arithmetic is paid on top of the
 // products; what the kernel saves is the HBM traffic of V and M.
@@ -70,8 +72,10 @@ __global__ __launch_bounds__(kFusedThreads, 1) void wino_onepass_kernel(const On
 
     // ---- step 1: thread = row i1 of the patch of tile tl1, channel c1 of the chunk
     const int tl1 = tid & 15, i1 = (tid >> 4) & 7, c1 = tid >> 7;
-    // The row is always fetched as the 8 floats xwin[0..7] that lie inside the image (a window
-    // clamped to the row); element j of the patch row is xwin[j + shift] where colMask has bit j.
+    // The row is fetched as the 8 floats xwin[0..7], of which those with a bit in colMask are inside the image; beside
+    // the image border the others belong to the rows before and after it and are dropped.  Where they would lie before
+    // the first or after the last element of x for any channel, the window is clamped to the row instead, and element j
+    // is xwin[j + shift].
     const float *xwin = p.x;
     uint32_t colMask = 0;     // bit j: column j of the patch row is inside the image
     int shift = 0;
@@ -85,9 +89,10 @@ __global__ __launch_bounds__(kFusedThreads, 1) void wino_onepass_kernel(const On
 #pragma unroll
                 for (int j = 0; j < 8; j++)
                     if (gx0 + j >= 0 && gx0 + j < p.W) colMask |= 1u << j;
-                const int gw = min(max(gx0, 0), p.W - 8);       // the host checks W >= 8
-                shift = gx0 - gw;
-                xwin = p.x + (((size_t)n * p.C + c1) * p.H + gy) * p.W + gw;
+                const long first = ((long)n * p.C * p.H + gy) * p.W + gx0, last = first + (long)(p.C - 1) * p.H * p.W + 7;
+                if (first < 0 || last >= (long)p.out.N * p.C * p.H * p.W)
+                    shift = gx0 - min(max(gx0, 0), p.W - 8);       // the host checks W >= 8
+                xwin = p.x + ((((long)n * p.C + c1) * p.H + gy) * p.W + gx0 - shift);
             }
         }
     }
@@ -137,22 +142,23 @@ __global__ __launch_bounds__(kFusedThreads, 1) void wino_onepass_kernel(const On
         for (int f = 0; f < kFW; f++)
             dst[f] = *reinterpret_cast<const floatx4 *>(reinterpret_cast<const char *>(src + f * planeU) + ubLane);
     };
-    // window (chunk q) -> patch row -> B along the row -> tmp[buf].  Rows that touch the image
-    // border are shifted and zero-filled through a private 8-float slot of LDS.
+    // window (chunk q) -> patch row -> B along the row -> tmp[buf].  Rows that touch the image border are zero-filled,
+    // those of a clamped window shifted before through a private 8-float slot of LDS.
     auto rowTransform = [&](int buf, const float (&win)[8], int q) {
         float d[8], o[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) d[j] = win[j];
         const uint32_t m = (q * kCB + c1 < p.C) ? colMask : 0u;
         if (m != 0xffu) {
-            float *slot = bounce + tid * 8;
-            reinterpret_cast<floatx4 *>(slot)[0] = floatx4{win[0], win[1], win[2], win[3]};
-            reinterpret_cast<floatx4 *>(slot)[1] = floatx4{win[4], win[5], win[6], win[7]};
+            if (shift != 0) {
+                float *slot = bounce + tid * 8;
+                reinterpret_cast<floatx4 *>(slot)[0] = floatx4{win[0], win[1], win[2], win[3]};
+                reinterpret_cast<floatx4 *>(slot)[1] = floatx4{win[4], win[5], win[6], win[7]};
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float v = slot[min(max(j + shift, 0), 7)];
-                d[j] = ((m >> j) & 1u) ? v : 0.f;
+                for (int j = 0; j < 8; j++) d[j] = slot[min(max(j + shift, 0), 7)];
             }
+#pragma unroll
+            for (int j = 0; j < 8; j++) d[j] = ((m >> j) & 1u) ? d[j] : 0.f;
         }
         bt8(d, o);
         floatx4 *dst = reinterpret_cast<floatx4 *>(tmp + buf * kTmpFloats + tmpW);
