@@ -31,7 +31,6 @@
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kCB = 4;                          // input channels per chunk
 constexpr int kTB = 16;                         // tiles per workgroup
@@ -260,7 +259,6 @@ __global__ __launch_bounds__(kFusedThreads, 1) void wino_onepass_kernel(const On
             const int rows = min(6, p.out.OH - (int)th * 6), ncols = min(6, p.out.OW - (int)tw * 6);
             const float bias = p.out.bias ? p.out.bias[k] : 0.f;
             float *dst = p.out.y + (((size_t)n * p.out.K + k) * p.out.OH + (size_t)th * 6) * p.out.OW + tw * 6;
-            const bool pairs = ncols == 6 && (p.out.OW & 1) == 0;    // 8-byte aligned row segments
 #pragma unroll
             for (int i = 0; i < 6; i++) {
                 float sres[6];
@@ -272,10 +270,8 @@ __global__ __launch_bounds__(kFusedThreads, 1) void wino_onepass_kernel(const On
                         if (p.out.relu) sres[jj] = __builtin_elementwise_maximum(sres[jj], 0.f);      // keeps a NaN, as the other epilogues do
                     }
                     float *drow = dst + (size_t)i * p.out.OW;
-                    if (pairs) {
-#pragma unroll
-                        for (int jj = 0; jj < 6; jj += 2)
-                            *reinterpret_cast<float2 *>(drow + jj) = make_float2(sres[jj], sres[jj + 1]);
+                    if (ncols == 6) {
+                        store_row6(drow, sres);
                     } else {
 #pragma unroll
                         for (int jj = 0; jj < 6; jj++)

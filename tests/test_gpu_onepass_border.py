@@ -1,5 +1,5 @@
 """Patch rows of the single-kernel Winograd path beside the image border: they are read past the image row and masked, or,
-at the ends of the tensor, clamped to the row and shifted."""
+at the ends of the tensor, clamped to the row and shifted.  And rows of y, stored six floats at a time wherever they start."""
 import numpy as np
 import pytest
 
@@ -17,6 +17,7 @@ SHAPES = [
     ((1, 6, 9, 8, 3), {"pl": 2, "pr": 2}),            # the smallest width
     ((2, 5, 8, 9, 4), {"pt": 2, "pb": 2, "pl": 2, "pr": 0}),
     ((2, 7, 12, 12, 5), {"pt": 9, "pb": 9, "pl": 9, "pr": 9}),      # whole tiles in the padding
+    ((2, 6, 13, 13, 65), {}), ((1, 8, 12, 15, 33), {}), ((1, 5, 9, 11, 3), {"pr": 2}),      # rows of 13, 15 and 12 floats
     ((1, 16, 12, 18, 64), {"pt": 0, "pb": 0, "pl": 0, "pr": 0}),    # no border inside a patch but in the ragged tiles
 ]
 
@@ -59,3 +60,11 @@ def test_what_lies_beyond_the_border_is_dropped(lib, shp, pads):
                     keep[:, :, 6 * th:6 * th + 6, 6 * tw:6 * tw + 6] = False
         assert keep.any() or y.shape[3] <= 12
         assert np.array_equal(y[keep], clean[keep])
+
+
+@pytest.mark.parametrize("shp,pads", SHAPES)
+def test_rows_of_the_fused_kernel_are_those_of_the_staged_pipeline(lib, shp, pads):
+    s = O.shape(*shp, **pads)
+    x, w = O.make_inputs(s, seed=shp[1])
+    print("fused rows", shp, pads, flush=True)
+    assert np.array_equal(lib.winograd_conv_fused(cshape(s), x, w), lib.winograd_conv(cshape(s), x, w))
