@@ -23,17 +23,6 @@ struct FusedOut {
     fc_fastdiv divTile, divTW;    // tiles per image, tiles per band
 };
 
-typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
-
-// Six floats of an output row, which start at any multiple of 4 bytes: 16 bytes and 8.  (A float at a time where rows are an
-// odd number of floats long, six stores in place of two, took, us: single kernel 64 -> 64 at 223x223 batch 32 573 / 472,
-// 64 -> 128 at 111x111 302 / 248, 32 -> 64 at 157x157 batch 20 142 / 104.)
-__device__ __forceinline__ void store_row6(float *row, const float (&v)[6]) {
-    *reinterpret_cast<floatx4u *>(row) = floatx4u{v[0], v[1], v[2], v[3]};
-    *reinterpret_cast<floatx2u *>(row + 4) = floatx2u{v[4], v[5]};
-}
-
 // Output channels kb*32 .. kb*32+31, tiles tb*32 .. tb*32+31.  Ml must be free for writing on
 // entry (callers put a barrier after their last LDS use).  Accumulator register i of lane l is
 // channel 8*(i/4) + 4*(l/32) + i%4, tile l%32: registers 0..7 are channels 0..15, 8..15 are

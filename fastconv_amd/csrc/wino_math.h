@@ -1,4 +1,4 @@
-// 1-D Winograd F(6,3) transforms shared by the transform kernels and the fused kernels.
+// 1-D Winograd F(6,3) transforms shared by the transform kernels and the fused kernels, and the fused kernels' store.
 #pragma once
 
 namespace {
@@ -48,6 +48,18 @@ __device__ __forceinline__ void g8(const float g[3], float w[8]) {
     w[5] = (h + two) * c180;
     w[6] = (h - two) * c180;
     w[7] = g[2];
+}
+
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
+
+// Six floats of an output row, which start at any multiple of 4 bytes: 16 bytes and 8.  (A float at a time where rows are an
+// odd number of floats long, six stores in place of two, took, us: single kernel 64 -> 64 at 223x223 batch 32 573 / 472,
+// 64 -> 128 at 111x111 302 / 248, 32 -> 64 at 157x157 batch 20 142 / 104; fused kernel 24 -> 256 at 49x49
+// batch 48 122 / 90; small-channel kernel 3 -> 64 at 223x223 batch 32 218 / 125.)
+__device__ __forceinline__ void store_row6(float *row, const float (&v)[6]) {
+    *reinterpret_cast<floatx4u *>(row) = floatx4u{v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<floatx2u *>(row + 4) = floatx2u{v[4], v[5]};
 }
 
 }  // namespace

@@ -241,9 +241,13 @@ __device__ __forceinline__ void sc_step(const SmallCParams &p, const UReg<C> &u,
                 if (q < st.srows[2] + tie) *reinterpret_cast<float2 *>(yrow + st.soff[2]) = a2;
             } else if (q < st.nRows + tie) {
                 float *row = st.ytile + (size_t)kprev * chanStride + (size_t)q * p.OW;
+                if (st.nCols + tie >= 6) {
+                    store_row6(row, o);
+                } else {
 #pragma unroll
-                for (int s = 0; s < 6; s++)
-                    if (s < st.nCols + tie) row[s] = o[s];
+                    for (int s = 0; s < 5; s++)
+                        if (s < st.nCols + tie) row[s] = o[s];
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);

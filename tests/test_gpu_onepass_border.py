@@ -68,3 +68,14 @@ def test_rows_of_the_fused_kernel_are_those_of_the_staged_pipeline(lib, shp, pad
     x, w = O.make_inputs(s, seed=shp[1])
     print("fused rows", shp, pads, flush=True)
     assert np.array_equal(lib.winograd_conv_fused(cshape(s), x, w), lib.winograd_conv(cshape(s), x, w))
+
+
+@pytest.mark.parametrize("shp", [(1, 3, 13, 13, 65), (2, 1, 12, 15, 16), (1, 4, 9, 11, 17), (3, 2, 14, 9, 5), (1, 2, 8, 67, 33)])
+def test_odd_rows_of_the_small_channel_kernel(lib, shp):
+    """Whole tiles six floats a row, ragged ones a float at a time."""
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=shp[1])
+    bias = O.rng_uniform(3, (s.K,))
+    print("odd rows", shp, flush=True)
+    y = lib.winograd_conv_onepass(cshape(s), x, w, bias=bias, relu=True)
+    assert O.max_rel_err(y, np.maximum(O.naive_conv_f64(s, x, w, bias), 0.0)) <= TOL_WINO
