@@ -782,8 +782,10 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
     fetch(sBegin);
     int s = sBegin;
     if constexpr (ROW) {
-        // stages of the first channel, where windows of the first image may start before x
-        const int stagesBefore = __builtin_amdgcn_readfirstlane(__any(before) ? (p.kh * ((p.kw + RUN - 1) / RUN) * RUN + 15) / 16 : 0);
+        // stages of the channels in which a run may start before x: its row is inside the image, so that its first column lies
+        // c * H * W - pl floats after the start of x at least (more than one channel where images are smaller than pl)
+        const int channels = min(p.C, 1 + max(p.pl - 1, 0) / (p.H * p.W));
+        const int stagesBefore = __builtin_amdgcn_readfirstlane(__any(before) ? (channels * p.kh * ((p.kw + RUN - 1) / RUN) * RUN + 15) / 16 : 0);
 #pragma unroll 1
         for (; s < sEnd && s < stagesBefore; s++) stage(s, s + 1 < sEnd, std::true_type());
 #pragma unroll 1

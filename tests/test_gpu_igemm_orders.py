@@ -25,6 +25,14 @@ SHAPES = [
     O.shape(1, 6, 9, 41, 64, 3, 11, 1, 1, 1),           # two runs a window row
     O.shape(2, 3, 19, 70, 64, 2, 31, 1, 1, 0),          # four runs, the widest window
     O.Shape(2, 20, 9, 9, 64, 3, 3, 1, 1, 0, 2, 2, 0),   # padding on two sides only
+    # images smaller than the left padding: windows start before the input in more channels than the first
+    O.Shape(2, 5, 1, 4, 64, 1, 15, 1, 1, 0, 0, 7, 7),   # two channels, two runs a window row
+    O.shape(2, 3, 1, 2, 64, 7, 7, 1, 1, 3),
+    O.shape(3, 3, 1, 1, 64, 5, 5, 1, 1, 2),
+    O.shape(2, 8, 1, 3, 64, 5, 5, 1, 1, 4),
+    O.shape(1, 20, 1, 1, 64, 5, 5, 1, 1, 4),            # four of twenty channels, split reduction
+    O.shape(2, 2, 1, 1, 33, 7, 7, 1, 1, 6),             # all channels
+    O.Shape(2, 70, 1, 2, 64, 2, 4, 1, 1, 1, 1, 3, 3),   # runs of 4
 ]
 
 
