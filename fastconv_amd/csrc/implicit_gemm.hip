@@ -5,6 +5,7 @@
 // it straight into LDS.  The filter is re-laid once to Wp[Kred_pad][K_pad]
 // (output channel fastest) so that its tiles are straight 16-byte copies, as in
 // the Winograd GEMM.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <mutex>
@@ -92,6 +93,9 @@ struct IgemmParams {
     long xBytes;                  // size of the input tensor
     int fastStore;                // K is a whole number of tiles, every output byte offset fits 32 bits, bias 16-byte aligned
     fc_fastdiv divOHW, divOW;
+    // row orders: pixels and stages past which no run of window columns starts before x (ig_before)
+    long pixBefore;
+    int stagesBefore;
 };
 
 template <int BM, int BN, int BK, int WGM, int WGN>
@@ -606,7 +610,6 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
 
     // pixels of this lane: byte offset of the window in the tensor, window rows and columns outside the image
     uint32_t pixByte[NI], rowBad[NI], colBad[NI];
-    bool before = false;      // a window that starts before the first element of x
 #pragma unroll
     for (int ni = 0; ni < NI; ni++) {
         const long pix = (long)pb * S::BN_ + wn0 + ni * 32 + lcol;
@@ -623,7 +626,6 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
                 for (int r = 0; r < p.kh; r++) rowBad[ni] &= (unsigned)(ih0 + r) < (unsigned)p.H ? ~(1u << r) : ~0u;
                 for (int q = 0; q < p.kw; q++) colBad[ni] &= (unsigned)(iw0 + q) < (unsigned)p.W ? ~(1u << q) : ~0u;
             }
-            before |= (int)pixByte[ni] < 0;
         }
     }
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.x), 0, (int)p.xBytes, 0x00020000);
@@ -782,10 +784,8 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
     fetch(sBegin);
     int s = sBegin;
     if constexpr (ROW) {
-        // stages of the channels in which a run may start before x: its row is inside the image, so that its first column lies
-        // c * H * W - pl floats after the start of x at least (more than one channel where images are smaller than pl)
-        const int channels = min(p.C, 1 + max(p.pl - 1, 0) / (p.H * p.W));
-        const int stagesBefore = __builtin_amdgcn_readfirstlane(__any(before) ? (channels * p.kh * ((p.kw + RUN - 1) / RUN) * RUN + 15) / 16 : 0);
+        // one number for the workgroup: all its wavefronts meet at the same barriers
+        const int stagesBefore = (long)pb * S::BN_ < p.pixBefore ? p.stagesBefore : 0;
 #pragma unroll 1
         for (; s < sEnd && s < stagesBefore; s++) stage(s, s + 1 < sEnd, std::true_type());
 #pragma unroll 1
@@ -916,6 +916,18 @@ int ig_order(const fc_conv_shape &s, const fc_gemm_config &c, long *rows) {
     return IG_ORDER_ROW4;
 }
 
+// Row orders, runs of `run` columns: which of them may start before x.  The row of such a run is inside the image, so that it
+// starts (n * C + c) * H * W + row * W - pl floats from the start of x or later: images, channels, rows below these bounds.
+void ig_before(const fc_conv_shape &s, int run, IgemmParams &p) {
+    p.pixBefore = 0;
+    p.stagesBefore = 0;
+    if (s.pl == 0) return;
+    const long last = s.pl - 1, image = (long)s.H * s.W;
+    const long n = last / (s.C * image), oh = (s.pt + last / s.W) / s.sh, channels = std::min<long>(s.C, 1 + last / image);
+    p.pixBefore = (n * p.OH + std::min<long>(p.OH, oh + 1)) * p.OW;
+    p.stagesBefore = (int)((channels * s.kh * ((s.kw + run - 1) / run) * run + 15) / 16);
+}
+
 template <class TL>
 void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, IgemmParams &p) {
     if constexpr (!std::is_void<typename IgSplitOf<TL>::type>::value) {
@@ -926,6 +938,7 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
             const dim3 grid((unsigned)(((long)p.nKB * p.nPB + 7) / 8 * 8), (unsigned)p.splitK), block(S::THREADS);
             long rows;
             const int order = ig_order(s, cfg, &rows);
+            ig_before(s, order == IG_ORDER_ROW8 ? 8 : 4, p);
             if (order == IG_ORDER_ROW8) igemm_split_kernel<S, SP_ROW8><<<grid, block, 0, ctx->stream>>>(p);
             else if (order == IG_ORDER_ROW4) igemm_split_kernel<S, SP_ROW4><<<grid, block, 0, ctx->stream>>>(p);
             else if (s.C % 16 != 0) igemm_split_kernel<S, SP_PAD><<<grid, block, 0, ctx->stream>>>(p);

@@ -33,6 +33,10 @@ SHAPES = [
     O.shape(1, 20, 1, 1, 64, 5, 5, 1, 1, 4),            # four of twenty channels, split reduction
     O.shape(2, 2, 1, 1, 33, 7, 7, 1, 1, 6),             # all channels
     O.Shape(2, 70, 1, 2, 64, 2, 4, 1, 1, 1, 1, 3, 3),   # runs of 4
+    # tiles of which some wavefronts hold such windows and others none
+    O.shape(1, 3, 9, 100, 64, 5, 5, 1, 1, 2),
+    O.shape(3, 3, 5, 70, 128, 7, 7, 1, 1, 3),
+    O.shape(1, 40, 1, 140, 64, 1, 7, 1, 1, 0, pl=150, pr=3),      # more than one image row before x, split reduction
 ]
 
 
