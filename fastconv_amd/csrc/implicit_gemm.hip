@@ -998,23 +998,30 @@ double ig_ws_us(const fc_conv_shape &s, const fc_gemm_config &c, long npix) {
     return 3.5 + (perCu * units * cycles + 52.8 * perCu * mt * nt * c.waves_k) / 2000;
 }
 
+// A plan whose partial sums fit the static workspace goes before any other, however much faster that is: the untuned plan is
+// what callers of fc_conv_implicit_gemm_static use.  Batch 32, us, fitting plan against the best one: 3x3/2 256->256@28 69.1 / 67.4,
+// 3x3 128->128@28 59.6 / 64.1, 512->512@14 209 / 193, 1x1/2 1024->2048@14 73.1 / 63.8.
 // A layer whose reduction the best tile would split over workgroups goes to the kernels that split it inside the workgroup
 // where those are expected ahead, from 9 parts on also where they are 15 % behind and from 21 on 50 %: the model then favours
-// the tiles (most of the layers that lost more than 15 % by it: 9 to 32 parts, reductions of 1000 to 9000 rows, 15 to 25 us).
+// the tiles (most of the layers that lost more than 15 % by it: 9 to 32 parts, reductions of 1000 to 9000 rows, 15 to 25 us);
+// and wherever no tile's partial sums fit.
 int ig_split_default_config(const fc_conv_shape *s) {
     int best = 3;
     double bestUs = 1e300;
+    bool bestFits = false;
     fc_igemm_plan plan, bestPlan = {};
     for (int id = 0; id < 4; id++) {
         if (fc_igemm_make_plan(s, id, &plan) != FC_OK) continue;
         const double us = ig_split_us(*s, id, plan);
-        if (us < bestUs) { bestUs = us; best = id; bestPlan = plan; }
+        const bool fits = plan.ws_bytes <= (size_t)FC_IGEMM_STATIC_WS_BYTES;
+        if (fits != bestFits ? fits : us < bestUs) { bestUs = us; best = id; bestPlan = plan; bestFits = fits; }
     }
     const int ws = bestPlan.split_k > 1 ? fc_igemm_ws_choose(s, plan.Npix) : -1;
     if (ws >= 0) {
         fc_gemm_config c;
         fc_igemm_ws_get_config(ws, kNumIgConfigs + ws, &c);
-        if (ig_ws_us(*s, c, plan.Npix) < bestUs * (bestPlan.split_k > 20 ? 1.5 : bestPlan.split_k > 8 ? 1.15 : 1.0)) return kNumIgConfigs + ws;
+        const double behind = bestPlan.split_k > 20 ? 1.5 : bestPlan.split_k > 8 ? 1.15 : 1.0;
+        if (!bestFits || ig_ws_us(*s, c, plan.Npix) < bestUs * behind) return kNumIgConfigs + ws;
     }
     return best;
 }
