@@ -876,7 +876,21 @@ const fc_gemm_config kIgConfigs[] = {
     FC_CFG(4, Ig4), FC_CFG(5, Ig5), FC_CFG(6, Ig6), FC_CFG(7, Ig7),
 #undef FC_CFG
 };
-const int kNumIgConfigs = sizeof(kIgConfigs) / sizeof(kIgConfigs[0]);
+constexpr int kNumIgConfigs = sizeof(kIgConfigs) / sizeof(kIgConfigs[0]);
+
+// Tiles that run in their place where products are split (0: none).
+struct IgTileSize {
+    int bm, bn;
+};
+template <class TL>
+constexpr IgTileSize ig_split_tile_size() {
+    typedef typename IgSplitOf<TL>::type S;
+    if constexpr (std::is_void<S>::value) return {0, 0};
+    else return {S::BM_, S::BN_};
+}
+const IgTileSize kIgSplitTiles[] = {ig_split_tile_size<Ig0>(), ig_split_tile_size<Ig1>(), ig_split_tile_size<Ig2>(), ig_split_tile_size<Ig3>(),
+                                    ig_split_tile_size<Ig4>(), ig_split_tile_size<Ig5>(), ig_split_tile_size<Ig6>(), ig_split_tile_size<Ig7>()};
+static_assert(sizeof(kIgSplitTiles) / sizeof(kIgSplitTiles[0]) == kNumIgConfigs, "one per configuration");
 
 // The column matrix of a pointwise layer is its input, read 16 bytes a lane where that is possible.
 bool ig_pointwise(const fc_conv_shape &s, int bk, bool x16) {
@@ -899,6 +913,12 @@ bool ig_splits(const fc_conv_shape &s, const fc_gemm_config &c) {
     if (c.waves_k > 1 || c.bm % 64 != 0 || 4l * s.N * s.C * s.H * s.W >= (1l << 31) || (long)s.C * s.kh * s.kw <= 48) return false;
     if (ig_pointwise(s, c.bk, true) && s.K <= 64) return false;
     return s.kh * s.kw <= 64 || (s.C % c.bk == 0 && ig_inside(s, c.bk));
+}
+
+// The tile that runs a layer under a configuration.
+IgTileSize ig_tile_size(const fc_conv_shape &s, const fc_gemm_config &c) {
+    if (c.id < kNumIgConfigs && ig_splits(s, c)) return kIgSplitTiles[c.id];
+    return {c.bm, c.bn};
 }
 
 // Order of the reduction rows and their number (before rounding up to a stage).
@@ -933,8 +953,6 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
     if constexpr (!std::is_void<typename IgSplitOf<TL>::type>::value) {
         if (ig_splits(s, cfg)) {
             typedef typename IgSplitOf<TL>::type S;
-            p.nKB = p.K_pad / S::BM_;
-            p.nPB = (int)((p.Npix + S::BN_ - 1) / S::BN_);
             const dim3 grid((unsigned)(((long)p.nKB * p.nPB + 7) / 8 * 8), (unsigned)p.splitK), block(S::THREADS);
             long rows;
             const int order = ig_order(s, cfg, &rows);
@@ -1095,7 +1113,8 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
         if (rows >= (1l << 28)) return FC_ERR_UNSUPPORTED;
     }
     plan->Kred_pad = (int)fc_round_up(rows, cfg.bk);
-    plan->K_pad = (int)fc_round_up(s->K, cfg.bm);
+    const IgTileSize tile = ig_tile_size(*s, cfg);
+    plan->K_pad = (int)fc_round_up(s->K, tile.bm);
     plan->Npix = npix;
     plan->config = config;
     // in fp32 and, where products are split, in three bf16 parts
@@ -1110,7 +1129,7 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
     }
     // Small layers do not fill 256 CUs with (K_pad/BM) x (Npix/BN) workgroups: split the
     // reduction until about three workgroups per CU exist, keeping >= 4 LDS stages per part.
-    const long blocks = (long)(plan->K_pad / cfg.bm) * ((npix + cfg.bn - 1) / cfg.bn);
+    const long blocks = (long)(plan->K_pad / tile.bm) * ((npix + tile.bn - 1) / tile.bn);
     const int stages = plan->Kred_pad / cfg.bk;
     int splitK = 1;
     // A grid of two to four workgroups per CU is placed unevenly by the dispatcher (some CUs get
@@ -1274,14 +1293,15 @@ static int igemm_run(fc_context *ctx, const fc_igemm_plan *plan, const float *x_
     p.kh = s.kh; p.kw = s.kw; p.sh = s.sh; p.sw = s.sw; p.pt = s.pt; p.pl = s.pl; p.relu = relu;
     p.Kred_pad = plan->Kred_pad; p.K_pad = plan->K_pad; p.Npix = plan->Npix;
     p.xBytes = 4l * s.N * s.C * s.H * s.W;
-    p.nKB = plan->K_pad / cfg.bm;
-    p.nPB = (int)((plan->Npix + cfg.bn - 1) / cfg.bn);
+    const IgTileSize tile = ig_tile_size(s, cfg);
+    p.nKB = plan->K_pad / tile.bm;
+    p.nPB = (int)((plan->Npix + tile.bn - 1) / tile.bn);
     p.divOHW = fc_make_fastdiv((uint32_t)(plan->OH * plan->OW));
     p.divOW = fc_make_fastdiv((uint32_t)plan->OW);
     p.splitK = plan->split_k;
     p.stagesPerSplit = ((plan->Kred_pad / cfg.bk) + plan->split_k - 1) / plan->split_k;
     p.ws = ws_dev;
-    p.fastStore = s.K % cfg.bm == 0 && 4.0 * s.N * s.K * plan->OH * plan->OW < 4294967296.0 &&
+    p.fastStore = s.K % tile.bm == 0 && 4.0 * s.N * s.K * plan->OH * plan->OW < 4294967296.0 &&
                   4.0 * plan->split_k * s.K * (double)plan->Npix < 4294967296.0 && ((uintptr_t)bias_dev & 15) == 0;
     if ((long)p.nKB * p.nPB >= (1l << 31)) return fail(FC_ERR_UNSUPPORTED, "grid too large");
     fc_stage_scope scope(ctx, timed ? FC_STAGE_IMPLICIT_GEMM : -1);

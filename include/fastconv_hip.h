@@ -347,6 +347,8 @@ int fc_wino_forward(fc_context *ctx, const fc_wino_plan *plan, const float *x_de
 
 int fc_igemm_num_configs(void);
 int fc_igemm_get_config(int id, fc_gemm_config *cfg);
+/* Where products are split (fc_igemm_splits_products) the tiles of 256x128, 128x256 and 64x256 run as
+ * 128x128, 128x128 and 64x128, and plans are made for those. */
 /* Untuned choice, as above (the role of mc=8, nc=256, kc=384 in
  * convLayer/im2colConv.h:17-18). */
 int fc_igemm_default_config(const fc_conv_shape *shape);

@@ -141,3 +141,17 @@ def test_layers_no_tile_of_which_fits_the_static_workspace(lib, c, without):
         assert lib.fc_igemm_make_plan(C.byref(s), i, C.byref(plan)) == 0 and plan.ws_bytes > capi.IGEMM_STATIC_WS_BYTES
     assert lib.fc_igemm_make_plan(C.byref(s), lib.fc_igemm_default_config(C.byref(s)), C.byref(plan)) == 0
     assert (plan.ws_bytes == 0) == without
+
+
+@pytest.mark.parametrize("geo", [(1, 256, 56, 56, 256, 3, 1, 1), (32, 256, 28, 28, 256, 3, 2, 1), (4, 512, 28, 28, 100, 1, 1, 0), (8, 3, 61, 61, 700, 7, 2, 3)])
+def test_plans_are_made_for_the_tile_that_runs(lib, geo):
+    """256x128, 128x256 and 64x256 run as 128x128, 128x128 and 64x128 where products are split."""
+    n, c, h, w, k, ks, st, p = geo
+    s, a, b = capi.ConvShape(n, c, h, w, k, ks, ks, st, st, p, p, p, p), capi.IgemmPlan(), capi.IgemmPlan()
+    for big, runs in ((5, 0), (6, 0), (7, 1)):
+        assert lib.fc_igemm_make_plan(C.byref(s), big, C.byref(a)) == 0 and lib.fc_igemm_make_plan(C.byref(s), runs, C.byref(b)) == 0
+        assert lib.fc_igemm_splits_products(C.byref(a)) == 1 and a.config == big
+        assert (a.K_pad, a.Kred_pad, a.split_k, a.ws_bytes, a.Wp_bytes) == (b.K_pad, b.Kred_pad, b.split_k, b.ws_bytes, b.Wp_bytes), big
+    whole = capi.ConvShape(n, 4, h, w, k, 3, 3, st, st, 1, 1, 1, 1)      # 36 rows: not split
+    assert lib.fc_igemm_make_plan(C.byref(whole), 5, C.byref(a)) == 0 and a.K_pad % 256 == 0
+    assert lib.fc_igemm_splits_products(C.byref(a)) == 0
