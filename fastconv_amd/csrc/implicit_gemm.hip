@@ -1016,9 +1016,13 @@ double ig_ws_us(const fc_conv_shape &s, const fc_gemm_config &c, long npix) {
     return 3.5 + (perCu * units * cycles + 52.8 * perCu * mt * nt * c.waves_k) / 2000;
 }
 
+// The kernel that adds up partial sums has one workgroup row per output channel.
+constexpr int kMaxReduceChannels = 65535;
+
 // A plan whose partial sums fit the static workspace goes before any other, however much faster that is: the untuned plan is
 // what callers of fc_conv_implicit_gemm_static use.  Batch 32, us, fitting plan against the best one: 3x3/2 256->256@28 69.1 / 67.4,
 // 3x3 128->128@28 59.6 / 64.1, 512->512@14 209 / 193, 1x1/2 1024->2048@14 73.1 / 63.8.
+// Plans that cannot run because of their partial sums (kMaxReduceChannels) are behind in the same way.
 // A layer whose reduction the best tile would split over workgroups goes to the kernels that split it inside the workgroup
 // where those are expected ahead, from 9 parts on also where they are 15 % behind and from 21 on 50 %: the model then favours
 // the tiles (most of the layers that lost more than 15 % by it: 9 to 32 parts, reductions of 1000 to 9000 rows, 15 to 25 us);
@@ -1031,7 +1035,7 @@ int ig_split_default_config(const fc_conv_shape *s) {
     for (int id = 0; id < 4; id++) {
         if (fc_igemm_make_plan(s, id, &plan) != FC_OK) continue;
         const double us = ig_split_us(*s, id, plan);
-        const bool fits = plan.ws_bytes <= (size_t)FC_IGEMM_STATIC_WS_BYTES;
+        const bool fits = plan.ws_bytes <= (size_t)FC_IGEMM_STATIC_WS_BYTES && (plan.split_k == 1 || s->K <= kMaxReduceChannels);
         if (fits != bestFits ? fits : us < bestUs) { bestUs = us; best = id; bestPlan = plan; bestFits = fits; }
     }
     const int ws = bestPlan.split_k > 1 ? fc_igemm_ws_choose(s, plan.Npix) : -1;
@@ -1319,7 +1323,7 @@ static int igemm_run(fc_context *ctx, const fc_igemm_plan *plan, const float *x_
     FC_LAUNCH_CHECK(ctx, "igemm_conv_kernel");
     if (plan->split_k > 1) {
         const dim3 rgrid((unsigned)((plan->Npix + 255) / 256), (unsigned)s.K);
-        if (rgrid.y > 65535) return fail(FC_ERR_UNSUPPORTED, "more than 65535 channels");
+        if (rgrid.y > kMaxReduceChannels) return fail(FC_ERR_UNSUPPORTED, "more than 65535 channels");
         igemm_reduce_kernel<<<rgrid, dim3(256), 0, ctx->stream>>>(ws_dev, bias_dev, y_dev, s.K, plan->Npix,
                                                                   plan->OH * plan->OW, plan->split_k, relu, p.divOHW);
         FC_LAUNCH_CHECK(ctx, "igemm_reduce_kernel");

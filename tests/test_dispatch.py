@@ -155,3 +155,11 @@ def test_plans_are_made_for_the_tile_that_runs(lib, geo):
     whole = capi.ConvShape(n, 4, h, w, k, 3, 3, st, st, 1, 1, 1, 1)      # 36 rows: not split
     assert lib.fc_igemm_make_plan(C.byref(whole), 5, C.byref(a)) == 0 and a.K_pad % 256 == 0
     assert lib.fc_igemm_splits_products(C.byref(a)) == 0
+
+
+@pytest.mark.parametrize("k", [65535, 65536, 70000, 100000])
+def test_untuned_plans_of_very_many_channels_can_run(lib, k):
+    """The sum over the parts of a split reduction takes 65535 output channels."""
+    s, plan = capi.ConvShape(1, 4096, 4, 4, k, 1, 1, 1, 1, 0, 0, 0, 0), capi.IgemmPlan()
+    assert lib.fc_igemm_make_plan(C.byref(s), lib.fc_igemm_default_config(C.byref(s)), C.byref(plan)) == 0
+    assert plan.split_k == 1 or k <= 65535
