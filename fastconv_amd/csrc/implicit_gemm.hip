@@ -40,37 +40,37 @@ __global__ __launch_bounds__(256) void igemm_pack_filter_kernel(const float *__r
                                                                 int kh, int kw, int H, int W, int rows,
                                                                 int Kred_pad, int K_pad, int order) {
     const int k = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int kred = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (kred >= Kred_pad) return;
-    int c = 0, r = 31, s = 31;
-    bool real = kred < rows;
-    if (real) {
-        if (order == IG_ORDER_TAP) {
-            const int t = kred / C;
-            c = kred - t * C;
-            r = t / kw;
-            s = t - r * kw;
-        } else if (order == IG_ORDER_BLOCK) {
-            const int stage = kred / 16, block = stage / (kh * kw), t = stage - block * (kh * kw);
-            c = block * 16 + kred % 16;
-            r = t / kw;
-            s = t - r * kw;
-            real = c < C;
-        } else {
-            const int run = order == IG_ORDER_ROW8 ? 8 : order == IG_ORDER_ROW4 ? 4 : 1;
-            const int width = (kw + run - 1) / run * run;      // rows of the reduction per window row
-            c = kred / (kh * width);
-            const int rs = kred - c * kh * width;
-            r = rs / width;
-            s = rs - r * width;
-            real = s < kw;
+    for (int kred = blockIdx.y * 4 + (threadIdx.x >> 6); kred < Kred_pad; kred += 4 * gridDim.y) {
+        int c = 0, r = 31, s = 31;
+        bool real = kred < rows;
+        if (real) {
+            if (order == IG_ORDER_TAP) {
+                const int t = kred / C;
+                c = kred - t * C;
+                r = t / kw;
+                s = t - r * kw;
+            } else if (order == IG_ORDER_BLOCK) {
+                const int stage = kred / 16, block = stage / (kh * kw), t = stage - block * (kh * kw);
+                c = block * 16 + kred % 16;
+                r = t / kw;
+                s = t - r * kw;
+                real = c < C;
+            } else {
+                const int run = order == IG_ORDER_ROW8 ? 8 : order == IG_ORDER_ROW4 ? 4 : 1;
+                const int width = (kw + run - 1) / run * run;      // rows of the reduction per window row
+                c = kred / (kh * width);
+                const int rs = kred - c * kh * width;
+                r = rs / width;
+                s = rs - r * width;
+                real = s < kw;
+            }
         }
-    }
-    if (k < K_pad)
-        Wp[(size_t)kred * K_pad + k] = (k < K && real) ? w[((size_t)k * C + c) * (kh * kw) + r * kw + s] : 0.f;
-    if (blockIdx.x == 0 && (threadIdx.x & 63) == 0) {
-        table[2 * kred] = real ? c * H * W + r * W + s : 0;
-        table[2 * kred + 1] = real ? (r << 16) | s : (31 << 16) | 31;
+        if (k < K_pad)
+            Wp[(size_t)kred * K_pad + k] = (k < K && real) ? w[((size_t)k * C + c) * (kh * kw) + r * kw + s] : 0.f;
+        if (blockIdx.x == 0 && (threadIdx.x & 63) == 0) {
+            table[2 * kred] = real ? c * H * W + r * W + s : 0;
+            table[2 * kred + 1] = real ? (r << 16) | s : (31 << 16) | 31;
+        }
     }
 }
 
@@ -1175,8 +1175,9 @@ extern "C" int fc_igemm_pack_filter(fc_context *ctx, const fc_igemm_plan *plan, 
     if (rc) return rc;
     if (!w_dev || !Wp_dev || !table_dev) return fc_set_error(ctx, FC_ERR_INVALID, "fc_igemm_pack_filter: null buffer", hipSuccess);
     const fc_conv_shape &s = plan->shape;
-    const dim3 grid((plan->K_pad + 63) / 64, (plan->Kred_pad + 3) / 4);
-    if (grid.y > 65535) return fc_set_error(ctx, FC_ERR_UNSUPPORTED, "fc_igemm_pack_filter: reduction too long", hipSuccess);
+    // (padded window rows or channels may take the rows of the packed filter past this)
+    if (fc_round_up(plan->Kred, 16) / 4 > 65535) return fc_set_error(ctx, FC_ERR_UNSUPPORTED, "fc_igemm_pack_filter: reduction too long", hipSuccess);
+    const dim3 grid((plan->K_pad + 63) / 64, std::min((plan->Kred_pad + 3) / 4, 65535));
     if (plan->config >= kNumIgConfigs) return fc_igemm_ws_pack(ctx, plan, w_dev, Wp_dev, table_dev);
     fc_gemm_config cfg;
     fc_igemm_get_config(plan->config, &cfg);

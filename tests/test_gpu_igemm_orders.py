@@ -56,3 +56,14 @@ def test_orders_of_the_reduction(lib, s):  # noqa: F811
         assert (np.abs(got - with_bias) <= tol + 2.0 ** -23 * (np.abs(truth) + 1)).all(), cfg.id
         seen += 1
     assert seen
+
+
+@pytest.mark.parametrize("c", [29120, 29125])
+def test_longest_reductions(lib, c):  # noqa: F811
+    """262125 rows of the filter, 262224 of the packed one; 29120 channels need no padding."""
+    s = O.shape(1, c, 3, 3, 33, 3, 3, 1, 1, 0)
+    x, w = O.make_inputs(s, seed=c)
+    truth, tol = O.naive_conv_f64(s, x, w), bound(s, x, w)
+    for cfg in (3, 4):
+        print("longest", c, cfg, flush=True)
+        assert (np.abs(lib.implicit_gemm_conv(cshape(s), x, w, config=cfg) - truth) <= tol).all()
