@@ -345,9 +345,18 @@ int main(int argc, char *argv[]) {
         size_t bytes = 4 * (in_elems + 2 * k_elems + out_elems) + ((size_t)64 << 20);
         if (options.algorithm == nnp_convolution_algorithm_winograd)
             bytes += 4 * 64 * (cpad * kpad + cpad * tpad + kpad * tpad);
-        else
-            bytes += 4 * ((k_elems / output_channels + 32) * kpad) + 8 * (k_elems / output_channels + 32) +
-                     std::min<size_t>(32 * 4 * out_elems, (size_t)1 << 30);   // split-reduction workspace of small layers
+        else {
+            // packed filter, gather table and split-reduction workspace of the tile shape that needs most
+            const fc_conv_shape shp = {(int)options.batch, (int)input_channels, (int)input_size.height, (int)input_size.width,
+                                       (int)output_channels, (int)kernel_size.height, (int)kernel_size.width,
+                                       (int)output_subsampling.height, (int)output_subsampling.width, (int)input_padding.top,
+                                       (int)input_padding.bottom, (int)input_padding.left, (int)input_padding.right};
+            size_t most = 0;
+            fc_igemm_plan plan;
+            for (int id = 0; id < fc_igemm_num_configs(); id++)
+                if (fc_igemm_make_plan(&shp, id, &plan) == FC_OK) most = std::max(most, plan.Wp_bytes + plan.table_bytes + plan.ws_bytes);
+            bytes += most;
+        }
         fastconv::Device::Configure(bytes);
     }
 

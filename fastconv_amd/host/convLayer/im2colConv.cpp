@@ -1,5 +1,6 @@
 #include "im2colConv.h"
 
+#include "../select_algorithm.h"
 #include "../utility/tuning_log.h"
 
 using fastconv::Device;
@@ -44,6 +45,11 @@ void ConvIm2colLayer::SetChannelBias(const float *bias_k, bool relu_) {
     relu = relu_;
 }
 
+// Whether the arena has room for what a plan needs (the arena hands out multiples of 256 bytes).
+static bool Fits(const fc_igemm_plan &plan) {
+    return plan.Wp_bytes + plan.table_bytes + plan.ws_bytes + 3 * 256 <= Device::Get().Left();
+}
+
 // Plans one tile shape and re-lays the filter for it (the one-time counterpart
 // of the reference's per-call pack_a, im2col/gemm_pack.cpp:192-260).
 void ConvIm2colLayer::AllocateFor(int cfg) {
@@ -54,7 +60,9 @@ void ConvIm2colLayer::AllocateFor(int cfg) {
         fprintf(stderr, "Error: no implicit-GEMM plan for this layer: %s\n", fc_status_string(rc));
         exit(EXIT_FAILURE);
     }
-    config = cfg;
+    // the filter of split products takes 10 bytes an element: without room for it, products on fp32 instructions
+    if (fc_igemm_splits_products(&plan) && !Fits(plan)) igemm_plan_of_fp32_filter(s, &plan);
+    config = plan.config;
     packed_kernel = (float *)d.Alloc(plan.Wp_bytes, "packed kernel");
     gather_table = (int32_t *)d.Alloc(plan.table_bytes, "gather table");
     workspace = plan.ws_bytes ? (float *)d.Alloc(plan.ws_bytes, "split-reduction workspace") : NULL;
@@ -74,6 +82,7 @@ int ConvIm2colLayer::Init() {
     dev.Acquire(input_data, in_elems, kernel_data, (size_t)M * K, output_elements());
     if (channel_bias) dev.SetBias(channel_bias, output_channels);
     AllocateFor(config_best);
+    config_best = config;
     fc_gemm_config c;
     fc_igemm_get_config(config, &c);
     printf("Testing M=%d N=%ld K=%d batch=%zu tile %dx%dx%d (cfg %d) reduction split %d over workgroups, %d over wavefronts\n",
@@ -132,6 +141,7 @@ int ConvIm2colLayer::Tuning() {
     for (int cfg = 0; cfg < fc_igemm_num_configs(); cfg++) {
         fc_igemm_plan probe;
         if (fc_igemm_make_plan(&s, cfg, &probe) != FC_OK) continue;      // a tile shape that cannot run this layer
+        if (fc_igemm_splits_products(&probe) && !Fits(probe)) continue;
         const size_t mark = d.Mark();
         AllocateFor(cfg);
         RunOnce();

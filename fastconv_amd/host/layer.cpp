@@ -61,6 +61,8 @@ int ConvolutionLayer::Init() {
         common_mempool->Request(m_off_ + (fused_ ? 0 : wplan_.M_bytes));
     } else {
         d.Check(fc_igemm_make_plan(&shape_, fc_igemm_default_config(&shape_), &iplan_), "fc_igemm_make_plan");
+        // products on fp32 instructions: slower, but 4 bytes an element of the filter in place of 10
+        if (no_split_filter_ && fc_igemm_splits_products(&iplan_)) igemm_plan_of_fp32_filter(shape_, &iplan_);
         // the largest tile whose workgroups split the reduction among themselves needs no partial sums in memory
         int area = 0;
         for (int id = 0; no_scratch_ && iplan_.ws_bytes && id < fc_igemm_num_configs(); id++) {
@@ -163,10 +165,14 @@ bool Net::InitLayers() {
 
 int Net::Init() {
     if (InitLayers()) return 0;
-    fprintf(stderr, "Net: the arena is too small for the shared scratch (%zu bytes); layers that can do without it will\n", common_->common_bytes());
-    common_->FreeAll();
-    for (size_t i = 0; i < layers_.size(); i++) layers_[i]->LeaveScratch();
-    if (InitLayers()) return 0;
+    for (int step = 1; step < 4; step++) {
+        const bool scratch = step != 2, split_filter = step != 1;
+        fprintf(stderr, "Net: the arena is too small (shared scratch %zu bytes); layers that can do without %s will\n", common_->common_bytes(),
+                !split_filter ? "scratch" : !scratch ? "a filter for split products" : "both");
+        common_->FreeAll();
+        for (size_t i = 0; i < layers_.size(); i++) layers_[i]->Leave(scratch, split_filter);
+        if (InitLayers()) return 0;
+    }
     fprintf(stderr, "Error: the arena is too small for the shared scratch (%zu bytes)\n", common_->common_bytes());
     return -1;
 }

@@ -39,13 +39,16 @@ class Layer {
     // Shapes (and allocates) the output blobs from the bottom blobs.
     virtual int GenerateTopBlobs() = 0;
     // Other initialisation: plans, filter transforms, scratch requests to the common pool.  Called again, after
-    // LeaveScratch(), when the arena has no room for the scratch of the fastest ways.
+    // Leave(), when the arena has no room for the fastest ways.
     virtual int Init() { return 0; }
-    // From now on without scratch where the layer has such a way; its buffers go back.
-    void LeaveScratch() {
+    // From now on without scratch, or without filters packed for split products, where the layer has such a way; its
+    // buffers go back.
+    void Leave(bool scratch, bool split_filter) {
         private_mempool->FreeAll();
-        no_scratch_ = true;
+        no_scratch_ = scratch;
+        no_split_filter_ = split_filter;
     }
+    void LeaveScratch() { Leave(true, false); }
     virtual int Forward() = 0;
 
     std::string name() { return _name; }
@@ -72,7 +75,7 @@ class Layer {
     CommonMemPool<float> *common_mempool;
     PrivateMemPool<float> *private_mempool;
     fastconv::RangeAllocator *_alloc = NULL;
-    bool no_scratch_ = false;
+    bool no_scratch_ = false, no_split_filter_ = false;
 };
 
 // kernel x kernel convolution, optional per-channel bias and ReLU fused into the epilogue.

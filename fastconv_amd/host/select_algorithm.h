@@ -25,3 +25,20 @@ inline enum nnp_convolution_algorithm select_algorithm(struct nnp_size kernel_si
     }
     return nnp_convolution_algorithm_im2col;
 }
+
+// The implicit-GEMM plan of a layer whose filter is packed in fp32 alone: 4 bytes an element, where split products take 10
+// (fc_igemm_splits_products).  Tiles that need no workspace go first, of those the tiles in LDS, of those the largest.
+inline bool igemm_plan_of_fp32_filter(const fc_conv_shape &shape, fc_igemm_plan *plan) {
+    int best = -1;
+    for (int id = 0; id < fc_igemm_num_configs(); id++) {
+        fc_gemm_config c;
+        fc_igemm_plan p;
+        if (fc_igemm_get_config(id, &c) != FC_OK || (c.waves_k != 1 && c.waves_k != 8)) continue;
+        if (fc_igemm_make_plan(&shape, id, &p) != FC_OK || fc_igemm_splits_products(&p)) continue;
+        const int rank = (p.ws_bytes == 0 ? 1 << 28 : 0) + (c.waves_k == 1 ? 1 << 27 : 0) + c.bm * c.bn;
+        if (rank <= best) continue;
+        best = rank;
+        *plan = p;
+    }
+    return best >= 0;
+}

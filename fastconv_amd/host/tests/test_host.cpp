@@ -142,6 +142,18 @@ static void test_select_algorithm() {
     CHECK(select_algorithm(k3, s1, wide, 64, 64, 8) == nnp_convolution_algorithm_im2col);
 }
 
+static void test_plan_of_fp32_filter() {
+    const fc_conv_shape shapes[] = {{16, 512, 28, 28, 512, 3, 3, 1, 1, 1, 1, 1, 1}, {1, 512, 14, 14, 512, 3, 3, 2, 2, 1, 1, 1, 1},
+                                    {32, 3, 224, 224, 64, 7, 7, 2, 2, 3, 3, 3, 3}, {2, 70, 9, 9, 33, 31, 1, 1, 1, 15, 15, 0, 0}};
+    for (size_t i = 0; i < sizeof shapes / sizeof shapes[0]; i++) {
+        fc_igemm_plan p, split;
+        CHECK(igemm_plan_of_fp32_filter(shapes[i], &p) && fc_igemm_make_plan(&shapes[i], 3, &split) == FC_OK);
+        CHECK(fc_igemm_splits_products(&split) && !fc_igemm_splits_products(&p));
+        CHECK(p.Wp_bytes == sizeof(float) * p.Kred_pad * p.K_pad && p.K_pad <= split.K_pad && p.Kred_pad <= split.Kred_pad);
+        CHECK(p.ws_bytes == 0);
+    }
+}
+
 static void test_conv_layer_geometry_and_naive() {
     // 8 channels of ones, 9x9, 3x3 kernel of ones, stride 2, pad 1: corner 32, centre 72
     const int C = 8, H = 9, K = 2;
@@ -222,6 +234,7 @@ int main(int argc, char **argv) {
     test_pools();
     test_tuning_log();
     test_select_algorithm();
+    test_plan_of_fp32_filter();
     test_conv_layer_geometry_and_naive();
     test_rng();
     if (failures) {

@@ -59,6 +59,12 @@ size_t Device::Mark() {
     return m;
 }
 
+size_t Device::Left() {
+    size_t capacity = 0, used = 0, peak = 0;
+    Check(fc_pool_stats(pool_, &capacity, &used, &peak), "fc_pool_stats");
+    return capacity - used;
+}
+
 void Device::Release(size_t mark) { Check(fc_pool_release(pool_, mark), "fc_pool_release"); }
 
 }  // namespace fastconv

@@ -25,6 +25,7 @@ class Device {
     void *Alloc(size_t bytes, const char *what);
     void Check(int status, const char *what);
     size_t Mark();
+    size_t Left();      // bytes of the arena not handed out
     void Release(size_t mark);
 
    private:

@@ -354,12 +354,15 @@ int fc_igemm_get_config(int id, fc_gemm_config *cfg);
 int fc_igemm_default_config(const fc_conv_shape *shape);
 
 /* Filter re-layout done once at Init: Wp[Kred_pad][K_pad], output channel
- * fastest, plus the per-row gather table.  The order of the reduction rows is
- * the library's business and depends on plan->config: the column matrix's
- * (c, r, s) (convLayer/im2colConv.cpp:285-309) in general, tap-major (r, s, c)
- * when C is a whole number of the configuration's reduction stages.  Treat Wp
- * and the table as opaque, hand them only to calls made with the same plan, and
- * pack them again when the configuration changes. */
+ * fastest, plus the per-row gather table; where products are split the filter
+ * follows a second time as operand words of its three bf16 parts, 10 bytes an
+ * element together (Wp_bytes says how many there are).  The order of the
+ * reduction rows and the rows added to it are the library's business and depend
+ * on plan->config: the column matrix's (c, r, s) (convLayer/im2colConv.cpp:285-309)
+ * or tap-major (r, s, c) on fp32 instructions, blocks of 16 channels or window
+ * rows in runs of 8 or 4 columns, both padded to whole ones, on split products.
+ * Treat Wp and the table as opaque, hand them only to calls made with the same
+ * plan, and pack them again when the configuration changes. */
 typedef struct {
     fc_conv_shape shape;
     int OH, OW;
@@ -372,8 +375,8 @@ typedef struct {
 } fc_igemm_plan;
 
 int fc_igemm_make_plan(const fc_conv_shape *shape, int config, fc_igemm_plan *plan);
-/* As fc_wino_gemm_splits_products, for x at a multiple of 16 bytes (else a pointwise layer of up to 64
- * output channels is split as well). */
+/* As fc_wino_gemm_splits_products.  Without room for the filter of split products, the configurations for which
+ * this is 0 (32x64, and those with waves_k above 1) keep it in fp32 alone. */
 int fc_igemm_splits_products(const fc_igemm_plan *plan);
 
 /* Replaces pack_a_v2 (im2col/gemm_pack.cpp:192-260) as a one-time step. */

@@ -200,6 +200,25 @@ def test_layer_graph_fits_an_arena_without_room_for_the_fastest_way():
     assert "PASS" in out and int(re.search(r"shared scratch (\d+) KB", out).group(1)) < 60 << 10
 
 
+def test_layer_graph_fits_an_arena_without_room_for_filters_of_split_products():
+    """No layer of this trunk has scratch; one runs on split products, whose filter takes 10 bytes an element (184 KB for
+    37).  Short of that room the layer runs on fp32 instructions."""
+    args = [_exe("net_test"), "-n", "32", "-is", "32", "-w", "2", "-i", "2"]
+    scratch, used = (int(v) for v in re.search(r"shared scratch (\d+) KB, arena used (\d+) KB", _run(args + ["--no-check"])).groups())
+    assert scratch == 0
+    out = _run(args + ["--arena", str(used - 100)])
+    assert "PASS" in out and int(re.search(r"arena used (\d+) KB", out).group(1)) <= used - 100
+
+
+@pytest.mark.parametrize("tuning", [[], ["-tn", "tuning"]])
+def test_im2col_layer_fits_an_arena_without_room_for_a_filter_of_split_products(tmp_path, monkeypatch, tuning):
+    """Input, filter and output of this layer and its filter packed in fp32 take 67.0 MiB, packed for split products 80.5."""
+    monkeypatch.setenv("FASTCONV_POOL_BYTES", str(69 << 20))
+    out = _run([_exe("conv_test"), "-ic", "512", "-oc", "512", "-is", "28", "28", "-ks", "3", "3", "-ip", "1", "-n", "16", "-i", "2",
+                "-t", "16", "--check-images", "1", "--strict", "-a", "im2col"] + tuning, cwd=str(tmp_path))
+    assert "PASS" in out and "FAIL" not in out
+
+
 def test_layer_graph_replayed_from_a_recording_matches_the_host_chain():
     out = _run([_exe("net_test"), "-n", "1", "-is", "64", "-w", "4", "-i", "3", "--graph"])
     m = re.search(r"Max relative error vs host chain: (\S+)", out)
