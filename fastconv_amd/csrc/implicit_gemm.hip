@@ -1019,31 +1019,27 @@ double ig_ws_us(const fc_conv_shape &s, const fc_gemm_config &c, long npix) {
 // The kernel that adds up partial sums has one workgroup row per output channel.
 constexpr int kMaxReduceChannels = 65535;
 
-// A plan whose partial sums fit the static workspace goes before any other, however much faster that is: the untuned plan is
-// what callers of fc_conv_implicit_gemm_static use.  Batch 32, us, fitting plan against the best one: 3x3/2 256->256@28 69.1 / 67.4,
-// 3x3 128->128@28 59.6 / 64.1, 512->512@14 209 / 193, 1x1/2 1024->2048@14 73.1 / 63.8.
-// Plans that cannot run because of their partial sums (kMaxReduceChannels) are behind in the same way.
+// Plans that cannot run because of their partial sums (kMaxReduceChannels) are behind all others.
 // A layer whose reduction the best tile would split over workgroups goes to the kernels that split it inside the workgroup
 // where those are expected ahead, from 9 parts on also where they are 15 % behind and from 21 on 50 %: the model then favours
-// the tiles (most of the layers that lost more than 15 % by it: 9 to 32 parts, reductions of 1000 to 9000 rows, 15 to 25 us);
-// and wherever no tile's partial sums fit.
+// the tiles (most of the layers that lost more than 15 % by it: 9 to 32 parts, reductions of 1000 to 9000 rows, 15 to 25 us).
 int ig_split_default_config(const fc_conv_shape *s) {
     int best = 3;
     double bestUs = 1e300;
-    bool bestFits = false;
+    bool bestRuns = false;
     fc_igemm_plan plan, bestPlan = {};
     for (int id = 0; id < 4; id++) {
         if (fc_igemm_make_plan(s, id, &plan) != FC_OK) continue;
         const double us = ig_split_us(*s, id, plan);
-        const bool fits = plan.ws_bytes <= (size_t)FC_IGEMM_STATIC_WS_BYTES && (plan.split_k == 1 || s->K <= kMaxReduceChannels);
-        if (fits != bestFits ? fits : us < bestUs) { bestUs = us; best = id; bestPlan = plan; bestFits = fits; }
+        const bool runs = plan.split_k == 1 || s->K <= kMaxReduceChannels;
+        if (runs != bestRuns ? runs : us < bestUs) { bestUs = us; best = id; bestPlan = plan; bestRuns = runs; }
     }
     const int ws = bestPlan.split_k > 1 ? fc_igemm_ws_choose(s, plan.Npix) : -1;
     if (ws >= 0) {
         fc_gemm_config c;
         fc_igemm_ws_get_config(ws, kNumIgConfigs + ws, &c);
         const double behind = bestPlan.split_k > 20 ? 1.5 : bestPlan.split_k > 8 ? 1.15 : 1.0;
-        if (!bestFits || ig_ws_us(*s, c, plan.Npix) < bestUs * behind) return kNumIgConfigs + ws;
+        if (!bestRuns || ig_ws_us(*s, c, plan.Npix) < bestUs * behind) return kNumIgConfigs + ws;
     }
     return best;
 }
@@ -1094,6 +1090,21 @@ extern "C" int fc_igemm_default_config(const fc_conv_shape *s) {
         if (ws >= 0) return kNumIgConfigs + ws;
     }
     return best;
+}
+
+// The reduction of a plan, `stages` long, in at most `parts` of equal length, none of them empty.
+static void ig_set_parts(fc_igemm_plan &plan, int stages, int parts) {
+    const int per = (stages + parts - 1) / parts;
+    plan.split_k = (stages + per - 1) / per;
+    plan.ws_bytes = plan.split_k > 1 ? sizeof(float) * (size_t)plan.split_k * plan.shape.K * plan.Npix : 0;
+}
+
+// In no more parts than have room for their sums: the packed filter does not depend on the number of parts.
+static void ig_split_to_fit(fc_igemm_plan &plan, size_t ws_bytes) {
+    fc_gemm_config cfg;
+    fc_igemm_get_config(plan.config, &cfg);
+    const size_t parts = ws_bytes / (sizeof(float) * (size_t)plan.shape.K * plan.Npix);
+    ig_set_parts(plan, plan.Kred_pad / cfg.bk, (int)std::max<size_t>(1, std::min<size_t>(plan.split_k, parts)));
 }
 
 extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_plan *plan) {
@@ -1148,9 +1159,7 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
         if (splitK > 32) splitK = 32;
         if (splitK < 1) splitK = 1;
     }
-    const int per = (stages + splitK - 1) / splitK;
-    plan->split_k = (stages + per - 1) / per;          // no empty parts
-    plan->ws_bytes = plan->split_k > 1 ? sizeof(float) * (size_t)plan->split_k * s->K * npix : 0;
+    ig_set_parts(*plan, stages, splitK);
     return FC_OK;
 }
 
@@ -1253,12 +1262,16 @@ extern "C" int fc_conv_implicit_gemm_static(fc_context *ctx, const fc_igemm_plan
                                             int relu, float *y_dev) {
     const int rc = ig_plan_check(ctx, plan);
     if (rc) return rc;
+    fc_igemm_plan fits = *plan;
     if (plan->ws_bytes > (size_t)FC_IGEMM_STATIC_WS_BYTES) {
-        char msg[200];
-        snprintf(msg, sizeof msg, "fc_conv_implicit_gemm_static: this layer needs %zu bytes of split-reduction workspace, "
-                 "the static one holds %d: use fc_conv_implicit_gemm with a workspace of the caller's", plan->ws_bytes,
-                 FC_IGEMM_STATIC_WS_BYTES);
-        return fc_set_error(ctx, FC_ERR_UNSUPPORTED, msg, hipSuccess);
+        if (plan->config != fc_igemm_default_config(&plan->shape)) {
+            char msg[200];
+            snprintf(msg, sizeof msg, "fc_conv_implicit_gemm_static: this layer needs %zu bytes of split-reduction workspace, "
+                     "the static one holds %d: use fc_conv_implicit_gemm with a workspace of the caller's", plan->ws_bytes,
+                     FC_IGEMM_STATIC_WS_BYTES);
+            return fc_set_error(ctx, FC_ERR_UNSUPPORTED, msg, hipSuccess);
+        }
+        ig_split_to_fit(fits, FC_IGEMM_STATIC_WS_BYTES);
     }
     if (!ctx->igemm_static_ws) return fc_set_error(ctx, FC_ERR_STATE, "fc_conv_implicit_gemm_static: static workspace not set up", hipSuccess);
     {
@@ -1271,7 +1284,7 @@ extern "C" int fc_conv_implicit_gemm_static(fc_context *ctx, const fc_igemm_plan
     }
     // Nothing has to start at zero: every partial sum the reduction reads ([split][k < K][pixel < Npix]) is
     // written by this call's GEMM kernel first.  No event brackets (creating an event may allocate).
-    return igemm_run(ctx, plan, x_dev, Wp_dev, table_dev, bias_dev, relu, ctx->igemm_static_ws, y_dev, false,
+    return igemm_run(ctx, &fits, x_dev, Wp_dev, table_dev, bias_dev, relu, ctx->igemm_static_ws, y_dev, false,
                      "fc_conv_implicit_gemm_static");
 }
 

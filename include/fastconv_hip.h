@@ -400,8 +400,9 @@ int fc_conv_implicit_gemm(fc_context *ctx, const fc_igemm_plan *plan, const floa
  * inside the library instead of a workspace of the caller's (each GPU the library runs on holds
  * that array until the process ends); the call allocates nothing and is never bracketed by
  * timing events.  A plan whose ws_bytes exceeds FC_IGEMM_STATIC_WS_BYTES is refused with
- * FC_ERR_UNSUPPORTED; the plan of fc_igemm_default_config is within it wherever a configuration
- * that might be chosen is.  All calls on one GPU share the array and calls that overlapped in time
+ * FC_ERR_UNSUPPORTED, but for the plan of fc_igemm_default_config, which then runs in as many
+ * parts as the array holds (one if need be): its result is that of fc_conv_implicit_gemm up to
+ * the order of the sums.  All calls on one GPU share the array and calls that overlapped in time
  * would race, so one context per GPU uses it at a time: the first context to make this call on a
  * GPU owns the array until fc_destroy, and the call is refused for any other context meanwhile
  * (FC_ERR_STATE); calls of one context are ordered on its stream and safe.  Other processes have

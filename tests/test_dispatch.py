@@ -112,37 +112,6 @@ def test_which_implicit_gemm_products_are_split(lib, geo, split):
             assert lib.fc_igemm_splits_products(C.byref(plan)) == (split if g.waves_k == 1 and g.bm % 64 == 0 else 0), i
 
 
-IGEMM_LAYERS = [      # ResNet-50 and the VGG-16 layers, (c, k, h, ks, stride)
-    (64, 64, 56, 3, 1), (128, 128, 28, 3, 1), (256, 256, 14, 3, 1), (512, 512, 7, 3, 1), (128, 128, 56, 3, 2), (256, 256, 28, 3, 2),
-    (512, 512, 14, 3, 2), (256, 64, 56, 1, 1), (64, 256, 56, 1, 1), (256, 128, 56, 1, 1), (512, 128, 28, 1, 1), (128, 512, 28, 1, 1),
-    (512, 256, 28, 1, 1), (1024, 256, 14, 1, 1), (256, 1024, 14, 1, 1), (1024, 512, 14, 1, 1), (2048, 512, 7, 1, 1), (512, 2048, 7, 1, 1),
-    (256, 512, 56, 1, 2), (512, 1024, 28, 1, 2), (1024, 2048, 14, 1, 2), (3, 64, 224, 7, 2), (64, 64, 224, 3, 1), (64, 128, 112, 3, 1),
-    (128, 128, 112, 3, 1), (128, 256, 56, 3, 1), (256, 256, 56, 3, 1), (256, 512, 28, 3, 1), (512, 512, 28, 3, 1), (512, 512, 14, 3, 1),
-    (592, 85, 60, 3, 1), (220, 56, 120, 7, 1)]
-
-
-@pytest.mark.parametrize("n", [1, 2, 4, 8, 16, 27, 32, 64])
-def test_untuned_implicit_gemm_plans_fit_the_static_workspace(lib, n):
-    """fc_conv_implicit_gemm_static refuses a plan whose partial sums do not, and callers hand it the untuned one."""
-    plan, split = capi.IgemmPlan(), 0
-    for c, k, h, ks, st in IGEMM_LAYERS:
-        s = capi.ConvShape(n, c, h, h, k, ks, ks, st, st, *([ks // 2] * 4))
-        assert lib.fc_igemm_make_plan(C.byref(s), lib.fc_igemm_default_config(C.byref(s)), C.byref(plan)) == 0
-        assert plan.ws_bytes <= capi.IGEMM_STATIC_WS_BYTES, (c, k, h, ks, st)
-        split += plan.split_k > 1
-    assert split or n == 1
-
-
-@pytest.mark.parametrize("c,without", [(1024, True), (1408, False)])
-def test_layers_no_tile_of_which_fits_the_static_workspace(lib, c, without):
-    """64x64 tiles in 3 parts: partial sums of 36 MB.  Up to 8 GFLOP the kernels that need no workspace take such a layer."""
-    s, plan = capi.ConvShape(1, c, 1, 46 * 256, 256, 1, 1, 1, 1, 0, 0, 0, 0), capi.IgemmPlan()
-    for i in range(4):
-        assert lib.fc_igemm_make_plan(C.byref(s), i, C.byref(plan)) == 0 and plan.ws_bytes > capi.IGEMM_STATIC_WS_BYTES
-    assert lib.fc_igemm_make_plan(C.byref(s), lib.fc_igemm_default_config(C.byref(s)), C.byref(plan)) == 0
-    assert (plan.ws_bytes == 0) == without
-
-
 @pytest.mark.parametrize("geo", [(1, 256, 56, 56, 256, 3, 1, 1), (32, 256, 28, 28, 256, 3, 2, 1), (4, 512, 28, 28, 100, 1, 1, 0), (8, 3, 61, 61, 700, 7, 2, 3)])
 def test_plans_are_made_for_the_tile_that_runs(lib, geo):
     """256x128, 128x256 and 64x256 run as 128x128, 128x128 and 64x128 where products are split."""

@@ -149,3 +149,36 @@ def test_static_workspace_entry_point_inside_a_recorded_graph():
             L.graph_destroy(g)
     finally:
         L.close()
+
+
+@pytest.mark.parametrize("shp,parts", [
+    ((1, 36, 139, 139, 534, 5, 5, 2, 2, 2), 3),      # of 5, channels past a block of 16
+    ((30, 128, 12, 12, 656, 3, 3, 1, 1, 1), 2),      # of 4
+    ((6, 21, 139, 139, 97, 7, 7, 2, 2, 3), 2),       # of 4, window rows in runs
+    ((51, 37, 16, 16, 454, 5, 5, 1, 1, 2), 1),       # of 2: no partial sums at all
+])
+def test_static_workspace_entry_point_takes_every_untuned_plan(shp, parts):
+    """Where the partial sums of the library's own choice pass 32 MiB the reduction runs in fewer parts."""
+    import fastconv_amd as F
+    from fastconv_amd import capi
+    from test_gpu_split_products import bound
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=parts)
+    bias = O.rng_uniform(parts, (s.K,))
+    with F.load(0, 1 << 30) as L:
+        plan = L.igemm_plan(cshape(s), L.igemm_default_config(cshape(s)))
+        assert plan.split_k > parts and plan.ws_bytes > capi.IGEMM_STATIC_WS_BYTES
+        assert parts == max(1, capi.IGEMM_STATIC_WS_BYTES // (4 * s.K * plan.Npix))
+        nout = s.N * s.K * plan.OH * plan.OW
+        dx, dw, db = L.upload(x), L.upload(w), L.upload(bias)
+        Wp, tab, y = L.alloc(plan.Wp_bytes), L.alloc(plan.table_bytes), L.alloc(4 * nout)
+        L.igemm_pack_filter(plan, dw, Wp, tab)
+        print("static workspace, fewer parts", shp, flush=True)
+        for b in (None, db):
+            L.conv_implicit_gemm_static(plan, dx, Wp, tab, y, b, b is not None)
+            got = L.download(y, (s.N, s.K, plan.OH, plan.OW))
+            truth, tol = O.naive_conv_f64(s, x, w), bound(s, x, w)
+            if b is not None:
+                tol = tol + 2.0 ** -23 * (np.abs(truth) + 1)
+                truth = np.maximum(truth + bias[None, :, None, None], 0.0)
+            assert (np.abs(got - truth) <= tol).all()
