@@ -625,15 +625,17 @@ def run_workload(name, steps, warmup, o, detail=True, offline_filter=None):
             g = L.igemm_configs()[l.iplan.config]
             if g.waves_k > 1:
                 return ("igemm_wavesplit_kernel", N, l.C, l.K, l.H, l.ks, l.st, "%dx%dx%dw%d" % (g.bm, g.bn, g.bk, g.waves_k))
-            return ("igemm_conv_kernel", N, l.C, l.K, l.H, l.ks, l.st, tile_name(g))
+            split = L.igemm_splits_products(l.iplan)
+            return ("igemm_split_kernel" if split else "igemm_conv_kernel", N, l.C, l.K, l.H, l.ks, l.st, tile_name(g))
         keys = [ig_key(l) for l in il]
         tr = None
         if all(k in traffic for k in keys):
             tr = round(sum(traffic[k] * l.repeats for k, l in zip(keys, il)) / sum(l.repeats for l in il))
-        n_ws = sum(l.repeats for l in il if L.igemm_configs()[l.iplan.config].waves_k > 1)
-        n_all = sum(l.repeats for l in il)
-        kname = ("igemm_conv_kernel" if n_ws == 0 else "igemm_wavesplit_kernel" if n_ws == n_all else
-                 "igemm_wavesplit_kernel (%d of %d launches per step), igemm_conv_kernel" % (n_ws, n_all))
+        n_of = {}
+        for k, l in zip(keys, il):
+            n_of[k[0]] = n_of.get(k[0], 0) + l.repeats
+        names = sorted(n_of, key=lambda k: -n_of[k])
+        kname = names[0] if len(names) == 1 else ", ".join("%s (%d of %d launches per step)" % (k, n_of[k], sum(n_of.values())) for k in names)
         roofline = dict(transforms["implicit_gemm"], kernel=kname, traffic=tr,
                         avg_launch_ms=round(igemm_stage[0] / igemm_stage[1], 5))
         if shader_clock:

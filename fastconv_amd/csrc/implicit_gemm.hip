@@ -561,13 +561,17 @@ __global__ __launch_bounds__(TL::THREADS, TL::MIN_WAVES) void igemm_conv_kernel(
 // wavefront that multiplies it and goes from memory to the matrix core without leaving its registers: a lane holds 8
 // consecutive reduction rows of one pixel, which is its share of a 32x32x16 product.  The filter has been split when it was
 // packed and goes to LDS by direct loads, one stage ahead, for all wavefronts of the workgroup.
-// What bounds it is the issue of vector memory: a load takes a CU about 20 cycles whatever its width, and a stage of a 128x128
-// tile takes 32 loads of columns and 12 of the filter, 880 cycles, beside 768 of products (both operands through registers,
-// 4 bytes a lane, took 64 loads).  Window rows in runs are 16 bytes a lane, 8 loads a stage.
-// Measured at batch 32, fp32 instructions -> both operands split in the kernel -> this: 256 -> 256 3x3/2 at 28x28 84 -> 75.5 -> 66.7
-// us, 7x7/2 stem 91 -> 79 -> 57, 64 -> 64 3x3 at 56x56 74 -> 62 -> 48, 256 -> 256 1x1 at 56x56 113 -> 83 -> 74.5, 512 -> 2048 1x1 at
-// 7x7 39 -> 32 -> 27.8; 32 -> 16 3x3 at 97x97, batch 55, (32 rows a tile) 112 -> 66.  Prefetch of the operands across a whole
-// stage with three LDS buffers in place of two: -3 to +8 %, two wavefronts a SIMD in place of four.
+// Four bytes a lane, a load costs the CU's address unit 18 to 21 cycles.  A stage of a 128x128 tile takes 32 loads of columns
+// and 12 of the filter, some 880 cycles, beside 768 of products; both operands through registers took 64 loads.  Counted on
+// 128 -> 128 3x3/2 at 56x56, batch 32: the address units are busy 81 % of the cycles and the matrix pipes 33 % with 64x64
+// tiles, 62 % and 39 % with 128x64, where a wavefront waits a third of its life for data or at a barrier.  Window rows in
+// runs are 16 bytes a lane, 8 loads a stage: on the 7x7/2 stem vector instructions take 59 % of the SIMD's cycles and the
+// matrix pipes 47 %, the address units 60 %.
+// Measured as calls in turn on one box, batch 32, fp32 instructions -> both operands split in the kernel -> this: 256 -> 256 3x3/2
+// at 28x28 94 -> 80 -> 70 us, 7x7/2 stem 106 -> 87 -> 62 (72 amid the layers of ResNet-50), 64 -> 64 3x3 at 56x56 83 -> 66 -> 52,
+// 256 -> 256 1x1 at 56x56 123 -> 93 -> 79, 512 -> 2048 1x1 at 7x7 42 -> 34 -> 29; 32 -> 16 3x3 at 97x97, batch 55, (32 rows a
+// tile) 124 -> 122 -> 73.  Prefetch of the operands across a whole stage with three LDS buffers in place of two: -3 to +8 %, two
+// wavefronts a SIMD in place of four.
 template <int BM, int BN, int WAVES>
 struct IgSplit {
     static constexpr int BM_ = BM, BN_ = BN, THREADS = 64 * WAVES;
@@ -904,11 +908,12 @@ bool ig_inside(const fc_conv_shape &s, int bk) {
     return s.pt == 0 && s.pl == 0 && (OH - 1) * s.sh + s.kh <= s.H && (OW - 1) * s.sw + s.kw <= s.W && (s.C * s.kh * s.kw) % bk == 0;
 }
 
-// Whether the products run on the bf16 matrix cores (a pointwise layer is a tap-major one whose only tap is inside): for
-// inputs below 2 GiB, but not for a pointwise layer of up to 64 output channels: that is bound by reading x, which the fp32
-// kernel does 16 bytes a lane (256 -> 64 channels at 56x56, batch 32: 35.8 us against 37.6; 64 -> 256: 35.0 against 34.4);
-// nor for a reduction of two or three stages, bound by its gathers and stores (3 -> 64 channels 3x3 at 224x224, batch 32:
-// 129 us against 139).
+// Whether the products run on the bf16 matrix cores (a pointwise layer is a block whose only tap is inside): for inputs below
+// 2 GiB, but not for pointwise layers of up to 64 output channels, whose x the fp32 kernel reads 16 bytes a lane, nor for
+// reductions of two or three stages.  Both lines were drawn when this kernel split both operands; at the kernel as it is, us,
+// best tile on fp32 / on split products, batch 32: 1x1 256 -> 64 at 56x56 33.3 / 27.5, 64 -> 64 12.4 / 11.5, 128 -> 32
+// 13.4 / 14.2, 512 -> 64 at 28x28 23.4 / 23.4; 3x3 3 -> 64 at 224x224 (27 rows) 129 / 137, batch 16 5 -> 64 (45 rows)
+// 68.4 / 60.1, 1x1 48 -> 256 at 56x56 29.4 / 25.0.  So both could be drawn lower.
 bool ig_splits(const fc_conv_shape &s, const fc_gemm_config &c) {
     if (c.waves_k > 1 || c.bm % 64 != 0 || 4l * s.N * s.C * s.H * s.W >= (1l << 31) || (long)s.C * s.kh * s.kw <= 48) return false;
     if (ig_pointwise(s, c.bk, true) && s.K <= 64) return false;
@@ -921,7 +926,10 @@ IgTileSize ig_tile_size(const fc_conv_shape &s, const fc_gemm_config &c) {
     return {c.bm, c.bn};
 }
 
-// Order of the reduction rows and their number (before rounding up to a stage).
+// Order of the reduction rows and their number (before rounding up to a stage).  A row in runs is taken at 0.85 (8 columns)
+// and 0.9 (4) of the time of one in blocks.  80 drawn layers without whole blocks (3x3, 5x5, 7x7), every order at its best
+// tile: 0.97 and 0.99 in the median, half-filled runs and blocks spread it from 0.76 to 1.58; the order so chosen is 0.5 %
+// behind the best of the three on average and 9 % at most.
 int ig_order(const fc_conv_shape &s, const fc_gemm_config &c, long *rows) {
     const long taps = (long)s.kh * s.kw;
     *rows = s.C * taps;
@@ -981,8 +989,9 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
 // Expected time of a layer on the bf16 matrix cores, in us, under one of the tile shapes 128x128, 64x128, 128x64 and 64x64
 // (configurations 0 to 3).  A CU takes a stage of a workgroup every `cycles` (block or row order), however many it holds, and
 // one workgroup takes at least `latency` for it; beside that the start of a round, memory, and for a split reduction the pass
-// over the partial sums.  Constants: least squares over 6348 times of 1894 layers (1x1, 3x3, 5x5 and 7x7, one to 64 images,
-// 1 to 1024 channels, 0.1 to 120 GFLOP), standard deviation 13 %; the choice among the four is 1.5 % behind the best of them.
+// over the partial sums.  The constants are a least squares fit.  On 217 drawn layers that it was not made on (1x1, 3x3, 5x5 and 7x7,
+// one to 64 images, 1 to 1024 channels, 0.1 to 60 GFLOP; profiles/igemm_untuned_choice.txt): standard deviation 12 %, the choice
+// among the four 1.7 % behind the best of them on average, 5.6 % or more on a tenth of the layers, 26 % at most.
 struct IgSplitCost {
     int bm, bn, perCu;
     double cyclesBlock, cyclesRow, latency, start;
@@ -1006,7 +1015,7 @@ double ig_split_us(const fc_conv_shape &s, int config, const fc_igemm_plan &plan
     return plan.split_k > 1 ? us + 3.4 + 2.0 * plan.ws_bytes / 6.65e6 : us;
 }
 
-// The same for a kernel that splits the reduction over the wavefronts of a workgroup (6001 times, 16 %).
+// The same for a kernel that splits the reduction over the wavefronts of a workgroup (same layers: 19 %).
 double ig_ws_us(const fc_conv_shape &s, const fc_gemm_config &c, long npix) {
     const double mt = c.bm / 16, nt = c.bn / 16, units = ceil((double)s.C * s.kh * s.kw / 16);
     const double perCu = ceil(ceil((double)s.K / c.bm) * ceil((double)npix / c.bn) / 256);
@@ -1022,7 +1031,8 @@ constexpr int kMaxReduceChannels = 65535;
 // Plans that cannot run because of their partial sums (kMaxReduceChannels) are behind all others.
 // A layer whose reduction the best tile would split over workgroups goes to the kernels that split it inside the workgroup
 // where those are expected ahead, from 9 parts on also where they are 15 % behind and from 21 on 50 %: the model then favours
-// the tiles (most of the layers that lost more than 15 % by it: 9 to 32 parts, reductions of 1000 to 9000 rows, 15 to 25 us).
+// the tiles.  Of the same 217 layers 77 go of 132 that would be split, at 0.72 of the tile's time on average (2 to 8 parts), 0.68
+// (9 to 20) and 0.79 (21 to 32); the seven that go by these lines alone take 0.72 to 1.20, 0.96 on average.
 int ig_split_default_config(const fc_conv_shape *s) {
     int best = 3;
     double bestUs = 1e300;
@@ -1062,7 +1072,9 @@ extern "C" int fc_igemm_get_config(int id, fc_gemm_config *cfg) {
 // evenly the grid fills the chip.
 extern "C" int fc_igemm_default_config(const fc_conv_shape *s) {
     if (!fc_shape_ok(s)) return FC_ERR_INVALID;
-    // (a 1x1 layer of at most 32 output channels is bound by reading x: 32 rows a tile and more workgroups are ahead there)
+    // (1x1 layers of at most 32 output channels have the choice below, with 32 rows a tile or the reduction split inside the
+    // workgroup.  Batch 32, us, that choice / best of the split tiles: stride 2 256 -> 32 at 56x56 15.4 / 18.7, 1024 -> 24
+    // at 27x27 20.9 / 24.6, 128 -> 32 at 56x56 13.4 / 14.2; 256 -> 32 at 55x55 23.0 / 20.2.)
     if (ig_splits(*s, kIgConfigs[3]) && !(s->kh * s->kw == 1 && s->K <= 32 && s->C % 16 == 0)) return ig_split_default_config(s);
     static const double kRate[] = {0.93, 0.81, 0.82, 1.00, 0.75, 0.60, 0.62, 0.84};
     static_assert(sizeof(kRate) / sizeof(kRate[0]) == sizeof(kIgConfigs) / sizeof(kIgConfigs[0]), "one rate per configuration");

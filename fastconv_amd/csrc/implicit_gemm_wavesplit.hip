@@ -384,7 +384,7 @@ bool fc_igemm_ws_supports(const fc_conv_shape *s) {
 // 8 wavefronts over the reduction, 4 when it is shorter than 16 units (16 wavefronts are ahead by 3-5 % on a
 // few long reductions at batch 8 to 16 and behind by 10 % on 256 -> 256 channels at 56x56: not chosen).  Beyond about 8 GFLOP (2 GFLOP for strided layers, whose
 // gathered rows use half of every cache line) the LDS-tiled kernels are level or ahead despite their second launch;
-// from 3.2 GFLOP on where their tiles waste nothing (fc_igemm_default_config).
+// where products are split the expected times decide below that (ig_split_default_config).
 int fc_igemm_ws_choose(const fc_conv_shape *s, long Npix) {
     if (!fc_igemm_ws_supports(s)) return -1;
     const double flops = 2.0 * Npix * s->K * (double)s->C * s->kh * s->kw;

@@ -418,24 +418,26 @@ extern "C" int fc_wino_prefer_onepass(const fc_conv_shape *s) {
     // What the pipelines with V and M in memory pay is bytes, what this one pays is products and, for every 64 output
     // channels, an input transform: the line is a number of bytes per input channel.  It lies higher for C*K > 8192, with
     // more output channels and from 49 input channels on the bf16 matrix cores.  Us here / staged, at (V+M in MB):
-    //   64 -> 256 56x56 n32 (262) 171 / 138, 64 -> 512 28x28 n64 (236) 184 / 126, 64 -> 1024 110x110 n6 (603) 406 / 343,
-    //   64 -> 256 112x112 n32 (946) 518 / 538, 48 -> 320 111x111 n5 (170) 139 / 96, 48 -> 512 218x218 n4 (785) 404 / 486,
-    //   32 -> 675 90x90 n5 (204) 116 / 104, 40 -> 812 215x215 n1 (283) 199 / 163, 24 -> 512 202x202 n2 (317) 123 / 148;
-    //   C*K <= 8192: 64 -> 64 53x53 n54 (143) 109 / 65, 63x63 n50 (198) 109 / 97, 119x119 n20 (262) 115 / 129,
-    //   32 -> 64 141x141 n6 (85) 48 / 45, 32 -> 128 66x66 n37 (183) 85 / 87.
+    //   64 -> 256 56x56 n32 (262) 169 / 139, 64 -> 512 28x28 n64 (236) 185 / 130, 64 -> 1024 110x110 n6 (603) 401 / 350,
+    //   64 -> 256 112x112 n32 (946) 519 / 549, 48 -> 320 111x111 n5 (170) 105 / 96, 48 -> 512 218x218 n4 (785) 392 / 485,
+    //   32 -> 675 90x90 n5 (212) 109 / 102, 40 -> 812 215x215 n1 (292) 157 / 162, 24 -> 512 202x202 n2 (322) 126 / 147;
+    //   C*K <= 8192: 64 -> 64 53x53 n54 (143) 89 / 68, 63x63 n50 (198) 89 / 95, 119x119 n20 (262) 95 / 128,
+    //   32 -> 64 141x141 n6 (85) 36 / 45, 32 -> 128 66x66 n37 (183) 83 / 88.
+    // (The lines are older than the wide stores of odd rows, which took 13 to 25 % off this kernel and nothing off the staged
+    // one: 63x63, 141x141 and 215x215 above are now on the staged side though they are faster here.)
     const double bytes = 256.0 * ((s->C + 15) / 16 * 16 + (s->K + 31) / 32 * 32) * (double)T;
     if (bytes <= ((long)s->C * s->K > 8192 ? 10e6 : 3.5e6) * s->C) return 0;
     // Few input and many output channels: the input transform of every 64 output channels outweighs writing V once, and
-    // the fused kernel needs no M.  Here / fused: 32 -> 256 62x62 n23 92 / 81, 159x159 n20 566 / 538, 32 -> 192 155x155
-    // n15 301 / 281, 24 -> 256 48x48 n48 78 / 70, 16 -> 512 112x112 n32 547 / 531; 32 -> 128 112x112 n32 169 / 183.
+    // the fused kernel needs no M.  Here / fused: 32 -> 256 62x62 n23 89 / 75, 159x159 n20 452 / 452, 32 -> 192 155x155
+    // n15 235 / 229, 24 -> 256 48x48 n48 74 / 63, 16 -> 512 112x112 n32 536 / 501; 32 -> 128 112x112 n32 171 / 178.
     return s->C <= 32 && s->K >= 192 && bytes <= 2e9 && fc_wino_prefer_fused(s) ? 0 : 1;
 }
 
 // Against the fused pipeline (V in memory) the line lies elsewhere.  One block of output channels: the fused kernel brings
 // half as many workgroups up to 32 of them and is level up to 64.  More: the input transform of every 64 output channels
-// outweighs writing V once, but for the layers above.  Us here / fused: 40 -> 24 112x112 n9 34.8 / 41.8, 48 -> 32 87x87 n17
-// 45.8 / 48.2, 32 -> 32 120x120 n10 33.1 / 35.0, 48 -> 64 87x87 n17 55.7 / 54.1, 64 -> 64 56x56 n32 51.2 / 52.2, 53x53 n54 108.2 /
-// 99.9, 63x63 n50 108.0 / 107.9; 48 -> 96 100x100 n10 75.6 / 69.3, 64 -> 256 56x56 n32 170 / 153, 64 -> 1024 110x110 n6 406 / 361.
+// outweighs writing V once, but for the layers above.  Us here / fused: 40 -> 24 112x112 n9 33.0 / 41.1, 48 -> 32 87x87 n17
+// 38.5 / 42.9, 32 -> 32 120x120 n10 31.7 / 33.5, 48 -> 64 87x87 n17 43.2 / 45.4, 64 -> 64 56x56 n32 48.9 / 51.0, 53x53 n54 88.5 /
+// 91.8, 63x63 n50 89.3 / 97.8; 48 -> 96 100x100 n10 70.9 / 66.0, 64 -> 256 56x56 n32 169 / 159, 64 -> 1024 110x110 n6 401 / 353.
 extern "C" int fc_wino_prefer_onepass_to_fused(const fc_conv_shape *s) {
     return onepass_fills(s) && (s->K <= kKB || fc_wino_prefer_onepass(s)) ? 1 : 0;
 }

@@ -477,12 +477,14 @@ extern "C" int fc_wino_make_plan(const fc_conv_shape *s, int gemm_config, fc_win
 }
 
 // Measured on MI355X (both algorithms at their best tile shape, whole-layer forward time, every 3x3
-// stride-1 layer of VGG-16 and ResNet-50 at batch 1, 4 and 32, the ResNet-50 ones also at 8 and 16): with
-// 16 or more input channels Winograd wins from 3.7 GFLOP of direct-convolution work on (by 1.1x to 3.2x;
-// two 512-channel layers are level there); at 1.85 GFLOP the two are level (seven layers, 0.97-1.36);
-// up to 0.92 GFLOP one implicit-GEMM launch, its reduction split inside the workgroups, is 1.3-2.2x ahead
-// of the three launches of the staged pipeline.  The 3-channel first layer: implicit GEMM 1.5-1.7x ahead
-// at batch 1 and 4, the two within 10 % at batch 32 (both bound by the stores of the output).
+// stride-1 layer of VGG-16 and ResNet-50 at batch 1, 4 and 32, the ResNet-50 ones also at 8 and 16;
+// profiles/auto_crossover_vgg16_resnet50.txt): with 16 or more input channels Winograd is level to 2.6x ahead from
+// 7.4 GFLOP of direct-convolution work on (512 -> 512 at 7x7, 3 % behind, excepted), at 3.7 GFLOP 1.34x ahead to 11 %
+// behind, at 1.85 GFLOP 5 % ahead to 26 % behind; up to 0.92 GFLOP one implicit-GEMM launch, its reduction split
+// inside the workgroups, is 1.3-2.2x ahead of the three launches of the staged pipeline.  The 3-channel first
+// layer: implicit GEMM 1.4-1.5x ahead at batch 1 and 4, 10 % behind at batch 32.  The line is older than the implicit
+// GEMM on split products as it is: of the 47 layers eight are on the slower side of it, by 2 to 11 % (512 -> 512 at
+// 7x7 and 64 -> 64 at 56x56, batch 16, 64 -> 64 at 224x224, batch 1, and the first layer at batch 32 by 10 and 11).
 extern "C" int fc_prefer_winograd(const fc_conv_shape *s) {
     if (!fc_shape_ok(s) || s->kh != 3 || s->kw != 3 || s->sh != 1 || s->sw != 1) return 0;
     const int OH = fc_out_dim(s->H, s->pt, s->pb, 3, 1), OW = fc_out_dim(s->W, s->pl, s->pr, 3, 1);
