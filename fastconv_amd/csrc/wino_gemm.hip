@@ -244,7 +244,7 @@ __device__ __forceinline__ void gemm_tile(const float *__restrict__ U, const flo
 }
 
 // The same tile on the bf16 matrix cores (see split_mfma.h): a wavefront takes 8 consecutive channels of 64 rows or
-// columns at a time, each lane one of them, splits the 8 floats it has fetched a stage ahead and writes one 16-byte
+// columns at a time, each lane one of them, splits the 8 floats it has fetched PF stages ahead and writes one 16-byte
 // word per part.  The split runs beside the products of the other wavefronts.  128x128 tiles take eight wavefronts of 64x32
 // (four wavefronts of 64x64: 179 us where eight take 166, as two a SIMD do not cover each other's barriers).
 // Batch 32, fp32 instructions -> this: 256 -> 256 channels at 56x56 225 -> 169 us (156 TFLOP/s; the matrix pipes are busy
@@ -256,6 +256,12 @@ struct SplitTile {
     static constexpr int ITEMS = 2 * (TL::BM_ + TL::BN_) / TL::THREADS;
     typedef fc_split_stage<TL::BM_, TL::BN_> Stage;
     static constexpr int LDS_WORDS = 2 * Stage::WORDS;
+    // Register sets of global prefetch: set u holds the stages s with s % PF == u, and a stage is fetched PF stages before it
+    // is split.  Where a stage is eight registers a second set leaves the wavefronts a SIMD holds as they are (128x128: 122
+    // registers of 128).  One / two / three / four sets, whole staged layer, us: 256 -> 256 channels at 56x56 batch 32 275 / 263 /
+    // 295 / 284, 128 -> 128 at 112x112 400 / 383 / 410 / 404, 512 -> 512 at 28x28 232 / 227 / 242 / 237, at 14x14 batch 4 42.5 /
+    // 40.3 / 40.5 / 40.2; one image 256 -> 256 at 56x56 30.1 / 28.7 / 29.2 / 29.8.  The wider tiles hold 24 registers a stage and keep one.
+    static constexpr int PF = ITEMS == 1 ? 2 : 1;
     static_assert(TL::BM_ % 64 == 0 && TL::BN_ % 64 == 0, "a wavefront fetches 64 rows or columns of one operand");
     static_assert(2 * (TL::BM_ + TL::BN_) % TL::THREADS == 0, "every wavefront fetches the same number of blocks");
     static_assert(TL::BK_ == 16, "one product of depth 16 per stage");
@@ -288,10 +294,11 @@ __device__ __forceinline__ void split_tile(const float *__restrict__ U, const fl
                                      : V + (size_t)f * C_pad * T_pad + (size_t)tb * BN) + (size_t)(8 * g) * ld[j] + c0);
         dst[j] = (isA[j] ? 0 : 3 * A_PLANE) + e;
     }
-    float r[ITEMS][8];
+    constexpr int PF = S::PF;
+    float r[PF][ITEMS][8];
     uint32_t laneOff = 4u * lane;
     // `more`: there is a stage to fetch (else the one before is fetched again, so that the loop has no branch)
-    auto fetch = [&](bool more) __attribute__((always_inline)) {
+    auto fetch = [&](float (&set)[ITEMS][8], bool more) __attribute__((always_inline)) {
         asm volatile("" : "+v"(laneOff));
 #pragma unroll
         for (int j = 0; j < ITEMS; j++) {
@@ -299,35 +306,40 @@ __device__ __forceinline__ void split_tile(const float *__restrict__ U, const fl
             const float *b = src[j];
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                r[j][i] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(b) + laneOff);
+                set[j][i] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(b) + laneOff);
                 b = uniform_ptr(b + ld[j]);
             }
         }
     };
-    auto park = [&](int buf) __attribute__((always_inline)) {
+    auto park = [&](const float (&set)[ITEMS][8], int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < ITEMS; j++) fc_split8(r[j], smem + buf * WORDS + dst[j] + lane, isA[j] ? A_PLANE : B_PLANE);
+        for (int j = 0; j < ITEMS; j++) fc_split8(set[j], smem + buf * WORDS + dst[j] + lane, isA[j] ? A_PLANE : B_PLANE);
     };
 
     floatx16 acc[MI][NI], small[MI][NI];
     fc_zero<MI, NI>(acc);
     fc_zero<MI, NI>(small);
 
-    fetch(false);
-    park(0);
-    fetch(nStages > 1);
+#pragma unroll
+    for (int u = 0; u < PF; u++) fetch(r[u], u > 0 && u < nStages);
+    park(r[0], 0);
+    fetch(r[0], PF < nStages);
     __syncthreads();
     const int aFrag = lrow * BM + wm0 + lcol, bFrag = 3 * A_PLANE + lrow * BN + wn0 + lcol;
-    int s = 0;
-    for (; s + 1 < nStages; s++) {
+    auto stage = [&](const int s, auto uc) __attribute__((always_inline)) {
+        constexpr int un = (decltype(uc)::value + 1) % PF;
         const fc_uintx4 *cur = smem + (s & 1) * WORDS;
         fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc, small);
-        park((s + 1) & 1);
-        fetch(s + 2 < nStages);
+        park(r[un], (s + 1) & 1);
+        fetch(r[un], s + 1 + PF < nStages);
         __syncthreads();
-    }
+    };
+    // all but the last stage
+    int s = 0;
+    for (; s + PF < nStages; s += PF) stage_group(stage, s, std::make_integer_sequence<int, PF>());
+    stage_rest(stage, s, nStages - 1, std::make_integer_sequence<int, PF - 1>());
     {
-        const fc_uintx4 *cur = smem + (s & 1) * WORDS;
+        const fc_uintx4 *cur = smem + ((nStages - 1) & 1) * WORDS;
         fc_split_products<MI, NI, A_PLANE, B_PLANE>(cur + aFrag, cur + bFrag, acc, small);
         __syncthreads();
     }
