@@ -593,7 +593,9 @@ template <class TL> struct IgSplitOf { typedef void type; };
 //   SP_PAD         the same with channels past the last one
 //   SP_ROW8        two runs of 8 columns of a window row of one channel: 16-byte loads
 //   SP_ROW4        four runs of 4 columns
-enum { SP_INSIDE, SP_MASKED, SP_PAD, SP_ROW8, SP_ROW4 };
+//   SP_POINT       pointwise layers under tiles of 64 rows: 16 channels, read four pixels a lane and turned through LDS
+//   SP_POINT32     the same with the packed filter in fp32, split on its way to LDS
+enum { SP_INSIDE, SP_MASKED, SP_PAD, SP_ROW8, SP_ROW4, SP_POINT, SP_POINT32 };
 
 template <int MI_, class S>
 struct IgSplitPart {
@@ -603,7 +605,7 @@ struct IgSplitPart {
 // One workgroup tile, of which the first MI blocks of 32 rows of each wavefront hold output channels.
 template <class S, int MODE, int MI>
 __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb, const int pb, fc_uintx4 *smem) {
-    constexpr bool ROW = MODE == SP_ROW8 || MODE == SP_ROW4;
+    constexpr bool ROW = MODE == SP_ROW8 || MODE == SP_ROW4, POINT = MODE == SP_POINT || MODE == SP_POINT32;
     constexpr int NI = S::NI, WAVES = S::THREADS / 64;
     constexpr uint32_t OUTSIDE = 0x80000000u;      // past the end of x whatever scalar offset is added: reads 0
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -619,7 +621,13 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
         const long pix = (long)pb * S::BN_ + wn0 + ni * 32 + lcol;
         pixByte[ni] = OUTSIDE;
         rowBad[ni] = colBad[ni] = ~0u;
-        if (pix < p.Npix) {
+        if (POINT) {      // pixels 4 * (lane % 8) .. + 3, channels lane / 8 and 8 on
+            const long first = (long)pb * S::BN_ + wn0 + ni * 32 + 4 * (lane & 7);
+            if (first < p.Npix) {
+                const uint32_t n = fc_div((uint32_t)first, p.divOHW), image = (uint32_t)(p.H * p.W);
+                pixByte[ni] = 4u * ((n * (uint32_t)p.C + (uint32_t)(lane >> 3)) * image + ((uint32_t)first - n * image));
+            }
+        } else if (pix < p.Npix) {
             const uint32_t n = fc_div((uint32_t)pix, p.divOHW);
             const uint32_t pp = (uint32_t)pix - n * (uint32_t)(p.OH * p.OW);
             const uint32_t oh = fc_div(pp, p.divOW), ow = pp - oh * p.OW;
@@ -691,6 +699,19 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
             table(min(s + 1, nStagesAll - 1));
             return;
         }
+        if (POINT) {
+            const int left = p.C - 16 * s - (lane >> 3);      // channels from the lane's first on that exist
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const floatx4 d = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                      xres, 8 * h < left ? pixByte[ni] : OUTSIDE, (uint32_t)min(16 * s + 8 * h, p.C - 1) * chanStep, 0));
+#pragma unroll
+                    for (int j = 0; j < 4; j++) raw[ni][4 * h + j] = d[j];
+                }
+            return;
+        }
         const int left = p.C - tapC - 8 * lrow;      // channels of the lane's 8 that exist
 #pragma unroll
         for (int i = 0; i < 8; i++) {
@@ -713,6 +734,18 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
     // readAgain: runs that start before x are read again, element by element (whether a 16-byte load there gives the elements
     // inside x is left open)
     auto split = [&](auto readAgain) __attribute__((always_inline)) {
+        if constexpr (POINT) {
+            // four pixels of one channel -> eight channels of one pixel, through this wavefront's own [16 channels][32 pixels]
+            float *const turn = reinterpret_cast<float *>(smem + S::LDS_WORDS) + wave * 512;
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) {
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    *reinterpret_cast<floatx4 *>(turn + 256 * h + 4 * lane) = floatx4{raw[ni][4 * h], raw[ni][4 * h + 1], raw[ni][4 * h + 2], raw[ni][4 * h + 3]};
+#pragma unroll
+                for (int i = 0; i < 8; i++) raw[ni][i] = turn[(8 * lrow + i) * 32 + lcol];
+            }
+        }
         if (ROW) {
             if constexpr (decltype(readAgain)::value) {
 #pragma unroll
@@ -751,6 +784,26 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
         fbase = uniform_ptr(fbase + fstep);
     };
 
+    // SP_POINT32: four rows of one channel to registers, and as halves of operand words to LDS a stage later
+    float rows[4];
+    auto filterRows = [&](const int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) rows[i] = p.Wp[(size_t)(16 * s + 4 * wave + i) * p.K_pad + lane];
+    };
+    auto filterSplit = [&](const int buf) __attribute__((always_inline)) {
+        typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
+        uintx2 part[3];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            uint32_t h, m, l;
+            fc_split2(rows[2 * i], rows[2 * i + 1], h, m, l);
+            part[0][i] = h; part[1][i] = m; part[2][i] = l;
+        }
+        uintx2 *const to = reinterpret_cast<uintx2 *>(smem + buf * S::STAGE_WORDS + lrow * kSplitBlockWords + (wave >> 1) * 32 + lcol) + (wave & 1);
+#pragma unroll
+        for (int i = 0; i < 3; i++) to[2 * i * 64] = part[i];
+    };
+
     floatx16 acc[MI][NI], small[MI][NI];
     fc_zero<MI, NI>(acc);
     fc_zero<MI, NI>(small);
@@ -758,7 +811,8 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
     auto stage = [&](const int s, const bool more, auto readAgain) __attribute__((always_inline)) {
         const int buf = (s - sBegin) & 1;
         split(readAgain);
-        __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): this wavefront's filter words of the stage are in LDS
+        if constexpr (MODE == SP_POINT32) filterSplit(buf);
+        if constexpr (MODE != SP_POINT32) __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): this wavefront's filter words of the stage are in LDS
         __syncthreads();                         // and those of the others, which have read the stage before
         const fc_uintx4 *as = smem + buf * S::STAGE_WORDS + lane;
         fc_bf16x8 a[3][MI];
@@ -767,7 +821,8 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
 #pragma unroll
             for (int mi = 0; mi < MI; mi++) a[q][mi] = __builtin_bit_cast(fc_bf16x8, as[mi * kSplitBlockWords + q * 64]);
         if (more) {      // (behind the reads: the compiler has reads of LDS wait for direct loads before them)
-            filter(buf ^ 1);
+            if constexpr (MODE == SP_POINT32) filterRows(s + 1);
+            else filter(buf ^ 1);
             fetch(s + 1);
         }
         constexpr int pa[5] = {2, 1, 0, 1, 0}, pb[5] = {0, 1, 2, 0, 1};
@@ -784,7 +839,8 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
             for (int ni = 0; ni < NI; ni++)
                 acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][mi], __builtin_bit_cast(fc_bf16x8, b[ni][0]), acc[mi][ni], 0, 0, 0);
     };
-    filter(0);
+    if constexpr (MODE == SP_POINT32) filterRows(sBegin);
+    else filter(0);
     fetch(sBegin);
     int s = sBegin;
     if constexpr (ROW) {
@@ -816,7 +872,7 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
 
 template <class S, int MODE>
 __global__ __launch_bounds__(S::THREADS, (MODE == SP_ROW4 || MODE == SP_INSIDE) && S::MIN_WAVES > 3 ? 3 : S::MIN_WAVES) void igemm_split_kernel(const IgemmParams p) {
-    __shared__ fc_uintx4 smem[S::LDS_WORDS];
+    __shared__ fc_uintx4 smem[S::LDS_WORDS + (MODE == SP_POINT || MODE == SP_POINT32 ? S::THREADS / 64 * 128 : 0)];
     int kb, pb;
     if (!ig_decode_tile(p, &kb, &pb)) return;
     // 32 rows of a 64-row tile past the last output channel are not multiplied
@@ -838,6 +894,8 @@ __global__ __launch_bounds__(256) void igemm_split_filter_kernel(const float *__
     for (int i = 0; i < 8; i++) v[i] = src[(size_t)i * K_pad];
     fc_split8(v, Ws + (size_t)block * kSplitBlockWords + lane, 64);
 }
+
+#include "implicit_gemm_short.h"
 
 // Sums the partial results of a split reduction in split order (so the result does
 // not depend on which workgroup finished first), adds bias, applies ReLU, writes NCHW.
@@ -897,10 +955,16 @@ const IgTileSize kIgSplitTiles[] = {ig_split_tile_size<Ig0>(), ig_split_tile_siz
 static_assert(sizeof(kIgSplitTiles) / sizeof(kIgSplitTiles[0]) == kNumIgConfigs, "one per configuration");
 
 // The column matrix of a pointwise layer is its input, read 16 bytes a lane where that is possible.
-bool ig_pointwise(const fc_conv_shape &s, int bk, bool x16) {
-    return s.kh == 1 && s.kw == 1 && s.sh == 1 && s.sw == 1 && s.pt == 0 && s.pb == 0 && s.pl == 0 && s.pr == 0 &&
-           (s.H * s.W) % 4 == 0 && s.C % bk == 0 && x16 && 4l * s.N * s.C * s.H * s.W < (1l << 32);
+bool ig_point(const fc_conv_shape &s) {
+    return s.kh == 1 && s.kw == 1 && s.sh == 1 && s.sw == 1 && s.pt == 0 && s.pb == 0 && s.pl == 0 && s.pr == 0;
 }
+bool ig_pointwise(const fc_conv_shape &s, int bk, bool x16) {
+    return ig_point(s) && (s.H * s.W) % 4 == 0 && s.C % bk == 0 && x16 && 4l * s.N * s.C * s.H * s.W < (1l << 32);
+}
+
+// Split products: four consecutive pixels of a pointwise layer lie in one image, so that they are one 16-byte load of a channel
+// (any alignment; beyond the last pixel of a single image it reads on into the next channel, or 0, for pixels that are not stored).
+bool ig_four_pixels(const fc_conv_shape &s) { return ig_point(s) && ((s.H * s.W) % 4 == 0 || s.N == 1); }
 
 // No tap of any window leaves the image, and the reduction has no padding rows.
 bool ig_inside(const fc_conv_shape &s, int bk) {
@@ -926,14 +990,13 @@ IgTileSize ig_tile_size(const fc_conv_shape &s, const fc_gemm_config &c) {
     return {c.bm, c.bn};
 }
 
-// Order of the reduction rows and their number (before rounding up to a stage).  A row in runs is taken at 0.85 (8 columns)
-// and 0.9 (4) of the time of one in blocks.  80 drawn layers without whole blocks (3x3, 5x5, 7x7), every order at its best
-// tile: 0.97 and 0.99 in the median, half-filled runs and blocks spread it from 0.76 to 1.58; the order so chosen is 0.5 %
-// behind the best of the three on average and 9 % at most.
-int ig_order(const fc_conv_shape &s, const fc_gemm_config &c, long *rows) {
+// Order of the reduction rows where products are split, and their number (before rounding up to a stage).  A row in runs is
+// taken at 0.85 (8 columns) and 0.9 (4) of the time of one in blocks.  80 drawn layers without whole blocks (3x3, 5x5, 7x7),
+// every order at its best tile: 0.97 and 0.99 in the median, half-filled runs and blocks spread it from 0.76 to 1.58; the order
+// so chosen is 0.5 % behind the best of the three on average and 9 % at most.
+int ig_split_order(const fc_conv_shape &s, long *rows) {
     const long taps = (long)s.kh * s.kw;
     *rows = s.C * taps;
-    if (!ig_splits(s, c)) return s.C % c.bk == 0 ? IG_ORDER_TAP : IG_ORDER_CHANNEL;
     if (s.C % 16 == 0) return IG_ORDER_BLOCK;
     const long block = fc_round_up(s.C, 16) * taps;
     const long row8 = 8l * s.C * s.kh * ((s.kw + 7) / 8), row4 = 4l * s.C * s.kh * ((s.kw + 3) / 4);
@@ -942,6 +1005,39 @@ int ig_order(const fc_conv_shape &s, const fc_gemm_config &c, long *rows) {
     if (costRow8 <= costRow4) { *rows = row8; return IG_ORDER_ROW8; }
     *rows = row4;
     return IG_ORDER_ROW4;
+}
+
+// Order of the reduction rows of a configuration and their number.
+int ig_order(const fc_conv_shape &s, const fc_gemm_config &c, long *rows) {
+    if (ig_splits(s, c)) return ig_split_order(s, rows);
+    *rows = (long)s.C * s.kh * s.kw;
+    return s.C % c.bk == 0 ? IG_ORDER_TAP : IG_ORDER_CHANNEL;
+}
+
+// Whether a layer runs in igemm_short_kernel: up to four stages of rows and at least 25 blocks of 32 channels and 32 pixels a CU
+// (below, a tile is as soon done as the filter is split, us: 1x1 26 -> 233 at 99x99, one image, 7.0 / 7.7, 31 -> 128 at 112x112 batch
+// 4 10.7 / 11.0, 3x3 3 -> 22 at 93x84 batch 23 11.9 / 13.0).  Window rows in runs, but for 49 to 64 output channels on few pixels,
+// which fill a tile and leave a walking wavefront one or two blocks (best tile / walking: 5 -> 64 3x3/2 at 112x112 batch 16 9.5 / 9.9,
+// 1 -> 58 7x7/2 at 93x147 batch 31 11.5 / 13.4).  Pointwise layers of more than 64 channels and at most three stages that the fp32
+// kernel does not read 16 bytes a lane, and those where two or three stages write 64 MB and more (32 -> 272 at 52x53 batch 36 55 / 36,
+// 48 -> 240 at 154x34 batch 18 47 / 32; below: 48 -> 256 at 56x56 batch 16 16.1 / 16.5, 32 -> 128 at 90x90 batch 8 10.3 / 11.1;
+// one stage: 16 -> 512 at 38x38 batch 62 49 / 57; four: 64 -> 304 at 111x111 batch 39 268 / 299).  With up to two stages and more
+// than 512 channels the pixels are read by many groups of workgroups: 2 -> 1005 at 165x91 batch 8 150 / 183.
+bool ig_short(const fc_conv_shape &s) {
+    long rows;
+    const int order = ig_split_order(s, &rows);
+    const long npix = (long)s.N * fc_out_dim(s.H, s.pt, s.pb, s.kh, s.sh) * fc_out_dim(s.W, s.pl, s.pr, s.kw, s.sw);
+    const double yBytes = 4.0 * s.K * (double)npix;
+    if (rows > 64 || s.kh * s.kw > 64 || 4l * s.N * s.C * s.H * s.W >= (1l << 31) || yBytes > kShortNoStore) return false;
+    if ((rows <= 32 && s.K > 512) || (npix + 31) / 32 * ((s.K + 31) / 32) < 25 * 256) return false;
+    if (order != IG_ORDER_BLOCK) return s.K <= 48 || s.K > 64 || npix >= 32 * 8192;
+    return ig_point(s) && s.K > 64 && rows <= 48 && (!ig_pointwise(s, 16, true) || (rows > 16 && yBytes >= 64e6));
+}
+
+// Pointwise layers of 33 to 64 output channels on many pixels: split from the fp32 filter.  Us, fp32 / this: 256 -> 64 at 56x56 batch 32
+// 38.7 / 36.3, 64 -> 64 12.5 / 12.2, 96 -> 64 at 102x102 batch 28 49.1 / 48.3; fewer pixels: 256 -> 64 at 200x200, one image, 16.5 / 17.8.
+bool ig_point_few(const fc_conv_shape &s) {
+    return ig_four_pixels(s) && s.K > 32 && s.K <= 64 && s.C > 48 && (long)s.N * s.H * s.W >= 768 * 128 && 4l * s.N * s.C * s.H * s.W < (1l << 31);
 }
 
 // Row orders, runs of `run` columns: which of them may start before x.  The row of such a run is inside the image, so that it
@@ -958,6 +1054,21 @@ void ig_before(const fc_conv_shape &s, int run, IgemmParams &p) {
 
 template <class TL>
 void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, IgemmParams &p) {
+    if (p.splitK == 1 && ig_point_few(s) && p.K_pad == 64) {
+        typedef IgSplit<64, 128, 4> S;
+        p.nKB = 1;
+        p.nPB = (int)((p.Npix + S::BN_ - 1) / S::BN_);
+        igemm_split_kernel<S, SP_POINT32><<<dim3((unsigned)((p.nPB + 7l) / 8 * 8)), dim3(S::THREADS), 0, ctx->stream>>>(p);
+        return;
+    }
+    if (p.splitK == 1 && ig_short(s)) {
+        long rows;
+        const int order = ig_split_order(s, &rows);
+        ig_before(s, order == IG_ORDER_ROW8 ? 8 : 4, p);
+        ig_short_launch(ctx, order == IG_ORDER_ROW8 ? SP_ROW8 : order == IG_ORDER_ROW4 ? SP_ROW4 : ig_four_pixels(s) ? SP_POINT : SP_PAD,
+                        rows, ig_splits(s, cfg), p);
+        return;
+    }
     if constexpr (!std::is_void<typename IgSplitOf<TL>::type>::value) {
         if (ig_splits(s, cfg)) {
             typedef typename IgSplitOf<TL>::type S;
@@ -967,6 +1078,10 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
             ig_before(s, order == IG_ORDER_ROW8 ? 8 : 4, p);
             if (order == IG_ORDER_ROW8) igemm_split_kernel<S, SP_ROW8><<<grid, block, 0, ctx->stream>>>(p);
             else if (order == IG_ORDER_ROW4) igemm_split_kernel<S, SP_ROW4><<<grid, block, 0, ctx->stream>>>(p);
+            // two 16-byte loads a stage and wavefront in place of eight of 4 bytes, whole layers of batch 32, us: 256 -> 64 at
+            // 56x56 28.2 / 26.0, 1024 -> 256 at 14x14 34.7 / 32.9, 112 -> 208 at 68x68 batch 4 13.4 / 12.3.  Tiles of 128 rows
+            // load half as often for their products: 64 -> 256 at 56x56 30.6 / 32.3, 144 -> 112 at 130x130 batch 35 173 / 178
+            else if (S::BM_ == 64 && ig_four_pixels(s)) igemm_split_kernel<S, SP_POINT><<<grid, block, 0, ctx->stream>>>(p);
             else if (s.C % 16 != 0) igemm_split_kernel<S, SP_PAD><<<grid, block, 0, ctx->stream>>>(p);
             else if (ig_inside(s, 16)) igemm_split_kernel<S, SP_INSIDE><<<grid, block, 0, ctx->stream>>>(p);
             else igemm_split_kernel<S, SP_MASKED><<<grid, block, 0, ctx->stream>>>(p);

@@ -375,7 +375,9 @@ typedef struct {
 } fc_igemm_plan;
 
 int fc_igemm_make_plan(const fc_conv_shape *shape, int config, fc_igemm_plan *plan);
-/* As fc_wino_gemm_splits_products.  Without room for the filter of split products, the configurations for which
+/* As fc_wino_gemm_splits_products: 1 where fc_igemm_pack_filter splits the filter.  (Some layers of short
+ * reductions, and pointwise ones of 33 to 64 output channels, keep their filter in fp32 and split it in the kernel;
+ * their results are no less exact.)  Without room for the filter of split products, the configurations for which
  * this is 0 (32x64, and those with waves_k above 1) keep it in fp32 alone. */
 int fc_igemm_splits_products(const fc_igemm_plan *plan);
 
