@@ -595,7 +595,9 @@ template <class TL> struct IgSplitOf { typedef void type; };
 //   SP_ROW4        four runs of 4 columns
 //   SP_POINT       pointwise layers under tiles of 64 rows: 16 channels, read four pixels a lane and turned through LDS
 //   SP_POINT32     the same with the packed filter in fp32, split on its way to LDS
-enum { SP_INSIDE, SP_MASKED, SP_PAD, SP_ROW8, SP_ROW4, SP_POINT, SP_POINT32 };
+//   SP_TRI         as SP_PAD, for windows of 3 columns and at most one column of left padding: the three stages of a window row and
+//                  16 channels from one 12-byte load a channel
+enum { SP_INSIDE, SP_MASKED, SP_PAD, SP_ROW8, SP_ROW4, SP_POINT, SP_POINT32, SP_TRI };
 
 template <int MI_, class S>
 struct IgSplitPart {
@@ -633,6 +635,7 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
             const uint32_t oh = fc_div(pp, p.divOW), ow = pp - oh * p.OW;
             const int ih0 = (int)oh * p.sh - p.pt, iw0 = (int)ow * p.sw - p.pl;
             pixByte[ni] = 4u * (n * (uint32_t)(p.C * p.H * p.W) + (uint32_t)(ih0 * p.W + iw0));
+            if (MODE == SP_TRI && iw0 < 0) pixByte[ni] += 4u;      // from its first column inside the image
             if (!ROW) pixByte[ni] += 8u * lrow * 4u * (uint32_t)(p.H * p.W);      // the lane's first channel of a stage
             if (MODE != SP_INSIDE) {
                 for (int r = 0; r < p.kh; r++) rowBad[ni] &= (unsigned)(ih0 + r) < (unsigned)p.H ? ~(1u << r) : ~0u;
@@ -645,7 +648,9 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xres, voff, soff, 0));
     };
 
+    typedef float floatx3 __attribute__((ext_vector_type(3)));
     float raw[NI][8];
+    floatx3 raw3[NI][8];      // SP_TRI: a window row of each channel
     // -- blocks of channels: the tap and the first channel of the stage, counted in scalar registers
     const uint32_t chanStep = 4u * (uint32_t)(p.H * p.W);
     int tapR = 0, tapS = 0, tapC = 0;
@@ -675,7 +680,7 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
         tapC = block * 16;
         tapR = t / p.kw;
         tapS = t - tapR * p.kw;
-        tap();
+        if (MODE != SP_TRI) tap();
     }
     // fetches stage s; stages are fetched in order
     auto fetch = [&](const int s) __attribute__((always_inline)) {
@@ -697,6 +702,22 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
                 }
             }
             table(min(s + 1, nStagesAll - 1));
+            return;
+        }
+        if constexpr (MODE == SP_TRI) {      // the window row that stage s begins or, at the first stage, lies in
+            const int left = p.C - tapC - 8 * lrow;      // channels of the lane's 8 that exist
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) {
+                const uint32_t vo = (rowBad[ni] >> tapR) & 1u ? OUTSIDE : pixByte[ni] + 4u * (uint32_t)(tapR * p.W);
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    raw3[ni][i] = __builtin_bit_cast(floatx3, __builtin_amdgcn_raw_buffer_load_b96(
+                                                                  xres, i < left ? vo : OUTSIDE, (uint32_t)min(tapC + i, p.C - 1) * chanStep, 0));
+            }
+            tapR++;
+            const bool all = tapR == p.kh;
+            tapR = all ? 0 : tapR;
+            tapC += all ? 16 : 0;
             return;
         }
         if (POINT) {
@@ -808,8 +829,22 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
     fc_zero<MI, NI>(acc);
     fc_zero<MI, NI>(small);
     // more: a stage follows
-    auto stage = [&](const int s, const bool more, auto readAgain) __attribute__((always_inline)) {
+    // column: of its window row, where three stages share their loads; fetch: the next stage's columns are not in registers yet
+    auto stage = [&](const int s, const bool more, auto readAgain, auto column) __attribute__((always_inline)) {
         const int buf = (s - sBegin) & 1;
+        if constexpr (MODE == SP_TRI) {
+            constexpr int q = decltype(column)::value;
+#pragma unroll
+            for (int ni = 0; ni < NI; ni++) {
+                const int keep = (int)(~colBad[ni] << (31 - q)) >> 31;
+                const bool shifted = colBad[ni] & 1u;
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const float v = q == 0 || shifted ? raw3[ni][i][q == 2 ? 1 : 0] : raw3[ni][i][q];
+                    raw[ni][i] = __builtin_bit_cast(float, __builtin_bit_cast(int, v) & keep);
+                }
+            }
+        }
         split(readAgain);
         if constexpr (MODE == SP_POINT32) filterSplit(buf);
         if constexpr (MODE != SP_POINT32) __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): this wavefront's filter words of the stage are in LDS
@@ -823,7 +858,7 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
         if (more) {      // (behind the reads: the compiler has reads of LDS wait for direct loads before them)
             if constexpr (MODE == SP_POINT32) filterRows(s + 1);
             else filter(buf ^ 1);
-            fetch(s + 1);
+            if (MODE != SP_TRI || decltype(column)::value == 2) fetch(s + 1);
         }
         constexpr int pa[5] = {2, 1, 0, 1, 0}, pb[5] = {0, 1, 2, 0, 1};
 #pragma unroll
@@ -847,13 +882,22 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
         // one number for the workgroup: all its wavefronts meet at the same barriers
         const int stagesBefore = (long)pb * S::BN_ < p.pixBefore ? p.stagesBefore : 0;
 #pragma unroll 1
-        for (; s < sEnd && s < stagesBefore; s++) stage(s, s + 1 < sEnd, std::true_type());
+        for (; s < sEnd && s < stagesBefore; s++) stage(s, s + 1 < sEnd, std::true_type(), std::integral_constant<int, 0>());
 #pragma unroll 1
-        for (; s < sEnd; s++) stage(s, s + 1 < sEnd, std::false_type());
+        for (; s < sEnd; s++) stage(s, s + 1 < sEnd, std::false_type(), std::integral_constant<int, 0>());
+    } else if constexpr (MODE == SP_TRI) {
+        // three stages a round; a part of a split reduction may begin and end within a window row
+        const int skip = tapS;
+#pragma unroll 1
+        for (s -= skip; s < sEnd; s += 3) {
+            if (s >= sBegin) stage(s, s + 1 < sEnd, std::false_type(), std::integral_constant<int, 0>());
+            if (s + 1 >= sBegin && s + 1 < sEnd) stage(s + 1, s + 2 < sEnd, std::false_type(), std::integral_constant<int, 1>());
+            if (s + 2 < sEnd) stage(s + 2, s + 3 < sEnd, std::false_type(), std::integral_constant<int, 2>());
+        }
     } else {
 #pragma unroll 1
-        for (; s + 1 < sEnd; s++) stage(s, true, std::false_type());
-        stage(s, false, std::false_type());
+        for (; s + 1 < sEnd; s++) stage(s, true, std::false_type(), std::integral_constant<int, 0>());
+        stage(s, false, std::false_type(), std::integral_constant<int, 0>());
     }
     fc_join<MI, NI>(acc, small);
     const bool again = __syncthreads_or(fc_not_finite<MI, NI>(acc));
@@ -871,7 +915,7 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
 }
 
 template <class S, int MODE>
-__global__ __launch_bounds__(S::THREADS, (MODE == SP_ROW4 || MODE == SP_INSIDE) && S::MIN_WAVES > 3 ? 3 : S::MIN_WAVES) void igemm_split_kernel(const IgemmParams p) {
+__global__ __launch_bounds__(S::THREADS, (MODE == SP_ROW4 || MODE == SP_INSIDE || MODE == SP_TRI) && S::MIN_WAVES > 3 ? 3 : S::MIN_WAVES) void igemm_split_kernel(const IgemmParams p) {
     __shared__ fc_uintx4 smem[S::LDS_WORDS + (MODE == SP_POINT || MODE == SP_POINT32 ? S::THREADS / 64 * 128 : 0)];
     int kb, pb;
     if (!ig_decode_tile(p, &kb, &pb)) return;
@@ -1082,6 +1126,10 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
             // 56x56 28.2 / 26.0, 1024 -> 256 at 14x14 34.7 / 32.9, 112 -> 208 at 68x68 batch 4 13.4 / 12.3.  Tiles of 128 rows
             // load half as often for their products: 64 -> 256 at 56x56 30.6 / 32.3, 144 -> 112 at 130x130 batch 35 173 / 178
             else if (S::BM_ == 64 && ig_four_pixels(s)) igemm_split_kernel<S, SP_POINT><<<grid, block, 0, ctx->stream>>>(p);
+            // strided layers under tiles of 128 rows, batch 32, us: 128 -> 128 at 56x56 76.0 / 71.9, 256 -> 256 at 28x28 69.6 / 67.0,
+            // 32 -> 448 at 100x100 batch 22 107.8 / 103.6.  (Stride 1 loads find their lines in the cache: 256 -> 256 at 56x56 batch 8
+            // 192 / 197; tiles of 64 rows lose a wavefront a SIMD to the registers: 64 -> 64 at 56x56 50.8 / 57.2)
+            else if (S::BM_ == 128 && s.kw == 3 && s.sw > 1 && s.pl <= 1) igemm_split_kernel<S, SP_TRI><<<grid, block, 0, ctx->stream>>>(p);
             else if (s.C % 16 != 0) igemm_split_kernel<S, SP_PAD><<<grid, block, 0, ctx->stream>>>(p);
             else if (ig_inside(s, 16)) igemm_split_kernel<S, SP_INSIDE><<<grid, block, 0, ctx->stream>>>(p);
             else igemm_split_kernel<S, SP_MASKED><<<grid, block, 0, ctx->stream>>>(p);
@@ -1101,12 +1149,24 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
     else igemm_conv_kernel<TL, IG_GATHER><<<grid, block, 0, ctx->stream>>>(p);
 }
 
+// Layers on split products whose reduction is cut into parts by their expected time: windows over whole blocks of channels, several
+// images, strided or 100 stages and more.  The others keep as many parts as fill the chip (ig_parts_to_fill): 1x1 layers as the
+// expected times do not tell their tiles apart so well (512 -> 2048 at 7x7 batch 32 28 / 33 us), window rows in runs and blocks with
+// channels missing as they are ahead and behind about as often (28 -> 38 at 9x45 batch 52 14.9 / 18.6, 548 -> 175 at 21x113 batch 10 235 /
+// 245, 168 -> 631 at 8x8 batch 18 36.9 / 31.9), and so that untuned plans with more than 32 MiB of partial sums stay what they were.
+bool ig_parts_by_time(const fc_conv_shape &s) {
+    const long taps = (long)s.kh * s.kw;
+    return taps > 1 && s.N > 1 && s.C % 16 == 0 && (s.sh > 1 || s.sw > 1 || s.C / 16 * taps >= 100);
+}
+
 // Expected time of a layer on the bf16 matrix cores, in us, under one of the tile shapes 128x128, 64x128, 128x64 and 64x64
 // (configurations 0 to 3).  A CU takes a stage of a workgroup every `cycles` (block or row order), however many it holds, and
 // one workgroup takes at least `latency` for it; beside that the start of a round, memory, and for a split reduction the pass
 // over the partial sums.  The constants are a least squares fit.  On 217 drawn layers that it was not made on (1x1, 3x3, 5x5 and 7x7,
 // one to 64 images, 1 to 1024 channels, 0.1 to 60 GFLOP; profiles/igemm_untuned_choice.txt): standard deviation 12 %, the choice
-// among the four 1.7 % behind the best of them on average, 5.6 % or more on a tenth of the layers, 26 % at most.
+// among the four 1.7 % behind the best of them on average, 5.6 % or more on a tenth of the layers, 26 % at most.  On 1495 layers under up to ten
+// numbers of parts each: 14 %, the choice among all of them 3.3 % behind the best on average (2.3 % in row orders, with 1.2 of `latency`), 11 % or more on a tenth; constants
+// fitted to those, for 1x1 layers apart, choose no better (3.1 %).
 struct IgSplitCost {
     int bm, bn, perCu;
     double cyclesBlock, cyclesRow, latency, start;
@@ -1121,8 +1181,10 @@ double ig_split_us(const fc_conv_shape &s, int config, const fc_igemm_plan &plan
     const double stages = ceil(ceil(rows / 16.0) / plan.split_k), kBlocks = ceil((double)s.K / c.bm);
     double cycles = order == IG_ORDER_BLOCK ? c.cyclesBlock : c.cyclesRow;
     if (c.bm == 64 && s.K % 64 != 0 && s.K % 64 <= 32) cycles *= (kBlocks - 1 + 0.59) / kBlocks;      // half of the last rows
-    const double blocks = kBlocks * ceil((double)plan.Npix / c.bn) * plan.split_k, slots = 256.0 * c.perCu;
-    auto round = [&](double perCu) { return stages * fmax(c.latency, perCu * cycles) + c.start * (1 + 2.3 * perCu); };
+    const double tiles = kBlocks * ceil((double)plan.Npix / c.bn);
+    // (as launched, in whole eights, where the number of parts is chosen by what fits the chip at once)
+    const double blocks = (ig_parts_by_time(s) ? ceil(tiles / 8) * 8 : tiles) * plan.split_k, slots = 256.0 * c.perCu;
+    auto round = [&](double perCu) { return stages * fmax(order == IG_ORDER_BLOCK ? c.latency : 1.2 * c.latency, perCu * cycles) + c.start * (1 + 2.3 * perCu); };
     const double full = floor(blocks / slots), rest = blocks - full * slots;
     const double compute = (full * round(c.perCu) + (rest > 0 ? round(ceil(rest / 256)) : 0)) / 2000;
     const double bytes = 4.0 * ((double)s.N * s.C * s.H * s.W / (s.kh * s.kw == 1 ? s.sh * s.sw : 1) + (double)s.K * plan.Npix);
@@ -1140,14 +1202,33 @@ double ig_ws_us(const fc_conv_shape &s, const fc_gemm_config &c, long npix) {
     return 3.5 + (perCu * units * cycles + 52.8 * perCu * mt * nt * c.waves_k) / 2000;
 }
 
+// Small layers do not fill 256 CUs with their tiles: the reduction in as many parts as make about three workgroups per CU,
+// keeping >= 4 LDS stages per part.
+int ig_parts_to_fill(long blocks, int stages) {
+    int splitK = 1;
+    // A grid of two to four workgroups per CU is placed unevenly by the dispatcher (some CUs get
+    // one more than their share and set the time of the launch): with a long reduction, splitting
+    // it to about six per CU is worth the second pass (measured: 3x3 stride-2 layers of ResNet-50
+    // at batch 32 -9 %, 2048 -> 512 at 7x7 -6 %; with a short reduction the second pass costs more).
+    const bool longReduction = stages >= 64;
+    const long below = longReduction ? 1024 : 512, target = longReduction ? 1536 : 768;
+    if (blocks < below) {
+        splitK = (int)((target + blocks - 1) / blocks);
+        if (splitK > stages / 4) splitK = stages / 4;
+        if (splitK > 32) splitK = 32;
+        if (splitK < 1) splitK = 1;
+    }
+    return splitK;
+}
+
 // The kernel that adds up partial sums has one workgroup row per output channel.
 constexpr int kMaxReduceChannels = 65535;
 
 // Plans that cannot run because of their partial sums (kMaxReduceChannels) are behind all others.
-// A layer whose reduction the best tile would split over workgroups goes to the kernels that split it inside the workgroup
-// where those are expected ahead, from 9 parts on also where they are 15 % behind and from 21 on 50 %: the model then favours
-// the tiles.  Of the same 217 layers 77 go of 132 that would be split, at 0.72 of the tile's time on average (2 to 8 parts), 0.68
-// (9 to 20) and 0.79 (21 to 32); the seven that go by these lines alone take 0.72 to 1.20, 0.96 on average.
+// A layer that the best tile would fill the chip with only in several parts (ig_parts_to_fill, whether it is then split or not) goes to
+// the kernels that split it inside the workgroup where those are expected ahead, from 9 parts on also where they are 15 % behind and
+// from 21 on 50 %: the model then favours the tiles.  Of 1495 drawn layers 321 go, at 0.71 of the tile's time on average; where they
+// take 20 us and more the two are level.
 int ig_split_default_config(const fc_conv_shape *s) {
     int best = 3;
     double bestUs = 1e300;
@@ -1159,11 +1240,13 @@ int ig_split_default_config(const fc_conv_shape *s) {
         const bool runs = plan.split_k == 1 || s->K <= kMaxReduceChannels;
         if (runs != bestRuns ? runs : us < bestUs) { bestUs = us; best = id; bestPlan = plan; bestRuns = runs; }
     }
-    const int ws = bestPlan.split_k > 1 ? fc_igemm_ws_choose(s, plan.Npix) : -1;
+    const IgSplitCost &tile = kIgSplitCost[best];
+    const int parts = ig_parts_to_fill((long)(bestPlan.K_pad / tile.bm) * ((bestPlan.Npix + tile.bn - 1) / tile.bn), bestPlan.Kred_pad / 16);
+    const int ws = parts > 1 ? fc_igemm_ws_choose(s, plan.Npix) : -1;
     if (ws >= 0) {
         fc_gemm_config c;
         fc_igemm_ws_get_config(ws, kNumIgConfigs + ws, &c);
-        const double behind = bestPlan.split_k > 20 ? 1.5 : bestPlan.split_k > 8 ? 1.15 : 1.0;
+        const double behind = parts > 20 ? 1.5 : parts > 8 ? 1.15 : 1.0;
         if (!bestRuns || ig_ws_us(*s, c, plan.Npix) < bestUs * behind) return kNumIgConfigs + ws;
     }
     return best;
@@ -1226,6 +1309,25 @@ static void ig_set_parts(fc_igemm_plan &plan, int stages, int parts) {
     plan.ws_bytes = plan.split_k > 1 ? sizeof(float) * (size_t)plan.split_k * plan.shape.K * plan.Npix : 0;
 }
 
+// In the parts that make enough workgroups (`fill`), or in the number of them, of at least four stages, that is expected to take the
+// least time where that is 6 % less (ig_parts_by_time).  128x128 tiles, of which a CU holds two, do best where all of them fit the chip
+// at once.  Batch 32, us, parts to fill / this: 256 -> 256 3x3/2 at 28x28 69 / 55, 128 -> 128 3x3/2 at 56x56 76 / 58, 512 -> 512 3x3/2 at
+// 14x14 70 / 55, 512 -> 512 3x3 at 28x28 batch 8 190 / 163, 208 -> 240 3x3 at 7x7 batch 42 37 / 26; 128 -> 80 3x3/2 at 106x106 batch 7 49 / 52.
+static void ig_expected_parts(fc_igemm_plan &plan, IgTileSize tile, int stages, int fill) {
+    int config = 0;      // the one of the four costed tiles that runs
+    while (kIgSplitCost[config].bm != tile.bm || kIgSplitCost[config].bn != tile.bn) config++;
+    ig_set_parts(plan, stages, fill);
+    int best = plan.split_k;
+    double bestUs = best > 1 && plan.shape.K > kMaxReduceChannels ? 1e300 : 0.94 * ig_split_us(plan.shape, config, plan);
+    for (int parts = 1; parts <= std::max(1, std::min(32, stages / 4)); parts++) {
+        ig_set_parts(plan, stages, parts);
+        if (plan.split_k != parts || (parts > 1 && plan.shape.K > kMaxReduceChannels)) continue;
+        const double us = ig_split_us(plan.shape, config, plan);
+        if (us < bestUs) { bestUs = us; best = parts; }
+    }
+    ig_set_parts(plan, stages, best);
+}
+
 // In no more parts than have room for their sums: the packed filter does not depend on the number of parts.
 static void ig_split_to_fit(fc_igemm_plan &plan, size_t ws_bytes) {
     fc_gemm_config cfg;
@@ -1269,24 +1371,13 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
         plan->ws_bytes = 0;
         return FC_OK;
     }
-    // Small layers do not fill 256 CUs with (K_pad/BM) x (Npix/BN) workgroups: split the
-    // reduction until about three workgroups per CU exist, keeping >= 4 LDS stages per part.
     const long blocks = (long)(plan->K_pad / tile.bm) * ((npix + tile.bn - 1) / tile.bn);
     const int stages = plan->Kred_pad / cfg.bk;
-    int splitK = 1;
-    // A grid of two to four workgroups per CU is placed unevenly by the dispatcher (some CUs get
-    // one more than their share and set the time of the launch): with a long reduction, splitting
-    // it to about six per CU is worth the second pass (measured: 3x3 stride-2 layers of ResNet-50
-    // at batch 32 -9 %, 2048 -> 512 at 7x7 -6 %; with a short reduction the second pass costs more).
-    const bool longReduction = stages >= 64;
-    const long below = longReduction ? 1024 : 512, target = longReduction ? 1536 : 768;
-    if (blocks < below) {
-        splitK = (int)((target + blocks - 1) / blocks);
-        if (splitK > stages / 4) splitK = stages / 4;
-        if (splitK > 32) splitK = 32;
-        if (splitK < 1) splitK = 1;
+    if (split && ig_parts_by_time(*s)) {
+        ig_expected_parts(*plan, tile, stages, ig_parts_to_fill(blocks, stages));
+        return FC_OK;
     }
-    ig_set_parts(*plan, stages, splitK);
+    ig_set_parts(*plan, stages, ig_parts_to_fill(blocks, stages));
     return FC_OK;
 }
 
