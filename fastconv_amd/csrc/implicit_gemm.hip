@@ -1125,7 +1125,9 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
             // two 16-byte loads a stage and wavefront in place of eight of 4 bytes, whole layers of batch 32, us: 256 -> 64 at
             // 56x56 28.2 / 26.0, 1024 -> 256 at 14x14 34.7 / 32.9, 112 -> 208 at 68x68 batch 4 13.4 / 12.3.  Tiles of 128 rows
             // load half as often for their products: 64 -> 256 at 56x56 30.6 / 32.3, 144 -> 112 at 130x130 batch 35 173 / 178
-            else if (S::BM_ == 64 && ig_four_pixels(s)) igemm_split_kernel<S, SP_POINT><<<grid, block, 0, ctx->stream>>>(p);
+            // (also where few wavefronts a CU walk a long reduction, whose every stage waits for the turn: 976 -> 96 at 40x77 batch 8, 61
+            // stages, 770 workgroups, 58.9 / 61.2, 720 -> 96 at 116x116 batch 2 39.2 / 42.8; 944 -> 80 at 164x164 batch 2, 1682, 88.5 / 82.7)
+            else if (S::BM_ == 64 && ig_four_pixels(s) && (p.stagesPerSplit <= 40 || (long)p.nKB * p.nPB * p.splitK * (S::THREADS / 128) >= 1024)) igemm_split_kernel<S, SP_POINT><<<grid, block, 0, ctx->stream>>>(p);
             // strided layers under tiles of 128 rows, batch 32, us: 128 -> 128 at 56x56 76.0 / 71.9, 256 -> 256 at 28x28 69.6 / 67.0,
             // 32 -> 448 at 100x100 batch 22 107.8 / 103.6.  (Stride 1 loads find their lines in the cache: 256 -> 256 at 56x56 batch 8
             // 192 / 197; tiles of 64 rows lose a wavefront a SIMD to the registers: 64 -> 64 at 56x56 50.8 / 57.2)
