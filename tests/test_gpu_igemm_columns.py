@@ -1,0 +1,57 @@
+"""Implicit GEMM on split products: columns read by wider loads (window rows of three taps, four pixels of a pointwise layer), at the
+edges of the image, of the tensor, of the channels and of the parts of a split reduction."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -24      # of a product and of an addition, as for the other kernels of split products
+
+
+@pytest.fixture(scope="module")
+def lib():
+    import fastconv_amd as F
+    L = F.load(0, 1 << 30)
+    yield L
+    L.close()
+
+
+def cshape(s):
+    import fastconv_amd as F
+    return F.ConvShape(*[getattr(s, n) for n, _ in F.ConvShape._fields_])
+
+
+WINDOWS = [      # tiles of 128 rows, strided, three columns
+    (3, 15, 11, 13, 130, 3, 3, 2, 2, 1),     # a channel missing, windows before x and past its end
+    (2, 47, 9, 30, 128, 3, 3, 2, 2, 0),      # no padding
+    (2, 32, 12, 11, 200, 3, 3, 3, 3, 1),     # stride 3: a column no window reads
+    (2, 16, 9, 8, 130, 5, 3, 1, 2, 1),       # five window rows
+    (4, 64, 15, 15, 256, 3, 3, 2, 2, 1),     # parts of the reduction that begin and end within a window row
+    (3, 208, 9, 9, 129, 3, 3, 2, 2, 1),
+    (1, 16, 3, 3, 129, 3, 3, 2, 2, 1),       # one image no larger than the window
+]
+POINTWISE = [      # tiles of 64 rows
+    (1, 64, 9, 7, 130, 1, 1, 1, 1, 0),       # one odd image: the last group reads past the last pixel, and past x
+    (3, 70, 6, 6, 96, 1, 1, 1, 1, 0),        # channels missing
+    (2, 100, 14, 14, 65, 1, 1, 1, 1, 0),     # four of the last eight channels missing
+    (5, 64, 2, 2, 72, 1, 1, 1, 1, 0),        # images of one group of pixels
+    (1, 49, 1, 3, 70, 1, 1, 1, 1, 0),        # fewer pixels than a group
+    (2, 720, 4, 4, 66, 1, 1, 1, 1, 0),       # 45 stages of few wavefronts: read a pixel a lane
+]
+
+
+@pytest.mark.parametrize("shp,configs", [(s, (0, 2)) for s in WINDOWS] + [(s, (1, 3)) for s in POINTWISE])
+def test_columns_against_fp64(lib, shp, configs):
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=sum(shp))
+    bias = O.rng_uniform(3, (s.K,))
+    # magnitudes over 2^40, as a product's rounding must not depend on the scale of its row
+    x = (x * np.exp2(np.arange(s.N * s.C) % 41 - 20).reshape(s.N, s.C, 1, 1)).astype(np.float32)
+    # products and the sums of them, of the parts of a split reduction (at most 32) and of the bias
+    tol = (s.C * s.kh * s.kw + 73) * EPS * (O.naive_conv_f64(s, np.abs(x), np.abs(w)) + np.abs(bias)[:, None, None]) + 1e-30
+    truth = O.naive_conv_f64(s, x, w) + bias[:, None, None]
+    for cfg in configs:
+        print("columns", shp, cfg, flush=True)
+        assert (np.abs(lib.implicit_gemm_conv(cshape(s), x, w, bias, False, config=cfg) - truth) <= tol).all(), cfg
