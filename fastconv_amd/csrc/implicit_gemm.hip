@@ -1242,6 +1242,7 @@ int ig_split_default_config(const fc_conv_shape *s) {
         const bool runs = plan.split_k == 1 || s->K <= kMaxReduceChannels;
         if (runs != bestRuns ? runs : us < bestUs) { bestUs = us; best = id; bestPlan = plan; bestRuns = runs; }
     }
+    if (bestUs == 1e300) return best;      // a layer that fc_igemm_make_plan refuses
     const IgSplitCost &tile = kIgSplitCost[best];
     const int parts = ig_parts_to_fill((long)(bestPlan.K_pad / tile.bm) * ((bestPlan.Npix + tile.bn - 1) / tile.bn), bestPlan.Kred_pad / 16);
     const int ws = parts > 1 ? fc_igemm_ws_choose(s, plan.Npix) : -1;

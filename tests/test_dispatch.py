@@ -1,10 +1,15 @@
 """Which Winograd pipeline the library advises (host code only): where the single-kernel path hands a layer to the
 pipelines with V and M in memory, they accept it."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import pytest
 
 from fastconv_amd import capi
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.fixture(scope="module")
@@ -146,3 +151,15 @@ def test_parts_of_a_reduction_put_the_large_tiles_on_the_chip_at_once(lib, geo, 
     assert plan.split_k == parts and 256 < -(-tiles // 8) * 8 * plan.split_k <= 512
     stages = plan.Kred_pad // 16
     assert -(-stages // -(-stages // parts)) == parts and plan.ws_bytes == 4 * parts * k * plan.Npix      # no part is empty
+
+
+@pytest.mark.parametrize("geo", [
+    (1, 16, 32, 32, 64, 32, 32, 1, 0), (1, 4, 8, 64, 64, 1, 33, 1, 0), (8, 16, 64, 64, 64, 33, 1, 2, 0), (1, 16, 64, 64, 64, 32, 1, 1, 16),      # windows of more than 31
+    (1, 65536, 8, 8, 64, 64, 64, 1, 32),      # and a reduction past the longest
+])
+def test_untuned_choice_answers_for_layers_that_have_no_plan(geo):
+    """fc_igemm_default_config is asked before a plan is made: the refusal is fc_igemm_make_plan's."""
+    code = ("import ctypes as C; from fastconv_amd import capi; lib = capi.load_cdll(); n, c, h, w, k, kh, kw, st, p = %r; "
+            "s = capi.ConvShape(n, c, h, w, k, kh, kw, st, st, p, p, p, p); d = lib.fc_igemm_default_config(C.byref(s)); "
+            "assert 0 <= d < lib.fc_igemm_num_configs(); assert lib.fc_igemm_make_plan(C.byref(s), d, C.byref(capi.IgemmPlan())) == -6") % (geo,)
+    assert subprocess.run([sys.executable, "-c", code], cwd=ROOT).returncode == 0
