@@ -1155,7 +1155,7 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
 // images, strided or 100 stages and more.  The others keep as many parts as fill the chip (ig_parts_to_fill): 1x1 layers as the
 // expected times do not tell their tiles apart so well (512 -> 2048 at 7x7 batch 32 28 / 33 us), window rows in runs and blocks with
 // channels missing as they are ahead and behind about as often (28 -> 38 at 9x45 batch 52 14.9 / 18.6, 548 -> 175 at 21x113 batch 10 235 /
-// 245, 168 -> 631 at 8x8 batch 18 36.9 / 31.9), and so that untuned plans with more than 32 MiB of partial sums stay what they were.
+// 245, 168 -> 631 at 8x8 batch 18 36.9 / 31.9).
 bool ig_parts_by_time(const fc_conv_shape &s) {
     const long taps = (long)s.kh * s.kw;
     return taps > 1 && s.N > 1 && s.C % 16 == 0 && (s.sh > 1 || s.sw > 1 || s.C / 16 * taps >= 100);
@@ -1176,21 +1176,23 @@ struct IgSplitCost {
 const IgSplitCost kIgSplitCost[] = {{128, 128, 2, 1121, 1032, 1602, 928}, {64, 128, 4, 756, 713, 1041, 535},
                                     {128, 64, 4, 621, 563, 1821, 711}, {64, 64, 8, 420, 398, 1031, 313}};
 
-double ig_split_us(const fc_conv_shape &s, int config, const fc_igemm_plan &plan) {
+// `refined`: with the grid as it is launched, in whole eights of tiles, where the number of parts is chosen by what fits the chip at once, and
+// with 1.2 of `latency` in row orders; the untuned tile is chosen without first (ig_split_default_config).
+double ig_split_us(const fc_conv_shape &s, int config, const fc_igemm_plan &plan, bool refined) {
     const IgSplitCost &c = kIgSplitCost[config];
     long rows;
     const int order = ig_order(s, kIgConfigs[config], &rows);
     const double stages = ceil(ceil(rows / 16.0) / plan.split_k), kBlocks = ceil((double)s.K / c.bm);
     double cycles = order == IG_ORDER_BLOCK ? c.cyclesBlock : c.cyclesRow;
     if (c.bm == 64 && s.K % 64 != 0 && s.K % 64 <= 32) cycles *= (kBlocks - 1 + 0.59) / kBlocks;      // half of the last rows
-    const double tiles = kBlocks * ceil((double)plan.Npix / c.bn);
-    // (as launched, in whole eights, where the number of parts is chosen by what fits the chip at once)
-    const double blocks = (ig_parts_by_time(s) ? ceil(tiles / 8) * 8 : tiles) * plan.split_k, slots = 256.0 * c.perCu;
-    auto round = [&](double perCu) { return stages * fmax(order == IG_ORDER_BLOCK ? c.latency : 1.2 * c.latency, perCu * cycles) + c.start * (1 + 2.3 * perCu); };
+    const double tiles = kBlocks * ceil((double)plan.Npix / c.bn), latency = refined && order != IG_ORDER_BLOCK ? 1.2 * c.latency : c.latency;
+    const double blocks = (refined && ig_parts_by_time(s) ? ceil(tiles / 8) * 8 : tiles) * plan.split_k, slots = 256.0 * c.perCu;
+    auto round = [&](double perCu) { return stages * fmax(latency, perCu * cycles) + c.start * (1 + 2.3 * perCu); };
     const double full = floor(blocks / slots), rest = blocks - full * slots;
     const double compute = (full * round(c.perCu) + (rest > 0 ? round(ceil(rest / 256)) : 0)) / 2000;
     const double bytes = 4.0 * ((double)s.N * s.C * s.H * s.W / (s.kh * s.kw == 1 ? s.sh * s.sw : 1) + (double)s.K * plan.Npix);
-    const double us = 4.5 + pow(pow(compute, 4) + pow(bytes / 4.99e6, 4), 0.25);
+    const double memory = bytes / 4.99e6;
+    const double us = 4.5 + sqrt(sqrt(compute * compute * compute * compute + memory * memory * memory * memory));
     return plan.split_k > 1 ? us + 3.4 + 2.0 * plan.ws_bytes / 6.65e6 : us;
 }
 
@@ -1231,26 +1233,42 @@ constexpr int kMaxReduceChannels = 65535;
 // the kernels that split it inside the workgroup where those are expected ahead, from 9 parts on also where they are 15 % behind and
 // from 21 on 50 %: the model then favours the tiles.  Of 1495 drawn layers 321 go, at 0.71 of the tile's time on average; where they
 // take 20 us and more the two are level.
+int ig_plan_to_fill(const fc_conv_shape *s, int config, fc_igemm_plan *plan);
 int ig_split_default_config(const fc_conv_shape *s) {
     int best = 3;
     double bestUs = 1e300;
     bool bestRuns = false;
     fc_igemm_plan plan, bestPlan = {};
     for (int id = 0; id < 4; id++) {
-        if (fc_igemm_make_plan(s, id, &plan) != FC_OK) continue;
-        const double us = ig_split_us(*s, id, plan);
+        if (ig_plan_to_fill(s, id, &plan) != FC_OK) continue;
+        const double us = ig_split_us(*s, id, plan, false);
         const bool runs = plan.split_k == 1 || s->K <= kMaxReduceChannels;
         if (runs != bestRuns ? runs : us < bestUs) { bestUs = us; best = id; bestPlan = plan; bestRuns = runs; }
     }
-    if (bestUs == 1e300) return best;      // a layer that fc_igemm_make_plan refuses
-    const IgSplitCost &tile = kIgSplitCost[best];
-    const int parts = ig_parts_to_fill((long)(bestPlan.K_pad / tile.bm) * ((bestPlan.Npix + tile.bn - 1) / tile.bn), bestPlan.Kred_pad / 16);
+    const int parts = bestPlan.split_k;      // 0: a layer that fc_igemm_make_plan refuses
     const int ws = parts > 1 ? fc_igemm_ws_choose(s, plan.Npix) : -1;
     if (ws >= 0) {
         fc_gemm_config c;
         fc_igemm_ws_get_config(ws, kNumIgConfigs + ws, &c);
         const double behind = parts > 20 ? 1.5 : parts > 8 ? 1.15 : 1.0;
         if (!bestRuns || ig_ws_us(*s, c, plan.Npix) < bestUs * behind) return kNumIgConfigs + ws;
+    }
+    // A second look where parts are chosen by time, and among layers in row orders that fill the chip unsplit: a tile that is expected ahead
+    // and asks for no more memory, so that callers who had room for the first one have it for this.  (The static workspace takes plans
+    // past its size of the untuned tile alone: the first one stays where its plan is such a one.)
+    const bool byTime = ig_parts_by_time(*s);
+    long rows;
+    if (parts == 0 || (!byTime && (parts > 1 || ig_split_order(*s, &rows) == IG_ORDER_BLOCK))) return best;
+    const size_t room = bestPlan.Wp_bytes + bestPlan.table_bytes + bestPlan.ws_bytes;
+    double least = (byTime ? 0.94 : 1.0) * ig_split_us(*s, best, bestPlan, true);
+    fc_igemm_make_plan(s, best, &plan);
+    if (plan.ws_bytes > (size_t)FC_IGEMM_STATIC_WS_BYTES) return best;
+    if (plan.split_k < parts) least = ig_split_us(*s, best, plan, true);
+    const int first = best;
+    for (int id = 0; id < 4; id++) {
+        if (id == first || fc_igemm_make_plan(s, id, &plan) != FC_OK || plan.Wp_bytes + plan.table_bytes + plan.ws_bytes > room) continue;
+        const double us = ig_split_us(*s, id, plan, true);
+        if (us < least) { least = us; best = id; }
     }
     return best;
 }
@@ -1312,25 +1330,6 @@ static void ig_set_parts(fc_igemm_plan &plan, int stages, int parts) {
     plan.ws_bytes = plan.split_k > 1 ? sizeof(float) * (size_t)plan.split_k * plan.shape.K * plan.Npix : 0;
 }
 
-// In the parts that make enough workgroups (`fill`), or in the number of them, of at least four stages, that is expected to take the
-// least time where that is 6 % less (ig_parts_by_time).  128x128 tiles, of which a CU holds two, do best where all of them fit the chip
-// at once.  Batch 32, us, parts to fill / this: 256 -> 256 3x3/2 at 28x28 69 / 55, 128 -> 128 3x3/2 at 56x56 76 / 58, 512 -> 512 3x3/2 at
-// 14x14 70 / 55, 512 -> 512 3x3 at 28x28 batch 8 190 / 163, 208 -> 240 3x3 at 7x7 batch 42 37 / 26; 128 -> 80 3x3/2 at 106x106 batch 7 49 / 52.
-static void ig_expected_parts(fc_igemm_plan &plan, IgTileSize tile, int stages, int fill) {
-    int config = 0;      // the one of the four costed tiles that runs
-    while (kIgSplitCost[config].bm != tile.bm || kIgSplitCost[config].bn != tile.bn) config++;
-    ig_set_parts(plan, stages, fill);
-    int best = plan.split_k;
-    double bestUs = best > 1 && plan.shape.K > kMaxReduceChannels ? 1e300 : 0.94 * ig_split_us(plan.shape, config, plan);
-    for (int parts = 1; parts <= std::max(1, std::min(32, stages / 4)); parts++) {
-        ig_set_parts(plan, stages, parts);
-        if (plan.split_k != parts || (parts > 1 && plan.shape.K > kMaxReduceChannels)) continue;
-        const double us = ig_split_us(plan.shape, config, plan);
-        if (us < bestUs) { bestUs = us; best = parts; }
-    }
-    ig_set_parts(plan, stages, best);
-}
-
 // In no more parts than have room for their sums: the packed filter does not depend on the number of parts.
 static void ig_split_to_fit(fc_igemm_plan &plan, size_t ws_bytes) {
     fc_gemm_config cfg;
@@ -1339,7 +1338,10 @@ static void ig_split_to_fit(fc_igemm_plan &plan, size_t ws_bytes) {
     ig_set_parts(plan, plan.Kred_pad / cfg.bk, (int)std::max<size_t>(1, std::min<size_t>(plan.split_k, parts)));
 }
 
-extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_plan *plan) {
+namespace {
+
+// A plan in the parts that fill the chip (ig_parts_to_fill).
+int ig_plan_to_fill(const fc_conv_shape *s, int config, fc_igemm_plan *plan) {
     if (!plan || !fc_shape_ok(s)) return FC_ERR_INVALID;
     fc_gemm_config cfg;
     const int rc = fc_igemm_get_config(config, &cfg);
@@ -1376,12 +1378,34 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
     }
     const long blocks = (long)(plan->K_pad / tile.bm) * ((npix + tile.bn - 1) / tile.bn);
     const int stages = plan->Kred_pad / cfg.bk;
-    if (split && ig_parts_by_time(*s)) {
-        ig_expected_parts(*plan, tile, stages, ig_parts_to_fill(blocks, stages));
-        return FC_OK;
-    }
     ig_set_parts(*plan, stages, ig_parts_to_fill(blocks, stages));
     return FC_OK;
+}
+
+// In the number of parts, at least four stages each and no more than fill the chip, that is expected to take the least time where that is 6 %
+// less (ig_parts_by_time).
+void ig_expected_parts(fc_igemm_plan &plan) {
+    const IgTileSize tile = kIgSplitTiles[plan.config];
+    int config = 0;      // the one of the four costed tiles that runs
+    while (kIgSplitCost[config].bm != tile.bm || kIgSplitCost[config].bn != tile.bn) config++;
+    const int stages = plan.Kred_pad / 16, fill = plan.split_k;
+    int best = fill;
+    double bestUs = plan.shape.K > kMaxReduceChannels ? 1e300 : 0.94 * ig_split_us(plan.shape, config, plan, true);
+    for (int parts = 1; parts < fill; parts++) {
+        ig_set_parts(plan, stages, parts);
+        if (plan.split_k != parts || (parts > 1 && plan.shape.K > kMaxReduceChannels)) continue;
+        const double us = ig_split_us(plan.shape, config, plan, true);
+        if (us < bestUs) { bestUs = us; best = parts; }
+    }
+    ig_set_parts(plan, stages, best);
+}
+
+}  // namespace
+
+extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_plan *plan) {
+    const int rc = ig_plan_to_fill(s, config, plan);
+    if (rc == FC_OK && plan->split_k > 1 && fc_igemm_splits_products(plan) && ig_parts_by_time(*s)) ig_expected_parts(*plan);
+    return rc;
 }
 
 extern "C" int fc_igemm_splits_products(const fc_igemm_plan *plan) {

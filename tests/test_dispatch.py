@@ -163,3 +163,42 @@ def test_untuned_choice_answers_for_layers_that_have_no_plan(geo):
             "s = capi.ConvShape(n, c, h, w, k, kh, kw, st, st, p, p, p, p); d = lib.fc_igemm_default_config(C.byref(s)); "
             "assert 0 <= d < lib.fc_igemm_num_configs(); assert lib.fc_igemm_make_plan(C.byref(s), d, C.byref(capi.IgemmPlan())) == -6") % (geo,)
     assert subprocess.run([sys.executable, "-c", code], cwd=ROOT).returncode == 0
+
+
+def parts_that_fill(plan, tile):
+    """About three workgroups a compute unit, six where the reduction is long, of at least four stages; no empty part."""
+    stages, blocks = plan.Kred_pad // 16, (plan.K_pad // tile[0]) * -(-plan.Npix // tile[1])
+    below, target = (1024, 1536) if stages >= 64 else (512, 768)
+    parts = max(1, min(-(-target // blocks), stages // 4, 32)) if blocks < below else 1
+    return -(-stages // -(-stages // parts))
+
+
+@pytest.mark.parametrize("geo", [
+    (5, 176, 136, 136, 336, 5, 2, 2), (6, 240, 154, 154, 64, 5, 1, 2), (8, 64, 16, 35, 736, 7, 1, 3), (32, 864, 44, 44, 752, 7, 2, 3),
+    (7, 432, 207, 207, 48, 3, 2, 1), (8, 464, 153, 153, 16, 5, 1, 2), (32, 256, 28, 28, 256, 3, 2, 1), (6, 389, 143, 109, 114, 7, 2, 3),
+    (8, 512, 28, 28, 512, 3, 1, 1), (32, 128, 28, 28, 512, 1, 1, 0), (43, 768, 18, 18, 112, 5, 2, 2), (3, 144, 92, 92, 528, 3, 2, 1),
+])
+def test_no_reduction_is_cut_into_more_parts_than_fill_the_chip(lib, geo):
+    """A caller with room for the partial sums of the parts that fill the chip has it for the plan; the static workspace takes the same plans."""
+    n, c, h, w, k, ks, st, p = geo
+    s, plan = capi.ConvShape(n, c, h, w, k, ks, ks, st, st, p, p, p, p), capi.IgemmPlan()
+    for i, tile in enumerate([(128, 128), (64, 128), (128, 64), (64, 64), None, (128, 128), (128, 128), (64, 128)]):
+        if tile and lib.fc_igemm_make_plan(C.byref(s), i, C.byref(plan)) == 0:
+            fill = parts_that_fill(plan, tile)
+            assert 1 <= plan.split_k <= fill and plan.ws_bytes == (4 * plan.split_k * k * plan.Npix if plan.split_k > 1 else 0), i
+
+
+@pytest.mark.parametrize("geo,ws_mb,static", [
+    # partial sums of the untuned plan in MiB at most; tiles whose plans fit the static workspace of 32 MiB or are the untuned ones
+    ((6, 240, 154, 154, 64, 5, 1, 2), 0, (0, 1, 2, 3, 5, 6, 7)), ((5, 176, 136, 136, 336, 5, 2, 2), 89, (1, 2, 3, 7)),
+    ((32, 864, 44, 44, 752, 7, 2, 3), 134, (1, 2, 3, 7)), ((7, 432, 207, 207, 48, 3, 2, 1), 42, (2, 3)), ((8, 64, 16, 35, 736, 7, 1, 3), 51, (2,)),
+    ((6, 389, 143, 109, 114, 7, 2, 3), 93, (0,)),
+])
+def test_plans_that_the_static_workspace_takes(lib, geo, ws_mb, static):
+    n, c, h, w, k, ks, st, p = geo
+    s, plan = capi.ConvShape(n, c, h, w, k, ks, ks, st, st, p, p, p, p), capi.IgemmPlan()
+    untuned = lib.fc_igemm_default_config(C.byref(s))
+    for i in (untuned,) + static:
+        assert lib.fc_igemm_make_plan(C.byref(s), i, C.byref(plan)) == 0
+        assert plan.ws_bytes <= capi.IGEMM_STATIC_WS_BYTES or i == untuned, i
+        assert i != untuned or plan.ws_bytes <= ws_mb << 20
