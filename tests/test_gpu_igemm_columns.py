@@ -55,3 +55,37 @@ def test_columns_against_fp64(lib, shp, configs):
     for cfg in configs:
         print("columns", shp, cfg, flush=True)
         assert (np.abs(lib.implicit_gemm_conv(cshape(s), x, w, bias, False, config=cfg) - truth) <= tol).all(), cfg
+
+
+@pytest.mark.parametrize("shp", [(4, 64, 15, 15, 256, 3, 3, 2, 2, 1), (2, 208, 9, 9, 129, 3, 3, 2, 2, 1)])
+def test_plans_in_other_parts_of_the_reduction_run_and_inconsistent_ones_do_not(lib, shp):
+    """A plan kept by a program, of a library that chose another number of parts; the packed filter does not depend on it."""
+    import fastconv_amd as F
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=sum(shp))
+    tol = (s.C * s.kh * s.kw + 73) * EPS * O.naive_conv_f64(s, np.abs(x), np.abs(w)) + 1e-30
+    truth = O.naive_conv_f64(s, x, w)
+    mark = lib.mark()
+    try:
+        for cfg in (0, 2, 3):
+            plan = lib.igemm_plan(cshape(s), cfg)
+            dx, dw, Wp, tab = lib.upload(x), lib.upload(w), lib.alloc(plan.Wp_bytes), lib.alloc(plan.table_bytes)
+            y, one = lib.alloc(4 * s.N * s.K * plan.OH * plan.OW), 4 * s.K * plan.Npix
+            ws = lib.alloc(32 * one)
+            lib.igemm_pack_filter(plan, dw, Wp, tab)
+            stages = plan.Kred_pad // 16
+            for parts in range(1, 34):
+                print("parts", shp, cfg, parts, flush=True)
+                plan.split_k, plan.ws_bytes = parts, parts * one if parts > 1 else 0
+                if parts <= stages // 4 and -(-stages // -(-stages // parts)) == parts:
+                    lib.conv_implicit_gemm(plan, dx, Wp, tab, y, None, False, ws)
+                    assert (np.abs(lib.download(y, (s.N, s.K, plan.OH, plan.OW)) - truth) <= tol).all(), (cfg, parts)
+                else:
+                    with pytest.raises(F.FastConvError):
+                        lib.conv_implicit_gemm(plan, dx, Wp, tab, y, None, False, ws)
+            for parts, nbytes in ((2, one), (2, 0), (1, one), (0, 0), (-1, 0)):
+                plan.split_k, plan.ws_bytes = parts, nbytes
+                with pytest.raises(F.FastConvError):
+                    lib.conv_implicit_gemm(plan, dx, Wp, tab, y, None, False, ws)
+    finally:
+        lib.release(mark)
