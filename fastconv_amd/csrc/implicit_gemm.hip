@@ -89,6 +89,7 @@ struct IgemmParams {
     long Npix;
     int nKB, nPB;
     int splitK, stagesPerSplit;   // reduction split over blockIdx.y; partial sums go to ws
+    int sumStages;                // split products in two levels of sums: stages added up in the first
     float *ws;                    // [splitK][K][Npix] when splitK > 1
     long xBytes;                  // size of the input tensor
     int fastStore;                // K is a whole number of tiles, every output byte offset fits 32 bits, bias 16-byte aligned
@@ -605,7 +606,12 @@ struct IgSplitPart {
 };
 
 // One workgroup tile, of which the first MI blocks of 32 rows of each wavefront hold output channels.
-template <class S, int MODE, int MI>
+// LEVELS (tiles of 128 rows): every p.sumStages stages the sum of the hi * hi products is added to a second one, and begun again.  A
+// product of 16 rows is rounded at the size of the sum it is added to, so that the error of one sum grows with its length; this way a reduction
+// in fewer parts has no larger one (ig_expected_parts).  Three of the second sum's four blocks of rows fit the registers two wavefronts a
+// SIMD leave, the last one lies in LDS (both in LDS: three 128x64 workgroups a CU in place of four, 256 -> 256 3x3/2 at 28x28 batch 32
+// 72 us / 57).  Columns of window rows of three taps (SP_TRI) leave no registers for it: 57 us would be 55.
+template <class S, int MODE, int MI, bool LEVELS>
 __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb, const int pb, fc_uintx4 *smem) {
     constexpr bool ROW = MODE == SP_ROW8 || MODE == SP_ROW4, POINT = MODE == SP_POINT || MODE == SP_POINT32;
     constexpr int NI = S::NI, WAVES = S::THREADS / 64;
@@ -874,6 +880,40 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
             for (int ni = 0; ni < NI; ni++)
                 acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][mi], __builtin_bit_cast(fc_bf16x8, b[ni][0]), acc[mi][ni], 0, 0, 0);
     };
+    constexpr int HELD = 3;      // blocks of the second sum in registers
+    static_assert(!LEVELS || (MI == HELD + 1 && NI == 1), "one block in LDS, four words a lane");
+    floatx16 second[HELD];
+    floatx4 *const secondLds = reinterpret_cast<floatx4 *>(smem + S::LDS_WORDS) + wave * 256 + lane;
+    if constexpr (LEVELS) {
+#pragma unroll
+        for (int mi = 0; mi < HELD; mi++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) second[mi][i] = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; q++) secondLds[64 * q] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    // the first sum to the second; at the end the whole to the first
+    auto carry = [&](const bool end) __attribute__((always_inline)) {
+        if constexpr (LEVELS) {
+#pragma unroll
+            for (int mi = 0; mi < HELD; mi++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    second[mi][i] += acc[mi][0][i];
+                    acc[mi][0][i] = end ? second[mi][i] : 0.f;
+                }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                floatx4 d = secondLds[64 * q];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    d[i] += acc[HELD][0][4 * q + i];
+                    acc[HELD][0][4 * q + i] = end ? d[i] : 0.f;
+                }
+                if (!end) secondLds[64 * q] = d;
+            }
+        }
+    };
     if constexpr (MODE == SP_POINT32) filterRows(sBegin);
     else filter(0);
     fetch(sBegin);
@@ -896,9 +936,17 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
         }
     } else {
 #pragma unroll 1
-        for (; s + 1 < sEnd; s++) stage(s, true, std::false_type(), std::integral_constant<int, 0>());
+        for (int left = p.sumStages; s + 1 < sEnd; s++) {
+            stage(s, true, std::false_type(), std::integral_constant<int, 0>());
+            if constexpr (LEVELS)
+                if (--left == 0) {
+                    carry(false);
+                    left = p.sumStages;
+                }
+        }
         stage(s, false, std::false_type(), std::integral_constant<int, 0>());
     }
+    if constexpr (LEVELS) carry(true);
     fc_join<MI, NI>(acc, small);
     const bool again = __syncthreads_or(fc_not_finite<MI, NI>(acc));
     ig_store_tile<IgSplitPart<MI, S>>(acc, p, again ? nullptr : p.bias, again ? 0 : p.relu, kb, pb, 0, wn0, lrow, lcol);
@@ -914,14 +962,14 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
     }
 }
 
-template <class S, int MODE>
+template <class S, int MODE, bool LEVELS = false>
 __global__ __launch_bounds__(S::THREADS, (MODE == SP_ROW4 || MODE == SP_INSIDE || MODE == SP_TRI) && S::MIN_WAVES > 3 ? 3 : S::MIN_WAVES) void igemm_split_kernel(const IgemmParams p) {
-    __shared__ fc_uintx4 smem[S::LDS_WORDS + (MODE == SP_POINT || MODE == SP_POINT32 ? S::THREADS / 64 * 128 : 0)];
+    __shared__ fc_uintx4 smem[S::LDS_WORDS + (LEVELS ? S::THREADS / 64 * 256 : 0) + (MODE == SP_POINT || MODE == SP_POINT32 ? S::THREADS / 64 * 128 : 0)];
     int kb, pb;
     if (!ig_decode_tile(p, &kb, &pb)) return;
     // 32 rows of a 64-row tile past the last output channel are not multiplied
-    if (S::BM_ == 64 && p.K - kb * 64 <= 32) ig_split_tile<S, MODE, 1>(p, kb, pb, smem);
-    else ig_split_tile<S, MODE, S::MI>(p, kb, pb, smem);
+    if (S::BM_ == 64 && p.K - kb * 64 <= 32) ig_split_tile<S, MODE, 1, false>(p, kb, pb, smem);
+    else ig_split_tile<S, MODE, S::MI, LEVELS>(p, kb, pb, smem);
 }
 
 // The packed filter as operand words: [stage][block of 32 output channels][part][half of the stage][channel], 16 bytes each,
@@ -1084,6 +1132,12 @@ bool ig_point_few(const fc_conv_shape &s) {
     return ig_four_pixels(s) && s.K > 32 && s.K <= 64 && s.C > 48 && (long)s.N * s.H * s.W >= 768 * 128 && 4l * s.N * s.C * s.H * s.W < (1l << 31);
 }
 
+// Stages of the first of two levels of sums.  Errors of sums in one level are smallest in parts of about the root of the number of stages
+// each; more than 15 give no time, fewer cost some: 256 -> 256 3x3/2 at 28x28 batch 32, 144 stages, in five parts 9 57.6 us and 8.9e-8 against
+// 64 bits, 15 56.6 and 9.6e-8 (one level, eight parts: 1.05e-7); 144 -> 832 3x3/2 at 44x22 batch 4, 81 stages, 9 8.3e-8, 15 9.2e-8 (eight
+// parts: 9.1e-8).
+int ig_sum_stages(int stages) { return std::max(4, std::min(15, (int)sqrt((double)stages))); }
+
 // Row orders, runs of `run` columns: which of them may start before x.  The row of such a run is inside the image, so that it
 // starts (n * C + c) * H * W + row * W - pl floats from the start of x or later: images, channels, rows below these bounds.
 void ig_before(const fc_conv_shape &s, int run, IgemmParams &p) {
@@ -1095,6 +1149,8 @@ void ig_before(const fc_conv_shape &s, int run, IgemmParams &p) {
     p.pixBefore = (n * p.OH + std::min<long>(p.OH, oh + 1)) * p.OW;
     p.stagesBefore = (int)((channels * s.kh * ((s.kw + run - 1) / run) * run + 15) / 16);
 }
+
+bool ig_sums_in_levels(const fc_conv_shape &s, IgTileSize tile, long blocks, int stages, int parts);
 
 template <class TL>
 void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, IgemmParams &p) {
@@ -1120,6 +1176,15 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
             long rows;
             const int order = ig_order(s, cfg, &rows);
             ig_before(s, order == IG_ORDER_ROW8 ? 8 : 4, p);
+            if constexpr (S::BM_ == 128) {
+                const int stages = p.Kred_pad / 16;
+                if (ig_sums_in_levels(s, {S::BM_, S::BN_}, (long)p.nKB * p.nPB, stages, p.splitK)) {
+                    p.sumStages = ig_sum_stages(stages);
+                    if (ig_inside(s, 16)) igemm_split_kernel<S, SP_INSIDE, true><<<grid, block, 0, ctx->stream>>>(p);
+                    else igemm_split_kernel<S, SP_MASKED, true><<<grid, block, 0, ctx->stream>>>(p);
+                    return;
+                }
+            }
             if (order == IG_ORDER_ROW8) igemm_split_kernel<S, SP_ROW8><<<grid, block, 0, ctx->stream>>>(p);
             else if (order == IG_ORDER_ROW4) igemm_split_kernel<S, SP_ROW4><<<grid, block, 0, ctx->stream>>>(p);
             // two 16-byte loads a stage and wavefront in place of eight of 4 bytes, whole layers of batch 32, us: 256 -> 64 at
@@ -1225,6 +1290,17 @@ int ig_parts_to_fill(long blocks, int stages) {
     return splitK;
 }
 
+// A reduction of `stages` in at most `parts` of equal length, none of them empty.
+int ig_whole_parts(int stages, int parts) {
+    const int per = (stages + parts - 1) / parts;
+    return (stages + per - 1) / per;
+}
+
+// Whether a tile adds up in two levels: cut by time into fewer parts than fill the chip.
+bool ig_sums_in_levels(const fc_conv_shape &s, IgTileSize tile, long blocks, int stages, int parts) {
+    return tile.bm == 128 && ig_parts_by_time(s) && parts < ig_whole_parts(stages, ig_parts_to_fill(blocks, stages));
+}
+
 // The kernel that adds up partial sums has one workgroup row per output channel.
 constexpr int kMaxReduceChannels = 65535;
 
@@ -1254,7 +1330,7 @@ int ig_split_default_config(const fc_conv_shape *s) {
         if (!bestRuns || ig_ws_us(*s, c, plan.Npix) < bestUs * behind) return kNumIgConfigs + ws;
     }
     // A second look where parts are chosen by time, and among layers in row orders that fill the chip unsplit: a tile that is expected ahead
-    // and asks for no more memory, so that callers who had room for the first one have it for this.  (The static workspace takes plans
+    // and asks for no more memory, so that callers who had room for the first one have it for this, and whose sums are no longer.  (The static workspace takes plans
     // past its size of the untuned tile alone: the first one stays where its plan is such a one.)
     const bool byTime = ig_parts_by_time(*s);
     long rows;
@@ -1267,6 +1343,9 @@ int ig_split_default_config(const fc_conv_shape *s) {
     const int first = best;
     for (int id = 0; id < 4; id++) {
         if (id == first || fc_igemm_make_plan(s, id, &plan) != FC_OK || plan.Wp_bytes + plan.table_bytes + plan.ws_bytes > room) continue;
+        const IgSplitCost &c = kIgSplitCost[id];
+        const long blocks = (long)(plan.K_pad / c.bm) * ((plan.Npix + c.bn - 1) / c.bn);
+        if (plan.split_k < parts && !ig_sums_in_levels(*s, {c.bm, c.bn}, blocks, plan.Kred_pad / 16, plan.split_k)) continue;
         const double us = ig_split_us(*s, id, plan, true);
         if (us < least) { least = us; best = id; }
     }
@@ -1323,10 +1402,9 @@ extern "C" int fc_igemm_default_config(const fc_conv_shape *s) {
     return best;
 }
 
-// The reduction of a plan, `stages` long, in at most `parts` of equal length, none of them empty.
+// The reduction of a plan in such parts.
 static void ig_set_parts(fc_igemm_plan &plan, int stages, int parts) {
-    const int per = (stages + parts - 1) / parts;
-    plan.split_k = (stages + per - 1) / per;
+    plan.split_k = ig_whole_parts(stages, parts);
     plan.ws_bytes = plan.split_k > 1 ? sizeof(float) * (size_t)plan.split_k * plan.shape.K * plan.Npix : 0;
 }
 
@@ -1383,11 +1461,15 @@ int ig_plan_to_fill(const fc_conv_shape *s, int config, fc_igemm_plan *plan) {
 }
 
 // In the number of parts, at least four stages each and no more than fill the chip, that is expected to take the least time where that is 6 %
-// less (ig_parts_by_time).
+// less (ig_parts_by_time), under tiles of 128 rows, which then add up in two levels.  Before / with this and the untuned tile after it, us, and
+// error against 64 bits: batch 32 256 -> 256 3x3/2 at 28x28, 128x64 tiles in 8 / 5 parts, 67.5 / 56.8, 1.05e-7 / 9.1e-8; 128 -> 128 3x3/2 at 56x56,
+// 128x64 in 4 / 128x128 in 2, 75.5 / 59.5, 9.8e-8 / 8.1e-8; 512 -> 512 3x3/2 at 14x14, 128x64 / 128x128 in 9, 69.9 / 58.3, 1.16e-7 / 1.05e-7.  The error
+// of none of 103 drawn layers that it changes is larger, and they take 0.90 of the time on average, 0.75 to 1.12 (496 -> 176 3x3 at 30x30 batch 4).
 void ig_expected_parts(fc_igemm_plan &plan) {
     const IgTileSize tile = kIgSplitTiles[plan.config];
     int config = 0;      // the one of the four costed tiles that runs
     while (kIgSplitCost[config].bm != tile.bm || kIgSplitCost[config].bn != tile.bn) config++;
+    if (tile.bm != 128) return;
     const int stages = plan.Kred_pad / 16, fill = plan.split_k;
     int best = fill;
     double bestUs = plan.shape.K > kMaxReduceChannels ? 1e300 : 0.94 * ig_split_us(plan.shape, config, plan, true);
@@ -1568,6 +1650,7 @@ static int igemm_run(fc_context *ctx, const fc_igemm_plan *plan, const float *x_
     p.divOW = fc_make_fastdiv((uint32_t)plan->OW);
     p.splitK = plan->split_k;
     p.stagesPerSplit = ((plan->Kred_pad / cfg.bk) + plan->split_k - 1) / plan->split_k;
+    p.sumStages = 0;
     p.ws = ws_dev;
     p.fastStore = s.K % tile.bm == 0 && 4.0 * s.N * s.K * plan->OH * plan->OW < 4294967296.0 &&
                   4.0 * plan->split_k * s.K * (double)plan->Npix < 4294967296.0 && ((uintptr_t)bias_dev & 15) == 0;

@@ -89,3 +89,35 @@ def test_plans_in_other_parts_of_the_reduction_run_and_inconsistent_ones_do_not(
                     lib.conv_implicit_gemm(plan, dx, Wp, tab, y, None, False, ws)
     finally:
         lib.release(mark)
+
+
+@pytest.mark.parametrize("shp,cfg,images", [
+    ((32, 256, 28, 28, 256, 3, 3, 2, 2, 1), 2, 3), ((32, 128, 56, 56, 128, 3, 3, 2, 2, 1), 0, 2), ((3, 144, 92, 92, 528, 3, 3, 2, 2, 0), 0, 1),
+    ((21, 256, 38, 38, 128, 5, 5, 2, 2, 2), 2, 4), ((12, 800, 10, 52, 128, 3, 3, 1, 1, 1), 0, 2), ((6, 144, 30, 30, 160, 3, 3, 2, 2, 1), 0, 4),
+])
+def test_a_reduction_in_fewer_parts_is_as_exact(lib, shp, cfg, images):
+    """Parts chosen by time against those that fill the chip, whose sums are shorter: root mean square of the differences from 64 bits, over
+    the first images."""
+    from test_dispatch import parts_that_fill
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=sum(shp))
+    truth = O.naive_conv_f64(O.shape(images, *shp[1:]), x[:images], w)
+    plan = lib.igemm_plan(cshape(s), cfg)
+    fill = parts_that_fill(plan, ((128, 128), None, (128, 64))[cfg])
+    assert plan.split_k < fill
+    mark = lib.mark()
+    try:
+        dx, dw, Wp, tab = lib.upload(x), lib.upload(w), lib.alloc(plan.Wp_bytes), lib.alloc(plan.table_bytes)
+        y, one, errors = lib.alloc(4 * s.K * plan.Npix), 4 * s.K * plan.Npix, []
+        ws = lib.alloc(fill * one)
+        lib.igemm_pack_filter(plan, dw, Wp, tab)
+        for parts in (plan.split_k, fill):
+            print("parts by time", shp, cfg, parts, flush=True)
+            plan.split_k, plan.ws_bytes = parts, parts * one if parts > 1 else 0
+            lib.conv_implicit_gemm(plan, dx, Wp, tab, y, None, False, ws)
+            errors.append(np.sqrt(np.mean((lib.download(y, (s.N,) + truth.shape[1:])[:images] - truth) ** 2)))
+    finally:
+        lib.release(mark)
+    # 100 000 values and more: each root mean square is known to about 1 / sqrt(2 * 100000), 0.3 %, of itself
+    print("rms", errors, flush=True)
+    assert truth.size >= 100000 and errors[0] <= 1.01 * errors[1], errors
