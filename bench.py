@@ -202,7 +202,7 @@ def takes_raw_filter_gemm(L, lay, filter_ready):
 def product_peak(L, lay, filter_ready=False):
     """Peak of the matrix instructions that form a layer's products."""
     if lay.algo == "im2col":
-        split = L.igemm_splits_products(lay.iplan)
+        split = L.igemm_on_bf16(lay.iplan)
     else:
         split = (lay.pipe != "onepass" and not takes_raw_filter_gemm(L, lay, filter_ready) and
                  L.wino_splits_products(lay.plan))
@@ -623,10 +623,8 @@ def run_workload(name, steps, warmup, o, detail=True, offline_filter=None):
         il = [l for l in layers if l.algo == "im2col"]
         def ig_key(l):
             g = L.igemm_configs()[l.iplan.config]
-            if g.waves_k > 1:
-                return ("igemm_wavesplit_kernel", N, l.C, l.K, l.H, l.ks, l.st, "%dx%dx%dw%d" % (g.bm, g.bn, g.bk, g.waves_k))
-            split = L.igemm_splits_products(l.iplan)
-            return ("igemm_split_kernel" if split else "igemm_conv_kernel", N, l.C, l.K, l.H, l.ks, l.st, tile_name(g))
+            tile = "%dx%dx%dw%d" % (g.bm, g.bn, g.bk, g.waves_k) if g.waves_k > 1 else tile_name(g)
+            return (L.igemm_kernel_name(l.iplan), N, l.C, l.K, l.H, l.ks, l.st, tile)
         keys = [ig_key(l) for l in il]
         tr = None
         if all(k in traffic for k in keys):

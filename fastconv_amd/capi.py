@@ -118,6 +118,8 @@ _ABI = {
     "fc_igemm_get_config": (C.c_int, [C.c_int, C.POINTER(GemmConfig)]),
     "fc_igemm_make_plan": (C.c_int, [C.POINTER(ConvShape), C.c_int, C.POINTER(IgemmPlan)]),
     "fc_igemm_splits_products": (C.c_int, [C.POINTER(IgemmPlan)]),
+    "fc_igemm_on_bf16": (C.c_int, [C.POINTER(IgemmPlan)]),
+    "fc_igemm_kernel_name": (C.c_char_p, [C.POINTER(IgemmPlan)]),
     "fc_igemm_pack_filter": (C.c_int, [_vp, C.POINTER(IgemmPlan), _vp, _vp, _vp]),
     "fc_conv_implicit_gemm": (C.c_int, [_vp, C.POINTER(IgemmPlan), _vp, _vp, _vp, _vp, C.c_int, _vp, _vp]),
     "fc_conv_implicit_gemm_static": (C.c_int, [_vp, C.POINTER(IgemmPlan), _vp, _vp, _vp, _vp, C.c_int, _vp]),
@@ -355,6 +357,14 @@ class Library:
         return bool(self.c.fc_igemm_splits_products(C.byref(plan)))
 
     # ---- Winograd stages
+
+    def igemm_on_bf16(self, plan):
+        """Whether the products are formed on the bf16 matrix cores, wherever the filter is split."""
+        return bool(self.c.fc_igemm_on_bf16(C.byref(plan)))
+
+    def igemm_kernel_name(self, plan):
+        return self.c.fc_igemm_kernel_name(C.byref(plan)).decode()
+
     def wino_filter_transform(self, plan, w, U):
         self._check(self.c.fc_wino_filter_transform(self.ctx, C.byref(plan), w, U))
 

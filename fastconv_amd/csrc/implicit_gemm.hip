@@ -1152,16 +1152,25 @@ void ig_before(const fc_conv_shape &s, int run, IgemmParams &p) {
 
 bool ig_sums_in_levels(const fc_conv_shape &s, IgTileSize tile, long blocks, int stages, int parts);
 
+// The kernels behind one plan of the LDS-tiled configurations.
+enum { IG_RUN_CONV, IG_RUN_SPLIT, IG_RUN_POINT_FEW, IG_RUN_SHORT };
+int ig_route(const fc_conv_shape &s, const fc_gemm_config &cfg, int K_pad, int splitK) {
+    if (splitK == 1 && ig_point_few(s) && K_pad == 64) return IG_RUN_POINT_FEW;
+    if (splitK == 1 && ig_short(s)) return IG_RUN_SHORT;
+    return ig_splits(s, cfg) ? IG_RUN_SPLIT : IG_RUN_CONV;
+}
+
 template <class TL>
 void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, IgemmParams &p) {
-    if (p.splitK == 1 && ig_point_few(s) && p.K_pad == 64) {
+    const int route = ig_route(s, cfg, p.K_pad, p.splitK);
+    if (route == IG_RUN_POINT_FEW) {
         typedef IgSplit<64, 128, 4> S;
         p.nKB = 1;
         p.nPB = (int)((p.Npix + S::BN_ - 1) / S::BN_);
         igemm_split_kernel<S, SP_POINT32><<<dim3((unsigned)((p.nPB + 7l) / 8 * 8)), dim3(S::THREADS), 0, ctx->stream>>>(p);
         return;
     }
-    if (p.splitK == 1 && ig_short(s)) {
+    if (route == IG_RUN_SHORT) {
         long rows;
         const int order = ig_split_order(s, &rows);
         ig_before(s, order == IG_ORDER_ROW8 ? 8 : 4, p);
@@ -1170,7 +1179,7 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
         return;
     }
     if constexpr (!std::is_void<typename IgSplitOf<TL>::type>::value) {
-        if (ig_splits(s, cfg)) {
+        if (route == IG_RUN_SPLIT) {
             typedef typename IgSplitOf<TL>::type S;
             const dim3 grid((unsigned)(((long)p.nKB * p.nPB + 7) / 8 * 8), (unsigned)p.splitK), block(S::THREADS);
             long rows;
@@ -1492,6 +1501,18 @@ extern "C" int fc_igemm_make_plan(const fc_conv_shape *s, int config, fc_igemm_p
 
 extern "C" int fc_igemm_splits_products(const fc_igemm_plan *plan) {
     return plan && plan->config >= 0 && plan->config < kNumIgConfigs && ig_splits(plan->shape, kIgConfigs[plan->config]) ? 1 : 0;
+}
+
+extern "C" const char *fc_igemm_kernel_name(const fc_igemm_plan *plan) {
+    if (!plan || plan->config < 0 || plan->config >= fc_igemm_num_configs()) return "";
+    if (plan->config >= kNumIgConfigs) return "igemm_wavesplit_kernel";
+    const int route = ig_route(plan->shape, kIgConfigs[plan->config], plan->K_pad, plan->split_k);
+    return route == IG_RUN_CONV ? "igemm_conv_kernel" : route == IG_RUN_SHORT ? "igemm_short_kernel" : "igemm_split_kernel";
+}
+
+extern "C" int fc_igemm_on_bf16(const fc_igemm_plan *plan) {
+    return plan && plan->config >= 0 && plan->config < kNumIgConfigs &&
+           ig_route(plan->shape, kIgConfigs[plan->config], plan->K_pad, plan->split_k) != IG_RUN_CONV ? 1 : 0;
 }
 
 static int ig_plan_check(fc_context *ctx, const fc_igemm_plan *plan) {

@@ -475,7 +475,7 @@ int main(int argc, char *argv[]) {
             fc_igemm_plan iplan;
             fc_wino_plan wplan;
             if (!wino) {
-                split = fc_igemm_make_plan(&shp, chosen_config, &iplan) == FC_OK && fc_igemm_splits_products(&iplan);
+                split = fc_igemm_make_plan(&shp, chosen_config, &iplan) == FC_OK && fc_igemm_on_bf16(&iplan);
             } else if (chosen_option != 0) {      // not the single kernel
                 if (chosen_option > 0) shp.N = chosen_option;
                 split = fc_wino_make_plan(&shp, chosen_config, &wplan) == FC_OK && fc_wino_gemm_splits_products(&wplan) &&

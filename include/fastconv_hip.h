@@ -380,6 +380,11 @@ int fc_igemm_make_plan(const fc_conv_shape *shape, int config, fc_igemm_plan *pl
  * their results are no less exact.)  Without room for the filter of split products, the configurations for which
  * this is 0 (32x64, and those with waves_k above 1) keep it in fp32 alone. */
 int fc_igemm_splits_products(const fc_igemm_plan *plan);
+/* 1 when the products of this plan are formed on the bf16 matrix cores, whether its filter is split when it is packed or in
+ * the kernel: the peak that a measured rate is a fraction of. */
+int fc_igemm_on_bf16(const fc_igemm_plan *plan);
+/* Name of the kernel that runs this plan, as a profiler shows it; "" for a plan that was not made. */
+const char *fc_igemm_kernel_name(const fc_igemm_plan *plan);
 
 /* Replaces pack_a_v2 (im2col/gemm_pack.cpp:192-260) as a one-time step. */
 int fc_igemm_pack_filter(fc_context *ctx, const fc_igemm_plan *plan, const float *w_dev,

@@ -202,3 +202,21 @@ def test_plans_that_the_static_workspace_takes(lib, geo, ws_mb, static):
         assert lib.fc_igemm_make_plan(C.byref(s), i, C.byref(plan)) == 0
         assert plan.ws_bytes <= capi.IGEMM_STATIC_WS_BYTES or i == untuned, i
         assert i != untuned or plan.ws_bytes <= ws_mb << 20
+
+
+@pytest.mark.parametrize("geo,kernel,bf16,split", [      # untuned plans
+    ((32, 3, 224, 224, 64, 3, 1, 1), "igemm_short_kernel", 1, 0), ((16, 18, 99, 99, 100, 1, 1, 0), "igemm_short_kernel", 1, 0),
+    ((3, 1, 223, 222, 200, 7, 2, 3), "igemm_short_kernel", 1, 1), ((32, 256, 56, 56, 64, 1, 1, 0), "igemm_split_kernel", 1, 0),
+    ((32, 256, 56, 56, 256, 1, 1, 0), "igemm_split_kernel", 1, 1), ((32, 256, 28, 28, 256, 3, 2, 1), "igemm_split_kernel", 1, 1),
+    ((16, 256, 56, 56, 64, 1, 1, 0), "igemm_conv_kernel", 0, 0), ((1, 256, 56, 56, 256, 3, 2, 1), "igemm_wavesplit_kernel", 0, 0),
+])
+def test_the_library_says_which_kernel_runs_a_plan_and_on_which_matrix_cores(lib, geo, kernel, bf16, split):
+    """What a rate is a fraction of: layers whose filter is split in the kernel run on the bf16 matrix cores too."""
+    n, c, h, w, k, ks, st, p = geo
+    s, plan = capi.ConvShape(n, c, h, w, k, ks, ks, st, st, p, p, p, p), capi.IgemmPlan()
+    assert lib.fc_igemm_make_plan(C.byref(s), lib.fc_igemm_default_config(C.byref(s)), C.byref(plan)) == 0
+    assert lib.fc_igemm_kernel_name(C.byref(plan)).decode() == kernel
+    assert (lib.fc_igemm_on_bf16(C.byref(plan)), lib.fc_igemm_splits_products(C.byref(plan))) == (bf16, split)
+    assert lib.fc_igemm_on_bf16(None) == 0 and lib.fc_igemm_kernel_name(None) == b""
+    plan.config = lib.fc_igemm_num_configs()
+    assert lib.fc_igemm_on_bf16(C.byref(plan)) == 0 and lib.fc_igemm_kernel_name(C.byref(plan)) == b""

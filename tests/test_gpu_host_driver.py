@@ -86,6 +86,17 @@ def test_json_line_names_the_peak_of_the_instructions_that_ran():
         assert j["split_products"] == 0 and j["gemm_frac_peak"] == pytest.approx(j["gemm_frac_mfma"], abs=2e-4)
 
 
+@pytest.mark.parametrize("args,split", [
+    (["-ic", "3", "-oc", "64", "-is", "224", "224", "-ks", "3", "3", "-ip", "1", "-n", "8"], 1),        # filter split in the kernel
+    (["-ic", "256", "-oc", "64", "-is", "56", "56", "-ks", "1", "1", "-n", "32"], 1),
+    (["-ic", "256", "-oc", "64", "-is", "56", "56", "-ks", "1", "1", "-n", "4"], 0),
+])
+def test_json_line_names_the_peak_of_filters_split_in_the_kernel(args, split):
+    j = _json_line(_run([_exe("conv_test"), "-i", "5", "-t", "16", "--check-images", "1", "--strict", "--json", "-a", "im2col"] + args))
+    assert j["split_products"] == split
+    assert j["gemm_frac_peak"] == pytest.approx(j["gemm_tflops"] / (2500 / 6 if split else 157.3), abs=2e-4)
+
+
 @pytest.mark.parametrize("variant", ["zc", "blocked"])
 @pytest.mark.parametrize("batch,C,H", [(64, 256, 56), (128, 256, 56), (64, 512, 28), (128, 512, 28), (64, 512, 14),
                                        (128, 512, 14)])
