@@ -1152,11 +1152,13 @@ void ig_before(const fc_conv_shape &s, int run, IgemmParams &p) {
 
 bool ig_sums_in_levels(const fc_conv_shape &s, IgTileSize tile, long blocks, int stages, int parts);
 
-// The kernels behind one plan of the LDS-tiled configurations.
+// The kernels behind the plans of the LDS-tiled configurations.  A layer that is left to the library goes to the kernels for short reductions
+// and for few output channels by the lines above; a caller's own configuration is the tile that it names, so that configurations can be
+// compared.
 enum { IG_RUN_CONV, IG_RUN_SPLIT, IG_RUN_POINT_FEW, IG_RUN_SHORT };
 int ig_route(const fc_conv_shape &s, const fc_gemm_config &cfg, int K_pad, int splitK) {
-    if (splitK == 1 && ig_point_few(s) && K_pad == 64) return IG_RUN_POINT_FEW;
-    if (splitK == 1 && ig_short(s)) return IG_RUN_SHORT;
+    const bool few = ig_point_few(s) && K_pad == 64;
+    if (splitK == 1 && (few || ig_short(s)) && cfg.id == fc_igemm_default_config(&s)) return few ? IG_RUN_POINT_FEW : IG_RUN_SHORT;
     return ig_splits(s, cfg) ? IG_RUN_SPLIT : IG_RUN_CONV;
 }
 

@@ -220,3 +220,19 @@ def test_the_library_says_which_kernel_runs_a_plan_and_on_which_matrix_cores(lib
     assert lib.fc_igemm_on_bf16(None) == 0 and lib.fc_igemm_kernel_name(None) == b""
     plan.config = lib.fc_igemm_num_configs()
     assert lib.fc_igemm_on_bf16(C.byref(plan)) == 0 and lib.fc_igemm_kernel_name(C.byref(plan)) == b""
+
+
+@pytest.mark.parametrize("geo", [(32, 3, 224, 224, 64, 3, 1, 1), (16, 18, 99, 99, 100, 1, 1, 0), (3, 1, 223, 222, 200, 7, 2, 3), (32, 256, 56, 56, 64, 1, 1, 0),
+                                 (6, 512, 128, 128, 64, 1, 1, 0)])
+def test_a_configuration_that_is_not_the_untuned_one_runs_its_own_tile(lib, geo):
+    """Tuning compares tiles: only the untuned plan of such layers goes to the kernels of short reductions and few output channels."""
+    n, c, h, w, k, ks, st, p = geo
+    s, plan = capi.ConvShape(n, c, h, w, k, ks, ks, st, st, p, p, p, p), capi.IgemmPlan()
+    untuned = lib.fc_igemm_default_config(C.byref(s))
+    for i in range(8):
+        assert lib.fc_igemm_make_plan(C.byref(s), i, C.byref(plan)) == 0
+        name, split = lib.fc_igemm_kernel_name(C.byref(plan)).decode(), lib.fc_igemm_splits_products(C.byref(plan))
+        if i == untuned:
+            assert name == "igemm_short_kernel" or (name == "igemm_split_kernel" and not split)
+        else:
+            assert name == ("igemm_split_kernel" if split else "igemm_conv_kernel"), i
