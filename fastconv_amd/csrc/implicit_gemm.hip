@@ -1126,8 +1126,12 @@ bool ig_short(const fc_conv_shape &s) {
     return ig_point(s) && s.K > 64 && rows <= 48 && (!ig_pointwise(s, 16, true) || (rows > 16 && yBytes >= 64e6));
 }
 
-// Pointwise layers of 33 to 64 output channels on many pixels: split from the fp32 filter.  Us, fp32 / this: 256 -> 64 at 56x56 batch 32
-// 38.7 / 36.3, 64 -> 64 12.5 / 12.2, 96 -> 64 at 102x102 batch 28 49.1 / 48.3; fewer pixels: 256 -> 64 at 200x200, one image, 16.5 / 17.8.
+// Pointwise layers of 33 to 64 output channels whose filter is packed in fp32, on three workgroups of 128 pixels a CU and more: split from
+// that filter.  Us, fp32 instructions / this: 256 -> 64 at 56x56 batch 32 38.7 / 36.3, 64 -> 64 12.5 / 12.2, 96 -> 64 at 102x102 batch 28 49.1 /
+// 48.3.  Eight layers of 88 000 to 97 000 pixels are 2 to 10 % faster too, sixteen of 50 000 to 82 000 between 4 % slower and 10 % faster
+// (256 -> 64 at 56x56 batch 16 20.2 / 18.4, batch 24 26.9 / 27.9), of 40 000 slower (64 -> 64 at 200x200 7.1 / 7.9, 512 -> 64 29.6 / 37.9).
+// A filter packed in parts is the faster one (this / packed in parts: 100 -> 64 at 102x102 batch 28 50.3 / 49.4, 900 -> 64 at 104x104 batch
+// 10 109 / 100, 200 -> 40 at 100x100 batch 12 31.4 / 29.4).
 bool ig_point_few(const fc_conv_shape &s) {
     return ig_four_pixels(s) && s.K > 32 && s.K <= 64 && s.C > 48 && (long)s.N * s.H * s.W >= 768 * 128 && 4l * s.N * s.C * s.H * s.W < (1l << 31);
 }
@@ -1157,7 +1161,7 @@ bool ig_sums_in_levels(const fc_conv_shape &s, IgTileSize tile, long blocks, int
 // compared.
 enum { IG_RUN_CONV, IG_RUN_SPLIT, IG_RUN_POINT_FEW, IG_RUN_SHORT };
 int ig_route(const fc_conv_shape &s, const fc_gemm_config &cfg, int K_pad, int splitK) {
-    const bool few = ig_point_few(s) && K_pad == 64;
+    const bool few = ig_point_few(s) && K_pad == 64 && !ig_splits(s, cfg);
     if (splitK == 1 && (few || ig_short(s)) && cfg.id == fc_igemm_default_config(&s)) return few ? IG_RUN_POINT_FEW : IG_RUN_SHORT;
     return ig_splits(s, cfg) ? IG_RUN_SPLIT : IG_RUN_CONV;
 }

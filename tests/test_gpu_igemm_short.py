@@ -74,3 +74,26 @@ def test_only_values_that_are_not_finite_are_formed_again(lib, shp, value):
     assert (np.abs(got[fin] - truth[fin]) <= (s.C * s.kh * s.kw + 40) * EPS * size[fin]).all()
     odd = hit & ~fin
     assert np.array_equal(got[odd], truth[odd].astype(np.float32), equal_nan=True)
+
+
+@pytest.mark.parametrize("shp", [SHAPES[12], SHAPES[13], (48, 72, 56, 56, 56, 1, 1, 1, 1, 0), (9, 68, 105, 104, 64, 1, 1, 1, 1, 0)])
+def test_a_filter_packed_in_parts_is_not_split_again_in_the_kernel(lib, shp):
+    """Few output channels, but channels that are no whole blocks or an odd image, so that the packed filter is split: the tile reads its
+    parts (and the fp32 filter before them only for values that are not finite)."""
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=5)
+    plan = lib.igemm_plan(cshape(s), lib.igemm_default_config(cshape(s)))
+    assert lib.igemm_splits_products(plan) and plan.split_k == 1 and lib.igemm_kernel_name(plan) == "igemm_split_kernel"
+    mark = lib.mark()
+    try:
+        dx, dw, Wp, tab = lib.upload(x), lib.upload(w), lib.alloc(plan.Wp_bytes), lib.alloc(plan.table_bytes)
+        y, got = lib.alloc(4 * s.K * plan.Npix), []
+        lib.igemm_pack_filter(plan, dw, Wp, tab)
+        for fp32 in (True, False):
+            if not fp32:
+                lib.fill_zero(Wp, 4 * plan.Kred_pad * plan.K_pad)
+            lib.conv_implicit_gemm(plan, dx, Wp, tab, y)
+            got.append(lib.download(y, (s.N, s.K, plan.OH, plan.OW)))
+    finally:
+        lib.release(mark)
+    assert np.abs(got[0]).max() > 0 and np.array_equal(got[0], got[1])
