@@ -1114,13 +1114,14 @@ int ig_order(const fc_conv_shape &s, const fc_gemm_config &c, long *rows) {
 // kernel does not read 16 bytes a lane, and those where two or three stages write 64 MB and more (32 -> 272 at 52x53 batch 36 55 / 36,
 // 48 -> 240 at 154x34 batch 18 47 / 32; below: 48 -> 256 at 56x56 batch 16 16.1 / 16.5, 32 -> 128 at 90x90 batch 8 10.3 / 11.1;
 // one stage: 16 -> 512 at 38x38 batch 62 49 / 57; four: 64 -> 304 at 111x111 batch 39 268 / 299).  With up to two stages and more
-// than 512 channels the pixels are read by many groups of workgroups: 2 -> 1005 at 165x91 batch 8 150 / 183.
+// than 512 channels the pixels are read by many groups of workgroups: 2 -> 1005 at 165x91 batch 8 150 / 183.  A single product is as exact on fp32
+// instructions as a float can be (2.52e-8 against 64 bits, this 2.58e-8; two products 3.12e-8 / 2.61e-8, 48 of them 1.24e-7 / 4.3e-8).
 bool ig_short(const fc_conv_shape &s) {
     long rows;
     const int order = ig_split_order(s, &rows);
     const long npix = (long)s.N * fc_out_dim(s.H, s.pt, s.pb, s.kh, s.sh) * fc_out_dim(s.W, s.pl, s.pr, s.kw, s.sw);
     const double yBytes = 4.0 * s.K * (double)npix;
-    if (rows > 64 || s.kh * s.kw > 64 || 4l * s.N * s.C * s.H * s.W >= (1l << 31) || yBytes > kShortNoStore) return false;
+    if ((long)s.C * s.kh * s.kw < 2 || rows > 64 || s.kh * s.kw > 64 || 4l * s.N * s.C * s.H * s.W >= (1l << 31) || yBytes > kShortNoStore) return false;
     if ((rows <= 32 && s.K > 512) || (npix + 31) / 32 * ((s.K + 31) / 32) < 25 * 256) return false;
     if (order != IG_ORDER_BLOCK) return s.K <= 48 || s.K > 64 || npix >= 32 * 8192;
     return ig_point(s) && s.K > 64 && rows <= 48 && (!ig_pointwise(s, 16, true) || (rows > 16 && yBytes >= 64e6));

@@ -97,3 +97,12 @@ def test_a_filter_packed_in_parts_is_not_split_again_in_the_kernel(lib, shp):
     finally:
         lib.release(mark)
     assert np.abs(got[0]).max() > 0 and np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("shp", [(8, 1, 112, 112, 100, 1, 1, 1, 1, 0), (9, 1, 140, 141, 40, 1, 1, 1, 1, 0), (16, 1, 223, 224, 70, 1, 1, 2, 2, 0)])
+def test_a_single_product_is_rounded_once(lib, shp):
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=3)
+    want = x[:, :, ::s.sh, ::s.sw] * w.reshape(1, s.K, 1, 1)
+    print("single product", shp, flush=True)
+    assert np.array_equal(lib.implicit_gemm_conv(cshape(s), x, w), want)
