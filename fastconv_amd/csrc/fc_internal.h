@@ -167,6 +167,16 @@ __device__ __forceinline__ uint32_t fc_div(uint32_t n, const fc_fastdiv f) {
     return (t + ((n - t) >> 1)) >> (f.shift - 1);
 }
 
+// Orders the LDS accesses of the lanes of one wavefront: the hardware executes a wavefront's LDS
+// instructions in order, so no instruction is needed, but the compiler must not move, merge or
+// drop them across this point (without it, it treats a lane's stores that the same lane never
+// reads back as dead).
+__device__ __forceinline__ void fc_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // A pointer that is the same for every lane, pinned to scalar registers: without the pin the
 // compiler turns a uniform base that advances in a loop into a 64-bit pointer per lane and pays
 // a vector add per access.

@@ -769,8 +769,10 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
 #pragma unroll
                 for (int h = 0; h < 2; h++)
                     *reinterpret_cast<floatx4 *>(turn + 256 * h + 4 * lane) = floatx4{raw[ni][4 * h], raw[ni][4 * h + 1], raw[ni][4 * h + 2], raw[ni][4 * h + 3]};
+                fc_wave_sync();      // lanes read what other lanes wrote
 #pragma unroll
                 for (int i = 0; i < 8; i++) raw[ni][i] = turn[(8 * lrow + i) * 32 + lcol];
+                fc_wave_sync();      // before the next block or stage is written
             }
         }
         if (ROW) {

@@ -152,8 +152,10 @@ __global__ __launch_bounds__(256, STAGES <= 2 ? 4 : STAGES == 3 ? 3 : 2) void ig
 #pragma unroll
                 for (int h = 0; h < 2; h++)
                     *reinterpret_cast<floatx4 *>(turn + 256 * h + 4 * lane) = floatx4{raw[s][4 * h], raw[s][4 * h + 1], raw[s][4 * h + 2], raw[s][4 * h + 3]};
+                fc_wave_sync();      // lanes read what other lanes wrote
 #pragma unroll
                 for (int i = 0; i < 8; i++) raw[s][i] = turn[(8 * lrow + i) * 32 + lcol];
+                fc_wave_sync();      // before the next stage is written
             }
             if constexpr (ROW) {
 #pragma unroll

@@ -155,16 +155,6 @@ __device__ __forceinline__ void column_products(const UReg<C> &u, const float (&
     for (int q = 0; q < 6; q++) r[q][j] = s[q];
 }
 
-// Orders the LDS accesses of the lanes of one wavefront: the hardware executes a wavefront's LDS
-// instructions in order, so no instruction is needed, but the compiler must not move, merge or
-// drop them across this point (without it, it treats a lane's stores that the same lane never
-// reads back as dead).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // What a lane needs to store its outputs.  Row stores: a row of the wavefront's tiles (6 floats
 // per lane) is written to the wavefront's LDS buffer and read back as pairs of floats in memory
 // order, so that a store instruction covers 512 contiguous bytes instead of 64 pieces of 8; pair
@@ -226,11 +216,11 @@ __device__ __forceinline__ void sc_step(const SmallCParams &p, const UReg<C> &u,
             for (int s = 0; s < 6; s++) o[s] = __builtin_elementwise_maximum(o[s], floorv);
             if (ROWST) {
                 float2 *sw = reinterpret_cast<float2 *>(st.stage) + lane * 3;
-                wave_sync();   // the previous row has been read by every lane
+                fc_wave_sync();   // the previous row has been read by every lane
                 sw[0] = make_float2(o[0], o[1]);
                 sw[1] = make_float2(o[2], o[3]);
                 sw[2] = make_float2(o[4], o[5]);
-                wave_sync();   // lanes read what other lanes wrote
+                fc_wave_sync();   // lanes read what other lanes wrote
                 const float2 *ld = reinterpret_cast<const float2 *>(st.stage) + lane;
                 const float2 a0 = ld[0], a1 = ld[64], a2 = ld[128];
                 float *yrow = yk + (size_t)q * p.OW;
