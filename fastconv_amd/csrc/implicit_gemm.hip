@@ -836,8 +836,7 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
     floatx16 acc[MI][NI], small[MI][NI];
     fc_zero<MI, NI>(acc);
     fc_zero<MI, NI>(small);
-    // more: a stage follows
-    // column: of its window row, where three stages share their loads; fetch: the next stage's columns are not in registers yet
+    // more: a stage follows; column: of its window row, where three stages share their loads
     auto stage = [&](const int s, const bool more, auto readAgain, auto column) __attribute__((always_inline)) {
         const int buf = (s - sBegin) & 1;
         if constexpr (MODE == SP_TRI) {
@@ -965,7 +964,7 @@ __device__ __forceinline__ void ig_split_tile(const IgemmParams &p, const int kb
 }
 
 template <class S, int MODE, bool LEVELS = false>
-__global__ __launch_bounds__(S::THREADS, (MODE == SP_ROW4 || MODE == SP_INSIDE || MODE == SP_TRI) && S::MIN_WAVES > 3 ? 3 : S::MIN_WAVES) void igemm_split_kernel(const IgemmParams p) {
+__global__ __launch_bounds__(S::THREADS, (MODE == SP_ROW4 || MODE == SP_INSIDE) && S::MIN_WAVES > 3 ? 3 : S::MIN_WAVES) void igemm_split_kernel(const IgemmParams p) {
     __shared__ fc_uintx4 smem[S::LDS_WORDS + (LEVELS ? S::THREADS / 64 * 256 : 0) + (MODE == SP_POINT || MODE == SP_POINT32 ? S::THREADS / 64 * 128 : 0)];
     int kb, pb;
     if (!ig_decode_tile(p, &kb, &pb)) return;
@@ -1194,31 +1193,34 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
             long rows;
             const int order = ig_order(s, cfg, &rows);
             ig_before(s, order == IG_ORDER_ROW8 ? 8 : 4, p);
-            if constexpr (S::BM_ == 128) {
+            auto run = [&](auto mode, auto levels) { igemm_split_kernel<S, decltype(mode)::value, decltype(levels)::value><<<grid, block, 0, ctx->stream>>>(p); };
+            constexpr std::false_type one{};
+            if (order == IG_ORDER_ROW8) return run(std::integral_constant<int, SP_ROW8>(), one);
+            if (order == IG_ORDER_ROW4) return run(std::integral_constant<int, SP_ROW4>(), one);
+            if constexpr (S::BM_ == 64) {
+                // two 16-byte loads a stage and wavefront in place of eight of 4 bytes, whole layers of batch 32, us: 256 -> 64 at
+                // 56x56 28.2 / 26.0, 1024 -> 256 at 14x14 34.7 / 32.9, 112 -> 208 at 68x68 batch 4 13.4 / 12.3.  Tiles of 128 rows
+                // load half as often for their products: 64 -> 256 at 56x56 30.6 / 32.3, 144 -> 112 at 130x130 batch 35 173 / 178.  Nor where
+                // few wavefronts a CU walk a long reduction, whose every stage waits for the turn: 976 -> 96 at 40x77 batch 8, 61 stages, 770
+                // workgroups, 58.9 / 61.2, 720 -> 96 at 116x116 batch 2 39.2 / 42.8; 944 -> 80 at 164x164 batch 2, 1682, 88.5 / 82.7.
+                const long pairs = (long)p.nKB * p.nPB * p.splitK * (S::THREADS / 128);
+                if (ig_four_pixels(s) && (p.stagesPerSplit <= 40 || pairs >= 1024)) return run(std::integral_constant<int, SP_POINT>(), one);
+            } else {
                 const int stages = p.Kred_pad / 16;
                 if (ig_sums_in_levels(s, {S::BM_, S::BN_}, (long)p.nKB * p.nPB, stages, p.splitK)) {
+                    constexpr std::true_type two{};
                     p.sumStages = ig_sum_stages(stages);
-                    if (ig_inside(s, 16)) igemm_split_kernel<S, SP_INSIDE, true><<<grid, block, 0, ctx->stream>>>(p);
-                    else igemm_split_kernel<S, SP_MASKED, true><<<grid, block, 0, ctx->stream>>>(p);
-                    return;
+                    if (ig_inside(s, 16)) return run(std::integral_constant<int, SP_INSIDE>(), two);
+                    return run(std::integral_constant<int, SP_MASKED>(), two);
                 }
+                // strided layers under tiles of 128 rows, batch 32, us: 128 -> 128 at 56x56 76.0 / 71.9, 256 -> 256 at 28x28 69.6 / 67.0,
+                // 32 -> 448 at 100x100 batch 22 107.8 / 103.6.  (Stride 1 loads find their lines in the cache: 256 -> 256 at 56x56 batch 8
+                // 192 / 197; tiles of 64 rows lose a wavefront a SIMD to the registers: 64 -> 64 at 56x56 50.8 / 57.2)
+                if (s.kw == 3 && s.sw > 1 && s.pl <= 1) return run(std::integral_constant<int, SP_TRI>(), one);
             }
-            if (order == IG_ORDER_ROW8) igemm_split_kernel<S, SP_ROW8><<<grid, block, 0, ctx->stream>>>(p);
-            else if (order == IG_ORDER_ROW4) igemm_split_kernel<S, SP_ROW4><<<grid, block, 0, ctx->stream>>>(p);
-            // two 16-byte loads a stage and wavefront in place of eight of 4 bytes, whole layers of batch 32, us: 256 -> 64 at
-            // 56x56 28.2 / 26.0, 1024 -> 256 at 14x14 34.7 / 32.9, 112 -> 208 at 68x68 batch 4 13.4 / 12.3.  Tiles of 128 rows
-            // load half as often for their products: 64 -> 256 at 56x56 30.6 / 32.3, 144 -> 112 at 130x130 batch 35 173 / 178
-            // (also where few wavefronts a CU walk a long reduction, whose every stage waits for the turn: 976 -> 96 at 40x77 batch 8, 61
-            // stages, 770 workgroups, 58.9 / 61.2, 720 -> 96 at 116x116 batch 2 39.2 / 42.8; 944 -> 80 at 164x164 batch 2, 1682, 88.5 / 82.7)
-            else if (S::BM_ == 64 && ig_four_pixels(s) && (p.stagesPerSplit <= 40 || (long)p.nKB * p.nPB * p.splitK * (S::THREADS / 128) >= 1024)) igemm_split_kernel<S, SP_POINT><<<grid, block, 0, ctx->stream>>>(p);
-            // strided layers under tiles of 128 rows, batch 32, us: 128 -> 128 at 56x56 76.0 / 71.9, 256 -> 256 at 28x28 69.6 / 67.0,
-            // 32 -> 448 at 100x100 batch 22 107.8 / 103.6.  (Stride 1 loads find their lines in the cache: 256 -> 256 at 56x56 batch 8
-            // 192 / 197; tiles of 64 rows lose a wavefront a SIMD to the registers: 64 -> 64 at 56x56 50.8 / 57.2)
-            else if (S::BM_ == 128 && s.kw == 3 && s.sw > 1 && s.pl <= 1) igemm_split_kernel<S, SP_TRI><<<grid, block, 0, ctx->stream>>>(p);
-            else if (s.C % 16 != 0) igemm_split_kernel<S, SP_PAD><<<grid, block, 0, ctx->stream>>>(p);
-            else if (ig_inside(s, 16)) igemm_split_kernel<S, SP_INSIDE><<<grid, block, 0, ctx->stream>>>(p);
-            else igemm_split_kernel<S, SP_MASKED><<<grid, block, 0, ctx->stream>>>(p);
-            return;
+            if (s.C % 16 != 0) return run(std::integral_constant<int, SP_PAD>(), one);
+            if (ig_inside(s, 16)) return run(std::integral_constant<int, SP_INSIDE>(), one);
+            return run(std::integral_constant<int, SP_MASKED>(), one);
         }
     }
     const bool x16 = ((uintptr_t)p.x & 15) == 0;

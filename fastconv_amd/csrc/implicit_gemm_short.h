@@ -248,9 +248,11 @@ static inline size_t ig_short_lds(int stages, int blocks, int mode) { return (si
 
 template <int STAGES>
 static void ig_short_launch_mode(fc_context *ctx, int mode, dim3 grid, size_t lds, const IgemmParams &p, const IgShortParams &q) {
-    if (mode == SP_POINT) igemm_short_kernel<STAGES, SP_POINT><<<grid, dim3(256), lds, ctx->stream>>>(p, q);
-    else if (mode == SP_PAD) igemm_short_kernel<STAGES, SP_PAD><<<grid, dim3(256), lds, ctx->stream>>>(p, q);
-    else if (mode == SP_ROW8) igemm_short_kernel<STAGES, SP_ROW8><<<grid, dim3(256), lds, ctx->stream>>>(p, q);
+    if constexpr (STAGES <= 3) {      // (pointwise layers have no more: ig_short)
+        if (mode == SP_POINT) return igemm_short_kernel<STAGES, SP_POINT><<<grid, dim3(256), lds, ctx->stream>>>(p, q);
+        if (mode == SP_PAD) return igemm_short_kernel<STAGES, SP_PAD><<<grid, dim3(256), lds, ctx->stream>>>(p, q);
+    }
+    if (mode == SP_ROW8) igemm_short_kernel<STAGES, SP_ROW8><<<grid, dim3(256), lds, ctx->stream>>>(p, q);
     else igemm_short_kernel<STAGES, SP_ROW4><<<grid, dim3(256), lds, ctx->stream>>>(p, q);
 }
 

@@ -236,3 +236,15 @@ def test_a_configuration_that_is_not_the_untuned_one_runs_its_own_tile(lib, geo)
             assert name == "igemm_short_kernel" or (name == "igemm_split_kernel" and not split)
         else:
             assert name == ("igemm_split_kernel" if split else "igemm_conv_kernel"), i
+
+
+def test_no_kernel_is_compiled_that_nothing_launches():
+    """Tile and mode of igemm_split_kernel, stages and mode of igemm_short_kernel, as their names are mangled (modes: 2
+    channels missing, 4 runs of four columns, 5 16-byte pointwise columns, 7 12-byte window rows)."""
+    built = open(capi.LIB_PATH, "rb").read()
+    for rows, cols, waves in ((64, 64, 2), (64, 128, 4), (128, 64, 2), (128, 128, 4)):
+        tile = b"IgSplitILi%dELi%dELi%dEEELi" % (rows, cols, waves)
+        assert tile + b"2E" in built
+        assert (tile + b"5E" in built) == (rows == 64) and (tile + b"7E" in built) == (rows == 128)
+    assert b"igemm_short_kernelILi4ELi4E" in built and b"igemm_short_kernelILi3ELi5E" in built
+    assert b"igemm_short_kernelILi4ELi5E" not in built and b"igemm_short_kernelILi4ELi2E" not in built
