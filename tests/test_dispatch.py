@@ -139,11 +139,12 @@ def test_untuned_plans_of_very_many_channels_can_run(lib, k):
     assert plan.split_k == 1 or k <= 65535
 
 
-@pytest.mark.parametrize("geo,parts", [
-    ((32, 256, 28, 28, 256, 3, 2, 1), 4), ((32, 128, 56, 56, 128, 3, 2, 1), 2), ((32, 512, 14, 14, 512, 3, 2, 1), 9),
+@pytest.mark.parametrize("geo,parts,untuned", [
+    ((32, 256, 28, 28, 256, 3, 2, 1), 4, (2, 5)), ((32, 128, 56, 56, 128, 3, 2, 1), 2, (0, 2)), ((32, 512, 14, 14, 512, 3, 2, 1), 9, (0, 9)),
 ])
-def test_parts_of_a_reduction_put_the_large_tiles_on_the_chip_at_once(lib, geo, parts):
-    """128x128 tiles, two a compute unit: at most 512 workgroups as launched, in whole eights of tiles, and more than half of that."""
+def test_parts_of_a_reduction_put_the_large_tiles_on_the_chip_at_once(lib, geo, parts, untuned):
+    """128x128 tiles, two a compute unit: at most 512 workgroups as launched, in whole eights of tiles, and more than half of that.  Left to
+    the library the first layer runs in tiles of 128x64, four a compute unit, all on the chip at once too."""
     n, c, h, w, k, ks, st, p = geo
     s, plan = capi.ConvShape(n, c, h, w, k, ks, ks, st, st, p, p, p, p), capi.IgemmPlan()
     assert lib.fc_igemm_make_plan(C.byref(s), 0, C.byref(plan)) == 0
@@ -151,6 +152,11 @@ def test_parts_of_a_reduction_put_the_large_tiles_on_the_chip_at_once(lib, geo, 
     assert plan.split_k == parts and 256 < -(-tiles // 8) * 8 * plan.split_k <= 512
     stages = plan.Kred_pad // 16
     assert -(-stages // -(-stages // parts)) == parts and plan.ws_bytes == 4 * parts * k * plan.Npix      # no part is empty
+    assert lib.fc_igemm_make_plan(C.byref(s), lib.fc_igemm_default_config(C.byref(s)), C.byref(plan)) == 0
+    assert (plan.config, plan.split_k) == untuned
+    if untuned[0] == 2:
+        tiles = (plan.K_pad // 128) * -(-plan.Npix // 64)
+        assert 512 < -(-tiles // 8) * 8 * plan.split_k <= 1024
 
 
 @pytest.mark.parametrize("geo", [

@@ -1,5 +1,5 @@
 """Implicit GEMM on split products: columns read by wider loads (window rows of three taps, four pixels of a pointwise layer), at the
-edges of the image, of the tensor, of the channels and of the parts of a split reduction."""
+edges of the image, of the tensor, of the channels and of the parts of a split reduction; parts chosen by time and their sums."""
 import numpy as np
 import pytest
 
@@ -38,11 +38,22 @@ POINTWISE = [      # tiles of 64 rows
     (2, 100, 14, 14, 65, 1, 1, 1, 1, 0),     # four of the last eight channels missing
     (5, 64, 2, 2, 72, 1, 1, 1, 1, 0),        # images of one group of pixels
     (1, 49, 1, 3, 70, 1, 1, 1, 1, 0),        # fewer pixels than a group
-    (2, 720, 4, 4, 66, 1, 1, 1, 1, 0),       # 45 stages of few wavefronts: read a pixel a lane
+    (2, 720, 4, 4, 66, 1, 1, 1, 1, 0),       # 45 stages in parts of five
+    (2, 720, 92, 92, 66, 1, 1, 1, 1, 0),     # 45 stages of few wavefronts: 64x64 tiles read a pixel a lane
+]
+LEVELS = [       # tiles of 128 rows cut by time: sums in two levels, the second begun within a part
+    (32, 64, 28, 28, 128, 3, 3, 2, 2, 1),
+    (6, 144, 92, 91, 272, 3, 3, 2, 2, 0),    # no padding, rows past the last channel
 ]
 
 
-@pytest.mark.parametrize("shp,configs", [(s, (0, 2)) for s in WINDOWS] + [(s, (1, 3)) for s in POINTWISE])
+def test_the_long_reduction_of_few_wavefronts_is_one(lib):
+    s = O.shape(*POINTWISE[-1])
+    plan = lib.igemm_plan(cshape(s), 3)
+    assert -(-(plan.Kred_pad // 16) // plan.split_k) > 40 and (plan.K_pad // 64) * -(-plan.Npix // 64) * plan.split_k < 1024
+
+
+@pytest.mark.parametrize("shp,configs", [(s, (0, 2)) for s in WINDOWS + LEVELS] + [(s, (1, 3)) for s in POINTWISE])
 def test_columns_against_fp64(lib, shp, configs):
     s = O.shape(*shp)
     x, w = O.make_inputs(s, seed=sum(shp))
@@ -55,6 +66,38 @@ def test_columns_against_fp64(lib, shp, configs):
     for cfg in configs:
         print("columns", shp, cfg, flush=True)
         assert (np.abs(lib.implicit_gemm_conv(cshape(s), x, w, bias, False, config=cfg) - truth) <= tol).all(), cfg
+        assert (np.abs(lib.implicit_gemm_conv(cshape(s), x, w, bias, True, config=cfg) - np.maximum(truth, 0.0)) <= tol).all(), cfg
+
+
+@pytest.mark.parametrize("shp", WINDOWS)
+def test_window_rows_give_the_bits_of_single_taps(lib, shp):
+    """Tiles of 64 rows read a tap at a time and add up the same products in the same order, in as many parts."""
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=sum(shp))
+    parts = [lib.igemm_plan(cshape(s), cfg).split_k for cfg in range(4)]
+    assert len(set(parts)) == 1
+    print("window rows", shp, parts, flush=True)
+    a, b, c, d = (lib.implicit_gemm_conv(cshape(s), x, w, config=cfg) for cfg in range(4))
+    assert np.abs(a).max() > 0 and np.array_equal(a, b) and np.array_equal(c, d) and np.array_equal(a, c)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3e38])
+@pytest.mark.parametrize("shp,cfg", [(WINDOWS[0], 0), (WINDOWS[4], 2), (WINDOWS[5], 2), (LEVELS[0], 2), (LEVELS[1], 0), (POINTWISE[1], 1), (POINTWISE[2], 3)])
+def test_only_values_that_are_not_finite_are_formed_again(lib, shp, cfg, value):
+    s = O.shape(*shp)
+    x, w = O.make_inputs(s, seed=11)
+    bad = x.copy()
+    bad[-1, s.C - 1, 4, 5] = value
+    truth, size = O.naive_conv_f64(s, bad, w), O.naive_conv_f64(s, np.abs(bad), np.abs(w))
+    hit = O.naive_conv_f64(s, (bad != x).astype(np.float32), np.ones_like(w)) > 0
+    print("poison", shp, cfg, value, flush=True)
+    clean, got = (lib.implicit_gemm_conv(cshape(s), v, w, config=cfg) for v in (x, bad))
+    assert hit.any() and np.array_equal(got[~hit], clean[~hit])
+    fin = hit & np.isfinite(truth) & np.isfinite(size)
+    # products and the sums of them and of at most 32 parts
+    assert (np.abs(got[fin] - truth[fin]) <= (s.C * s.kh * s.kw + 72) * EPS * size[fin]).all()
+    odd = hit & ~fin
+    assert np.array_equal(got[odd], truth[odd].astype(np.float32), equal_nan=True)
 
 
 @pytest.mark.parametrize("shp", [(4, 64, 15, 15, 256, 3, 3, 2, 2, 1), (2, 208, 9, 9, 129, 3, 3, 2, 2, 1)])

@@ -27,8 +27,8 @@ def cshape(s):
 SHAPES = [
     (1, 1, 140, 143, 321, 3, 3, 1, 1, 1),    # one channel, a part of a block of channels and of pixels
     (9, 3, 150, 151, 33, 3, 3, 1, 1, 1),     # runs of four, windows before x, more blocks than wavefronts: every one walks
-    (2, 4, 89, 88, 1030, 3, 3, 2, 2, 1),     # many groups of channels
-    (3, 5, 101, 103, 100, 3, 3, 1, 1, 0),    # four stages, as many rows as are padded
+    (4, 4, 89, 88, 1030, 3, 3, 2, 2, 1),     # many groups of channels
+    (6, 5, 101, 103, 100, 3, 3, 1, 1, 0),    # four stages in runs of four, as many rows as are padded
     (3, 1, 223, 222, 200, 7, 7, 2, 2, 3),    # runs of eight
     (8, 1, 99, 98, 97, 5, 5, 1, 1, 2),       # runs of eight in three stages, the last one half filled
     (1, 18, 231, 297, 85, 1, 1, 1, 1, 0),    # four pixels a lane, odd image
@@ -36,15 +36,30 @@ SHAPES = [
     (3, 48, 131, 133, 129, 1, 1, 1, 1, 0),   # images that are no whole groups of four pixels
     (2, 16, 101, 101, 330, 1, 1, 1, 1, 0),   # one stage, many channels
     (2, 32, 130, 130, 500, 1, 1, 1, 1, 0),   # 64 MB of y
-    (5, 64, 140, 141, 64, 1, 1, 1, 1, 0),    # 64 channels, split in the kernel from the fp32 filter
-    (2, 100, 223, 224, 40, 1, 1, 1, 1, 0),   # the same with 32 of its rows unused in part, channels past the last
-    (1, 52, 333, 331, 33, 1, 1, 1, 1, 0),
+]
+FEW = [      # of 33 to 64 output channels
+    (5, 64, 140, 141, 64, 1, 1, 1, 1, 0),    # split in the kernel from the fp32 filter
+    (2, 112, 223, 224, 40, 1, 1, 1, 1, 0),   # the same with 32 of its rows unused in part
+    (1, 64, 332, 331, 33, 1, 1, 1, 1, 0),    # and all but one of them
+]
+PACKED = [   # the same, of which the filter is packed in parts
+    (2, 100, 223, 224, 40, 1, 1, 1, 1, 0),   # channels past the last
+    (1, 52, 333, 331, 33, 1, 1, 1, 1, 0),    # images that are no whole groups of four pixels
 ]
 
 
-@pytest.mark.parametrize("shp", SHAPES)
+def kernel_of(lib, s):
+    plan = lib.igemm_plan(cshape(s), lib.igemm_default_config(cshape(s)))
+    return lib.igemm_kernel_name(plan), lib.igemm_splits_products(plan)
+
+
+@pytest.mark.parametrize("shp", SHAPES + FEW + PACKED)
 def test_short_reductions_against_fp64(lib, shp):
     s = O.shape(*shp)
+    if shp in SHAPES:
+        assert kernel_of(lib, s)[0] == "igemm_short_kernel"
+    else:
+        assert kernel_of(lib, s) == ("igemm_split_kernel", shp in PACKED)
     x, w = O.make_inputs(s, seed=sum(shp))
     bias = O.rng_uniform(3, (s.K,))
     # magnitudes over 2^40, as a product's rounding must not depend on the scale of its row
@@ -59,7 +74,7 @@ def test_short_reductions_against_fp64(lib, shp):
 
 
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3e38, 1e30])
-@pytest.mark.parametrize("shp", [SHAPES[1], SHAPES[4], SHAPES[7], SHAPES[8], SHAPES[12]])
+@pytest.mark.parametrize("shp", [SHAPES[1], SHAPES[3], SHAPES[4], SHAPES[7], SHAPES[8], FEW[1], PACKED[0]])
 def test_only_values_that_are_not_finite_are_formed_again(lib, shp, value):
     s = O.shape(*shp)
     x, w = O.make_inputs(s, seed=11)
@@ -76,7 +91,7 @@ def test_only_values_that_are_not_finite_are_formed_again(lib, shp, value):
     assert np.array_equal(got[odd], truth[odd].astype(np.float32), equal_nan=True)
 
 
-@pytest.mark.parametrize("shp", [SHAPES[12], SHAPES[13], (48, 72, 56, 56, 56, 1, 1, 1, 1, 0), (9, 68, 105, 104, 64, 1, 1, 1, 1, 0)])
+@pytest.mark.parametrize("shp", PACKED + [(48, 72, 56, 56, 56, 1, 1, 1, 1, 0), (9, 68, 106, 104, 64, 1, 1, 1, 1, 0)])
 def test_a_filter_packed_in_parts_is_not_split_again_in_the_kernel(lib, shp):
     """Few output channels, but channels that are no whole blocks or an odd image, so that the packed filter is split: the tile reads its
     parts (and the fp32 filter before them only for values that are not finite)."""
