@@ -1,6 +1,7 @@
 """The measurement summaries under profiles/ say which tree they were taken at, and the one bench.py reads
 numbers from (measured HBM traffic per GEMM launch) must have been taken with the GEMM kernels of this tree."""
 import os
+import re
 
 from fastconv_amd import provenance
 
@@ -28,10 +29,21 @@ def test_digest_follows_the_sources():
 
 
 def test_traffic_summary_was_measured_on_the_gemm_kernels_of_this_tree():
-    """When wino_gemm.hip or implicit_gemm.hip change, profiles/gemm_hbm_traffic_pmc.txt has to be taken again
+    """When the sources of the GEMM kernels change, headers included, profiles/gemm_hbm_traffic_pmc.txt has to be taken again
     (its commands are in its header); until then bench.py reports roofline.traffic as null."""
     path = os.path.join(PROFILES, "gemm_hbm_traffic_pmc.txt")
     commit, _, sources_digest, sources = provenance.parse(path)
     assert sources and sources_digest
+    # the files of the kernels it names, with the headers that they include
+    text = {n: open(os.path.join(provenance.CSRC, n)).read() for n in os.listdir(provenance.CSRC) if n.endswith((".hip", ".h"))}
+    kernels = set(re.findall(r"^traffic kernel=(\w+)", open(path).read(), re.M))
+    need = {n for n in text for k in kernels if n.endswith(".hip") and re.search(r"__global__[^;{]*\b%s\(" % k, text[n])}
+    assert len(kernels) >= 3 and len(need) == len(kernels)
+    while True:
+        more = {h for n in need for h in re.findall(r'#include "(\w+\.h)"', text[n]) if h in text} - need
+        if not more:
+            break
+        need |= more
+    assert need <= set(sources), sorted(need - set(sources))
     assert provenance.sources_current(path), (
         "%s changed since commit %s: measure the HBM traffic of the GEMM kernels again" % (", ".join(sources), commit))
