@@ -977,7 +977,7 @@ def test_untuned_tile_choice_is_close_to_the_best_of_a_search(lib, geo):
     (fc_wino_gemm_default_config for the staged Winograd pipeline, fc_igemm_default_config for the implicit GEMM)
     takes at most 10 % (Winograd) or 15 % (implicit GEMM, whose search has 25 configurations and 10-20 us launches;
     measured 0-9 %) longer than the best configuration of a search over all of them (20 launches back to back, best
-    of three rounds)."""
+    of three rounds, and of three more in turn for the two that are compared)."""
     N, C, H, W, K, ks, st, pad = geo
     s = O.shape(N, C, H, W, K, ks, ks, st, st, pad)
     cs = cshape(s)
@@ -987,33 +987,47 @@ def test_untuned_tile_choice_is_close_to_the_best_of_a_search(lib, geo):
         dx, dw = lib.upload(x), lib.upload(w)
         oh, ow = O.out_hw(s)
         y = lib.alloc(4 * N * K * oh * ow)
-        if ks == 3 and st == 1:
-            times = {}
-            for g in lib.wino_configs():
-                plan = lib.wino_plan(cs, g.id)
-                if plan.K_pad > 2 * K and g.bm > 32:
-                    continue
-                m2 = lib.mark()
-                U, V, M = lib.alloc(plan.U_bytes), lib.alloc(plan.V_bytes), lib.alloc(plan.M_bytes)
-                times[g.id] = _launch_us(lib, lambda: lib.wino_forward(plan, dx, dw, U, V, M, y))
-                lib.release(m2)
-            d = lib.wino_default_config(cs)
-            announce("winograd", geo, "untuned config", d, "%.1f us" % times[d], "best", min(times, key=times.get), "%.1f us" % min(times.values()))
-            assert times[d] <= 1.10 * min(times.values()), (geo, times)
-        times = {}
-        for g in lib.igemm_configs():
-            try:
-                plan = lib.igemm_plan(cs, g.id)
-            except Exception:
-                continue
+
+        def wino_us(i):
+            plan = lib.wino_plan(cs, i)
+            m2 = lib.mark()
+            U, V, M = lib.alloc(plan.U_bytes), lib.alloc(plan.V_bytes), lib.alloc(plan.M_bytes)
+            us = _launch_us(lib, lambda: lib.wino_forward(plan, dx, dw, U, V, M, y))
+            lib.release(m2)
+            return us
+
+        def igemm_us(i):
+            plan = lib.igemm_plan(cs, i)
             m2 = lib.mark()
             Wp, tab = lib.alloc(plan.Wp_bytes), lib.alloc(plan.table_bytes)
             ws = lib.alloc(plan.ws_bytes) if plan.ws_bytes else None
             lib.igemm_pack_filter(plan, dw, Wp, tab)
-            times[g.id] = _launch_us(lib, lambda: lib.conv_implicit_gemm(plan, dx, Wp, tab, y, ws=ws))
+            us = _launch_us(lib, lambda: lib.conv_implicit_gemm(plan, dx, Wp, tab, y, ws=ws))
             lib.release(m2)
+            return us
+
+        def against_best(times, d, us):
+            """Both of them again in turn: the search times its configurations one after another, at clocks that move by a tenth."""
+            best = min(times, key=times.get)
+            for _ in range(3):
+                for i in (d, best):
+                    times[i] = min(times[i], us(i))
+            return "untuned config", d, "%.1f us" % times[d], "best", best, "%.1f us" % min(times.values())
+
+        if ks == 3 and st == 1:
+            times = {g.id: wino_us(g.id) for g in lib.wino_configs() if g.bm <= 32 or lib.wino_plan(cs, g.id).K_pad <= 2 * K}
+            d = lib.wino_default_config(cs)
+            announce("winograd", geo, *against_best(times, d, wino_us))
+            assert times[d] <= 1.10 * min(times.values()), (geo, times)
+        times = {}
+        for g in lib.igemm_configs():
+            try:
+                lib.igemm_plan(cs, g.id)
+            except Exception:
+                continue
+            times[g.id] = igemm_us(g.id)
         d = lib.igemm_default_config(cs)
-        announce("implicit gemm", geo, "untuned config", d, "%.1f us" % times[d], "best", min(times, key=times.get), "%.1f us" % min(times.values()))
+        announce("implicit gemm", geo, *against_best(times, d, igemm_us))
         assert times[d] <= 1.15 * min(times.values()), (geo, times)
     finally:
         lib.release(mark)
