@@ -1065,12 +1065,11 @@ bool ig_inside(const fc_conv_shape &s, int bk) {
     return s.pt == 0 && s.pl == 0 && (OH - 1) * s.sh + s.kh <= s.H && (OW - 1) * s.sw + s.kw <= s.W && (s.C * s.kh * s.kw) % bk == 0;
 }
 
-// Whether the products run on the bf16 matrix cores (a pointwise layer is a block whose only tap is inside): for inputs below
-// 2 GiB, but not for pointwise layers of up to 64 output channels, whose x the fp32 kernel reads 16 bytes a lane, nor for
-// reductions of two or three stages.  Both lines were drawn when this kernel split both operands; at the kernel as it is, us,
-// best tile on fp32 / on split products, batch 32: 1x1 256 -> 64 at 56x56 33.3 / 27.5, 64 -> 64 12.4 / 11.5, 128 -> 32
-// 13.4 / 14.2, 512 -> 64 at 28x28 23.4 / 23.4; 3x3 3 -> 64 at 224x224 (27 rows) 129 / 137, batch 16 5 -> 64 (45 rows)
-// 68.4 / 60.1, 1x1 48 -> 256 at 56x56 29.4 / 25.0.  So both could be drawn lower.
+// Whether a tile of this configuration runs on the bf16 matrix cores with its filter packed in parts (a pointwise layer is a block whose only
+// tap is inside): for inputs below 2 GiB, but not for pointwise layers of up to 64 output channels, whose x the fp32 kernel reads 16 bytes a
+// lane, nor for reductions of two or three stages; their filter is packed in fp32, and those of many pixels are split from it in the kernel
+// (ig_point_few, ig_short).  For the others of them, best tile on fp32 / on a filter in parts, batch 32, us: 1x1 128 -> 32 at 56x56 13.4 / 14.2,
+// 512 -> 64 at 28x28 23.4 / 23.4, 64 -> 64 at 56x56 12.4 / 11.5.
 bool ig_splits(const fc_conv_shape &s, const fc_gemm_config &c) {
     if (c.waves_k > 1 || c.bm % 64 != 0 || 4l * s.N * s.C * s.H * s.W >= (1l << 31) || (long)s.C * s.kh * s.kw <= 48) return false;
     if (ig_pointwise(s, c.bk, true) && s.K <= 64) return false;

@@ -257,10 +257,13 @@ struct SplitTile {
     typedef fc_split_stage<TL::BM_, TL::BN_> Stage;
     static constexpr int LDS_WORDS = 2 * Stage::WORDS;
     // Register sets of global prefetch: set u holds the stages s with s % PF == u, and a stage is fetched PF stages before it
-    // is split.  Where a stage is eight registers a second set leaves the wavefronts a SIMD holds as they are (128x128: 122
-    // registers of 128).  One / two / three / four sets, whole staged layer, us: 256 -> 256 channels at 56x56 batch 32 275 / 263 /
-    // 295 / 284, 128 -> 128 at 112x112 400 / 383 / 410 / 404, 512 -> 512 at 28x28 232 / 227 / 242 / 237, at 14x14 batch 4 42.5 /
-    // 40.3 / 40.5 / 40.2; one image 256 -> 256 at 56x56 30.1 / 28.7 / 29.2 / 29.8.  The wider tiles hold 24 registers a stage and keep one.
+    // is split.  128x128 tiles hold a second set in as many wavefronts a SIMD, four, with 122 registers of 128; 64x64 tiles go from 72 to 90
+    // registers and from six wavefronts, which is what LDS holds, to five.  One / two / three / four sets, whole staged layer, us: 256 -> 256
+    // channels at 56x56 batch 32 275 / 263 / 295 / 284, 128 -> 128 at 112x112 400 / 383 / 410 / 404, 512 -> 512 at 28x28 232 / 227 / 242 / 237,
+    // at 14x14 batch 4 42.5 / 40.3 / 40.5 / 40.2; one image 256 -> 256 at 56x56 30.1 / 28.7 / 29.2 / 29.8.  64x64 tiles with one set in six
+    // wavefronts / two in five / two in six (80 registers): 512 -> 512 at 14x14 batch 32 118.4 / 117.5 / 117.0, batch 16 81.9 / 82.2 / 81.0, batch 4
+    // 45.2 / 41.7 / 43.0, 96 -> 160 at 48x48 batch 2 17.6 / 16.8 / 17.1, 11 layers 0.980 / 1 / 1.000 of the speed.  The wider tiles hold 24
+    // registers a stage and keep one.
     static constexpr int PF = ITEMS == 1 ? 2 : 1;
     static_assert(TL::BM_ % 64 == 0 && TL::BN_ % 64 == 0, "a wavefront fetches 64 rows or columns of one operand");
     static_assert(2 * (TL::BM_ + TL::BN_) % TL::THREADS == 0, "every wavefront fetches the same number of blocks");
