@@ -1239,7 +1239,9 @@ void launch(fc_context *ctx, const fc_conv_shape &s, const fc_gemm_config &cfg, 
 // images, strided or 100 stages and more.  The others keep as many parts as fill the chip (ig_parts_to_fill): 1x1 layers as the
 // expected times do not tell their tiles apart so well (512 -> 2048 at 7x7 batch 32 28 / 33 us), window rows in runs and blocks with
 // channels missing as they are ahead and behind about as often (28 -> 38 at 9x45 batch 52 14.9 / 18.6, 548 -> 175 at 21x113 batch 10 235 /
-// 245, 168 -> 631 at 8x8 batch 18 36.9 / 31.9).
+// 245, 168 -> 631 at 8x8 batch 18 36.9 / 31.9).  Neither several images nor 100 stages is where it ceases to pay: 24 layers of one image take 0.93 of the
+// time by it, 24 of several at stride 1 with fewer stages 0.96 (0.80 to 1.08 each; 192 -> 360 5x5/2 at 100x115 85 / 69, 128 -> 672 3x3 at 10x8 batch
+// 51 67 / 55, 16 -> 384 at 33x33 batch 16 17.9 / 19.4), so that the line could be drawn lower.
 bool ig_parts_by_time(const fc_conv_shape &s) {
     const long taps = (long)s.kh * s.kw;
     return taps > 1 && s.N > 1 && s.C % 16 == 0 && (s.sh > 1 || s.sw > 1 || s.C / 16 * taps >= 100);
